@@ -411,4 +411,151 @@ GH_HD inline double sinc_ratio(double x)
     return fma(p, x2, 1.0);
 }
 
+// One Horner step of M polynomials with the same coefficients: the scalar
+// pair of a coefficient is set once for all M.
+template <int M>
+GH_HD inline void horner(double (&p)[M], const double (&z)[M], double coef)
+{
+    const double k = kc(coef);
+    for (int m = 0; m < M; m++) p[m] = fma(p[m], z[m], k);
+}
+
+// sin and cos of M arguments up to one common sign: x = k pi + r, |r| <=
+// pi/2, s = sin r, c = cos r, and flip has bit 31 set where k is odd, so
+// that (sin x, cos x) = flip_sign(s, flip), flip_sign(c, flip).  A caller
+// that multiplies both by an amplitude applies the sign to that once: no
+// quadrant swap, 30 instructions an argument against sincos_red's 45.
+// k comes from the low bits of x / pi + 1.5 * 2^52.  pi in two parts: k < 2^28
+// leaves a third part's share below 1e-24.  Minimax polynomials in r^2 (own
+// Remez fits, coefficients rounded in turn: sin 2.4e-19 and cos 4.4e-18
+// absolute).  Domain |x| < 2^29; outside it (and for NaN) the results are NaN.
+template <int M>
+GH_HD inline void sincos_half(const double (&x)[M], double (&s)[M], double (&c)[M], unsigned (&flip)[M])
+{
+    const double INV_PI = 0.31830988618379067154;
+    const double C1 = 3.141592653589793116;        // pi rounded
+    const double C2 = 1.2246467991473531772e-16;   // pi - C1
+    const double SHIFT = 6755399441055744.0;       // 1.5 * 2^52
+    double r[M], z[M], ps[M], pc[M];
+    for (int m = 0; m < M; m++)
+    {
+        const double t = fma(x[m], INV_PI, SHIFT);
+        const double k = t - SHIFT;
+        unsigned long long b;
+        __builtin_memcpy(&b, &t, sizeof b);
+        flip[m] = (unsigned)b << 31;
+        r[m] = fma(-k, C1, x[m]);
+        r[m] = fma(-k, C2, r[m]);
+        if (!(fabs(x[m]) < 536870912.0)) r[m] = __builtin_nan("");
+        z[m] = r[m] * r[m];
+        ps[m] = 2.7205053073271883e-15;
+        pc[m] = 4.6104367203077217e-14;
+    }
+    horner(ps, z, -7.6429275697811245e-13);
+    horner(pc, z, -1.1463055248591474e-11);
+    horner(ps, z, 1.6058937286791798e-10);
+    horner(pc, z, 2.0876568461140048e-09);
+    horner(ps, z, -2.5052106827316448e-08);
+    horner(pc, z, -2.7557316542332734e-07);
+    horner(ps, z, 2.7557319210711158e-06);
+    horner(pc, z, 2.4801587279376377e-05);
+    horner(ps, z, -0.00019841269841207673);
+    horner(pc, z, -0.0013888888888787317);
+    horner(ps, z, 0.0083333333333331962);
+    horner(pc, z, 0.04166666666666443);
+    horner(ps, z, -0.16666666666666666);
+    horner(pc, z, -0.49999999999999983);
+    for (int m = 0; m < M; m++)
+    {
+        s[m] = fma(r[m] * z[m], ps[m], r[m]);
+        c[m] = fma(pc[m], z[m], 1.0);
+    }
+}
+
+// sin(x)/x (s), cos x (c) and, if D, the derivative of sin(x)/x (d) of M
+// arguments: minimax polynomials in x^2 on |x| <= 1.75 (own Remez fits: s
+// 2e-18, c 9e-20, d 2e-18 absolute).  wide (the same for the whole workgroup:
+// a template above ~27 mHz, sinc_wide): larger arguments may be among them;
+// they enter the polynomials less a multiple of pi.  Otherwise no lane takes
+// another path.
+template <bool D, int M>
+GH_HD inline void sinc_values(const double (&x)[M], bool wide, double (&s)[M], double (&c)[M], double (&d)[M])
+{
+    double z[M], r[M], k[M];
+    for (int m = 0; m < M; m++)
+    {
+        r[m] = x[m];
+        k[m] = 0.0;
+    }
+    if (wide)
+        for (int m = 0; m < M; m++)
+        {
+            k[m] = rint(x[m] * 0.31830988618379067154);
+            r[m] = fma(-k[m], 1.2246467991473531772e-16, fma(-k[m], 3.141592653589793116, x[m]));
+        }
+    for (int m = 0; m < M; m++)
+    {
+        z[m] = r[m] * r[m];
+        s[m] = 2.6980953427936517e-15;
+        c[m] = -1.5026701985826183e-16;
+        d[m] = -1.3377466686687439e-16;
+    }
+    horner(c, z, 4.7758396494203246e-14);
+    horner(s, z, -7.6405781270510619e-13);
+    if (D) horner(d, z, 4.4836650306213241e-14);
+    horner(c, z, -1.1470623327874561e-11);
+    horner(s, z, 1.6058837462977408e-10);
+    if (D) horner(d, z, -1.0705308753469852e-11);
+    horner(c, z, 2.0876754553270967e-09);
+    horner(s, z, -2.5052104628865737e-08);
+    if (D) horner(d, z, 1.9270833004095398e-09);
+    horner(c, z, -2.7557319194947931e-07);
+    horner(s, z, 2.755731918410767e-06);
+    if (D) horner(d, z, -2.5052108076159289e-07);
+    horner(c, z, 2.4801587301388157e-05);
+    horner(s, z, -0.0001984126984103551);
+    if (D) horner(d, z, 2.2045855376394339e-05);
+    horner(c, z, -0.0013888888888888189);
+    horner(s, z, 0.0083333333333326671);
+    if (D) horner(d, z, -0.0011904761904748447);
+    horner(c, z, 0.041666666666666657);
+    horner(s, z, -0.1666666666666666);
+    if (D) horner(d, z, 0.033333333333333041);
+    if (D) horner(d, z, -0.33333333333333331);
+    for (int m = 0; m < M; m++)
+    {
+        s[m] = fma(s[m], z[m], 1.0);
+        c[m] = fma(fma(c[m], z[m], -0.5), z[m], 1.0);
+        if (D) d[m] *= r[m];
+    }
+    if (wide)
+        for (int m = 0; m < M; m++)
+            if (k[m] != 0.0)
+            {
+                const double e = 1.0 - 2.0 * fabs(k[m] - 2.0 * rint(0.5 * k[m]));  // (-1)^k
+                const double i = 1.0 / x[m];
+                s[m] = e * (r[m] * s[m]) * i;
+                c[m] = e * c[m];
+                if (D) d[m] = (c[m] - s[m]) * i;
+            }
+}
+
+// sin(x)/x exp(-i x), the transfer function of a link: fr + i fi = s c - i x s s.
+template <int M>
+GH_HD inline void sinc_phase(const double (&x)[M], bool wide, double (&fr)[M], double (&fi)[M])
+{
+    double s[M], c[M], d[M];
+    sinc_values<false>(x, wide, s, c, d);
+    for (int m = 0; m < M; m++)
+    {
+        fr[m] = s[m] * c[m];
+        fi[m] = -(x[m] * s[m]) * s[m];
+    }
+}
+
+// Whether the transfer-function arguments of a template may leave |x| <=
+// 1.75, from its largest |f|/f*: they reach (1 + k.r/L)/2 times it, up to
+// 1.25 with the arm half as long again as L.
+GH_HD inline bool sinc_wide(double fmax) { return !(1.25 * fmax <= 1.75); }
+
 }  // namespace glass

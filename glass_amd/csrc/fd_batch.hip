@@ -40,6 +40,24 @@ constexpr int kMaxSrcDefault = 8;   // source slots per chain of glass_hip_fd_ba
 constexpr int kMaxSrcLimit = 64;    // largest max_src of glass_hip_fd_batch_create_ex
 constexpr int kNClass = 8;     // BW = 32 << k, k = 0..7 (32..4096)
 constexpr int kPosN = 4096;    // positions table samples (largest BW)
+constexpr int kAlignOne = 256; // items of one align_kernel workgroup
+
+// Where an item's template meets its chain: written once per item by
+// align_kernel, read by scalar loads where the class kernels need it.  A class
+// kernel that followed item -> chain -> window -> offsets itself waited for
+// five dependent loads before its first sample, and held every pointer in
+// scalar registers (spilled to vector lanes) until its last bin.
+struct EvalRec
+{
+    double2* tmpl;      // the source's stored template, 3 rows of cap
+    double2* R;         // the chain's residual, 3 rows of W
+    const double* iC;   // the window's invC, 6 rows of W
+    double logl;        // the chain's logL
+    int W, cap;
+    int imin;           // first window bin of the new template
+    int imin_o, bw_o;   // ... and of the stored one, with its bins
+    int cls;            // BW class; kNClass: none holds it, -1: left out
+};
 
 struct BatchDev
 {
@@ -67,6 +85,7 @@ struct BatchDev
     int bwcap;                // largest g_cap
     int maxsrc;               // source slots per chain in sparams / s_bw / s_imin
     UcbConst* pc;             // per-item template constants, written by align_kernel
+    struct EvalRec* rec;      // per-item places, written by align_kernel
     // constants
     double T, t0, L, fstar;
     const double* pos;      // positions table, kPosN samples
@@ -75,12 +94,38 @@ struct BatchDev
     int fmt;
 };
 
-// Positions for fd_link_bins at N bins: the structure-of-arrays block of N
-// for the split shape (coalesced coordinate loads), else the record table.
-template <int N, int NTHR>
-__device__ __forceinline__ const double* batch_pos(const BatchDev& B)
+// What the class kernels read: kernel arguments, few enough to stay in
+// scalar registers.
+struct EvalArgs
 {
-    return fd_split(N, NTHR) ? B.pos_soa + pos_soa_offset(N) : B.pos;
+    const UcbConst* pc;
+    const EvalRec* rec;
+    const double* pos;  // the class's structure-of-arrays positions (coalesced loads)
+    const double2* tw;
+    double2* stg;       // optional staging of the templates (Items)
+    double* logl;
+    double* snr;
+    int bwcap, fmt;
+};
+
+// A scalar load of memory no kernel in flight writes; p uniform.
+__device__ __forceinline__ int scalar_load(const int* p)
+{
+    return *(const __attribute__((address_space(4))) int*)p;
+}
+
+// One item's EvalRec by scalar loads (LoadedConst's way).
+__device__ __forceinline__ EvalRec load_rec(const EvalRec* p)
+{
+    static_assert(sizeof(EvalRec) % 8 == 0, "read as 64-bit words");
+    auto g = (const __attribute__((address_space(4))) unsigned long long*)uniform_ptr(p);
+    asm volatile("" : "+s"(g));
+    unsigned long long w[sizeof(EvalRec) / 8];
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(EvalRec) / 8); i++) w[i] = g[i];
+    EvalRec r;
+    __builtin_memcpy(&r, w, sizeof r);
+    return r;
 }
 
 // Work items: item e refers to entry q = sel ? sel[e] : e of the
@@ -120,12 +165,13 @@ __global__ void zero_int_kernel(int* p, int n)
 // bucketing by BW class.  Class slots are reserved per block (an LDS
 // histogram, then one global atomic per class per block) so the class
 // counters are not hammered by every item.  Items whose BW falls outside
-// the classes are counted in *err and left out.
-__global__ __launch_bounds__(256) void align_kernel(int n, Items it, BatchDev B, int* __restrict__ bw_out,
-                                                    int* __restrict__ imin_out, int* __restrict__ cls_count,
-                                                    int* __restrict__ cls_list, int cls_stride, int* __restrict__ err,
-                                                    double* __restrict__ logl_out = nullptr,
-                                                    double* __restrict__ snr_out = nullptr)
+// the classes are counted in *err (cls_count[kNClass]) and left out.  One
+// workgroup alone writes the counts; more add to counts cleared before.
+__global__ __launch_bounds__(kAlignOne) void align_kernel(int n, Items it, BatchDev B, int* __restrict__ bw_out,
+                                                          int* __restrict__ imin_out, int* __restrict__ cls_count,
+                                                          int* __restrict__ cls_list, int cls_stride,
+                                                          double* __restrict__ logl_out,
+                                                          double* __restrict__ snr_out)
 {
     __shared__ int hist[kNClass + 1], base[kNClass + 1];
     if (threadIdx.x <= kNClass) hist[threadIdx.x] = 0;
@@ -147,8 +193,19 @@ __global__ __launch_bounds__(256) void align_kernel(int n, Items it, BatchDev B,
         int qmin = (int)(f0 * B.T) - BW / 2;
         bw_out[e] = BW;
         imin_out[e] = qmin - B.g_qmin[g];
-        // the template constants of the class kernels, once per item
+        // the template constants and places of the class kernels, once per item
         ucb_setup(p, 8, B.T, B.t0, B.L, B.fstar, B.pc[e]);
+        const int s = item_src(it, e), so = c * B.maxsrc + s;
+        EvalRec r;
+        r.tmpl = src_tmpl(B, c, s);
+        r.R = B.resid + (size_t)B.c_roff[c] * 3;
+        r.iC = B.invC + (size_t)B.g_off[g] * 6;
+        r.logl = B.logl[c];
+        r.W = W;
+        r.cap = B.g_cap[g];
+        r.imin = qmin - B.g_qmin[g];
+        r.imin_o = B.s_imin[so];
+        r.bw_o = B.s_bw[so];
         k = 31 - __clz(BW) - 5;  // log2(BW) - 5
         if (BW > B.g_cap[g] || k < 0 || k >= kNClass || (BW & (BW - 1)))
         {
@@ -158,11 +215,22 @@ __global__ __launch_bounds__(256) void align_kernel(int n, Items it, BatchDev B,
             if (logl_out) logl_out[e] = -INFINITY;
             if (snr_out) snr_out[e] = 0.0;
         }
+        r.cls = k;
+        B.rec[e] = r;
         slot = atomicAdd(&hist[k], 1);
     }
+    else if (e < n)
+        B.rec[e].cls = -1;
     __syncthreads();
-    if (threadIdx.x < kNClass && hist[threadIdx.x]) base[threadIdx.x] = atomicAdd(&cls_count[threadIdx.x], hist[threadIdx.x]);
-    if (threadIdx.x == kNClass && hist[kNClass]) atomicAdd(err, hist[kNClass]);
+    if (threadIdx.x <= kNClass)
+    {
+        const int h = hist[threadIdx.x];
+        base[threadIdx.x] = 0;
+        if (gridDim.x == 1)
+            cls_count[threadIdx.x] = h;
+        else if (h)
+            base[threadIdx.x] = atomicAdd(&cls_count[threadIdx.x], h);
+    }
     __syncthreads();
     if (k >= 0 && k < kNClass) cls_list[k * cls_stride + base[k] + slot] = e;
 }
@@ -172,6 +240,15 @@ __global__ __launch_bounds__(256) void align_kernel(int n, Items it, BatchDev B,
 // and the body has no loop, so nothing is hoisted across templates and the
 // register footprint stays that of one template), or a grid sized to a
 // multiple of the resident capacity striding over the class list.
+
+// half of bform(u, u, w): the cross terms once
+__device__ inline double qform(const double2* u, const double* w)
+{
+    auto re = [](double2 a, double2 b) { return a.x * b.x + a.y * b.y; };
+    const double d = w[0] * re(u[0], u[0]) + w[1] * re(u[1], u[1]) + w[2] * re(u[2], u[2]);
+    const double o = w[3] * re(u[0], u[1]) + w[4] * re(u[0], u[2]) + w[5] * re(u[1], u[2]);
+    return d + 2.0 * o;
+}
 
 // symmetric 3x3 weighted bilinear form of complex 3-vectors:
 // 2 * sum_ab Re(u_a conj v_b) w_ab, w planes XX,YY,ZZ,XY,XZ,YZ
@@ -187,112 +264,112 @@ __device__ inline double bform(const double2* u, const double2* v, const double*
 __device__ inline void load_w(const double* __restrict__ iC, int W, int j, double* w)
 {
 #pragma unroll
-    for (int q = 0; q < 6; q++) w[q] = iC[(size_t)q * W + j];
+    for (int q = 0; q < 6; q++) w[q] = gload(iC + (size_t)q * W + j);
 }
 
-// Fused waveform + delta-logL + snr of class-list entry w.
-template <int N, int NTHR>
-__device__ __forceinline__ void eval_item(int w, double2* lds, const int* __restrict__ list, Items it,
-                                          BatchDev B, const int* __restrict__ p_imin,
-                                          double* __restrict__ logl_out, double* __restrict__ snr_out)
+// Fused waveform + delta-logL + snr of item e.
+template <int N>
+__device__ __forceinline__ void eval_item(int e, double2* lds, const EvalArgs& A)
 {
-    {
-        const int e = list[w];
-        const int c = item_chain(it, e), s = item_src(it, e);
-        const int g = B.c_group[c];
-        const int W = B.g_W[g];
-        // the constants straight into scalar registers (uniform loads):
-        // no LDS copy and no barriers around it, and the slow series reads
-        // them as scalar operands (3% faster at 512 bins than through LDS)
-        UcbConst kc = B.pc[e];
-        make_uniform(kc);
-        const UcbConst& k = kc;
-
-        const int so = c * B.maxsrc + s;
-        const int imin_n = p_imin[e];
-        const int imin_o = B.s_imin[so], bw_o = B.s_bw[so];
-        const int cap = B.g_cap[g];
-        const double2* ho = src_tmpl(B, c, s);
-        const double2* R = B.resid + (size_t)B.c_roff[c] * 3;
-        const double* iC = B.invC + (size_t)B.g_off[g] * 6;
-        double acc = 0.0, s2 = 0.0;
-        // the old template's values at bin m, loaded before the bin's
-        // transform (their latency, an HBM read per source, overlaps the FFT)
-        double2 hpre[3];
-        auto pre = [&](int m) {
-            const int j = imin_n + m, mo = j - imin_o;
-            const bool inold = j >= 0 && j < W && mo >= 0 && mo < bw_o;
+    constexpr int NTHR = fd_threads(N);
+    // the constants and places by scalar loads where they are used: no LDS
+    // copy and no barriers around it, and the slow series reads them as
+    // scalar operands
+    const LoadedConst k{A.pc + e};
+    const EvalRec* rec = A.rec + e;
+    // the record's cache line is fetched beside the constants'; held whole
+    // from here it would push vector values out of 79 registers
+    const int warm = scalar_load(&rec->W);
+    double acc = 0.0, s2 = 0.0;
+    // the old template's values at bin m, loaded before the bin's transform
+    // (their latency, an HBM read per source, overlaps the FFT) where no
+    // other series wait in registers meanwhile, else with the bin
+    constexpr bool EARLY = fd_series(N) == 1;
+    double2 hpre[3];
+    auto old_bin = [&](const EvalRec& r, int m) {
+        const int j = r.imin + m, mo = j - r.imin_o;
+        const bool inold = j >= 0 && j < r.W && mo >= 0 && mo < r.bw_o;
 #pragma unroll
-            for (int ch = 0; ch < 3; ch++) hpre[ch] = inold ? ho[ch * cap + mo] : make_double2(0.0, 0.0);
-        };
-        // new-template bins (and the old template where they overlap)
-        // no tail barrier: the reduction's barrier below separates this
-        // item's last LDS reads from the next item's writes
-        fd_link_bins<N, NTHR, fd_split(N, NTHR), fd_split(N, NTHR), false>(
-            k, lds, opaque(batch_pos<N, NTHR>(B)), kPosN / N, opaque(B.tw), kTwN / N, pre,
-            [&](int m, const double2* dl) {
-                double2 v[5];
-                fd_tdi<N>(k, m, B.fmt, dl, v);
-                if (it.stg)
+        for (int ch = 0; ch < 3; ch++) hpre[ch] = inold ? gload(r.tmpl + ch * r.cap + mo) : make_double2(0.0, 0.0);
+    };
+    auto pre = [&](int m) {
+        asm volatile("" ::"s"(warm));
+        if constexpr (EARLY) old_bin(load_rec(rec), m);
+    };
+    // new-template bins (and the old template where they overlap)
+    // no tail barrier: the reduction's barrier below separates this
+    // item's last LDS reads from the next item's writes
+    fd_link_bins<N, true>(
+        k, lds, opaque(A.pos), 0, opaque(A.tw), kTwN / N, pre, [&](int, int m, const double2* dl) {
+            double2 v[5];
+            fd_tdi<N>(k(), m, A.fmt, dl, v);
+            if (A.stg)
 #pragma unroll
-                    for (int ch = 0; ch < 3; ch++) it.stg[(size_t)e * 3 * B.bwcap + ch * N + m] = v[ch];
-                double wq[6];
-                load_w(iC, W, m, wq);  // snr: template bin m against window bin m
-                s2 += bform(v, v, wq);
-                const int j = imin_n + m;
-                if (j >= 0 && j < W)
-                {
-                    double2 d[3], r[3];
-#pragma unroll
-                    for (int ch = 0; ch < 3; ch++)
-                    {
-                        const double2 h0 = hpre[ch];  // zero outside the old template
-                        d[ch] = make_double2(v[ch].x - h0.x, v[ch].y - h0.y);
-                        r[ch] = R[(size_t)ch * W + j];
-                    }
-                    load_w(iC, W, j, wq);
-                    acc += bform(r, d, wq) - 0.5 * bform(d, d, wq);
-                }
-            });
-        // old-template bins outside the new support: dh = -h_old
-        for (int mo = threadIdx.x; mo < bw_o; mo += NTHR)
-        {
-            const int j = imin_o + mo;
-            if (j < 0 || j >= W || (j >= imin_n && j < imin_n + N)) continue;
-            double2 d[3], r[3];
+                for (int ch = 0; ch < 3; ch++) A.stg[(size_t)e * 3 * A.bwcap + ch * N + m] = v[ch];
+            const EvalRec r = load_rec(rec);
+            if constexpr (!EARLY) old_bin(r, m);
             double wq[6];
-#pragma unroll
-            for (int ch = 0; ch < 3; ch++)
+            load_w(r.iC, r.W, m, wq);  // snr: template bin m against window bin m
+            s2 += qform(v, wq);
+            const int j = r.imin + m;
+            if (j >= 0 && j < r.W)
             {
-                double2 h0 = ho[ch * cap + mo];
-                d[ch] = make_double2(-h0.x, -h0.y);
-                r[ch] = R[(size_t)ch * W + j];
+                double2 d[3], x[3];
+#pragma unroll
+                for (int ch = 0; ch < 3; ch++)
+                {
+                    const double2 h0 = hpre[ch];  // zero outside the old template
+                    d[ch] = make_double2(v[ch].x - h0.x, v[ch].y - h0.y);
+                    // (r|d) - (d|d)/2 = (r - d/2|d)
+                    x[ch] = gload(r.R + (size_t)ch * r.W + j);
+                    x[ch].x = fma(-0.5, d[ch].x, x[ch].x);
+                    x[ch].y = fma(-0.5, d[ch].y, x[ch].y);
+                }
+                load_w(r.iC, r.W, j, wq);
+                acc += bform(x, d, wq);
             }
-            load_w(iC, W, j, wq);
-            acc += bform(r, d, wq) - 0.5 * bform(d, d, wq);
-        }
-        // both sums over the workgroup behind one barrier (block_sum's
-        // order: wave sums, then the waves' partials in turn); thread 0
-        // writes the logL, thread 1 the snr.  The partials are next written
-        // by the following item's reduction, many barriers later.
-        constexpr int NW = (NTHR < 64 ? 64 : NTHR) / 64;
-        __shared__ double part[NW][2];
-        const double wa = wave_sum(acc), ws = wave_sum(s2);
-        if ((threadIdx.x & 63) == 0)
+        });
+    // old-template bins outside the new support: dh = -h_old
+    const EvalRec r = load_rec(rec);
+    for (int mo = threadIdx.x; mo < r.bw_o; mo += NTHR)
+    {
+        const int j = r.imin_o + mo;
+        if (j < 0 || j >= r.W || (j >= r.imin && j < r.imin + N)) continue;
+        double2 d[3], x[3];
+        double wq[6];
+#pragma unroll
+        for (int ch = 0; ch < 3; ch++)
         {
-            part[threadIdx.x >> 6][0] = wa;
-            part[threadIdx.x >> 6][1] = ws;
+            const double2 h0 = gload(r.tmpl + ch * r.cap + mo);
+            d[ch] = make_double2(-h0.x, -h0.y);
+            x[ch] = gload(r.R + (size_t)ch * r.W + j);
+            x[ch].x = fma(0.5, h0.x, x[ch].x);
+            x[ch].y = fma(0.5, h0.y, x[ch].y);
         }
-        __syncthreads();
-        if (threadIdx.x < 2)
-        {
-            double r = 0.0;
-            for (int i = 0; i < NW; i++) r += part[i][threadIdx.x];
-            if (threadIdx.x == 0)
-                logl_out[e] = B.logl[c] + r;
-            else
-                snr_out[e] = sqrt(r);
-        }
+        load_w(r.iC, r.W, j, wq);
+        acc += bform(x, d, wq);
+    }
+    // both sums over the workgroup behind one barrier (block_sum's
+    // order: wave sums, then the waves' partials in turn); thread 0
+    // writes the logL, thread 1 the snr.  The partials are next written
+    // by the following item's reduction, many barriers later.
+    constexpr int NW = NTHR / 64;
+    __shared__ double part[NW][2];
+    const double wa = wave_sum(acc), ws = wave_sum(s2);
+    if ((threadIdx.x & 63) == 0)
+    {
+        part[threadIdx.x >> 6][0] = wa;
+        part[threadIdx.x >> 6][1] = ws;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2)
+    {
+        double q = 0.0;
+        for (int i = 0; i < NW; i++) q += part[i][threadIdx.x];
+        if (threadIdx.x == 0)
+            A.logl[e] = r.logl + q;
+        else
+            A.snr[e] = sqrt(2.0 * q);
     }
 }
 
@@ -303,76 +380,95 @@ __device__ __forceinline__ void eval_item(int w, double2* lds, const int* __rest
 // MINW: waves per SIMD the register allocation must allow (1: the
 // compiler's choice; more trades register spills for resident waves).
 template <int N, int NTHR, bool LOOP, int MINW>
-__global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(MINW, 8))) void eval_kernel(const int* __restrict__ list, const int* __restrict__ count,
-                                                    Items it, BatchDev B, const int* __restrict__ p_imin,
-                                                    double* __restrict__ logl_out, double* __restrict__ snr_out)
+__global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(MINW, 8))) void eval_kernel(
+    const int* __restrict__ list, const int* __restrict__ count, EvalArgs A)
 {
-    __shared__ double2 lds[FdShape<N, NTHR, fd_split(N, NTHR)>::LDS];
-    const int cnt = *count;
+    __shared__ double2 lds[FdShape<N>::LDS];
+    const int cnt = scalar_load(count);
     if constexpr (LOOP)
     {
-        for (int w = blockIdx.x; w < cnt; w += gridDim.x)
-            eval_item<N, NTHR>(w, lds, list, it, B, p_imin, logl_out, snr_out);
+        for (int w = blockIdx.x; w < cnt; w += gridDim.x) eval_item<N>(scalar_load(list + w), lds, A);
     }
     else
     {
-        if (blockIdx.x < cnt) eval_item<N, NTHR>(blockIdx.x, lds, list, it, B, p_imin, logl_out, snr_out);
+        if ((int)blockIdx.x < cnt) eval_item<N>(scalar_load(list + blockIdx.x), lds, A);
     }
 }
 
 // Compiled launch shapes of the class kernels (tile candidates), default
 // first: (class k, template bins N, workgroup threads, waves per SIMD).
-// From 128 to 1024 bins the default is the split shape (N/2 threads, two
-// bins each, half the LDS of one sample per thread): at 126 VGPRs it keeps
-// 4 waves per SIMD, so BW 1024 fits two workgroups per CU instead of one and
-// BW 512 four 256-thread workgroups instead of three.  The N-thread shapes
-// (one sample per thread, ~94 VGPRs) and their 5- and 6-wave variants
-// (spilling some registers for more waves in flight across the FFT
-// barriers) remain candidates.  The decimated classes (N >= 2048) keep
-// their accumulators in registers only at 512 (and 1024 for N = 2048)
-// threads.
+#ifndef GH_EVAL_TILES
 #define GH_EVAL_TILES(X)                                                                                      \
-    X(0, 32, 64, 1) X(1, 64, 64, 1) X(1, 64, 64, 6) X(2, 128, 64, 1) X(2, 128, 128, 1) X(2, 128, 128, 6)     \
-    X(3, 256, 128, 1) X(3, 256, 128, 4) X(3, 256, 256, 1) X(3, 256, 256, 5) X(3, 256, 256, 6)                \
-    X(4, 512, 256, 1) X(4, 512, 512, 1) X(4, 512, 512, 6) X(5, 1024, 512, 4) X(5, 1024, 512, 1)              \
-    X(5, 1024, 1024, 1) X(5, 1024, 256, 1)                                                                   \
-    X(6, 2048, 512, 1) X(6, 2048, 1024, 1) X(7, 4096, 512, 1)
+    X(0, 32, 64, 1) X(1, 64, 64, 1) X(1, 64, 64, 6) X(2, 128, 128, 1) X(2, 128, 128, 6) X(3, 256, 256, 1)    \
+    X(3, 256, 256, 6) X(3, 256, 256, 8) X(4, 512, 512, 6) X(4, 512, 512, 1) X(4, 512, 512, 8)                \
+    X(5, 1024, 512, 4) X(5, 1024, 512, 5) X(6, 2048, 1024, 1) X(7, 4096, 1024, 1)
+#endif
 
 // Template of each listed item into its source's slot.  LOOP: the grid
 // strides over the class list (large rebuilds, where one workgroup per
-// item would mostly launch workgroups that exit at once).
-template <int N, int NTHR>
-__device__ __forceinline__ void tmpl_item(int w, double2* lds, const int* __restrict__ list, Items it, BatchDev B)
+// item would mostly launch workgroups that exit at once).  use(rec, m, v):
+// called with each bin m's X, Y, Z.
+template <int N, typename Use>
+__device__ __forceinline__ void tmpl_item(int e, double2* lds, const EvalArgs& A, Use&& use)
 {
-    const int e = list[w];
-    UcbConst kc = B.pc[e];  // into scalar registers, as in eval_item
-    make_uniform(kc);
-    const UcbConst& k = kc;
-    const int c = item_chain(it, e), cap = chain_cap(B, c);
-    double2* o = src_tmpl(B, c, item_src(it, e));
-    fd_link_bins<N, NTHR, fd_split(N, NTHR), fd_split(N, NTHR)>(k, lds, opaque(batch_pos<N, NTHR>(B)), kPosN / N,
-                                                                opaque(B.tw), kTwN / N,
-                                             [&](int m, const double2* dl) {
-                                                 double2 v[5];
-                                                 fd_tdi<N>(k, m, B.fmt, dl, v);
+    const LoadedConst k{A.pc + e};
+    const EvalRec* rec = A.rec + e;
+    fd_link_bins<N, true>(
+        k, lds, opaque(A.pos), 0, opaque(A.tw), kTwN / N, [](int) {}, [&](int, int m, const double2* dl) {
+            double2 v[5];
+            fd_tdi<N>(k(), m, A.fmt, dl, v);
+            const EvalRec r = load_rec(rec);
 #pragma unroll
-                                                 for (int ch = 0; ch < 3; ch++) o[ch * cap + m] = v[ch];
-                                             });
+            for (int ch = 0; ch < 3; ch++) gstore(r.tmpl + ch * r.cap + m, v[ch]);
+            use(r, m, v);
+        });
 }
+constexpr auto kNoUse = [](const EvalRec&, int, const double2*) {};
 
-template <int N, int NTHR, bool LOOP>
-__global__ __launch_bounds__(NTHR) void tmpl_kernel(const int* __restrict__ list, const int* __restrict__ count,
-                                                    Items it, BatchDev B)
+template <int N, bool LOOP>
+__global__ __launch_bounds__(fd_threads(N)) void tmpl_kernel(const int* __restrict__ list, const int* __restrict__ count,
+                                                    EvalArgs A)
 {
-    __shared__ double2 lds[FdShape<N, NTHR, fd_split(N, NTHR)>::LDS];
-    const int cnt = *count;
+    __shared__ double2 lds[FdShape<N>::LDS];
+    const int cnt = scalar_load(count);
     if constexpr (LOOP)
     {
-        for (int w = blockIdx.x; w < cnt; w += gridDim.x) tmpl_item<N, NTHR>(w, lds, list, it, B);
+        for (int w = blockIdx.x; w < cnt; w += gridDim.x)
+        {
+            tmpl_item<N>(scalar_load(list + w), lds, A, kNoUse);
+            __syncthreads();  // its last LDS reads before the next item's writes
+        }
     }
     else
     {
-        if ((int)blockIdx.x < cnt) tmpl_item<N, NTHR>(blockIdx.x, lds, list, it, B);
+        if ((int)blockIdx.x < cnt) tmpl_item<N>(scalar_load(list + blockIdx.x), lds, A, kNoUse);
+    }
+}
+
+// residual += h_old over the stored template's support
+__device__ __forceinline__ void accept_add_old(double2* R, int W, const double2* ho, int cap, int io, int bo)
+{
+    for (int j = max(0, io) + threadIdx.x; j < min(W, io + bo); j += blockDim.x)
+        for (int ch = 0; ch < 3; ch++)
+        {
+            double2 v = R[(size_t)ch * W + j];
+            v.x += ho[ch * cap + j - io].x;
+            v.y += ho[ch * cap + j - io].y;
+            R[(size_t)ch * W + j] = v;
+        }
+}
+
+// The source of accepted item a takes its parameters and alignment.
+__device__ __forceinline__ void accept_source(const Items& it, int a, const BatchDev& B, int bw, int imin,
+                                              const double* __restrict__ logl_new)
+{
+    const int c = item_chain(it, a), so = c * B.maxsrc + item_src(it, a);
+    if (threadIdx.x < 8) B.sparams[(size_t)so * 8 + threadIdx.x] = item_params(it, a)[threadIdx.x];
+    if (threadIdx.x == 0)
+    {
+        B.s_bw[so] = bw;
+        B.s_imin[so] = imin;
+        B.logl[c] = logl_new[item_q(it, a)];
     }
 }
 
@@ -434,17 +530,7 @@ __global__ __launch_bounds__(256) void accept_add_old_kernel(int nacc, Items it,
     if (a >= nacc || (it.dn && a >= *it.dn)) return;
     const int c = item_chain(it, a), s = item_src(it, a), so = c * B.maxsrc + s;
     const int g = B.c_group[c], W = B.g_W[g], cap = B.g_cap[g];
-    const int io = B.s_imin[so], bo = B.s_bw[so];
-    double2* R = B.resid + (size_t)B.c_roff[c] * 3;
-    const double2* ho = src_tmpl(B, c, s);
-    for (int j = max(0, io) + threadIdx.x; j < min(W, io + bo); j += blockDim.x)
-        for (int ch = 0; ch < 3; ch++)
-        {
-            double2 v = R[(size_t)ch * W + j];
-            v.x += ho[ch * cap + j - io].x;
-            v.y += ho[ch * cap + j - io].y;
-            R[(size_t)ch * W + j] = v;
-        }
+    accept_add_old(B.resid + (size_t)B.c_roff[c] * 3, W, src_tmpl(B, c, s), cap, B.s_imin[so], B.s_bw[so]);
 }
 
 __global__ __launch_bounds__(256) void accept_sub_new_kernel(int nacc, Items it, BatchDev B,
@@ -454,7 +540,7 @@ __global__ __launch_bounds__(256) void accept_sub_new_kernel(int nacc, Items it,
 {
     const int a = blockIdx.x;
     if (a >= nacc || (it.dn && a >= *it.dn)) return;
-    const int c = item_chain(it, a), s = item_src(it, a), so = c * B.maxsrc + s;
+    const int c = item_chain(it, a), s = item_src(it, a);
     const int g = B.c_group[c], W = B.g_W[g], cap = B.g_cap[g];
     const int in = imin_new[a], bn = bw_new[a];
     double2* R = B.resid + (size_t)B.c_roff[c] * 3;
@@ -467,13 +553,7 @@ __global__ __launch_bounds__(256) void accept_sub_new_kernel(int nacc, Items it,
             v.y -= hn[ch * cap + j - in].y;
             R[(size_t)ch * W + j] = v;
         }
-    if (threadIdx.x < 8) B.sparams[(size_t)so * 8 + threadIdx.x] = item_params(it, a)[threadIdx.x];
-    if (threadIdx.x == 0)
-    {
-        B.s_bw[so] = bn;
-        B.s_imin[so] = in;
-        B.logl[c] = logl_new[item_q(it, a)];
-    }
+    accept_source(it, a, B, bn, in, logl_new);
 }
 
 }  // namespace glass
@@ -599,16 +679,12 @@ static int dalloc(glass_hip_fd_batch* P, T** p, size_t n)
     return GLASS_HIP_OK;
 }
 
-#define GH_NTHR_(N) (::glass::fd_batch_threads(N))
-#define GH_NTHR(N) GH_NTHR_(N)
-
 // Workgroups of a class kernel resident per CU, as bounded by LDS (160 KB)
 // and by the waves per SIMD the register allocation allows (4 by default,
 // `waves` when forced higher).
 static int resident_per_cu(int N, int nthr, int waves)
 {
-    const int ns = fd_split(N, nthr) ? N / 2 : (N <= 1024 ? N : GH_DECIM_NS);
-    const int lds = (int)sizeof(double2) * 6 * ns + 512;
+    const int lds = (int)sizeof(double2) * kNLink * wave_fft_stride(N < 512 ? N : 512) + 512;
     int per = (160 * 1024) / lds;
     const int wv = 4 * (waves > 4 ? waves : 4) / ((nthr + 63) / 64);
     if (wv < per) per = wv;
@@ -616,9 +692,11 @@ static int resident_per_cu(int N, int nthr, int waves)
 }
 
 // Waves per SIMD of the default tiles (the first candidate of each class):
-// 4 at 1024 bins, where the compiler's choice lands a few VGPRs above the
-// 128 that four waves allow.
-constexpr int batch_default_waves(int N) { return N == 1024 ? 4 : 1; }
+// 6 at 512 bins, where the compiler's choice of 81 vector registers is one
+// above what three workgroups per CU allow (130,042 evaluations 2.60 -> 2.28
+// ms), and 4 at 1024, two workgroups per CU (41,400 in 1.77 ms, 2.47 before
+// the series were cut to 512 points; with 5 the spills make it 2.36).
+constexpr int batch_default_waves(int N) { return N == 512 ? 6 : (N == 1024 ? 4 : 1); }
 
 static int setup_grids(glass_hip_fd_batch* P)
 {
@@ -626,14 +704,14 @@ static int setup_grids(glass_hip_fd_batch* P)
     for (int k = 0; k < kNClass; k++)
     {
         const int N = 32 << k;
-        P->tgrid[k] = P->ncu * resident_per_cu(N, fd_batch_threads(N), batch_default_waves(N));
-        P->tile[k] = glass_hip_tile{fd_batch_threads(N), 0, batch_default_waves(N)};
+        P->tgrid[k] = P->ncu * resident_per_cu(N, fd_threads(N), batch_default_waves(N));
+        P->tile[k] = glass_hip_tile{fd_threads(N), 0, batch_default_waves(N)};
     }
     return GLASS_HIP_OK;
 }
 
 // Grid multipliers of the tile candidates: 0 = one workgroup per proposal
-// slot, m > 0 = m x (resident workgroups per CU) x CUs, striding.
+// slot (striding 4 x the resident ones where eval_strides), m > 0 = m x (resident workgroups per CU) x CUs, striding.
 constexpr int kGmul[] = {0, 1, 2, 4};
 constexpr int kNGmul = sizeof(kGmul) / sizeof(kGmul[0]);
 
@@ -646,11 +724,39 @@ static bool tile_compiled(int k, int nthr, int waves)
     return false;
 }
 
+// Shapes of class k that earlier builds compiled (other thread counts of the
+// same kernels): a caller's saved choice of one runs as the default shape
+// with its grid multiplier.
+static bool tile_retired(int k, int nthr, int waves)
+{
+    static constexpr int shape[][3] = {{2, 64, 1},  {3, 128, 1},  {3, 128, 4}, {3, 256, 5}, {4, 256, 1},
+                                       {5, 512, 1}, {5, 1024, 1}, {5, 256, 1}, {6, 512, 1}, {7, 512, 1}};
+    for (const auto& x : shape)
+        if (x[0] == k && x[1] == nthr && x[2] == waves) return true;
+    return false;
+}
+
+// Classes whose default grid strides.  The grid cannot know how many of the n
+// proposals are in a class; a slot that is not costs the launch of an empty
+// workgroup, 0.2 ns of 64 threads and 0.7 ns of 1024 (0.07 and 0.22 ms of
+// 327,680), while striding costs the 128- to 1024-bin kernels 6 to 10% an
+// item (the loop holds 30 more vector registers).  Striding against one
+// workgroup per slot, of 327,680: 74 of 32 bins 0.013 / 0.081 ms, 20,188 of
+// 64 bins 0.050 / 0.111, 23,671 of 2048 bins 2.85 / 3.13, 379 of 4096 bins
+// 0.24 / 0.46; but 130,042 of 512 bins 2.59 / 2.35.
+constexpr bool eval_strides(int k) { return k < 2 || k > 5; }
+
 static int tile_grid(const glass_hip_fd_batch* P, int k, glass_hip_tile t, int n)
 {
-    if (t.gmul <= 0) return n;
-    const long long g = (long long)t.gmul * P->ncu * resident_per_cu(32 << k, t.nthr, t.waves);
+    if (t.gmul <= 0 && !eval_strides(k)) return n;
+    const long long g = (long long)(t.gmul > 0 ? t.gmul : 4) * P->ncu * resident_per_cu(32 << k, t.nthr, t.waves);
     return (int)(g < n ? g : n);
+}
+
+static EvalArgs eval_args(const glass_hip_fd_batch* P, int N, const Items& it, double* logl_out, double* snr_out)
+{
+    const BatchDev& B = P->B;
+    return EvalArgs{B.pc, B.rec, B.pos_soa + pos_soa_offset(N), B.tw, it.stg, logl_out, snr_out, B.bwcap, B.fmt};
 }
 
 // The class-k eval kernel under tile t over the n proposal slots.
@@ -661,16 +767,26 @@ static int launch_eval(glass_hip_fd_batch* P, int k, glass_hip_tile t, int n, co
 #define GH_X(kk, N, T, MW)                                                                                       \
     if (k == kk && t.nthr == T && t.waves == MW)                                                                 \
     {                                                                                                            \
-        if (t.gmul > 0)                                                                                          \
-            eval_kernel<N, T, true, MW><<<g, T, 0, s>>>(list, cnt, it, P->B, P->p_imin, logl_out, snr_out);      \
+        const EvalArgs A = eval_args(P, N, it, logl_out, snr_out);                                               \
+        if (t.gmul > 0 || eval_strides(k))                                                                       \
+            eval_kernel<N, T, true, MW><<<g, T, 0, s>>>(list, cnt, A);                                           \
         else                                                                                                     \
-            eval_kernel<N, T, false, MW><<<g, T, 0, s>>>(list, cnt, it, P->B, P->p_imin, logl_out, snr_out);     \
+            eval_kernel<N, T, eval_strides(kk), MW><<<g, T, 0, s>>>(list, cnt, A);                               \
         return GLASS_HIP_OK;                                                                                     \
     }
     GH_EVAL_TILES(GH_X)
 #undef GH_X
     set_error("batch: no compiled tile for class %d with %d threads, %d waves", k, t.nthr, t.waves);
     return GLASS_HIP_EINVAL;
+}
+
+// alignment and class lists of the items
+static void launch_align(glass_hip_fd_batch* P, int n, const Items& it, double* logl_out, double* snr_out,
+                         hipStream_t s)
+{
+    if (n > kAlignOne) zero_int_kernel<<<1, 64, 0, s>>>(P->cls, kNClass + 1);
+    align_kernel<<<(n + kAlignOne - 1) / kAlignOne, kAlignOne, 0, s>>>(n, it, P->B, P->p_bw, P->p_imin, P->cls,
+                                                                       P->cls_list, P->cls_cap, logl_out, snr_out);
 }
 
 // alignment + per-class launches for items; mode 0: eval, 1: templates
@@ -683,10 +799,7 @@ static int launch_items(glass_hip_fd_batch* P, int n, const Items& it, int mode,
         set_error("batch: %d items exceed capacity %d", n, P->cls_cap);
         return GLASS_HIP_EINVAL;
     }
-    zero_int_kernel<<<1, 64, 0, s>>>(P->cls, kNClass + 1);
-    align_kernel<<<(n + 255) / 256, 256, 0, s>>>(n, it, P->B, P->p_bw, P->p_imin, P->cls, P->cls_list, P->cls_cap,
-                                                 P->cls + kNClass, mode == 0 ? logl_out : nullptr,
-                                                 mode == 0 ? snr_out : nullptr);
+    launch_align(P, n, it, mode == 0 ? logl_out : nullptr, mode == 0 ? snr_out : nullptr, s);
     // the per-class timings of the profiling mode need the classes in turn
     const bool par = P->concurrent && !(P->prof && mode == 0);
     if (par)
@@ -721,9 +834,11 @@ static int launch_items(glass_hip_fd_batch* P, int n, const Items& it, int mode,
 #define GH_L(kk, N)                                                                               \
     case kk:                                                                                      \
         if (loop)                                                                                 \
-            tmpl_kernel<N, GH_NTHR(N), true><<<g, GH_NTHR(N), 0, sk>>>(list, cnt, it, P->B);      \
+            tmpl_kernel<N, true><<<g, fd_threads(N), 0, sk>>>(                                    \
+                list, cnt, eval_args(P, N, it, nullptr, nullptr));                                \
         else                                                                                      \
-            tmpl_kernel<N, GH_NTHR(N), false><<<g, GH_NTHR(N), 0, sk>>>(list, cnt, it, P->B);     \
+            tmpl_kernel<N, false><<<g, fd_threads(N), 0, sk>>>(                                   \
+                list, cnt, eval_args(P, N, it, nullptr, nullptr));                                \
         break;
             switch (k)
             {
@@ -928,7 +1043,7 @@ extern "C" int glass_hip_fd_batch_create_ex(glass_hip_fd_batch** plan, const gla
         (rc = dalloc(P, &P->p_logl, P->cls_cap)) || (rc = dalloc(P, &P->p_snr, P->cls_cap)) ||
         (rc = dalloc(P, &P->p_bw, P->cls_cap)) || (rc = dalloc(P, &P->p_imin, P->cls_cap)) ||
         (rc = dalloc(P, &P->cls, kNClass + 1)) || (rc = dalloc(P, &P->cls_list, (size_t)kNClass * P->cls_cap)) ||
-        (rc = dalloc(P, &P->B.pc, P->cls_cap)) ||
+        (rc = dalloc(P, &P->B.pc, P->cls_cap)) || (rc = dalloc(P, &P->B.rec, P->cls_cap)) ||
         (rc = dalloc(P, &P->i_chain, P->ninit)) || (rc = dalloc(P, &P->i_src, P->ninit)) ||
         (rc = dalloc(P, &P->i_slot, P->ninit)) || (rc = dalloc(P, &P->i_params, (size_t)P->ninit * 8)) ||
         (rc = dalloc(P, &P->D.pidx, P->cls_cap)) || (rc = dalloc(P, &P->D.imin, P->cls_cap)) ||
@@ -1107,7 +1222,6 @@ extern "C" int glass_hip_fd_batch_accept(glass_hip_fd_batch* P, int nacc, const 
     hipStream_t s = (hipStream_t)stream;
     Items it{d_chain, d_src, d_params, d_idx};
     int rc;
-    // new templates into the scratch slots 0..nacc (item a -> slot a)
     accept_add_old_kernel<<<nacc, 256, 0, s>>>(nacc, it, P->B);
     if ((rc = launch_items(P, nacc, it, 1, nullptr, nullptr, s))) return rc;
     accept_sub_new_kernel<<<nacc, 256, 0, s>>>(nacc, it, P->B, P->p_bw, P->p_imin, d_logL);
@@ -1357,16 +1471,22 @@ extern "C" int glass_hip_fd_batch_set_tiles(glass_hip_fd_batch* P, const glass_h
         set_error("fd_batch_set_tiles: bad arguments");
         return GLASS_HIP_EINVAL;
     }
+    glass_hip_tile use[kNClass];
     for (int k = 0; k < kNClass; k++)
-        if (!tile_compiled(k, tiles[k].nthr, tiles[k].waves) || tiles[k].gmul < 0 || tiles[k].gmul > 64)
+    {
+        use[k] = tiles[k];
+        if (tile_retired(k, use[k].nthr, use[k].waves))
+            use[k] = glass_hip_tile{fd_threads(32 << k), tiles[k].gmul, batch_default_waves(32 << k)};
+        if (!tile_compiled(k, use[k].nthr, use[k].waves) || use[k].gmul < 0 || use[k].gmul > 64)
         {
             set_error("fd_batch_set_tiles: class %d (BW %d): no compiled tile with %d threads, %d waves, grid x%d",
                       k, 32 << k, tiles[k].nthr, tiles[k].waves, tiles[k].gmul);
             return GLASS_HIP_EINVAL;
         }
+    }
     GH_CHECK(hipSetDevice(P->device));
     if (int rc = drop_graph(P)) return rc;
-    for (int k = 0; k < kNClass; k++) P->tile[k] = tiles[k];
+    for (int k = 0; k < kNClass; k++) P->tile[k] = use[k];
     return GLASS_HIP_OK;
 }
 
@@ -1383,9 +1503,7 @@ extern "C" int glass_hip_fd_batch_autotune(glass_hip_fd_batch* P, int nprop, con
     hipStream_t s = (hipStream_t)stream;
     Items it{d_chain, d_src, d_params, nullptr};
     // class lists of these proposals, as an eval builds them
-    zero_int_kernel<<<1, 64, 0, s>>>(P->cls, kNClass + 1);
-    align_kernel<<<(nprop + 255) / 256, 256, 0, s>>>(nprop, it, P->B, P->p_bw, P->p_imin, P->cls, P->cls_list,
-                                                     P->cls_cap, P->cls + kNClass);
+    launch_align(P, nprop, it, nullptr, nullptr, s);
     GH_CHECK(hipGetLastError());
     int cnt[kNClass + 1];
     GH_CHECK(hipMemcpyAsync(cnt, P->cls, sizeof(cnt), hipMemcpyDeviceToHost, s));

@@ -50,9 +50,8 @@ int launch_derivs(int N, const DerivArgs& A, int grid, hipStream_t s);
 // The BW 2048 and 4096 kernels: grid workgroups striding over A.list (or
 // over items 0..A.nitems-1 without a list), workgroup w with a scratch
 // slice of deriv_scratch(N) complex at hs + w slice.
-constexpr int kDeriv2048Threads = 512;
 constexpr size_t kDeriv2048Scratch = 18 * 2048;
-constexpr size_t kDeriv4096Scratch = 24 * 4096;
+constexpr size_t kDeriv4096Scratch = 18 * 4096;
 constexpr size_t deriv_scratch(int N) { return N == 2048 ? kDeriv2048Scratch : (N == 4096 ? kDeriv4096Scratch : 0); }
 int launch_derivs_2048(const DerivArgs& A, int grid, double2* hs, hipStream_t s);
 int launch_derivs_4096(const DerivArgs& A, int grid, double2* hs, hipStream_t s);

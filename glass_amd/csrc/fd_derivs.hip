@@ -8,12 +8,14 @@
 //   dL/dtheta_k = (R - h | dh/dtheta_k),   Gamma_kl = (dh_k | dh_l),
 // with ( | ) the 3-channel noise-weighted product of gaussian_log_likelihood
 // (utils/src/glass_model.c:758-767).  One workgroup per source: the six
-// series sets of fd_tangent.h go through LDS in as few passes as 96 KB
-// allows, each pass FFT'd and TDI'd into per-bin registers; then every
-// thread accumulates L, the 8 gradient entries and the 36 distinct Fisher
-// entries of its bins and the workgroup reduces the 45 sums.
+// series sets of fd_tangent.h go through LDS and FFT in passes of a few sets,
+// each TDI'd into per-bin values u_q; every thread then adds its bins'
+// Hermitian Gram G_qr = u_q^H W u_r (36 real numbers) and projections
+// P_q = (W (R - h))^H u_q (12), and the workgroup reduces the 48 sums.  All
+// eight dh/dtheta are fixed complex combinations of the six u_q, so L, the
+// gradient and the Fisher matrix follow from them: 420 multiply-adds a bin
+// where the 45 real products of the dh/dtheta took 1250.
 #include <cmath>
-#include <type_traits>
 
 #include "../../include/glass_hip_batch.h"
 #include "fd_derivs.h"
@@ -25,215 +27,100 @@ namespace glass {
 
 int parse_format(const char* format);
 
-constexpr int kNSum = 45;  // L, grad[8], Fisher upper triangle[36]
+// Sums of one source: G_qq (6), Re and Im of G_qr for q < r (15 pairs), Re
+// and Im of P_q (6 pairs), and in mode 1 h^H W h with the likelihood's weights.
+constexpr int kNSum = 49, kNMain = 48, kGOff = 6, kPOff = 36;
+__host__ __device__ constexpr int gram_index(int q, int r) { return kGOff + 2 * (q * 5 - q * (q - 1) / 2 + r - q - 1); }
 
-// B(u,v) = 2 sum_ab Re(u_a conj v_b) w_ab with w = XX,YY,ZZ,XY,XZ,YZ
-__device__ inline double bf3(const double2* u, const double2* v, const double* w)
-{
-    auto re = [](double2 a, double2 b) { return a.x * b.x + a.y * b.y; };
-    return 2.0 * (w[0] * re(u[0], v[0]) + w[1] * re(u[1], v[1]) + w[2] * re(u[2], v[2]) +
-                  w[3] * (re(u[0], v[1]) + re(u[1], v[0])) + w[4] * (re(u[0], v[2]) + re(u[2], v[0])) +
-                  w[5] * (re(u[1], v[2]) + re(u[2], v[1])));
-}
+// Series sets per pass.  Three up to 512 bins (two passes; 138 KB of LDS at
+// 512, two workgroups per CU at 256): each pass evaluates the sample's
+// common part again.  One above, where a thread holds P results of every
+// series through its samples.
+constexpr int deriv_sets(int N) { return N <= 512 ? 3 : 1; }
 
-template <int NTHR>
-__device__ inline void block_sum_vec(double (&v)[kNSum], double* out)
+// One pass: series sets [S0, S0+NS) of the slow samples -> LDS -> FFT ->
+// TDI: out(r, set, X, Y, Z) for the thread's bins m = P t + r.
+template <int N, int S0, int NS, typename Out>
+__device__ __forceinline__ void deriv_pass(const UcbConst& c, const UcbDiff& dd, double2* lds, const DerivArgs& A,
+                                           Out&& out)
 {
-    constexpr int NW = (NTHR + 63) / 64;
-    __shared__ double part[NW][kNSum];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    // the 45 wave sums by transposition: lane k ends with value k's sum
-    constexpr int GROUP = 64 / pow2_at_least(kNSum);  // lanes holding one sum
-    const double x = wave_sum_transpose<kNSum>(v);
-    const int k = lane / GROUP;
-    if (k < kNSum && lane % GROUP == 0) part[w][k] = x;
-    __syncthreads();
-    if (threadIdx.x < kNSum)
+    using S = FdShape<N, 1>;
+    constexpr int P = S::P, NT = S::NT, PN = S::PN, L = NS * kNLink;
+    const int t = threadIdx.x;
+    const bool on = NT >= 64 || t < NT;
+    const int ts = wave_fft_slot(t);
+    const double2* tw = opaque(A.tw);
+    const double* pos = opaque(A.pos);
+    double2 x[P][L];
+    if constexpr (P == 1)
     {
-        double s = 0.0;
-        for (int i = 0; i < NW; i++) s += part[i][threadIdx.x];
-        out[threadIdx.x] = s;
+        if (on)
+            ucb_sample_sets_to<S0, NS>(c, dd, ucb_sample_time(c.T, c.t0, t, N), pos + (size_t)t * (4096 / N) * 9,
+                                       [&](int q, int l, double2 v) { lds[((q - S0) * kNLink + l) * PN + ts] = v; });
     }
-    __syncthreads();
-}
-
-// LDS bytes for the series sets of one pass: sets per pass = this / 96 N
-// (at least one).  48 KB up to 256 bins (two or more workgroups per CU at
-// ~250 VGPRs), 96 KB above (one workgroup per CU either way, fewer passes).
-constexpr int deriv_lds_budget(int N) { return N <= 256 ? 49152 : 98304; }
-
-// One pass of series sets [S0, S0+NS): samples -> LDS -> FFT -> TDI into H.
-template <int N, int NTHR, int S0, int NS>
-__device__ inline void deriv_pass(const UcbConst& c, const UcbDiff& dd, double2* lds, const DerivArgs& A,
-                                  double2 (&H)[FdShape<N, NTHR>::PER][6][3])
-{
-    using S = FdShape<N, NTHR>;
-    for (int j = threadIdx.x; j < N; j += NTHR)
+    else
     {
-        const double t = ucb_sample_time(c.T, c.t0, j, N);
-        ucb_sample_sets<S0, NS>(c, dd, t, A.pos + (size_t)j * (4096 / N) * 9, lds, N, j);
-    }
-    __syncthreads();
-    lds_fft<N, 6 * NS, NTHR>(lds, A.tw, kTwN / N);
-    const double inv2N = 1. / (double)(2 * N);
 #pragma unroll
-    for (int k = 0; k < S::PER; k++)
-    {
-        const int m = threadIdx.x + k * NTHR;
-        if (m >= N) continue;
-        const int s = (m + N / 2) & (N - 1);
+        for (int p = 0; p < P; p++)
 #pragma unroll
-        for (int q = 0; q < NS; q++)
+            for (int l = 0; l < L; l++) x[p][l] = make_double2(0.0, 0.0);
+#pragma unroll 1
+        for (int p = 0; p < P; p++)
         {
-            double2 d6[6], o5[5];
+            const int n = t + NT * p;
+            ucb_sample_sets_to<S0, NS>(c, dd, ucb_sample_time(c.T, c.t0, n, N), pos + (size_t)n * (4096 / N) * 9,
+                                       [&](int q, int l, double2 v) {
+                                           const int k = (q - S0) * kNLink + l;
 #pragma unroll
-            for (int l = 0; l < 6; l++)
-            {
-                double2 v = lds[(q * 6 + l) * N + s];
-                d6[l] = make_double2(v.x * inv2N, v.y * inv2N);
-            }
-            fd_tdi<N>(c, m, A.fmt, d6, o5);
-#pragma unroll
-            for (int ch = 0; ch < 3; ch++) H[k][S0 + q][ch] = o5[ch];
+                                           for (int j = 0; j + 1 < P; j++) x[j][k] = x[j + 1][k];
+                                           x[P - 1][k] = v;
+                                       });
         }
+        fd_dif<N, L>(x, tw, kTwN / N, t);
+#pragma unroll
+        for (int l = 0; l < L; l++) lds[l * PN + ts] = x[0][l];
     }
     __syncthreads();
-}
-
-// Passes over the sets below S1, the highest first: the tangent sets (2-5,
-// the costly samples) run while few TDI values of earlier passes are held in
-// registers, the basis sets (0, 1) last.
-template <int N, int NTHR, int S1>
-__device__ inline void deriv_passes(const UcbConst& c, const UcbDiff& dd, double2* lds, const DerivArgs& A,
-                                    double2 (&H)[FdShape<N, NTHR>::PER][6][3])
-{
-    constexpr int CAP = (deriv_lds_budget(N) / (96 * N)) < 1 ? 1 : (deriv_lds_budget(N) / (96 * N));
-    constexpr int NS = S1 < CAP ? S1 : CAP;
-    deriv_pass<N, NTHR, S1 - NS, NS>(c, dd, lds, A, H);
-    if constexpr (S1 - NS > 0) deriv_passes<N, NTHR, S1 - NS>(c, dd, lds, A, H);
-}
-
-// Waves per SIMD the register allocation must allow (the launch bound's
-// second argument; 1 = the compiler's choice).  Only 256 bins can use more:
-// their 50 KB of LDS fits three workgroups per CU, the larger and smaller
-// sizes are held to two waves per SIMD by LDS.  Three waves cap the kernel
-// at 168 VGPRs (from 195, with 144 B of spill) and run the 256-bin Fisher
-// batch about 2% faster.
-#ifndef GH_DERIV_W256
-#define GH_DERIV_W256 3
-#endif
-constexpr int deriv_min_waves(int N) { return N == 256 ? GH_DERIV_W256 : 1; }
-
-template <int N, int NTHR>
-__global__ __launch_bounds__(NTHR, deriv_min_waves(N)) void deriv_kernel(DerivArgs A)
-{
-    using S = FdShape<N, NTHR>;
-    constexpr int CAP = (deriv_lds_budget(N) / (96 * N)) < 1 ? 1 : (deriv_lds_budget(N) / (96 * N));
-    constexpr int NSMAX = CAP < 6 ? CAP : 6;
-    __shared__ double2 lds[6 * NSMAX * N];
-    __shared__ UcbDiff sdd;
-    __shared__ double red[kNSum];
-    int e = blockIdx.x;
-    if (A.list)
+    const int k = wave_fft_slot((t + NT / 2) & (NT - 1));
+#pragma unroll
+    for (int r = 0; r < P; r++)
     {
-        if (e >= *A.count) return;  // uniform over the workgroup
-        e = A.list[e];
-    }
-    const double* p = A.params + (size_t)(A.pidx ? A.pidx[e] : e) * 8;
-    // the template constants and their derivatives set up at once on two
-    // waves (one workgroup per source: nothing of a previous source to wait for)
-    __shared__ UcbConst sc;
-    if (threadIdx.x == 0) ucb_setup(p, 8, A.T, A.t0, A.L, A.fstar, sc);
-    if (threadIdx.x == (NTHR >= 128 ? 64 : 0)) ucb_diff_setup(p, A.T, sdd);
-    __syncthreads();
-    // the constants into scalar registers for the passes (2% faster than
-    // reading them from LDS; the derivative constants stay in LDS, where
-    // the scalar copies would spill)
-    UcbConst cr = sc;
-    make_uniform(cr);
-    const UcbConst& c = cr;
-    const UcbDiff& dd = sdd;
-    double2 H[S::PER][6][3];
-    deriv_passes<N, NTHR, 6>(c, dd, lds, A, H);
-
-    const double2* R = A.iroff ? A.resid + A.iroff[e] : A.resid + (size_t)e * (A.rstride / 2);
-    const double* iC = A.iioff ? A.invC + A.iioff[e] : A.invC + (size_t)e * A.istride;
-    const int W = A.iW ? A.iW[e] : A.W, imin = A.imin[e];
-    const double2* Ha = A.tadd ? A.tadd + A.taddoff[e] : nullptr;
-    const int hcap = A.tadd ? A.taddcap[e] : 0;
-    const double2 DP = make_double2(c.DPr, c.DPi), DC = make_double2(c.DCr, c.DCi);
-    const double2 DP4 = make_double2(dd.DPr4, dd.DPi4), DC4 = make_double2(dd.DCr4, dd.DCi4);
-    const double2 DP5 = make_double2(dd.DPr5, dd.DPi5), DC5 = make_double2(dd.DCr5, dd.DCi5);
-    double acc[kNSum];
+        wave_fft<NT, L, S::NTHR>(lds, opaque(A.tw), P * (kTwN / N));
+        double2 d[L];
+        if (on)
 #pragma unroll
-    for (int k = 0; k < kNSum; k++) acc[k] = 0.0;
+            for (int l = 0; l < L; l++) d[l] = lds[l * PN + k];
+        __syncthreads();
+        if (r + 1 < P)
 #pragma unroll
-    for (int k = 0; k < S::PER; k++)
-    {
-        const int m = threadIdx.x + k * NTHR;
-        if (m >= N) continue;
-        const int j = imin + m;
-        const int wi = A.mode == 1 ? m : j;  // weight index
-        if (wi < 0 || wi >= W) continue;
-        double w[6];
-#pragma unroll
-        for (int q = 0; q < 6; q++) w[q] = iC[(size_t)q * W + wi];
-        double2 h[3], dh[8][3], r[3];
-#pragma unroll
-        for (int ch = 0; ch < 3; ch++)
+            for (int l = 0; l < L; l++) lds[l * PN + ts] = x[r + 1][l];
+        if (on)
         {
-            const double2 hp = H[k][0][ch], hc = H[k][1][ch];
-            h[ch] = make_double2(cmulc(DP, hp).x + cmulc(DC, hc).x, cmulc(DP, hp).y + cmulc(DC, hc).y);
-            dh[0][ch] = H[k][2][ch];
-            dh[1][ch] = H[k][3][ch];
-            dh[2][ch] = H[k][4][ch];
-            dh[3][ch] = h[ch];                                  // d/d ln A
-            dh[4][ch] = make_double2(cmulc(DP4, hp).x + cmulc(DC4, hc).x, cmulc(DP4, hp).y + cmulc(DC4, hc).y);
-            dh[5][ch] = make_double2(cmulc(DP5, hp).x + cmulc(DC5, hc).x, cmulc(DP5, hp).y + cmulc(DC5, hc).y);
-            dh[6][ch] = make_double2(h[ch].y, -h[ch].x);        // d/d phi0 = -i h
-            dh[7][ch] = H[k][5][ch];
-            const bool inwin = j >= 0 && j < W;
-            r[ch] = (A.resid && inwin) ? R[(size_t)ch * W + j] : make_double2(0.0, 0.0);
-            if (Ha && inwin)
+            const int m = P * t + r;
+            double s1, c1;
+            fd_tdi_phase<N>(c, m, c1, s1);
+            const double2 pf = fd_tdi_prefactor<N>(c, m, A.fmt, c1, s1);
+#pragma unroll
+            for (int q = 0; q < NS; q++)
             {
-                // the residual of the whole model plus this source's stored
-                // template: the residual without the source
-                r[ch].x += Ha[(size_t)ch * hcap + m].x;
-                r[ch].y += Ha[(size_t)ch * hcap + m].y;
+                double2 X, Y, Z;
+                fd_tdi_xyz(c1, s1, pf, d + q * kNLink, X, Y, Z);
+                out(r, S0 + q, X, Y, Z);
             }
         }
-        // likelihood terms only where the template lands in the window
-        if (A.mode == 0 || (j >= 0 && j < W))
-        {
-            double wj[6];
-            if (A.mode == 1)
-            {
-                for (int q = 0; q < 6; q++) wj[q] = (j >= 0 && j < W) ? iC[(size_t)q * W + j] : 0.0;
-            }
-            const double* ww = A.mode == 1 ? wj : w;
-            acc[0] += bf3(r, h, ww) - 0.5 * bf3(h, h, ww);
-            double2 rh[3];
-#pragma unroll
-            for (int ch = 0; ch < 3; ch++) rh[ch] = make_double2(r[ch].x - h[ch].x, r[ch].y - h[ch].y);
-#pragma unroll
-            for (int a = 0; a < 8; a++) acc[1 + a] += bf3(rh, dh[a], ww);
-        }
-        int idx = 9;
-#pragma unroll
-        for (int a = 0; a < 8; a++)
-#pragma unroll
-            for (int b = a; b < 8; b++) acc[idx++] += bf3(dh[a], dh[b], w);
+        if (r + 1 < P) __syncthreads();
     }
-    block_sum_vec<NTHR>(acc, red);
-    if (threadIdx.x < 64)
-    {
-        const int a = threadIdx.x / 8, b = threadIdx.x % 8;
-        const int lo = a < b ? a : b, hi = a < b ? b : a;
-        const int idx = 9 + lo * 8 - lo * (lo - 1) / 2 + (hi - lo);
-        A.fisher[(size_t)e * 64 + threadIdx.x] = red[idx];
-        if (threadIdx.x < 8) A.grad[(size_t)e * 8 + threadIdx.x] = red[1 + threadIdx.x];
-        if (threadIdx.x == 0) A.outL[e] = red[0];
-    }
+}
+
+// All passes, the highest sets first: the tangent sets (2-5, the costly
+// samples) run while few TDI values of earlier passes are held in registers.
+template <int N, int S1, typename Out>
+__device__ __forceinline__ void deriv_passes(const UcbConst& c, const UcbDiff& dd, double2* lds, const DerivArgs& A,
+                                             Out&& out)
+{
+    constexpr int NS = S1 < deriv_sets(N) ? S1 : deriv_sets(N);
+    deriv_pass<N, S1 - NS, NS>(c, dd, lds, A, out);
+    if constexpr (S1 - NS > 0) deriv_passes<N, S1 - NS>(c, dd, lds, A, out);
 }
 
 // The window and residual of item e.
@@ -257,195 +144,284 @@ __device__ __forceinline__ DerivItem deriv_item(const DerivArgs& A, int e)
     return it;
 }
 
-// Adds template bin m's terms to the 45 sums from its six series-set TDI
-// values Hb[set][channel]: h and the eight dh/dtheta (sets 0,1 the plus /
-// cross basis, 2..5 the tangent sets), L, the gradient and the Fisher
-// upper triangle.
-__device__ __forceinline__ void deriv_bin(const UcbConst& c, const UcbDiff& dd, const DerivArgs& A, const DerivItem& it, int m,
-                                 const double2 (&Hb)[6][3], double (&acc)[kNSum])
+// y = W u for the symmetric weights w = XX, YY, ZZ, XY, XZ, YZ
+__device__ __forceinline__ void wmul(const double* w, const double2* u, double2* y)
 {
-    const int W = it.W;
-    const int j = it.imin + m;
-    const int wi = A.mode == 1 ? m : j;  // weight index
+    y[0] = make_double2(w[0] * u[0].x + w[3] * u[1].x + w[4] * u[2].x, w[0] * u[0].y + w[3] * u[1].y + w[4] * u[2].y);
+    y[1] = make_double2(w[3] * u[0].x + w[1] * u[1].x + w[5] * u[2].x, w[3] * u[0].y + w[1] * u[1].y + w[5] * u[2].y);
+    y[2] = make_double2(w[4] * u[0].x + w[5] * u[1].x + w[2] * u[2].x, w[4] * u[0].y + w[5] * u[1].y + w[2] * u[2].y);
+}
+
+// Adds template bin m's terms to the sums from its six sets' TDI values u.
+__device__ __forceinline__ void deriv_bin(const UcbConst& c, const DerivArgs& A, const DerivItem& it, int m,
+                                          const double2 (&u)[6][3], double (&acc)[kNSum])
+{
+    const int W = it.W, j = it.imin + m;
+    const int wi = A.mode == 1 ? m : j;  // Fisher weight index
+    const bool inwin = j >= 0 && j < W;
     if (wi < 0 || wi >= W) return;
-    const double2 DP = make_double2(c.DPr, c.DPi), DC = make_double2(c.DCr, c.DCi);
-    const double2 DP4 = make_double2(dd.DPr4, dd.DPi4), DC4 = make_double2(dd.DCr4, dd.DCi4);
-    const double2 DP5 = make_double2(dd.DPr5, dd.DPi5), DC5 = make_double2(dd.DCr5, dd.DCi5);
     double w[6];
 #pragma unroll
     for (int q = 0; q < 6; q++) w[q] = it.iC[(size_t)q * W + wi];
-    double2 h[3], dh[8][3], r[3];
+    if (inwin)
+    {
+        // likelihood terms only where the template lands in the window
+        double2 h[3], x[3], z[3];
 #pragma unroll
-    for (int ch = 0; ch < 3; ch++)
-    {
-        const double2 hp = Hb[0][ch], hc = Hb[1][ch];
-        h[ch] = make_double2(cmulc(DP, hp).x + cmulc(DC, hc).x, cmulc(DP, hp).y + cmulc(DC, hc).y);
-        dh[0][ch] = Hb[2][ch];
-        dh[1][ch] = Hb[3][ch];
-        dh[2][ch] = Hb[4][ch];
-        dh[3][ch] = h[ch];                                  // d/d ln A
-        dh[4][ch] = make_double2(cmulc(DP4, hp).x + cmulc(DC4, hc).x, cmulc(DP4, hp).y + cmulc(DC4, hc).y);
-        dh[5][ch] = make_double2(cmulc(DP5, hp).x + cmulc(DC5, hc).x, cmulc(DP5, hp).y + cmulc(DC5, hc).y);
-        dh[6][ch] = make_double2(h[ch].y, -h[ch].x);        // d/d phi0 = -i h
-        dh[7][ch] = Hb[5][ch];
-        const bool inwin = j >= 0 && j < W;
-        r[ch] = (A.resid && inwin) ? it.R[(size_t)ch * W + j] : make_double2(0.0, 0.0);
-        if (it.Ha && inwin)
+        for (int ch = 0; ch < 3; ch++)
         {
-            // the residual of the whole model plus this source's stored
-            // template: the residual without the source
-            r[ch].x += it.Ha[(size_t)ch * it.hcap + m].x;
-            r[ch].y += it.Ha[(size_t)ch * it.hcap + m].y;
+            const double2 a = u[0][ch], b = u[1][ch];
+            h[ch] = make_double2(c.DPr * a.x - c.DPi * a.y + c.DCr * b.x - c.DCi * b.y,
+                                 c.DPr * a.y + c.DPi * a.x + c.DCr * b.y + c.DCi * b.x);
+            double2 r = A.resid ? it.R[(size_t)ch * W + j] : make_double2(0.0, 0.0);
+            if (it.Ha)
+            {
+                // the residual of the whole model plus this source's stored
+                // template: the residual without the source
+                r.x += it.Ha[(size_t)ch * it.hcap + m].x;
+                r.y += it.Ha[(size_t)ch * it.hcap + m].y;
+            }
+            x[ch] = make_double2(r.x - h[ch].x, r.y - h[ch].y);
         }
-    }
-    // likelihood terms only where the template lands in the window
-    if (A.mode == 0 || (j >= 0 && j < W))
-    {
-        double wj[6];
         if (A.mode == 1)
         {
-            for (int q = 0; q < 6; q++) wj[q] = (j >= 0 && j < W) ? it.iC[(size_t)q * W + j] : 0.0;
+            double wj[6];
+#pragma unroll
+            for (int q = 0; q < 6; q++) wj[q] = it.iC[(size_t)q * W + j];
+            wmul(wj, x, z);
+            double2 y[3];
+            wmul(wj, h, y);
+#pragma unroll
+            for (int ch = 0; ch < 3; ch++) acc[kNMain] += h[ch].x * y[ch].x + h[ch].y * y[ch].y;
         }
-        const double* ww = A.mode == 1 ? wj : w;
-        acc[0] += bf3(r, h, ww) - 0.5 * bf3(h, h, ww);
-        double2 rh[3];
+        else
+            wmul(w, x, z);
 #pragma unroll
-        for (int ch = 0; ch < 3; ch++) rh[ch] = make_double2(r[ch].x - h[ch].x, r[ch].y - h[ch].y);
+        for (int q = 0; q < 6; q++)
 #pragma unroll
-        for (int a = 0; a < 8; a++) acc[1 + a] += bf3(rh, dh[a], ww);
+            for (int ch = 0; ch < 3; ch++)
+            {
+                acc[kPOff + 2 * q] += z[ch].x * u[q][ch].x + z[ch].y * u[q][ch].y;
+                acc[kPOff + 2 * q + 1] += z[ch].x * u[q][ch].y - z[ch].y * u[q][ch].x;
+            }
     }
-    int idx = 9;
 #pragma unroll
-    for (int a = 0; a < 8; a++)
+    for (int r = 0; r < 6; r++)
+    {
+        double2 y[3];
+        wmul(w, u[r], y);
 #pragma unroll
-        for (int b = a; b < 8; b++) acc[idx++] += bf3(dh[a], dh[b], w);
+        for (int ch = 0; ch < 3; ch++) acc[r] += u[r][ch].x * y[ch].x + u[r][ch].y * y[ch].y;
+#pragma unroll
+        for (int q = 0; q < r; q++)
+#pragma unroll
+            for (int ch = 0; ch < 3; ch++)
+            {
+                acc[gram_index(q, r)] += u[q][ch].x * y[ch].x + u[q][ch].y * y[ch].y;
+                acc[gram_index(q, r) + 1] += u[q][ch].x * y[ch].y - u[q][ch].y * y[ch].x;
+            }
+    }
 }
 
-// Workgroup reduction of the 45 sums and the outputs of item e.
-template <int NTHR>
-__device__ __forceinline__ void deriv_write(const DerivArgs& A, int e, double (&acc)[kNSum], double* red)
+// Workgroup sums of the per-thread sums into red[kNSum] through LDS: CH
+// values at a time are laid out one row per value (rows a double apart in
+// banks), each thread adds CH entries of one row, the lanes of a row add up
+// by two or three exchanges and the waves' partials in order.  170
+// instructions a thread for 48 values; the transposed shuffles took 500.
+// Fixed order.  buf: the FFT buffer (its readers have passed a barrier).
+template <int NTHR, int CH>
+__device__ __forceinline__ void deriv_reduce(const double (&acc)[kNSum], double* buf, double* red, bool extra)
 {
-    block_sum_vec<NTHR>(acc, red);
-    if (threadIdx.x < 64)
+    static_assert(kNMain % CH == 0 && 64 % CH == 0, "whole chunks");
+    constexpr int NW = NTHR / 64, ROW = NTHR + 1;
+    __shared__ double part[kNSum][NW];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+#pragma unroll
+    for (int k0 = 0; k0 < kNMain; k0 += CH)
     {
-        const int a = threadIdx.x / 8, b = threadIdx.x % 8;
-        const int lo = a < b ? a : b, hi = a < b ? b : a;
-        const int idx = 9 + lo * 8 - lo * (lo - 1) / 2 + (hi - lo);
-        A.fisher[(size_t)e * 64 + threadIdx.x] = red[idx];
-        if (threadIdx.x < 8) A.grad[(size_t)e * 8 + threadIdx.x] = red[1 + threadIdx.x];
-        if (threadIdx.x == 0) A.outL[e] = red[0];
+        if (k0) __syncthreads();
+#pragma unroll
+        for (int v = 0; v < CH; v++) buf[v * ROW + t] = acc[k0 + v];
+        __syncthreads();
+        const int v = t % CH;
+        const double* row = buf + v * ROW + (t / CH) * CH;
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < CH; i++) s += row[i];
+#pragma unroll
+        for (int d = CH; d < 64; d *= 2) s += __shfl_xor(s, d, 64);
+        if (lane < CH) part[k0 + v][wave] = s;
+    }
+    if (extra)
+    {
+        const double s = wave_sum(acc[kNMain]);
+        if (lane == 0) part[kNMain][wave] = s;
+    }
+    __syncthreads();
+    if (t < kNSum)
+    {
+        double s = 0.0;
+        if (t < kNMain || extra)
+            for (int i = 0; i < NW; i++) s += part[t][i];
+        red[t] = s;
     }
     __syncthreads();
 }
 
-// N = 2048: the six link series of one set take 196 KB, more than a CU's
-// LDS, so each set is built by decimation in time as in fd_link_spectra's
-// N >= 2048 branch (two 1024-point sub-series, six 1024-point link FFTs in
-// 96 KB of LDS, folded in registers), one set per pass; each set's TDI
-// values go to the workgroup's slice of hs (6 sets x 3 channels x N
-// complex) and are read back bin by bin for the sums.  Grid-striding over
-// the class list (A.list / A.count required).
-template <int NTHR>
-__global__ __launch_bounds__(NTHR) void deriv_kernel_2048(DerivArgs A, double2* __restrict__ hs)
+// L, gradient and Fisher matrix of item e from the reduced sums: dh/dtheta_a
+// = A u_q + B u_s with at most two sets.
+__device__ __forceinline__ void deriv_write(const UcbConst& c, const UcbDiff& dd, const DerivArgs& A, int e,
+                                            const double* red)
 {
-    constexpr int N = 2048, NS = 1024, P = N / NS, U = NS / NTHR, PER = N / NTHR;
-    static_assert(NS % NTHR == 0, "decimated shape");
-    __shared__ double2 lds[6 * NS];
+    if (threadIdx.x >= 64) return;
+    auto coef = [&](int a, int& q, double2& ca, double2& cb) {
+        const int set[8] = {2, 3, 4, 0, 0, 0, 0, 5};
+        q = set[a];
+        ca = make_double2(1.0, 0.0);
+        cb = make_double2(0.0, 0.0);
+        const double2 DP = make_double2(c.DPr, c.DPi), DC = make_double2(c.DCr, c.DCi);
+        if (a == 3) ca = DP, cb = DC;                                                        // ln A: h
+        if (a == 4) ca = make_double2(dd.DPr4, dd.DPi4), cb = make_double2(dd.DCr4, dd.DCi4);
+        if (a == 5) ca = make_double2(dd.DPr5, dd.DPi5), cb = make_double2(dd.DCr5, dd.DCi5);
+        if (a == 6) ca = make_double2(DP.y, -DP.x), cb = make_double2(DC.y, -DC.x);          // phi0: -i h
+    };
+    auto G = [&](int q, int r) {
+        if (q == r) return make_double2(red[q], 0.0);
+        const int k = gram_index(q < r ? q : r, q < r ? r : q);
+        return make_double2(red[k], q < r ? red[k + 1] : -red[k + 1]);
+    };
+    // Re conj(a) g b
+    auto re3 = [](double2 a, double2 g, double2 b) {
+        const double2 ab = make_double2(a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x);
+        return ab.x * g.x - ab.y * g.y;
+    };
+    const int a = threadIdx.x / 8, b = threadIdx.x % 8;
+    const int lo = a < b ? a : b, hi = a < b ? b : a;  // both triangles alike, bit for bit
+    int qa, qb;
+    double2 a0, a1, b0, b1;
+    coef(lo, qa, a0, a1);
+    coef(hi, qb, b0, b1);
+    double f = re3(a0, G(qa, qb), b0);
+    if (qb == 0) f += re3(a0, G(qa, 1), b1);
+    if (qa == 0) f += re3(a1, G(1, qb), b0);
+    if (qa == 0 && qb == 0) f += re3(a1, G(1, 1), b1);
+    A.fisher[(size_t)e * 64 + threadIdx.x] = 2.0 * f;
+    auto proj = [&](int k) {
+        int q;
+        double2 ca, cb;
+        coef(k, q, ca, cb);
+        double g = ca.x * red[kPOff + 2 * q] - ca.y * red[kPOff + 2 * q + 1];
+        if (q == 0) g += cb.x * red[kPOff + 2] - cb.y * red[kPOff + 3];
+        return 2.0 * g;
+    };
+    if (threadIdx.x < 8) A.grad[(size_t)e * 8 + threadIdx.x] = proj(threadIdx.x);
+    // (R|h) - (h|h)/2 = (R - h|h) + (h|h)/2; thread 27 holds (3, 3) = (h|h)
+    if (threadIdx.x == 27) A.outL[e] = proj(3) + (A.mode == 1 ? red[kNMain] : f);
+}
+
+// Waves per SIMD the register allocation must allow (1 = the compiler's
+// choice, at least the two that eight waves per CU need).
+#ifndef GH_DERIV_WAVES
+#define GH_DERIV_WAVES 1
+#endif
+
+// The constants of the workgroup's source and their derivatives on lanes of
+// two waves, so the two serial setups overlap.
+template <int NTHR>
+__device__ __forceinline__ void deriv_setup(const double* p, const DerivArgs& A, UcbConst& sc, UcbDiff& sdd)
+{
+    if (threadIdx.x == 0) ucb_setup(p, 8, A.T, A.t0, A.L, A.fstar, sc);
+    if (threadIdx.x == (NTHR >= 128 ? 64 : 0)) ucb_diff_setup(p, A.T, sdd);
+    __syncthreads();
+}
+
+template <int N>
+__global__ __launch_bounds__(fd_threads(N), GH_DERIV_WAVES) void deriv_kernel(DerivArgs A)
+{
+    using S = FdShape<N, 1>;
+    constexpr int P = S::P, NTHR = S::NTHR;
+    constexpr int LDS = deriv_sets(N) * kNLink * S::PN;
+    constexpr int CH = 16 * (NTHR + 1) <= 2 * LDS ? 16 : 8;
+    static_assert(CH * (NTHR + 1) <= 2 * LDS, "the reduction's rows fit the FFT buffer");
+    __shared__ double2 lds[LDS];
     __shared__ UcbDiff sdd;
+    __shared__ UcbConst sc;
     __shared__ double red[kNSum];
-    double2* H = hs + (size_t)blockIdx.x * 18 * N;
+    int e = blockIdx.x;
+    if (A.list)
+    {
+        if (e >= *A.count) return;  // uniform over the workgroup
+        e = A.list[e];
+    }
+    deriv_setup<NTHR>(A.params + (size_t)(A.pidx ? A.pidx[e] : e) * 8, A, sc, sdd);
+    // the constants into scalar registers for the passes (the derivative
+    // constants stay in LDS, where the scalar copies would spill)
+    UcbConst c = sc;
+    c.np = 8;
+    make_uniform(c);
+    double2 u[P][6][3];
+    deriv_passes<N, 6>(c, sdd, lds, A, [&](int r, int q, double2 X, double2 Y, double2 Z) {
+        u[r][q][0] = X;
+        u[r][q][1] = Y;
+        u[r][q][2] = Z;
+    });
+    double acc[kNSum];
+#pragma unroll
+    for (int k = 0; k < kNSum; k++) acc[k] = 0.0;
+    const DerivItem it = deriv_item(A, e);
+    if (S::NT >= 64 || threadIdx.x < S::NT)
+#pragma unroll
+        for (int r = 0; r < P; r++) deriv_bin(c, A, it, P * threadIdx.x + r, u[r], acc);
+    deriv_reduce<NTHR, CH>(acc, (double*)lds, red, A.mode == 1);
+    deriv_write(c, sdd, A, e, red);
+}
+
+// N = 2048, 4096: the same with the TDI values of a source (18 N complex) in
+// the workgroup's slice of hs, read back bin by bin for the sums (each
+// thread reads only what it wrote).  Grid-striding over the class list.
+template <int N>
+__global__ __launch_bounds__(fd_threads(N, 1)) void deriv_kernel_long(DerivArgs A, double2* __restrict__ hs)
+{
+    using S = FdShape<N, 1>;
+    constexpr int P = S::P, NTHR = S::NTHR;
+    constexpr int LDS = deriv_sets(N) * kNLink * S::PN;
+    constexpr int CH = 8;
+    static_assert(CH * (NTHR + 1) <= 2 * LDS, "the reduction's rows fit the FFT buffer");
+    __shared__ double2 lds[LDS];
+    __shared__ UcbDiff sdd;
+    __shared__ UcbConst sc;
+    __shared__ double red[kNSum];
+    double2* H = hs + (size_t)blockIdx.x * deriv_scratch(N);
     const int cnt = A.list ? *A.count : A.nitems;
     const int t = threadIdx.x;
-    const int twstride = kTwN / N;
-    const double inv2N = 1. / (double)(2 * N);
     for (int w = blockIdx.x; w < cnt; w += gridDim.x)
     {
         const int e = A.list ? A.list[w] : w;
-        const double* p = A.params + (size_t)(A.pidx ? A.pidx[e] : e) * 8;
-        const UcbConst& c = ucb_setup_shared(p, 8, A.T, A.t0, A.L, A.fstar);
-        if (t == 0) ucb_diff_setup(p, A.T, sdd);
-        __syncthreads();
-        const UcbDiff& dd = sdd;
-        auto one_set = [&](auto set_tag) {
-            constexpr int S = decltype(set_tag)::value;
-            double2 X[U][P][6];
-#pragma unroll
-            for (int u = 0; u < U; u++)
-#pragma unroll
-                for (int r = 0; r < P; r++)
-#pragma unroll
-                    for (int l = 0; l < 6; l++) X[u][r][l] = make_double2(0.0, 0.0);
-#pragma unroll 1
-            for (int ph = 0; ph < P; ph++)
-            {
-                for (int j = t; j < NS; j += NTHR)
-                {
-                    const int n = P * j + ph;
-                    const double ts = ucb_sample_time(c.T, c.t0, n, N);
-                    ucb_sample_sets<S, 1>(c, dd, ts, A.pos + (size_t)n * (4096 / N) * 9, lds, NS, j);
-                }
-                __syncthreads();
-                lds_fft<NS, 6, NTHR>(lds, A.tw, twstride * P);
-#pragma unroll
-                for (int u = 0; u < U; u++)
-                {
-                    const int j = t + u * NTHR;
-                    const double2 wj = A.tw[(ph * j) * twstride];
-#pragma unroll
-                    for (int l = 0; l < 6; l++)
-                    {
-                        const double2 v = cmul(lds[l * NS + j], wj);
-#pragma unroll
-                        for (int r = 0; r < P; r++)
-                        {
-                            const double2 q = cmul(v, A.tw[((ph * r) % P) * NS * twstride]);
-                            X[u][r][l].x += q.x;
-                            X[u][r][l].y += q.y;
-                        }
-                    }
-                }
-                __syncthreads();
-            }
-            // FFT index s = j + NS r (j = t + u NTHR) is template bin
-            // m = (s + N/2) mod N = t + k NTHR
-#pragma unroll
-            for (int u = 0; u < U; u++)
-#pragma unroll
-                for (int r = 0; r < P; r++)
-                {
-                    const int k = (u + U * r + N / (2 * NTHR)) % PER;
-                    const int m = t + k * NTHR;
-                    double2 d6[6], o5[5];
-#pragma unroll
-                    for (int l = 0; l < 6; l++) d6[l] = make_double2(X[u][r][l].x * inv2N, X[u][r][l].y * inv2N);
-                    fd_tdi<N>(c, m, A.fmt, d6, o5);
-#pragma unroll
-                    for (int ch = 0; ch < 3; ch++) H[(size_t)(S * 3 + ch) * N + m] = o5[ch];
-                }
-        };
-        one_set(std::integral_constant<int, 0>{});
-        one_set(std::integral_constant<int, 1>{});
-        one_set(std::integral_constant<int, 2>{});
-        one_set(std::integral_constant<int, 3>{});
-        one_set(std::integral_constant<int, 4>{});
-        one_set(std::integral_constant<int, 5>{});
-        // each thread reads back only the bins it wrote: no barrier needed
-        DerivItem it = deriv_item(A, e);
+        __syncthreads();  // the last item's readers of sc, sdd and red
+        deriv_setup<NTHR>(A.params + (size_t)(A.pidx ? A.pidx[e] : e) * 8, A, sc, sdd);
+        const UcbConst& c = sc;
+        deriv_passes<N, 6>(c, sdd, lds, A, [&](int r, int q, double2 X, double2 Y, double2 Z) {
+            double2* o = H + (size_t)(q * 3 * P + r) * NTHR + t;
+            o[0] = X;
+            o[P * NTHR] = Y;
+            o[2 * P * NTHR] = Z;
+        });
         double acc[kNSum];
 #pragma unroll
-        for (int q = 0; q < kNSum; q++) acc[q] = 0.0;
+        for (int k = 0; k < kNSum; k++) acc[k] = 0.0;
+        const DerivItem it = deriv_item(A, e);
 #pragma unroll 1
-        for (int k = 0; k < PER; k++)
+        for (int r = 0; r < P; r++)
         {
-            const int m = t + k * NTHR;
-            double2 Hb[6][3];
+            double2 u[6][3];
 #pragma unroll
-            for (int S = 0; S < 6; S++)
+            for (int q = 0; q < 6; q++)
 #pragma unroll
-                for (int ch = 0; ch < 3; ch++) Hb[S][ch] = H[(size_t)(S * 3 + ch) * N + m];
-            deriv_bin(c, dd, A, it, m, Hb, acc);
+                for (int ch = 0; ch < 3; ch++) u[q][ch] = H[(size_t)((q * 3 + ch) * P + r) * NTHR + t];
+            deriv_bin(c, A, it, P * t + r, u, acc);
         }
-        deriv_write<NTHR>(A, e, acc, red);
+        deriv_reduce<NTHR, CH>(acc, (double*)lds, red, A.mode == 1);
+        deriv_write(c, sdd, A, e, red);
     }
 }
 
@@ -457,119 +433,9 @@ int launch_derivs_2048(const DerivArgs& A, int grid, double2* hs, hipStream_t s)
         set_error("fd derivs: BW 2048 needs a class list or an item count, and scratch");
         return GLASS_HIP_EINVAL;
     }
-    deriv_kernel_2048<kDeriv2048Threads><<<grid, kDeriv2048Threads, 0, s>>>(A, hs);
+    deriv_kernel_long<2048><<<grid, fd_threads(2048, 1), 0, s>>>(A, hs);
     GH_CHECK(hipGetLastError());
     return GLASS_HIP_OK;
-}
-
-// N = 4096: the 2048 kernel's decimation in time with P = 4 phases of
-// 1024-point sub-series, but the P x 6 link accumulators of a thread's
-// sub-bins (four times the 2048 kernel's, past any register budget) live in
-// the workgroup's global scratch slice: acc[l][s] (6 x N complex), summed
-// over the phases in order, then TDI'd into H[set][ch][m] (18 x N).  Each
-// thread reads back only the accumulators and bins it wrote (FFT index
-// s = j + NS r and bin m = (s + N/2) mod N keep j mod NTHR), so the slice
-// needs no barrier.
-template <int NTHR>
-__global__ __launch_bounds__(NTHR) void deriv_kernel_4096(DerivArgs A, double2* __restrict__ hs)
-{
-    constexpr int N = 4096, NS = 1024, P = N / NS, U = NS / NTHR, PER = N / NTHR;
-    static_assert(NS % NTHR == 0 && (N / 2) % NTHR == 0, "decimated shape");
-    __shared__ double2 lds[6 * NS];
-    __shared__ UcbDiff sdd;
-    __shared__ double red[kNSum];
-    double2* Acc = hs + (size_t)blockIdx.x * kDeriv4096Scratch;
-    double2* H = Acc + 6 * N;
-    const int cnt = A.list ? *A.count : A.nitems;
-    const int t = threadIdx.x;
-    const int twstride = kTwN / N;
-    const double inv2N = 1. / (double)(2 * N);
-    for (int w = blockIdx.x; w < cnt; w += gridDim.x)
-    {
-        const int e = A.list ? A.list[w] : w;
-        const double* p = A.params + (size_t)(A.pidx ? A.pidx[e] : e) * 8;
-        const UcbConst& c = ucb_setup_shared(p, 8, A.T, A.t0, A.L, A.fstar);
-        if (t == 0) ucb_diff_setup(p, A.T, sdd);
-        __syncthreads();
-        const UcbDiff& dd = sdd;
-        auto one_set = [&](auto set_tag) {
-            constexpr int S = decltype(set_tag)::value;
-#pragma unroll 1
-            for (int ph = 0; ph < P; ph++)
-            {
-                for (int j = t; j < NS; j += NTHR)
-                {
-                    const int n = P * j + ph;
-                    const double ts = ucb_sample_time(c.T, c.t0, n, N);
-                    ucb_sample_sets<S, 1>(c, dd, ts, A.pos + (size_t)n * (4096 / N) * 9, lds, NS, j);
-                }
-                __syncthreads();
-                lds_fft<NS, 6, NTHR>(lds, A.tw, twstride * P);
-#pragma unroll
-                for (int u = 0; u < U; u++)
-                {
-                    const int j = t + u * NTHR;
-                    const double2 wj = A.tw[(ph * j) * twstride];
-#pragma unroll
-                    for (int l = 0; l < 6; l++)
-                    {
-                        const double2 v = cmul(lds[l * NS + j], wj);
-#pragma unroll
-                        for (int r = 0; r < P; r++)
-                        {
-                            const double2 q = cmul(v, A.tw[((ph * r) % P) * NS * twstride]);
-                            double2* a = Acc + (size_t)l * N + j + NS * r;
-                            if (ph == 0)
-                                *a = q;
-                            else
-                                *a = make_double2(a->x + q.x, a->y + q.y);
-                        }
-                    }
-                }
-                __syncthreads();
-            }
-#pragma unroll 1
-            for (int u = 0; u < U; u++)
-#pragma unroll 1
-                for (int r = 0; r < P; r++)
-                {
-                    const int sidx = t + u * NTHR + NS * r;
-                    const int m = (sidx + N / 2) & (N - 1);
-                    double2 d6[6], o5[5];
-#pragma unroll
-                    for (int l = 0; l < 6; l++)
-                    {
-                        const double2 a = Acc[(size_t)l * N + sidx];
-                        d6[l] = make_double2(a.x * inv2N, a.y * inv2N);
-                    }
-                    fd_tdi<N>(c, m, A.fmt, d6, o5);
-#pragma unroll
-                    for (int ch = 0; ch < 3; ch++) H[(size_t)(S * 3 + ch) * N + m] = o5[ch];
-                }
-        };
-        one_set(std::integral_constant<int, 0>{});
-        one_set(std::integral_constant<int, 1>{});
-        one_set(std::integral_constant<int, 2>{});
-        one_set(std::integral_constant<int, 3>{});
-        one_set(std::integral_constant<int, 4>{});
-        one_set(std::integral_constant<int, 5>{});
-        DerivItem it = deriv_item(A, e);
-        double acc[kNSum];
-#pragma unroll
-        for (int q = 0; q < kNSum; q++) acc[q] = 0.0;
-#pragma unroll 1
-        for (int k = 0; k < PER; k++)
-        {
-            const int m = t + k * NTHR;
-            double2 Hb[6][3];
-#pragma unroll
-            for (int S = 0; S < 6; S++)
-#pragma unroll
-                for (int ch = 0; ch < 3; ch++) Hb[S][ch] = H[(size_t)(S * 3 + ch) * N + m];
-            deriv_bin(c, dd, A, it, m, Hb, acc);
-        }
-        deriv_write<NTHR>(A, e, acc, red);
-    }
 }
 
 int launch_derivs_4096(const DerivArgs& A, int grid, double2* hs, hipStream_t s)
@@ -580,7 +446,7 @@ int launch_derivs_4096(const DerivArgs& A, int grid, double2* hs, hipStream_t s)
         set_error("fd derivs: BW 4096 needs a class list or an item count, and scratch");
         return GLASS_HIP_EINVAL;
     }
-    deriv_kernel_4096<kDeriv2048Threads><<<grid, kDeriv2048Threads, 0, s>>>(A, hs);
+    deriv_kernel_long<4096><<<grid, fd_threads(4096, 1), 0, s>>>(A, hs);
     GH_CHECK(hipGetLastError());
     return GLASS_HIP_OK;
 }
@@ -592,7 +458,7 @@ int launch_derivs(int N, const DerivArgs& A, int grid, hipStream_t s)
     {
 #define GH_D(NN)                                                                   \
     case NN:                                                                       \
-        deriv_kernel<NN, fd_threads(NN)><<<grid, fd_threads(NN), 0, s>>>(A);       \
+        deriv_kernel<NN><<<grid, fd_threads(NN), 0, s>>>(A);       \
         break;
         GH_D(32) GH_D(64) GH_D(128) GH_D(256) GH_D(512) GH_D(1024)
 #undef GH_D

@@ -21,22 +21,16 @@ __global__ __launch_bounds__(NTHR) void fd_waveform_kernel(const double* __restr
                                                            const double2* __restrict__ tw, int twstride,
                                                            int fmt, double2* __restrict__ out)
 {
-    using S = FdShape<N, NTHR>;
-    __shared__ double2 lds[S::LDS];
+    __shared__ double2 lds[FdShape<N>::LDS];
     const UcbConst& c = ucb_setup_shared(params + (size_t)blockIdx.x * np, np, T, t0, L, fstar);
-    double2 d[S::PER][6];
-    fd_link_spectra<N, NTHR>(c, lds, pos, posstride, tw, twstride, d);
     double2* o = out + (size_t)blockIdx.x * 5 * N;
+    fd_link_bins<N, false>(
+        HeldConst{c}, lds, pos, posstride, tw, twstride, [](int) {}, [&](int, int m, const double2* d) {
+            double2 v[5];
+            fd_tdi<N>(c, m, fmt, d, v);
 #pragma unroll
-    for (int k = 0; k < S::PER; k++)
-    {
-        const int m = threadIdx.x + k * NTHR;
-        if (m >= N) continue;
-        double2 v[5];
-        fd_tdi<N>(c, m, fmt, d[k], v);
-#pragma unroll
-        for (int ch = 0; ch < 5; ch++) o[ch * N + m] = v[ch];
-    }
+            for (int ch = 0; ch < 5; ch++) o[ch * N + m] = v[ch];
+        });
 }
 
 template <int N>

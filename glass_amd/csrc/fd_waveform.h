@@ -1,66 +1,64 @@
 // fd_waveform.h -- device building blocks of the frequency-domain UCB
-// template: slow series -> six LDS FFTs -> fftshift/normalise -> TDI.
+// template: slow series -> LDS FFTs -> fftshift/normalise -> TDI.
 // ucb/src/glass_ucb_waveform.c:738-1001; TDI utils/src/glass_lisa.c:458-710.
 //
-// Work split: one workgroup of NTHR threads per template of N bins; thread
-// t owns output bins m = t + k*NTHR (k < PER).
-//  * N <= 1024: NTHR = max(N, 64) threads, one slow sample each, written
-//    straight into LDS (6 links x N complex = 96 N bytes <= 96 KB), six
-//    FFTs, then every thread reads its bin's six link values.
-//  * N <= 1024 with NTHR = N/2 (fd_link_bins): thread t folds samples t
-//    and t + N/2 by one radix-2 decimation-in-frequency step; the even-bin
-//    series goes to LDS, the odd-bin series waits in registers, and the two
-//    half-length transforms run in turn (48 N bytes of LDS).  Bins are
-//    handed out per pass, one per thread (m = 2t, then 2t + 1), so only
-//    one bin's six link values are live at a time.
-//  * N = 2048 with NTHR = 512 (fd_link_bins): the split step on two sample
-//    pairs per thread, the two 1024-point half-length transforms in turn.
-//  * N = P*NS (N >= 2048, NS = 1024): decimation in time.  The samples
-//    n = P*j + p of each phase p form an NS-point series; its six FFTs run
-//    in LDS in turn and each thread folds X_{j+NS r} += w_N^{p j} w_P^{p r}
-//    S_p[j] into registers for its sub-bins j, so LDS stays at 6*NS*16
-//    bytes and no sample is held in registers across passes.
+// Five series, not six: every TDI channel is made of differences of link
+// series, so the series e_l = d_l - d_23 of the other five links carry them
+// all (a sixth of the FFT work, LDS and TDI reads less).  Order: 12, 21, 31,
+// 13, 32.
+//
+// Work split: one workgroup per template of N = P NT bins, NT <= 512
+// threads (64 at least).  Thread t evaluates the samples n = t + NT p; a
+// P-point decimation-in-frequency step in registers turns them into P series
+// of NT points (X[P k + r] = FFT_NT(w_N^{r t} sum_p x_p w_P^{r p})[k]), which
+// are transformed in LDS one after the other, the others waiting in
+// registers.  Each pass hands one bin per thread to the caller (m = P t + r),
+// so one bin's five values are live at a time.  NT = 512 is the length that
+// one wave transforms in three radix-8 passes (wave_fft).  At 2048 bins two
+// groups of threads share the P samples (FdShape).
 #pragma once
 #include "fft_lds.h"
 #include "ucb_common.h"
 
-#ifndef GH_NTHR_1024
-#define GH_NTHR_1024 512
-#endif
-#ifndef GH_DECIM_NS
-#define GH_DECIM_NS 1024
-#endif
-#ifndef GH_NTHR_DECIM
-#define GH_NTHR_DECIM 512
-#endif
-
 namespace glass {
 
-// Workgroup size for a template of N bins: one sample per thread up to 512,
-// two at N = 1024 (keeps the 256-VGPR budget of 8-wave workgroups), and
-// 1024 threads for the decimated N >= 2048 path.
-constexpr int fd_threads(int N) { return N < 64 ? 64 : (N <= 512 ? N : (N == 1024 ? GH_NTHR_1024 : GH_NTHR_DECIM)); }
+constexpr int kNLink = 5;  // series of a template
 
-// Default workgroup size of the batched template kernels (fd_link_bins):
-// the split shape, N/2 threads with two bins each, from 128 to 1024 bins.
-constexpr int fd_batch_threads(int N) { return N <= 64 ? 64 : (N <= 1024 ? N / 2 : GH_NTHR_DECIM); }
+// Groups of 512 threads per template: two from 2048 bins, where the four or
+// eight series of one group would take 233 VGPRs and more (one workgroup of
+// eight waves per CU, the vector units 34% busy); each group holds half.
+// 23,671 fused evaluations of 2048 bins 2.93 -> 2.81 ms, 379 of 4096 bins 0.39
+// -> 0.24 ms.
+constexpr int fd_groups(int N) { return N >= 2048 ? 2 : 1; }
 
-// SPLIT (fd_link_bins only, N <= 2048 with NTHR = N/2): one radix-2
-// decimation-in-frequency step in registers, then the even- and odd-bin
-// half-length transforms in LDS one after the other (half the LDS).
-template <int N, int NTHR, bool SPLIT = false>
+// Series of a template of N bins (P).
+constexpr int fd_series(int N) { return N <= 512 ? 1 : N / 512; }
+
+// Workgroup size for a template of N bins.
+constexpr int fd_threads(int N, int G) { return N < 64 ? 64 : (N <= 512 ? N : 512 * G); }
+constexpr int fd_threads(int N) { return fd_threads(N, fd_groups(N)); }
+
+template <int N, int GROUPS = fd_groups(N)>
 struct FdShape
 {
-    static_assert(!SPLIT || (N <= 2048 && N >= 8 && 2 * NTHR == N), "split shape: N <= 2048, N/2 threads");
-    static constexpr int PER = (N + NTHR - 1) / NTHR;  // bins per thread
-    // FFT length in LDS: the whole template up to 1024 bins (half of it
-    // when split), else the sub-series length of the decimated path
-    static constexpr int NS = SPLIT ? N / 2 : (N <= 1024 ? N : GH_DECIM_NS);
-    static constexpr int LDS = 6 * NS;                  // double2 elements
+    static_assert(N >= 16 && N <= 4096 && (N & (N - 1)) == 0, "16 to 4096 bins");
+    static_assert(GROUPS == 1 || (GROUPS == 2 && N >= 2048), "two groups: two or four samples a thread");
+    static constexpr int G = GROUPS;
+    static constexpr int P = fd_series(N);
+    static constexpr int Q = P / G;                   // samples and bins per thread
+    static constexpr int NT = N / P;                  // points of an LDS series
+    static constexpr int NTHR = fd_threads(N, G);
+    static constexpr int PN = wave_fft_stride(NT);
+    static constexpr int LDS = G * kNLink * PN;       // double2 elements
+    // the thread's place in its group, and its bin in pass s: P t + the
+    // residue, of which the group g of two takes j = g Q/2 .. and j + Q
+    static __device__ __forceinline__ int lane() { return G == 1 ? threadIdx.x : threadIdx.x & 511; }
+    static __device__ __forceinline__ int group() { return G == 1 ? 0 : threadIdx.x >> 9; }
+    static __device__ __forceinline__ int residue(int s) { return G == 1 ? s : group() * (Q / 2) + s / 2 + Q * (s % 2); }
+    static __device__ __forceinline__ int bin(int s) { return P * lane() + residue(s); }
+    // where the series of pass s waits
+    static constexpr int slot(int s) { return G == 1 ? s : s / 2 + (Q / 2) * (s % 2); }
 };
-
-// Split launch shapes: two bins per thread up to 2048 bins.
-constexpr bool fd_split(int N, int NTHR) { return N <= 2048 && N >= 8 && 2 * NTHR == N; }
 
 // Move a value that every lane holds identically into a scalar register.
 __device__ inline double uniform(double x)
@@ -80,7 +78,50 @@ __device__ inline void make_uniform(UcbConst& c)
     c.q = ((long)__builtin_amdgcn_readfirstlane((int)(c.q >> 32)) << 32) |
           (unsigned)__builtin_amdgcn_readfirstlane((int)(c.q & 0xffffffff));
     c.np = __builtin_amdgcn_readfirstlane(c.np);
+    c.wide = __builtin_amdgcn_readfirstlane(c.wide);
 }
+
+// A pointer that every lane holds identically, in scalar registers.
+template <typename T>
+__device__ __forceinline__ const T* uniform_ptr(const T* p)
+{
+    const unsigned long long v = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return (const T*)(((unsigned long long)hi << 32) | lo);
+}
+
+// The constants of one template as the building blocks below take them: a
+// callable that returns them.  One that is held (in LDS or registers):
+struct HeldConst
+{
+    const UcbConst& c;
+    __device__ const UcbConst& operator()() const { return c; }
+};
+// ... and one read again by scalar loads at each use (8 parameters).  The
+// constants, pointers and masks of a fused kernel are more than the ~100
+// scalar registers; held throughout, 370 moves a wave go to spilling them
+// into vector lanes.  The pointer passes through an empty asm, so that no
+// value of one use stays live until the next.
+struct LoadedConst
+{
+    const UcbConst* p;
+    __device__ __forceinline__ UcbConst operator()() const
+    {
+        auto g = (const __attribute__((address_space(4))) double*)uniform_ptr(p);
+        asm volatile("" : "+s"(g));
+        UcbConst c;
+        double* f = &c.T;
+        constexpr int nd = (int)((offsetof(UcbConst, q)) / sizeof(double));
+#pragma unroll
+        for (int i = 0; i < nd; i++) f[i] = g[i];
+        auto w = (const __attribute__((address_space(4))) int*)g;
+        c.q = (long)c.qd;
+        c.np = 8;
+        c.wide = w[offsetof(UcbConst, wide) / sizeof(int)];
+        return c;
+    }
+};
 
 // Per-template constants computed once per workgroup (by thread 0) into
 // LDS; every thread reads them from there.  Synchronises the workgroup on
@@ -95,340 +136,224 @@ __device__ inline const UcbConst& ucb_setup_shared(const double* p, int np, doub
     return sc;
 }
 
-// Slow samples of one phase into LDS: sample n = P*j + p at LDS slot j.
-template <int N, int NTHR, int P>
-__device__ inline void fd_samples_to_lds(const UcbConst& c, double2* lds, const double* __restrict__ pos,
-                                         int posstride, int p)
+// The P-point decimation-in-frequency step of thread t's samples x_p (sample
+// t + NT p) in place: x[r] becomes the thread's point of series r.
+template <int N, int L>
+__device__ __forceinline__ void fd_dif(double2 (&x)[fd_series(N)][L], const double2* __restrict__ tw, int tws, int t)
 {
-    constexpr int NS = N / P;
-    for (int j = threadIdx.x; j < NS; j += NTHR)
+    constexpr int P = fd_series(N);
+    double2 w[P > 1 ? P - 1 : 1];
+#pragma unroll
+    for (int r = 1; r < P; r++) w[r - 1] = tw[(r * t) * tws];
+#pragma unroll
+    for (int l = 0; l < L; l++)
     {
-        const int n = P * j + p;
-        double t = ucb_sample_time(c.T, c.t0, n, N);
-        ucb_slow_sample(c, t, pos + (size_t)n * posstride * 9, lds, NS, j);
+        double2 v[P], y[P];
+#pragma unroll
+        for (int p = 0; p < P; p++) v[p] = x[p][l];
+        radix_butterfly<P>(v, y);
+        x[0][l] = y[0];
+#pragma unroll
+        for (int r = 1; r < P; r++) x[r][l] = cmul(y[r], w[r - 1]);
+    }
+}
+
+// The same with the samples of a point on two threads: group g of two holds
+// x_{g + 2q}, q < Q.  Each thread transforms its own (A_j from the even samples,
+// B_j from the odd, j < Q), hands half of the results to its partner through
+// LDS and combines the other half: X_j = A_j + w_P^j B_j, X_{j+Q} = A_j - w_P^j B_j,
+// left in the slots of FdShape.  lds: the groups' series rows.
+template <int N>
+__device__ __forceinline__ void fd_dif2(double2 (&x)[fd_series(N) / 2][kNLink], double2* lds,
+                                        const double2* __restrict__ tw, int tws)
+{
+    using S = FdShape<N, 2>;
+    constexpr int Q = S::Q, H = Q / 2;
+    const bool g = S::group() != 0;
+    const int t = S::lane();
+    // by value: a choice between array elements would put the array in memory
+    auto pick = [](bool c, double2 a, double2 b) { return make_double2(c ? a.x : b.x, c ? a.y : b.y); };
+    double2* mine = lds + g * kNLink * S::PN;
+    const double2* other = lds + (1 - g) * kNLink * S::PN;
+#pragma unroll
+    for (int l = 0; l < kNLink; l++)
+    {
+        double2 v[Q], y[Q];
+#pragma unroll
+        for (int q = 0; q < Q; q++) v[q] = x[q][l];
+        radix_butterfly<Q>(v, y);
+#pragma unroll
+        for (int q = 0; q < Q; q++) x[q][l] = y[q];
+    }
+#pragma unroll
+    for (int i = 0; i < H; i++)
+    {
+        if (i) __syncthreads();
+#pragma unroll
+        for (int l = 0; l < kNLink; l++) mine[l * S::PN + t] = pick(g, x[i][l], x[H + i][l]);
+        __syncthreads();
+        const int j = g * H + i;
+        const double2 wp = tw[j * S::NT * tws];  // w_P^j
+        const double2 w1 = tw[(j * t) * tws], w2 = tw[((j + Q) * t) * tws];
+#pragma unroll
+        for (int l = 0; l < kNLink; l++)
+        {
+            const double2 o = other[l * S::PN + t], h = pick(g, x[H + i][l], x[i][l]);
+            const double2 a = pick(g, o, h), b = cmul(pick(g, h, o), wp);
+            x[i][l] = cmul(make_double2(a.x + b.x, a.y + b.y), w1);
+            x[H + i][l] = cmul(make_double2(a.x - b.x, a.y - b.y), w2);
+        }
     }
     __syncthreads();
 }
 
-// Build the six shifted, normalised link spectra of one template: on return
-// d[k][l] holds link l at output bin m = threadIdx.x + k*NTHR, i.e.
-// FFT_l[(m + N/2) mod N] / (2N)  (glass_ucb_waveform.c:940-962).
-// Link order 12, 21, 31, 13, 23, 32.  Ends with a barrier, so lds may be
-// reused immediately.
-template <int N, int NTHR>
-__device__ inline void fd_link_spectra(const UcbConst& c, double2* lds, const double* __restrict__ pos,
-                                       int posstride, const double2* __restrict__ tw, int twstride,
-                                       double2 (&d)[FdShape<N, NTHR>::PER][6])
+// f(s, m, d) for every output bin m = FdShape::bin(s) of this thread: d[l] =
+// series l at bin m, FFT_l[(m + N/2) mod N] (glass_ucb_waveform.c:940-962);
+// the reference's 1/(2N) is part of fd_tdi's prefactor.  SOA: pos is the
+// N-sample structure-of-arrays block (9 rows of N samples); else the record
+// table read with stride posstride.  tws = entries of tw per N-th root.
+// pre(m) is called before the transform of bin m's pass, so that global
+// loads the caller issues there are in flight during it.  No barrier after
+// the last LDS reads: the caller passes one of its own before anything
+// writes lds again.
+template <int N, bool SOA, int GROUPS = fd_groups(N), typename K, typename Pre, typename F>
+__device__ __forceinline__ void fd_link_bins(const K& kget, double2* lds, const double* __restrict__ pos,
+                                             int posstride, const double2* __restrict__ tw, int tws, Pre&& pre, F&& f)
 {
-    using S = FdShape<N, NTHR>;
-    const double inv2N = 1. / (double)(2 * N);
-    if constexpr (N <= 1024)
+    using S = FdShape<N, GROUPS>;
+    constexpr int P = S::P, Q = S::Q, NT = S::NT, PN = S::PN;
+    constexpr int KS = SOA ? N : 1;
+    const int t = S::lane();
+    const bool on = NT >= 64 || t < NT;
+    const int ts = wave_fft_slot(t);
+    double2* rows = lds + S::group() * kNLink * PN;
+    auto sample = [&](int n, auto&& out) {
+        const UcbConst& c = kget();
+        ucb_slow_sample_to<KS>(c, ucb_sample_time(c.T, c.t0, n, N), SOA ? pos + n : pos + (size_t)n * posstride * 9,
+                               out);
+    };
+    double2 x[Q][kNLink];
+    if constexpr (P == 1)
     {
-        fd_samples_to_lds<N, NTHR, 1>(c, lds, pos, posstride, 0);
-        lds_fft<N, 6, NTHR>(lds, tw, twstride);
-#pragma unroll
-        for (int k = 0; k < S::PER; k++)
-        {
-            const int m = threadIdx.x + k * NTHR;
-            const int s = (m + N / 2) & (N - 1);
-            if (m < N)
-#pragma unroll
-                for (int l = 0; l < 6; l++)
-                {
-                    double2 v = lds[l * N + s];
-                    d[k][l] = make_double2(v.x * inv2N, v.y * inv2N);
-                }
-        }
-        __syncthreads();
+        if (on) sample(t, [&](int l, double2 v) { rows[l * PN + ts] = v; });
     }
     else
     {
-        // decimation in time: P phases of NS-point sub-series
-        constexpr int NS = S::NS, P = N / NS, U = NS / NTHR;
-        static_assert(NS % NTHR == 0 && N % NS == 0, "decimated shape");
-        const int t = threadIdx.x;
-        double2 X[U][P][6];
+        // the samples shifted in: a loop whose body is one sample, so that
+        // one sample's temporaries are live beside the Q results
 #pragma unroll
-        for (int u = 0; u < U; u++)
+        for (int p = 0; p < Q; p++)
 #pragma unroll
-            for (int r = 0; r < P; r++)
-#pragma unroll
-                for (int l = 0; l < 6; l++) X[u][r][l] = make_double2(0.0, 0.0);
+            for (int l = 0; l < kNLink; l++) x[p][l] = make_double2(0.0, 0.0);
 #pragma unroll 1
-        for (int p = 0; p < P; p++)
+        for (int p = 0; p < Q; p++)
+            sample(t + NT * (S::group() + S::G * p), [&](int l, double2 v) {
+#pragma unroll
+                for (int q = 0; q + 1 < Q; q++) x[q][l] = x[q + 1][l];
+                x[Q - 1][l] = v;
+            });
+        if constexpr (S::G == 2)
+            fd_dif2<N>(x, lds, tw, tws);
+        else
+            fd_dif<N, kNLink>(x, tw, tws, t);
+#pragma unroll
+        for (int l = 0; l < kNLink; l++) rows[l * PN + ts] = x[0][l];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < Q; s++)
+    {
+        // fresh indices per pass (as in wave_fft): kept, they fill registers
+        int u = t;
+        if constexpr (P > 1) asm volatile("" : "+v"(u));
+        // bin m = P t + r is FFT index (m + N/2) mod N = P k + r
+        const int k = wave_fft_slot((u + NT / 2) & (NT - 1));
+        const int m = P * u + S::residue(s);
+        if (on) pre(m);
+        wave_fft<NT, S::G * kNLink, S::NTHR, (P > 1)>(lds, opaque(tw), P * tws);
+        double2 d[kNLink];
+#pragma unroll
+        for (int l = 0; l < kNLink; l++) d[l] = rows[l * PN + k];
+        if (s + 1 < Q)
         {
-            fd_samples_to_lds<N, NTHR, P>(c, lds, opaque(pos), posstride, p);
-            tw = opaque(tw);
-            lds_fft<NS, 6, NTHR>(lds, tw, twstride * P);
-#pragma unroll
-            for (int u = 0; u < U; u++)
-            {
-                const int j = t + u * NTHR;
-                // w_N^{p j}; the radix-P rotations are w_P^{p r}
-                const double2 wj = tw[(p * j) * twstride];
-#pragma unroll
-                for (int l = 0; l < 6; l++)
-                {
-                    const double2 v = cmul(lds[l * NS + j], wj);
-#pragma unroll
-                    for (int r = 0; r < P; r++)
-                    {
-                        const double2 w = tw[((p * r) % P) * NS * twstride];
-                        const double2 q = cmul(v, w);
-                        X[u][r][l].x += q.x;
-                        X[u][r][l].y += q.y;
-                    }
-                }
-            }
             __syncthreads();
+            // the next series takes the LDS before this bin's work, so it is
+            // not held in registers across that work
+#pragma unroll
+            for (int l = 0; l < kNLink; l++) rows[l * PN + wave_fft_slot(u)] = x[S::slot(s + 1)][l];
         }
-        // FFT index s = j + NS r, j = t + u NTHR, is output bin
-        // m = (s + N/2) mod N = t + k NTHR with k as below
-#pragma unroll
-        for (int u = 0; u < U; u++)
-#pragma unroll
-            for (int r = 0; r < P; r++)
-            {
-                const int k = (u + U * r + N / (2 * NTHR)) % (N / NTHR);
-#pragma unroll
-                for (int l = 0; l < 6; l++) d[k][l] = make_double2(X[u][r][l].x * inv2N, X[u][r][l].y * inv2N);
-            }
+        if (on) f(s, m, d);
+        if (s + 1 < Q) __syncthreads();
     }
 }
 
-// f(m, d) for every output bin m of this thread, d[l] = link l at bin m
-// as fd_link_spectra leaves it.  Ends with a barrier (TAIL below).  SOA (split shape
-// only): pos is the N-sample structure-of-arrays block (9 rows of N
-// samples) and posstride is unused; else pos is the record table read with
-// stride posstride.
-// pre(m) is called for each bin m before f(m, d) of that bin, as early as
-// the shape allows: in the split shape at the start of the bin's pass,
-// before its transform, so that global loads the caller issues there for
-// bin m are in flight during the FFT stages.  TAIL = false (split shape):
-// no barrier after the last LDS reads; the caller then passes a barrier of
-// its own before anything writes lds again.
-template <int N, int NTHR, bool SPLIT, bool SOA = false, bool TAIL = true, typename Pre, typename F>
-__device__ inline void fd_link_bins(const UcbConst& c, double2* lds, const double* __restrict__ pos, int posstride,
-                                    const double2* __restrict__ tw, int twstride, Pre&& pre, F&& f)
+// exp(-i x) of x = f/f* at template bin m (f = (q + m - N/2)/T,
+// glass_lisa.c:664): the template's own value at bin q (ucb_setup) turned by
+// the few bins between, a small angle, 14 instructions instead of a full
+// sine and cosine per bin (50).  Where N/2 bins are more than 1/64 rad (a
+// T below ~1e7 s for long templates) the angle is evaluated directly.  The
+// reference steps it with a rotation recurrence (glass_lisa.c:403-415),
+// which agrees to ~N ulp.
+template <int N>
+__device__ __forceinline__ void fd_tdi_phase(const UcbConst& c, int m, double& c1, double& s1)
 {
-    static_assert(SPLIT || !SOA, "structure-of-arrays positions: split shape only");
-    // 2048 bins on 512 threads: the split step on two sample pairs per
-    // thread (n = t, t + 512 with partners n + 1024), the odd-bin series in
-    // registers during the even-bin transform; no decimated accumulators
-    // (3% faster than the decimated form, 173 VGPRs instead of ~235)
-    constexpr bool SPLIT2 = !SPLIT && N == 2048 && NTHR == 512;
-    if constexpr (SPLIT2)
+    const double dm = (double)(m - N / 2);
+    if (c.tdx * (N / 2) <= 0.015625)
     {
-        constexpr int H = N / 2, Q = H / NTHR;
-        const double inv2N = 1. / (double)(2 * N);
-        const int t = threadIdx.x;
-        double2 ya[Q][3], yb[Q][3];
-#pragma unroll
-        for (int q = 0; q < Q; q++)
-        {
-            const int n = t + q * NTHR;
-            ucb_slow_sample(c, ucb_sample_time(c.T, c.t0, n, N), pos + (size_t)n * posstride * 9, lds, H, n);
-            const double2 w = tw[n * twstride];
-            ucb_slow_sample_to<false>(c, ucb_sample_time(c.T, c.t0, n + H, N), pos + (size_t)(n + H) * posstride * 9,
-                                      [&](int l, double2 x1) {
-                                          const double2 x0 = lds[l * H + n];
-                                          lds[l * H + n] = make_double2(x0.x + x1.x, x0.y + x1.y);
-                                          const double2 dv = cmul(make_double2(x0.x - x1.x, x0.y - x1.y), w);
-                                          if (l < 3)
-                                          {
-                                              ya[q][0] = ya[q][1];
-                                              ya[q][1] = ya[q][2];
-                                              ya[q][2] = dv;
-                                          }
-                                          else
-                                          {
-                                              yb[q][0] = yb[q][1];
-                                              yb[q][1] = yb[q][2];
-                                              yb[q][2] = dv;
-                                          }
-                                      });
-        }
-        __syncthreads();
-#pragma unroll
-        for (int pass = 0; pass < 2; pass++)
-        {
-            lds_fft<H, 6, NTHR>(lds, opaque(tw), 2 * twstride);
-            double2 d[Q][6];
-#pragma unroll
-            for (int q = 0; q < Q; q++)
-            {
-                // bin m = 2n + pass is FFT index (m + H) mod N, of parity pass
-                const int m = 2 * (t + q * NTHR) + pass;
-                const int sl = ((m + H) & (N - 1)) >> 1;
-#pragma unroll
-                for (int l = 0; l < 6; l++)
-                {
-                    const double2 v = lds[l * H + sl];
-                    d[q][l] = make_double2(v.x * inv2N, v.y * inv2N);
-                }
-            }
-            if (!pass || TAIL) __syncthreads();
-            if (!pass)
-#pragma unroll
-                for (int q = 0; q < Q; q++)
-#pragma unroll
-                    for (int l = 0; l < 3; l++)
-                    {
-                        lds[l * H + t + q * NTHR] = ya[q][l];
-                        lds[(l + 3) * H + t + q * NTHR] = yb[q][l];
-                    }
-#pragma unroll
-            for (int q = 0; q < Q; q++)
-            {
-                const int m = 2 * (t + q * NTHR) + pass;
-                pre(m);
-                f(m, d[q]);
-            }
-            if (!pass) __syncthreads();
-        }
-    }
-    else if constexpr (!SPLIT)
-    {
-        using S = FdShape<N, NTHR>;
-        double2 dl[S::PER][6];
-        fd_link_spectra<N, NTHR>(c, lds, pos, posstride, tw, twstride, dl);
-#pragma unroll
-        for (int k = 0; k < S::PER; k++)
-        {
-            const int m = threadIdx.x + k * NTHR;
-            if (m < N)
-            {
-                pre(m);
-                f(m, dl[k]);
-            }
-        }
+        const double d = dm * c.tdx, z = d * d;
+        const double sd = d * fma(z, fma(z, 1.0 / 120.0, -1.0 / 6.0), 1.0);
+        const double cd = fma(z, fma(z, fma(z, -1.0 / 720.0, 1.0 / 24.0), -0.5), 1.0);
+        c1 = c.ttc * cd - c.tts * sd;
+        s1 = c.tts * cd + c.ttc * sd;
     }
     else
-    {
-        // X[2k] = FFT_H(x[n] + x[n+H]), X[2k+1] = FFT_H((x[n] - x[n+H]) w_N^n),
-        // H = N/2 = NTHR
-        constexpr int H = N / 2;
-        // swizzled LDS layout of the half-length series (conflict-free
-        // Stockham writes) at 1024 bins: 4.5% faster there; at 256 and 512
-        // bins the extra index arithmetic cancels the gain (measured)
-        constexpr bool SW = H == 512;
-        const double inv2N = 1. / (double)(2 * N);
-        const int t = threadIdx.x;
-        const int ts = lds_slot<SW>(t);
-        constexpr int KS = SOA ? N : 1;
-        const double* p0 = SOA ? pos + t : pos + (size_t)t * posstride * 9;
-        const double* p1 = SOA ? pos + t + H : pos + (size_t)(t + H) * posstride * 9;
-        ucb_slow_sample<KS>(c, ucb_sample_time(c.T, c.t0, t, N), p0, lds, H, ts);
-        // links 0-2 and 3-5 of the odd-bin series, shifted in as the
-        // spacecraft loop produces them (l < 3 is known per unrolled link)
-        const double2 w = tw[t * twstride];
-        double2 ya[3], yb[3];
-        ucb_slow_sample_to<false, KS>(c, ucb_sample_time(c.T, c.t0, t + H, N), p1,
-                                  [&](int l, double2 x1) {
-                                      const double2 x0 = lds[l * H + ts];
-                                      lds[l * H + ts] = make_double2(x0.x + x1.x, x0.y + x1.y);
-                                      const double2 dv = cmul(make_double2(x0.x - x1.x, x0.y - x1.y), w);
-                                      if (l < 3)
-                                      {
-                                          ya[0] = ya[1];
-                                          ya[1] = ya[2];
-                                          ya[2] = dv;
-                                      }
-                                      else
-                                      {
-                                          yb[0] = yb[1];
-                                          yb[1] = yb[2];
-                                          yb[2] = dv;
-                                      }
-                                  });
-        __syncthreads();
-#pragma unroll
-        for (int pass = 0; pass < 2; pass++)
-        {
-            // bin m = 2t + pass is FFT index (m + H) mod N, of parity pass
-            const int m = 2 * t + pass;
-            pre(m);
-            lds_fft<H, 6, NTHR, SW>(lds, opaque(tw), 2 * twstride);
-            const int s = lds_slot<SW>(((m + H) & (N - 1)) >> 1);
-            double2 d[6];
-#pragma unroll
-            for (int l = 0; l < 6; l++)
-            {
-                const double2 v = lds[l * H + s];
-                d[l] = make_double2(v.x * inv2N, v.y * inv2N);
-            }
-            if (!pass || TAIL) __syncthreads();
-            if (!pass)
-            {
-                // the odd-bin series takes the LDS before the even bins'
-                // work, so it is not held in registers across that work
-#pragma unroll
-                for (int l = 0; l < 3; l++)
-                {
-                    lds[l * H + ts] = ya[l];
-                    lds[(l + 3) * H + ts] = yb[l];
-                }
-            }
-            f(m, d);
-            if (!pass) __syncthreads();
-        }
-    }
+        sincos_red((c.qd + dm) * c.invT * c.invfstar, &s1, &c1);
 }
 
-template <int N, int NTHR, bool SPLIT, bool SOA = false, typename F>
-__device__ inline void fd_link_bins(const UcbConst& c, double2* lds, const double* __restrict__ pos, int posstride,
-                                    const double2* __restrict__ tw, int twstride, F&& f)
-{
-    fd_link_bins<N, NTHR, SPLIT, SOA>(c, lds, pos, posstride, tw, twstride, [](int) {}, f);
-}
-
-// TDI of template bin m from its six link values d (link order 12, 21, 31,
-// 13, 23, 32).  out: X, Y, Z, A, E.  Trig of f/f* is evaluated directly per
-// bin; the reference steps it with a rotation recurrence
-// (glass_lisa.c:403-415), which agrees to ~N ulp.
+// The prefactor P of a channel P (a exp(-ix) + b), a = d_ij - d_ik and b =
+// d_ji - d_ki, with the 1/(2N) of the link spectra (a power of two):
+//   sangria (glass_lisa.c:645-710): pf [a e^{-2ix} + b e^{-ix}],
+//     pf = 4 sqrt(T) (f/f*) sin(f/f*), so P = pf e^{-ix};
+//   phase, frequency (:458-643): pf [a e^{-3ix} + b e^{-2ix} - a e^{-ix} - b],
+//     pf = sqrt(T) or sqrt(T) 2 f/f*, so P = pf (e^{-2ix} - 1).
 template <int N>
-__device__ inline void fd_tdi(const UcbConst& c, int m, int fmt, const double2* d, double2* out)
+__device__ __forceinline__ double2 fd_tdi_prefactor(const UcbConst& c, int m, int fmt, double c1, double s1)
 {
-    const double2 d12 = d[0], d21 = d[1], d31 = d[2], d13 = d[3], d23 = d[4], d32 = d[5];
-    // f = (q + m - N/2)/T (glass_lisa.c:664); amplitude path, so the
-    // reciprocal is folded in
-    const double f = ((double)(c.q + m - N / 2)) * c.invT;
-    const double fonfs = f * c.invfstar;
-    double s1, c1;
-    sincos_red(fonfs, &s1, &c1);
-    const double c2 = 2. * c1 * c1 - 1.0, s2 = 2. * s1 * c1;
-    const double sqT = c.sqT;
-    // link combinations a = d_ij - d_ik, b = d_ji - d_ki per channel
-    const double2 aX = make_double2(d12.x - d13.x, d12.y - d13.y), bX = make_double2(d21.x - d31.x, d21.y - d31.y);
-    const double2 aY = make_double2(d23.x - d21.x, d23.y - d21.y), bY = make_double2(d32.x - d12.x, d32.y - d12.y);
-    const double2 aZ = make_double2(d31.x - d32.x, d31.y - d32.y), bZ = make_double2(d13.x - d23.x, d13.y - d23.y);
-    double2 X, Y, Z;
+    constexpr double inv2N = 1. / (double)(2 * N);
+    const double x = (c.qd + (double)(m - N / 2)) * c.tdx;
     if (fmt == TDI_SANGRIA)
     {
-        // glass_lisa.c:645-710: pf [a e^{-2ix} + b e^{-ix}], pf = 4 sqrt(T) (f/f*) sin(f/f*)
-        const double pf = f * (4.0 * c.invfstar * sqT) * s1;
-        auto ch = [&](double2 a, double2 b) {
-            return make_double2(pf * (a.x * c2 + a.y * s2 + b.x * c1 + b.y * s1),
-                                pf * (a.y * c2 - a.x * s2 + b.y * c1 - b.x * s1));
-        };
-        X = ch(aX, bX);
-        Y = ch(aY, bY);
-        Z = ch(aZ, bZ);
+        const double pf = x * (4.0 * inv2N * c.sqT) * s1;
+        return make_double2(pf * c1, -pf * s1);
     }
-    else
-    {
-        // glass_lisa.c:458-643: pf [a e^{-3ix} + b e^{-2ix} - a e^{-ix} - b],
-        // pf = sqrt(T) ("phase") or sqrt(T) 2 f/f* ("frequency")
-        const double c3 = 2. * c1 * c2 - c1, s3 = 2. * s1 * c2 + s1;
-        const double pf = (fmt == TDI_PHASE) ? sqT : sqT * (2. * fonfs);
-        auto ch = [&](double2 a, double2 b) {
-            return make_double2(pf * (a.x * c3 + a.y * s3 + b.x * c2 + b.y * s2 - a.x * c1 - a.y * s1 - b.x),
-                                pf * (a.y * c3 - a.x * s3 + b.y * c2 - b.x * s2 - a.y * c1 + a.x * s1 - b.y));
-        };
-        X = ch(aX, bX);
-        Y = ch(aY, bY);
-        Z = ch(aZ, bZ);
-    }
+    const double pf = -2.0 * inv2N * c.sqT * s1 * (fmt == TDI_PHASE ? 1.0 : 2.0 * x);
+    return make_double2(pf * s1, pf * c1);
+}
+
+// The channel combinations of the series (kNLink order): aX = d12 - d13, bX
+// = d21 - d31, aY = d23 - d21, bY = d32 - d12, aZ = d31 - d32, bZ = d13 - d23.
+// TDI of template bin m from its five series values.  out: X, Y, Z, A, E.
+// From exp(-ix) and the prefactor P of the bin.
+__device__ __forceinline__ void fd_tdi_xyz(double c1, double s1, double2 P, const double2* d, double2& X, double2& Y,
+                                           double2& Z)
+{
+    auto ch = [&](double ax, double ay, double bx, double by) {
+        const double vx = fma(ax, c1, fma(ay, s1, bx)), vy = fma(ay, c1, fma(-ax, s1, by));
+        return make_double2(vx * P.x - vy * P.y, vx * P.y + vy * P.x);
+    };
+    X = ch(d[0].x - d[3].x, d[0].y - d[3].y, d[1].x - d[2].x, d[1].y - d[2].y);
+    Y = ch(-d[1].x, -d[1].y, d[4].x - d[0].x, d[4].y - d[0].y);
+    Z = ch(d[2].x - d[4].x, d[2].y - d[4].y, d[3].x, d[3].y);
+}
+
+template <int N>
+__device__ __forceinline__ void fd_tdi(const UcbConst& c, int m, int fmt, const double2* d, double2* out)
+{
+    double s1, c1;
+    fd_tdi_phase<N>(c, m, c1, s1);
+    const double2 P = fd_tdi_prefactor<N>(c, m, fmt, c1, s1);
+    double2 X, Y, Z;
+    fd_tdi_xyz(c1, s1, P, d, X, Y, Z);
     double2 A = make_double2((Z.x - X.x) * kSQRT1_2, (Z.y - X.y) * kSQRT1_2);
     double2 E = make_double2((X.x - 2 * Y.x + Z.x) * kINVSQ6, (X.y - 2 * Y.y + Z.y) * kINVSQ6);
     if (fmt == TDI_PHASE)

@@ -8,7 +8,7 @@
 // exponent, radix 4 for the rest.
 // Each stage reads every butterfly's inputs into registers, synchronises,
 // then writes the outputs into the same buffer, so a single LDS buffer
-// suffices (96*N bytes for the six link series of a template).
+// suffices.  Transforms of up to 512 points that one wave holds: wave_fft.
 //
 // Twiddles come from a table tw[k] = exp(-2 pi i k / NTW) of NTW entries
 // (NTW a multiple of N: 4096 or 16384 for N = 2^a, 12288 for N = 3*2^a) built once
@@ -34,6 +34,27 @@ __device__ inline double2 cmul(double2 a, double2 b)
 // origin would turn every table read into a flat load, which the hardware
 // counts against the LDS wait counter as well, so each FFT stage's LDS
 // wait would also wait for its twiddle loads.
+// Loads through a pointer that came out of memory: global ones, which the
+// compiler cannot infer there (generic loads are flat and wait with the LDS's).
+__device__ __forceinline__ double2 gload(const double2* p)
+{
+    typedef double v2 __attribute__((ext_vector_type(2)));
+    const v2 v = *(const __attribute__((address_space(1))) v2*)p;
+    return make_double2(v.x, v.y);
+}
+__device__ __forceinline__ double gload(const double* p)
+{
+    return *(const __attribute__((address_space(1))) double*)p;
+}
+__device__ __forceinline__ void gstore(double2* p, double2 x)
+{
+    typedef double v2 __attribute__((ext_vector_type(2)));
+    v2 v;
+    v.x = x.x;
+    v.y = x.y;
+    *(__attribute__((address_space(1))) v2*)p = v;
+}
+
 template <typename T>
 __device__ inline const T* opaque(const T* p)
 {
@@ -42,35 +63,35 @@ __device__ inline const T* opaque(const T* p)
     return (const T*)g;
 }
 
-// LDS slot of complex element i of a buffer transformed with the swizzled
-// layout (SWZ = true below): bits 0-3 of i XOR-ed with bits 2-5 and bit 0
-// also with bit 3.  The map is linear over GF(2) (slot(a ^ b) = slot(a) ^
-// slot(b)) and a bijection of every aligned block of 64 elements.  With it
-// the reads of consecutive elements stay conflict-free and so do the
-// strided writes of the first Stockham stages (64 bytes apart per lane at
-// Ns = 1, runs of four lanes 256 bytes apart at Ns = 4), which in the plain
-// layout put 2-4 lanes of every 8 or 16 on the same LDS banks.  Linearity
-// lets a butterfly swizzle its base index once: its R elements sit at
-// disjoint-bit offsets m*span, whose slots are compile-time constants.
-__device__ __forceinline__ int lds_swz(int i) { return i ^ ((i >> 2) & 15) ^ ((i >> 3) & 1); }
-template <bool SWZ>
-__device__ __forceinline__ int lds_slot(int i)
-{
-    return SWZ ? lds_swz(i) : i;
-}
-// Slot of a + c for a and c with no set bit in common, from the slot of a.
-template <bool SWZ>
-__device__ __forceinline__ int lds_slot_add(int slot_a, int c)
-{
-    return SWZ ? (slot_a ^ lds_swz(c)) : slot_a + c;
-}
-
-// Radix-R butterfly (R = 2, 3, 4) of twiddled inputs v into y:
+// Radix-R butterfly (R = 2, 3, 4, 8) of twiddled inputs v into y:
 // y[m] = sum_q v[q] exp(-2 pi i q m / R).
 template <int R>
 __device__ inline void radix_butterfly(const double2 (&v)[R], double2 (&y)[R])
 {
-    if constexpr (R == 3)
+    if constexpr (R == 8)
+    {
+        const double h = 0.70710678118654752440;
+        double2 e[4], o[4], ye[4], yo[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+        {
+            e[q] = make_double2(v[q].x + v[q + 4].x, v[q].y + v[q + 4].y);
+            o[q] = make_double2(v[q].x - v[q + 4].x, v[q].y - v[q + 4].y);
+        }
+        // odd outputs: o[q] times exp(-2 pi i q/8)
+        o[1] = make_double2(h * (o[1].x + o[1].y), h * (o[1].y - o[1].x));
+        o[2] = make_double2(o[2].y, -o[2].x);
+        o[3] = make_double2(h * (o[3].y - o[3].x), -h * (o[3].x + o[3].y));
+        radix_butterfly<4>(e, ye);
+        radix_butterfly<4>(o, yo);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+        {
+            y[2 * q] = ye[q];
+            y[2 * q + 1] = yo[q];
+        }
+    }
+    else if constexpr (R == 3)
     {
         // w = exp(-2 pi i/3): y1 = a0 - s/2 - i(sqrt3/2) d, y2 = conj rotation
         const double h3 = 0.86602540378443864676;
@@ -124,11 +145,10 @@ __device__ __forceinline__ void wave_lds_sync()
 // wave, the same wave as in the neighbouring stages (lds_fft decides), so
 // the stage's two synchronisations are wave-level; LAST: its final one is a
 // workgroup barrier all the same (the caller reads across waves after it).
-template <int N, int NL, int R, int NTHR, bool SWZ = false, bool WAVE = false, bool LAST = true>
+template <int N, int NL, int R, int NTHR, bool WAVE = false, bool LAST = true>
 __device__ __forceinline__ void stockham_stage(double2* buf, int Ns, const double2* __restrict__ tw, int twstride,
                                                int tid = threadIdx.x)
 {
-    static_assert(!SWZ || (N % 64 == 0 && R != 3), "swizzled layout: power-of-two N >= 64");
     constexpr int NB = NL * (N / R);                 // butterflies in the stage
     constexpr int PER = (NB + NTHR - 1) / NTHR;      // per thread
     constexpr bool SAMEJ = NTHR % (N / R) == 0;
@@ -154,9 +174,8 @@ __device__ __forceinline__ void stockham_stage(double2* buf, int Ns, const doubl
         if (NB % NTHR == 0 || b < NB)
         {
             int l = b / (N / R), j = b % (N / R);
-            const int sj = lds_slot<SWZ>(j);  // j < N/R: disjoint from m*(N/R)
 #pragma unroll
-            for (int m = 0; m < R; m++) v[p][m] = buf[l * N + lds_slot_add<SWZ>(sj, m * (N / R))];
+            for (int m = 0; m < R; m++) v[p][m] = buf[l * N + j + m * (N / R)];
         }
     }
     if constexpr (WAVE)
@@ -176,10 +195,9 @@ __device__ __forceinline__ void stockham_stage(double2* buf, int Ns, const doubl
                 for (int m = 1; m < R; m++) v[p][m] = cmul(v[p][m], w[SAMEJ ? 0 : p][m - 1]);
             double2 y[R];
             radix_butterfly<R>(v[p], y);
-            // base has no bits in [log2 Ns, log2 (R Ns)), where m*Ns lives
-            const int sb = lds_slot<SWZ>((j / Ns) * Ns * R + k);
+            const int base = (j / Ns) * Ns * R + k;
 #pragma unroll
-            for (int m = 0; m < R; m++) buf[l * N + lds_slot_add<SWZ>(sb, m * Ns)] = y[m];
+            for (int m = 0; m < R; m++) buf[l * N + base + m * Ns] = y[m];
         }
     }
     if constexpr (WAVE && !LAST)
@@ -189,23 +207,14 @@ __device__ __forceinline__ void stockham_stage(double2* buf, int Ns, const doubl
 }
 
 // Full forward FFT of NL length-N series in LDS. twstride = NTW / N.
-// SWZ: element n of series l lives at buf[l*N + lds_swz(n)] on entry and
-// on return.
-template <int N, int NL, int NTHR, bool SWZ = false>
+template <int N, int NL, int NTHR>
 __device__ __forceinline__ void lds_fft(double2* buf, const double2* __restrict__ tw, int twstride)
 {
     constexpr bool R3 = N % 3 == 0;
     constexpr int P2 = R3 ? N / 3 : N;
     static_assert((P2 & (P2 - 1)) == 0 && N >= 4, "N = 2^a or 3*2^a");
     constexpr int LOG2 = __builtin_ctz(P2);
-    int tid = threadIdx.x;
-    if constexpr (SWZ)
-    {
-        // a fresh thread index per transform: its swizzled addresses are
-        // not shared with another transform's, so none stays live between
-        asm volatile("" : "+v"(tid));
-        tid &= 1023;  // the range threadIdx.x has
-    }
+    const int tid = threadIdx.x;
     int Ns = 1;
     if (R3)
     {
@@ -214,7 +223,7 @@ __device__ __forceinline__ void lds_fft(double2* buf, const double2* __restrict_
     }
     if (LOG2 & 1)
     {
-        stockham_stage<N, NL, 2, NTHR, SWZ>(buf, Ns, tw, twstride, tid);
+        stockham_stage<N, NL, 2, NTHR>(buf, Ns, tw, twstride, tid);
         Ns *= 2;
     }
     // radix-4 stages only, N/4 <= 64 butterflies per series: butterfly b =
@@ -226,11 +235,121 @@ __device__ __forceinline__ void lds_fft(double2* buf, const double2* __restrict_
     for (int s = 0; s < LOG2 / 2; s++)
     {
         if (s == LOG2 / 2 - 1)
-            stockham_stage<N, NL, 4, NTHR, SWZ, WAVE, true>(buf, Ns, tw, twstride, tid);
+            stockham_stage<N, NL, 4, NTHR, WAVE, true>(buf, Ns, tw, twstride, tid);
         else
-            stockham_stage<N, NL, 4, NTHR, SWZ, WAVE, false>(buf, Ns, tw, twstride, tid);
+            stockham_stage<N, NL, 4, NTHR, WAVE, false>(buf, Ns, tw, twstride, tid);
         Ns *= 4;
     }
+}
+
+// Transforms of up to 512 points, each held by one wave: NL series of N
+// points in LDS, N = 16..512, in the padded layout below.  A unit is 512
+// points (512/N series); a wave takes a unit through all stages, eight
+// points a lane, so the stages of a transform need no workgroup barrier and
+// only three passes go through LDS at 512 points (radix 8; radix 4 takes
+// five).  What bounds the fused template kernels is LDS traffic and vector
+// issue in turn: with radix 4 and barriers the LDS was active 55% of the
+// time, a quarter of it bank conflicts.
+//
+// Padded layout: point n of series l at l * wave_fft_stride(N) + n + n/8.
+// The writes of a radix-8 stage are 8 points apart (9 slots: eight lanes on
+// eight different 16-byte columns), the other accesses run along the lanes;
+// and all eight slots of a butterfly are constants away from the first, so
+// they are instruction offsets.
+__host__ __device__ constexpr int wave_fft_slot(int n) { return n + (n >> 3); }
+__host__ __device__ constexpr int wave_fft_stride(int N) { return N + N / 8; }
+
+template <int N, int NL, int R, int NTHR>
+__device__ __forceinline__ void wave_fft_stage(double2* buf, int Ns, const double2* __restrict__ tw, int twstride,
+                                               int unit, int lane)
+{
+    constexpr int SPW = 512 / N;      // series in a unit
+    constexpr int NB = N / R;         // butterflies in a series
+    constexpr int PER = 8 / R;        // butterflies a lane
+    constexpr int PN = wave_fft_stride(N);
+    double2 v[PER][R];
+    double2 w[PER][R - 1];
+    if (Ns > 1)
+#pragma unroll
+        for (int p = 0; p < PER; p++)
+        {
+            const int k = ((lane + 64 * p) % NB) % Ns;
+            const int step = k * twstride * (N / (R * Ns));
+#pragma unroll
+            for (int m = 1; m < R; m++) w[p][m - 1] = tw[m * step];
+        }
+#pragma unroll
+    for (int p = 0; p < PER; p++)
+    {
+        const int b = lane + 64 * p, l = unit * SPW + b / NB, j = b % NB;
+        if (NL % SPW == 0 || l < NL)
+        {
+            // slot(j + m NB) = slot(j) + slot(m NB): j < NB, and NB is 4 or
+            // a multiple of 8
+            const double2* src = buf + l * PN + wave_fft_slot(j);
+#pragma unroll
+            for (int m = 0; m < R; m++) v[p][m] = src[wave_fft_slot(m * NB)];
+        }
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int p = 0; p < PER; p++)
+    {
+        const int b = lane + 64 * p, l = unit * SPW + b / NB, j = b % NB;
+        if (NL % SPW == 0 || l < NL)
+        {
+            if (Ns > 1)
+#pragma unroll
+                for (int m = 1; m < R; m++) v[p][m] = cmul(v[p][m], w[p][m - 1]);
+            double2 y[R];
+            radix_butterfly<R>(v[p], y);
+            const int base = (j / Ns) * Ns * R + j % Ns;
+            // likewise: base has no bits in [log2 Ns, log2 R Ns), and its
+            // bits below Ns and those of m Ns share no octet unless Ns is 1 or
+            // 4, where both stay within one
+            double2* dst = buf + l * PN + wave_fft_slot(base);
+#pragma unroll
+            for (int m = 0; m < R; m++) dst[wave_fft_slot(m * Ns)] = y[m];
+        }
+    }
+    wave_lds_sync();
+}
+
+// All units of NL series.  The caller has synchronised the input; ends with
+// a workgroup barrier.  TIGHT: a stage's twiddles are loaded in that stage
+// and not before (28 registers instead of up to 56), for callers that hold
+// other series meanwhile.
+template <int N, int NL, int NTHR, bool TIGHT = false>
+__device__ __forceinline__ void wave_fft(double2* buf, const double2* __restrict__ tw, int twstride)
+{
+    static_assert(N >= 16 && N <= 512 && (N & (N - 1)) == 0 && NTHR % 64 == 0, "powers of two, 16 to 512 points");
+    constexpr int SPW = 512 / N, UNITS = (NL + SPW - 1) / SPW, NW = NTHR / 64;
+    constexpr int LOG2 = __builtin_ctz(N);
+    // radix 8 first, then one or two of radix 4
+    constexpr int N4 = LOG2 % 3 == 0 ? 0 : (LOG2 % 3 == 2 ? 1 : 2), N8 = (LOG2 - 2 * N4) / 3;
+    // a fresh lane index per transform: its addresses are not shared with
+    // another transform's, so none stays live between them
+    int lane = threadIdx.x & 63;
+    if constexpr (TIGHT) asm volatile("" : "+v"(lane));
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+#pragma unroll 1
+    for (int u = wave; u < UNITS; u += NW)
+    {
+        int Ns = 1;
+#pragma unroll
+        for (int s = 0; s < N8; s++)
+        {
+            wave_fft_stage<N, NL, 8, NTHR>(buf, Ns, TIGHT ? opaque(tw) : tw, twstride, u, lane);
+            Ns *= 8;
+        }
+#pragma unroll
+        for (int s = 0; s < N4; s++)
+        {
+            wave_fft_stage<N, NL, 4, NTHR>(buf, Ns, TIGHT ? opaque(tw) : tw, twstride, u, lane);
+            Ns *= 4;
+        }
+    }
+    __syncthreads();
 }
 
 // One Stockham stage of radix R from src to dst (two buffers, any memory:

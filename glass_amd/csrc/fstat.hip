@@ -164,14 +164,14 @@ template <int N, int NTHR>
 __global__ __launch_bounds__(NTHR) void fstat_kernel(const int* __restrict__ list, const int* __restrict__ count,
                                                      FstatDev D, Cells C)
 {
-    using S = FdShape<N, NTHR>;
-    __shared__ double2 lds[S::LDS];
+    constexpr int PER = (N + NTHR - 1) / NTHR;  // bins per thread
+    __shared__ double2 lds[FdShape<N>::LDS];
     if ((int)blockIdx.x >= *count) return;
     const int e = list[blockIdx.x];
     const double f0 = C.cell[(size_t)e * 4], fdot = C.cell[(size_t)e * 4 + 1];
     const double theta = C.cell[(size_t)e * 4 + 2], phi = C.cell[(size_t)e * 4 + 3];
     const long q = (long)(f0 * D.T);
-    double2 hx[S::PER][4], ha[S::PER][4], he[S::PER][4];
+    double2 hx[PER][4], ha[PER][4], he[PER][4];
     // the four filters' constants, one lane each (the same code on four lanes
     // of the first wave: one setup's latency instead of four in turn)
     __shared__ UcbConst sc4[4];
@@ -186,19 +186,15 @@ __global__ __launch_bounds__(NTHR) void fstat_kernel(const int* __restrict__ lis
     for (int fi = 0; fi < 4; fi++)
     {
         const UcbConst& k = sc4[fi];
-        double2 dl[S::PER][6];
-        fd_link_spectra<N, NTHR>(k, lds, D.pos, kPosNF / N, D.tw, kTwN / N, dl);
-#pragma unroll
-        for (int kk = 0; kk < S::PER; kk++)
-        {
-            const int m = threadIdx.x + kk * NTHR;
-            if (m >= N) continue;
-            double2 v[5];
-            fd_tdi<N>(k, m, D.fmt, dl[kk], v);
-            hx[kk][fi] = v[0];
-            ha[kk][fi] = v[3];
-            he[kk][fi] = v[4];
-        }
+        if (fi) __syncthreads();  // the last filter's LDS reads
+        fd_link_bins<N, false>(
+            HeldConst{k}, lds, D.pos, kPosNF / N, D.tw, kTwN / N, [](int) {}, [&](int kk, int m, const double2* dl) {
+                double2 v[5];
+                fd_tdi<N>(k, m, D.fmt, dl, v);
+                hx[kk][fi] = v[0];
+                ha[kk][fi] = v[3];
+                he[kk][fi] = v[4];
+            });
     }
     // projections and Gram sums (get_N, get_M), the reference's term order
     double nx[4] = {0, 0, 0, 0}, nae[4] = {0, 0, 0, 0}, mx[10], mae[10];
@@ -207,9 +203,9 @@ __global__ __launch_bounds__(NTHR) void fstat_kernel(const int* __restrict__ lis
     {
 #pragma clang fp contract(off)
 #pragma unroll
-        for (int kk = 0; kk < S::PER; kk++)
+        for (int kk = 0; kk < PER; kk++)
         {
-            const int m = threadIdx.x + kk * NTHR;
+            const int m = FdShape<N>::bin(kk);
             const long kb = qo + m - N / 2;
             if (m >= N || !(kb > 0 && kb < D.NFFT)) continue;
             const double c = D.C00[kb];

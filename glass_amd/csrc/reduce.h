@@ -1,66 +1,32 @@
-// reduce.h -- deterministic FP64 block reductions (wave64 shuffles + LDS).
+// reduce.h -- deterministic FP64 block reductions (DPP within a wave, then LDS).
 #pragma once
 #include <hip/hip_runtime.h>
 
 namespace glass {
 
+// v + (v of the lane a DPP control names, 0 where it names none).
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ double dpp_add(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+    return v + __hiloint2double(hi, lo);
+}
+
+// Sum over the wave, the same in every lane: shifts within the rows of 16
+// lanes, then the rows' sums handed on (18 vector instructions, no LDS; the
+// six exchanges through LDS they replace waited for each other).
 __device__ inline double wave_sum(double v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    return v;  // valid in lane 0
-}
-
-// The least power of two >= k (k >= 1).  Written as a loop, and used only
-// to initialise constexpr variables, so it is always evaluated at compile
-// time: a recursive helper called at run time would make the calling kernel's
-// stack size unbounded.
-constexpr int pow2_at_least(int k)
-{
-    int p = 1;
-    while (p < k) p *= 2;
-    return p;
-}
-
-// One exchange step at distance D of wave_sum_transpose with N values left.
-template <int D, int N, int P>
-__device__ __forceinline__ void wave_sum_transpose_step(double (&a)[P], int lane)
-{
-    if constexpr (N > 1)
-    {
-        constexpr int H = N / 2;
-        const bool up = (lane & D) != 0;
-#pragma unroll
-        for (int i = 0; i < H; i++)
-        {
-            const double send = up ? a[i] : a[i + H];
-            const double keep = up ? a[i + H] : a[i];
-            a[i] = keep + __shfl_xor(send, D, 64);
-        }
-    }
-    else
-        a[0] += __shfl_xor(a[0], D, 64);
-    if constexpr (D > 1) wave_sum_transpose_step<D / 2, (N > 1 ? N / 2 : 1), P>(a, lane);
-}
-
-// K per-lane values summed over the wave by transposition: at each exchange
-// step (partner lane ^ d, d = 32, 16, ...) a lane keeps half of its values,
-// the lower half where bit d of the lane is clear, and adds the partner's
-// copies of them; with one value left, the remaining steps are plain
-// butterflies.  K values padded to P = 2^p cost P - 1 double shuffles (63
-// for 45 values against 270 for 45 separate tree sums).  Lane L returns the
-// sum of value index L / (64 / P) (every lane of that group holds it).
-// Fixed order: reproducible run to run.
-template <int K>
-__device__ inline double wave_sum_transpose(const double (&v)[K])
-{
-    static_assert(K >= 1 && K <= 64, "at most 64 values");
-    constexpr int P = pow2_at_least(K);
-    double a[P];
-#pragma unroll
-    for (int i = 0; i < P; i++) a[i] = i < K ? v[i] : 0.0;
-    wave_sum_transpose_step<32, P, P>(a, threadIdx.x & 63);
-    return a[0];
+    v = dpp_add<0x111>(v);       // row_shr:1
+    v = dpp_add<0x112>(v);       // row_shr:2
+    v = dpp_add<0x114>(v);       // row_shr:4
+    v = dpp_add<0x118>(v);       // row_shr:8: lane 15 of each row has its sum
+    v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
+    return __hiloint2double(hi, lo);
 }
 
 // K sums over the block at once: each wave's tree sum of each value, one

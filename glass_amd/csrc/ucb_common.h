@@ -42,11 +42,16 @@ struct UcbConst
     double halfd2;  // 0.5*d2fdt2
     double DPr, DPi, DCr, DCi;
     double k[3];
-    double ep[6], ec[6];  // symmetric tensors: xx, yy, zz, xy, xz, yz
+    double ua[3], va[2], ka[3];  // u, v (v_z = 0) and k over the arm length L
+    double f0h, dfh, d2h;        // f0, dfdt, d2fdt2/2 over 2 f*
+    double aevq;                 // aevc/4
     double invfstar, fstar, invL;
     double sqT, invT;  // sqrt(T), 1/T (TDI prefactor and bin frequency)
+    double qd;               // q
+    double tdx, ttc, tts;    // f/f* per bin, cos and sin of f/f* at bin q (fd_tdi)
     long q;
     int np;
+    int wide;  // transfer-function arguments above 1.75 (sinc_wide)
 };
 
 // glass_ucb_waveform.c:804-837 + LISA_polarization_tensor (glass_lisa.c:1566-1596)
@@ -82,116 +87,138 @@ __host__ __device__ inline void ucb_setup(const double* p, int np, double T, dou
     double sinth = sqrt(1.0 - costh * costh);
     double cosph = cos(phi), sinph = sin(phi);
     double u0 = costh * cosph, u1 = costh * sinph, u2 = -sinth;
-    double v0 = sinph, v1 = -cosph, v2 = 0.;
+    double v0 = sinph, v1 = -cosph;
     c.k[0] = -sinth * cosph;
     c.k[1] = -sinth * sinph;
     c.k[2] = -costh;
-    c.ep[0] = v0 * v0 - u0 * u0;  c.ec[0] = u0 * v0 + v0 * u0;
-    c.ep[1] = v1 * v1 - u1 * u1;  c.ec[1] = u1 * v1 + v1 * u1;
-    c.ep[2] = v2 * v2 - u2 * u2;  c.ec[2] = u2 * v2 + v2 * u2;
-    c.ep[3] = v0 * v1 - u0 * u1;  c.ec[3] = u0 * v1 + v0 * u1;
-    c.ep[4] = v0 * v2 - u0 * u2;  c.ec[4] = u0 * v2 + v0 * u2;
-    c.ep[5] = v1 * v2 - u1 * u2;  c.ec[5] = u1 * v2 + v1 * u2;
     c.fstar = fstar;
     c.invfstar = 1. / fstar;
     c.invL = 1. / L;
     c.sqT = sqrt(T);
     c.invT = 1. / T;
+    c.ua[0] = u0 * c.invL;  c.ua[1] = u1 * c.invL;  c.ua[2] = u2 * c.invL;
+    c.va[0] = v0 * c.invL;  c.va[1] = v1 * c.invL;
+    for (int i = 0; i < 3; i++) c.ka[i] = c.k[i] * c.invL;
+    // times reach t0 + T and a light travel time of 1 AU beyond
+    const double tm = fabs(t0) + T + 1000.0;
+    c.wide = sinc_wide((fabs(c.f0) + (fabs(c.dfdt) + fabs(c.halfd2) * tm) * tm) * c.invfstar);
+    c.f0h = 0.5 * c.f0 * c.invfstar;
+    c.dfh = 0.5 * c.dfdt * c.invfstar;
+    c.d2h = 0.5 * c.halfd2 * c.invfstar;
+    c.aevq = 0.25 * c.aevc;
+    c.qd = (double)c.q;
+    c.tdx = c.invT * c.invfstar;
+    sincos_red(c.qd * c.invT * c.invfstar, &c.tts, &c.ttc);
 }
 
-// r^T E r for a symmetric 3x3 tensor stored as xx,yy,zz,xy,xz,yz
-__device__ inline double quad3(const double* E, double a, double b, double cc)
-{
-    return E[0] * a * a + E[1] * b * b + E[2] * cc * cc + 2.0 * (E[3] * a * b + E[4] * a * cc + E[5] * b * cc);
-}
-
-// One slow-series sample of the six links at time t: out(l, value) receives
-// link l in the order 12, 21, 31, 13, 23, 32.
+// One slow-series sample at time t: out(l, value) receives the links 12, 21,
+// 31, 13, 32 (l = 0..4, a compile-time constant once inlined) less link 23.
 // pos: spacecraft positions x1,x2,x3,y1,y2,y3,z1,z2,z3 at t (metres), KS
 // doubles apart (1 in a sample record, N in a structure-of-arrays table).
 // glass_ucb_waveform.c:843-936, LISA_detector_tensor glass_lisa.c:1521-1564.
-// The loop runs over the sending spacecraft i; its two links (i,j) share
-// xi_i, arg2_i and the frequency at spacecraft i.  UNROLL unrolls it so that
-// l is a compile-time index (values may then stay in registers).
-template <bool UNROLL, int KS = 1, typename Out>
-__device__ inline void ucb_slow_sample_to(const UcbConst& c, double t, const double* __restrict__ pos, Out&& out)
+//
+// The vector issue rate bounds this code, so the sample is arranged for few
+// instructions (about 400; 850 before, which with fd_tdi_phase took 130,042
+// fused 512-bin evaluations from 3.12 to 2.65 ms, 74,247 of 256 bins from
+// 0.93 to 0.77 ms and 23,671 of 2048 bins from 3.87 to 2.96 ms):
+//  * r.E.r of the rank-two polarisation tensors from the projections on u
+//    and v: d+ = (r.v)^2 - (r.u)^2, dx = 2 (r.u)(r.v); the arm's d+ DP + dx DC
+//    is shared by its two links;
+//  * a link is T1 exp(i arg2) [sinc(arg1) exp(-i arg1)]: one full-range sine
+//    and cosine per spacecraft instead of one per link, and the bracket, of
+//    small argument, from two polynomials without range reduction;
+//  * the spacecraft unrolled, no selects, each polynomial coefficient set
+//    once for all arguments that use it.
+template <int KS = 1, typename Out>
+__device__ __forceinline__ void ucb_slow_sample_to(const UcbConst& c, double t, const double* __restrict__ pos,
+                                                   Out&& out)
 {
-    const double x1 = pos[0], x2 = pos[KS], x3 = pos[2 * KS];
-    const double y1 = pos[3 * KS], y2 = pos[4 * KS], y3 = pos[5 * KS];
-    const double z1 = pos[6 * KS], z2 = pos[7 * KS], z3 = pos[8 * KS];
-
-    // unit arm vectors (amplitude path)
-    const double r12a = (x2 - x1) * c.invL, r12b = (y2 - y1) * c.invL, r12c = (z2 - z1) * c.invL;
-    const double r13a = (x3 - x1) * c.invL, r13b = (y3 - y1) * c.invL, r13c = (z3 - z1) * c.invL;
-    const double r23a = (x3 - x2) * c.invL, r23b = (y3 - y2) * c.invL, r23c = (z3 - z2) * c.invL;
-    const double dp12 = quad3(c.ep, r12a, r12b, r12c), dc12 = quad3(c.ec, r12a, r12b, r12c);
-    const double dp13 = quad3(c.ep, r13a, r13b, r13c), dc13 = quad3(c.ec, r13a, r13b, r13c);
-    const double dp23 = quad3(c.ep, r23a, r23b, r23c), dc23 = quad3(c.ec, r23a, r23b, r23c);
-    const double k12 = c.k[0] * r12a + c.k[1] * r12b + c.k[2] * r12c;
-    const double k13 = c.k[0] * r13a + c.k[1] * r13b + c.k[2] * r13c;
-    const double k23 = c.k[0] * r23a + c.k[1] * r23b + c.k[2] * r23c;
+    double x[3], y[3], z[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+    {
+        x[i] = pos[i * KS];
+        y[i] = pos[(3 + i) * KS];
+        z[i] = pos[(6 + i) * KS];
+    }
+    double a2[3], hf[3], ae[3];
     double dft;
     {
 #pragma clang fp contract(off)
         dft = c.df * t;
     }
-#pragma unroll(UNROLL ? 3 : 1)
+#pragma unroll
     for (int i = 0; i < 3; i++)
     {
-        const double px = i == 0 ? x1 : (i == 1 ? x2 : x3);
-        const double py = i == 0 ? y1 : (i == 1 ? y2 : y3);
-        const double pz = i == 0 ? z1 : (i == 1 ? z2 : z3);
-        double a2, fon, ae;
+        double xi;
         {
 #pragma clang fp contract(off)
             // the quotient by c, as IEEE division gives it (div_by_recip)
-            double kdotx = div_by_recip(px * c.k[0] + py * c.k[1] + pz * c.k[2], kCLIGHT, kInvCLIGHT);
-            double xi = t - kdotx;
-            double fi = c.f0;
-            a2 = c.pi2f0 * xi - c.phi0 - dft;
-            ae = 1.0;
-            if (c.np > 7)
-            {
-                fi += c.dfdt * xi;
-                a2 += c.pidfdt * xi * xi;
-                ae += c.aevc * xi;
-            }
-            if (c.np > 8)
-            {
-                fi += c.halfd2 * xi * xi;
-                a2 += c.pid2 * xi * xi * xi;
-            }
-            fon = fi * c.invfstar;
+            const double kdotx = div_by_recip(x[i] * c.k[0] + y[i] * c.k[1] + z[i] * c.k[2], kCLIGHT, kInvCLIGHT);
+            xi = t - kdotx;
+            a2[i] = c.pi2f0 * xi - c.phi0 - dft;
+            a2[i] += c.pidfdt * xi * xi;
+            if (c.np > 8) a2[i] += c.pid2 * xi * xi * xi;
         }
-        // links (i, j) of spacecraft i: kdotr antisymmetric, d+/dx symmetric
-        const double kra = i == 0 ? k12 : (i == 1 ? -k12 : -k13);
-        const double krb = i == 0 ? k13 : (i == 1 ? k23 : -k23);
-        const double dpa = i == 0 ? dp12 : (i == 1 ? dp12 : dp13);
-        const double dpb = i == 0 ? dp13 : (i == 1 ? dp23 : dp23);
-        const double dca = i == 0 ? dc12 : (i == 1 ? dc12 : dc13);
-        const double dcb = i == 0 ? dc13 : (i == 1 ? dc23 : dc23);
+        // half the frequency over f*, and a quarter of the amplitude
+        hf[i] = fma(c.dfh, xi, c.f0h);
+        if (c.np > 8) hf[i] = fma(c.d2h * xi, xi, hf[i]);
+        ae[i] = fma(c.aevq, xi, 0.25);
+    }
+    // arms 12, 13, 23: k.r and T1 = d+ DP + dx DC
+    double kr[3], t1r[3], t1i[3];
+    const double dcr = 2.0 * c.DCr, dci = 2.0 * c.DCi;
+#pragma unroll
+    for (int m = 0; m < 3; m++)
+    {
+        const int i0 = m < 2 ? 0 : 1, i1 = m == 0 ? 1 : 2;
+        const double r0 = x[i1] - x[i0], r1 = y[i1] - y[i0], r2 = z[i1] - z[i0];
+        const double ru = r0 * c.ua[0] + r1 * c.ua[1] + r2 * c.ua[2];
+        const double rv = r0 * c.va[0] + r1 * c.va[1];
+        kr[m] = r0 * c.ka[0] + r1 * c.ka[1] + r2 * c.ka[2];
+        const double dp = rv * rv - ru * ru, dc = ru * rv;
+        t1r[m] = dp * c.DPr + dc * dcr;
+        t1i[m] = dp * c.DPi + dc * dci;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // exp(i arg2) times the amplitude
+    double wr[3], wi[3];
+    {
+        double sn[3], cs[3];
+        unsigned fl[3];
+        sincos_half<3>(a2, sn, cs, fl);
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+        {
+            const double a = flip_sign(ae[i], fl[i]);
+            wr[i] = a * cs[i];
+            wi[i] = a * sn[i];
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    double2 d23;
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+    {
+        const int i = q == 0 ? 1 : (q == 1 ? 0 : 2);  // spacecraft 2 first: link 23
+        // links (i, j) of spacecraft i: k.r_ij antisymmetric, T1 symmetric
+        const double ka = i == 0 ? kr[0] : (i == 1 ? -kr[0] : -kr[1]), kb = i == 0 ? kr[1] : (i == 1 ? kr[2] : -kr[2]);
+        const double arg[2] = {fma(hf[i], ka, hf[i]), fma(hf[i], kb, hf[i])};
+        double fr[2], fi[2];
+        sinc_phase<2>(arg, c.wide, fr, fi);
+        double2 d[2];
 #pragma unroll
         for (int h = 0; h < 2; h++)
         {
-            const double kr = h ? krb : kra, dp = h ? dpb : dpa, dc = h ? dcb : dca;
-            const double arg1 = 0.5 * fon * (1.0 + kr);
-            const double sinc = 0.25 * sinc_ratio(arg1);
-            const double t1r = ae * (dp * c.DPr + dc * c.DCr);
-            const double t1i = ae * (dp * c.DPi + dc * c.DCi);
-            double s2, c2;
-            sincos_red(arg1 - a2, &s2, &c2);
-            out(i + 3 * h, make_double2(sinc * (t1r * c2 + t1i * s2), sinc * (-t1r * s2 + t1i * c2)));
+            const int m = i == 0 ? h : (i == 1 ? 2 * h : 1 + h);
+            const double pr = t1r[m] * wr[i] - t1i[m] * wi[i], pi = t1r[m] * wi[i] + t1i[m] * wr[i];
+            d[h] = make_double2(pr * fr[h] - pi * fi[h], pr * fi[h] + pi * fr[h]);
         }
-        if constexpr (UNROLL) __builtin_amdgcn_sched_barrier(0);
+        if (i == 1) d23 = d[1];
+        out(i, make_double2(d[0].x - d23.x, d[0].y - d23.y));
+        if (i != 1) out(i == 0 ? 3 : 4, make_double2(d[1].x - d23.x, d[1].y - d23.y));
+        __builtin_amdgcn_sched_barrier(0);
     }
-}
-
-// The sample written to lds[l*stride + j].
-template <int KS = 1>
-__device__ inline void ucb_slow_sample(const UcbConst& c, double t, const double* __restrict__ pos,
-                                       double2* lds, int stride, int j)
-{
-    ucb_slow_sample_to<false, KS>(c, t, pos, [&](int l, double2 v) { lds[l * stride + j] = v; });
 }
 
 // Time of slow sample n (0-based) of a BW-sample series:

@@ -134,11 +134,12 @@ int glass_hip_fd_batch_set_concurrent(glass_hip_fd_batch *plan, int on);
 /* Launch shape ("tile") of one BW class's fused eval kernel (no reference
  * counterpart): nthr threads per workgroup (one template per workgroup;
  * fewer threads than template bins take several bins each), the grid
- * (gmul 0 = one workgroup per proposal slot, gmul > 0 = gmul x (workgroups
- * resident per CU) x CUs workgroups striding over the class's proposals),
- * and waves: the waves per SIMD the kernel's register allocation must
- * allow (1 = the compiler's own choice; 5 or 6 spill registers to keep more
- * workgroups resident).  Class k covers BW = 32 << k, k = 0..7.  Every
+ * (gmul 0 = the class's own: one workgroup per proposal slot at BW 128 to
+ * 1024, at the others 4 x the resident workgroups, striding; gmul > 0 =
+ * gmul x (workgroups resident per CU) x CUs workgroups striding over the
+ * class's proposals), and waves: the waves per SIMD the kernel's register
+ * allocation must allow (1 = the compiler's own choice).  Shapes that no
+ * build compiles any more run as the class's default shape.  Class k covers BW = 32 << k, k = 0..7.  Every
  * tile gives the same results up to the order of the final sums (~1e-16
  * relative). */
 typedef struct glass_hip_tile
@@ -190,7 +191,7 @@ int glass_hip_fd_batch_state(glass_hip_fd_batch *plan, double *logL, double *src
  * template with invC at window bin imin+m; mode 1 reproduces the
  * reference's Fisher alignment (invC at window bin m).  BW: a power of two,
  * 32..4096.  BW 2048 and 4096 run decimated kernels over at most one
- * workgroup per CU with a scratch slice each (0.6 / 1.6 MB) that the
+ * workgroup per CU with a scratch slice each (0.6 / 1.2 MB) that the
  * calling host thread keeps (grown with hipMalloc on first use; calls of
  * one host thread on different streams must not overlap). */
 int glass_hip_fd_source_derivs(const glass_hip_orbit *orbit, const char *format, double T,
