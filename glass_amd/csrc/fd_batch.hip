@@ -5,7 +5,8 @@
 // (ucb/src/glass_ucb_sampler.c:139-155): regenerate one source's template
 // and evaluate the chain's likelihood and the template's snr.  The sweep is
 // a fixed launch sequence with no host synchronisation:
-//   1. zero the BW-class counters (a kernel, not a memset: graph-safe)
+//   1. zero the BW-class counters (a kernel, not a memset: graph-safe),
+//      where more than one align workgroup adds to them
 //   2. align_kernel: ucb_alignment per proposal on the device; each block
 //      histograms its proposals into the 8 BW classes (32..4096) in LDS and
 //      reserves its slots with one atomic per class
@@ -14,10 +15,11 @@
 //      workgroup per proposal slot, or a multiple of the resident capacity
 //      striding over the class list), chosen by glass_hip_fd_batch_autotune
 //      from the compiled candidates: each workgroup takes an entry of its
-//      class list, builds the template in LDS (slow series, 6 FFTs, TDI)
+//      class list, builds the template in LDS (slow series, 5 FFTs, TDI)
 //      and reduces (r|dh) - (dh|dh)/2 over the union of the old and new
 //      supports only, reading the chain residual, the group's invC and the
-//      source's stored template with coalesced loads.
+//      source's stored template with coalesced loads.  Up to kFewItems
+//      proposals run in one launch for all classes instead.
 // The full-window likelihood is therefore never re-read per proposal: the
 // algorithmic HBM traffic per proposal is ~144 bytes per template bin, and
 // proposals of one chain find their window in L2.
@@ -234,12 +236,6 @@ __global__ __launch_bounds__(kAlignOne) void align_kernel(int n, Items it, Batch
     __syncthreads();
     if (k >= 0 && k < kNClass) cls_list[k * cls_stride + base[k] + slot] = e;
 }
-
-// Work distribution of the class kernels: one workgroup per proposal slot
-// (grid = proposal count; workgroups beyond the class count exit at once,
-// and the body has no loop, so nothing is hoisted across templates and the
-// register footprint stays that of one template), or a grid sized to a
-// multiple of the resident capacity striding over the class list.
 
 // half of bform(u, u, w): the cross terms once
 __device__ inline double qform(const double2* u, const double* w)
@@ -472,6 +468,77 @@ __device__ __forceinline__ void accept_source(const Items& it, int a, const Batc
     }
 }
 
+// f(integral constant N) of class k's template bins, the classes of at most
+// NTHR threads a workgroup; the waves past a class's own threads end, and its
+// barriers wait for the others.
+template <int NTHR, typename F>
+__device__ __forceinline__ void with_class(int k, F&& f)
+{
+#define GH_K(kk, N)                                                                 \
+    case kk:                                                                        \
+        if constexpr (fd_threads(N) <= NTHR)                                        \
+            if ((int)threadIdx.x < fd_threads(N)) f(std::integral_constant<int, N>()); \
+        break;
+    switch (k)
+    {
+        GH_K(0, 32) GH_K(1, 64) GH_K(2, 128) GH_K(3, 256) GH_K(4, 512) GH_K(5, 1024) GH_K(6, 2048) GH_K(7, 4096)
+    }
+#undef GH_K
+}
+
+// A few proposals (one sampler step of some chains): all classes in one
+// launch, workgroup e evaluates item e.  The launches bound it: eight over
+// four streams with their fork and join took 90 us of host and queue time for
+// 20 us of work (evaluate and accept 12 proposals: 309 -> 148 us).  NTHR: the
+// largest class's threads.  A.pos: the whole table.
+template <int NTHR>
+__global__ __launch_bounds__(NTHR) void eval_few_kernel(EvalArgs A)
+{
+    __shared__ double2 lds[FdShape<NTHR == 512 ? 1024 : 4096>::LDS];
+    const int e = blockIdx.x;
+    with_class<NTHR>(scalar_load(&A.rec[e].cls), [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        EvalArgs a = A;
+        a.pos += pos_soa_offset(N);
+        eval_item<N>(e, lds, a);
+    });
+}
+
+// ... and accepted: the three passes of the accept kernels below with the
+// template between them, workgroup e for item e.  Per bin r + h_old - h_new.
+template <int NTHR>
+__global__ __launch_bounds__(NTHR) void accept_few_kernel(Items it, BatchDev B, EvalArgs A,
+                                                          const double* __restrict__ logl_new)
+{
+    __shared__ double2 lds[FdShape<NTHR == 512 ? 1024 : 4096>::LDS];
+    const int e = blockIdx.x;
+    const EvalRec* rec = A.rec + e;
+    const int cls = scalar_load(&rec->cls);
+    if (cls < 0 || cls >= kNClass) return;  // no class holds it: the source stays
+    {
+        const EvalRec r = load_rec(rec);
+        accept_add_old(r.R, r.W, r.tmpl, r.cap, r.imin_o, r.bw_o);
+    }
+    __syncthreads();  // before the old template's slot and the residual are written again
+    with_class<NTHR>(cls, [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        EvalArgs a = A;
+        a.pos += pos_soa_offset(N);
+        tmpl_item<N>(e, lds, a, [&](const EvalRec& r, int m, const double2* v) {
+            const int j = r.imin + m;
+            if (j < 0 || j >= r.W) return;
+#pragma unroll
+            for (int ch = 0; ch < 3; ch++)
+            {
+                double2* R = r.R + (size_t)ch * r.W + j;
+                const double2 x = gload(R);
+                gstore(R, make_double2(x.x - v[ch].x, x.y - v[ch].y));
+            }
+        });
+        accept_source(it, e, B, N, load_rec(rec).imin, logl_new);
+    });
+}
+
 // r_c = d_g - sum_s h_cs (add_ucb_model, ucb/src/glass_ucb_model.c:192-232)
 // One workgroup per chain (grid = chain count), striding over its window.
 __global__ __launch_bounds__(256) void resid_kernel(BatchDev B)
@@ -698,6 +765,12 @@ static int resident_per_cu(int N, int nthr, int waves)
 // the series were cut to 512 points; with 5 the spills make it 2.36).
 constexpr int batch_default_waves(int N) { return N == 512 ? 6 : (N == 1024 ? 4 : 1); }
 
+static bool default_tile(int k, glass_hip_tile t)
+{
+    const int N = 32 << k;
+    return t.nthr == fd_threads(N) && t.gmul == 0 && t.waves == batch_default_waves(N);
+}
+
 static int setup_grids(glass_hip_fd_batch* P)
 {
     GH_CHECK(hipDeviceGetAttribute(&P->ncu, hipDeviceAttributeMultiprocessorCount, P->device));
@@ -789,6 +862,22 @@ static void launch_align(glass_hip_fd_batch* P, int n, const Items& it, double* 
                                                                        P->cls_list, P->cls_cap, logl_out, snr_out);
 }
 
+// Items that one launch of all classes takes: four per CU.  Evaluating
+// proposals of 2- and 4-year windows (512 to 4096 bins) in one launch against
+// eight launches of the classes, eager and replayed as a graph: 12 in 20, 37 /
+// 89, 81 us; 252 in 43, 47 / 94, 83; 1020 in 97, 104 / 139, 123; but 2040 in
+// 214, 222 / 206, 189, where the waves that end leave the CUs half empty.  The
+// class kernels run for a caller's own tiles and in the profiling mode, which
+// times them.
+constexpr int kFewItems = 1024;
+static bool few_items(const glass_hip_fd_batch* P, int n)
+{
+    if (n > kFewItems || P->prof) return false;
+    for (int k = 0; k < kNClass; k++)
+        if (!default_tile(k, P->tile[k])) return false;
+    return true;
+}
+
 // alignment + per-class launches for items; mode 0: eval, 1: templates
 static int launch_items(glass_hip_fd_batch* P, int n, const Items& it, int mode, double* logl_out, double* snr_out,
                         hipStream_t s)
@@ -800,6 +889,17 @@ static int launch_items(glass_hip_fd_batch* P, int n, const Items& it, int mode,
         return GLASS_HIP_EINVAL;
     }
     launch_align(P, n, it, mode == 0 ? logl_out : nullptr, mode == 0 ? snr_out : nullptr, s);
+    if (mode == 0 && few_items(P, n))
+    {
+        EvalArgs A = eval_args(P, 32, it, logl_out, snr_out);
+        A.pos = P->B.pos_soa;
+        if (P->B.bwcap <= 1024)
+            eval_few_kernel<512><<<n, 512, 0, s>>>(A);
+        else
+            eval_few_kernel<1024><<<n, 1024, 0, s>>>(A);
+        GH_CHECK(hipGetLastError());
+        return GLASS_HIP_OK;
+    }
     // the per-class timings of the profiling mode need the classes in turn
     const bool par = P->concurrent && !(P->prof && mode == 0);
     if (par)
@@ -1222,6 +1322,18 @@ extern "C" int glass_hip_fd_batch_accept(glass_hip_fd_batch* P, int nacc, const 
     hipStream_t s = (hipStream_t)stream;
     Items it{d_chain, d_src, d_params, d_idx};
     int rc;
+    if (few_items(P, nacc))
+    {
+        launch_align(P, nacc, it, nullptr, nullptr, s);
+        EvalArgs A = eval_args(P, 32, it, nullptr, nullptr);
+        A.pos = P->B.pos_soa;
+        if (P->B.bwcap <= 1024)
+            accept_few_kernel<512><<<nacc, 512, 0, s>>>(it, P->B, A, d_logL);
+        else
+            accept_few_kernel<1024><<<nacc, 1024, 0, s>>>(it, P->B, A, d_logL);
+        GH_CHECK(hipGetLastError());
+        return GLASS_HIP_OK;
+    }
     accept_add_old_kernel<<<nacc, 256, 0, s>>>(nacc, it, P->B);
     if ((rc = launch_items(P, nacc, it, 1, nullptr, nullptr, s))) return rc;
     accept_sub_new_kernel<<<nacc, 256, 0, s>>>(nacc, it, P->B, P->p_bw, P->p_imin, d_logL);
