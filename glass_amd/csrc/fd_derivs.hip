@@ -223,48 +223,14 @@ __device__ __forceinline__ void deriv_bin(const UcbConst& c, const DerivArgs& A,
     }
 }
 
-// Workgroup sums of the per-thread sums into red[kNSum] through LDS: CH
-// values at a time are laid out one row per value (rows a double apart in
-// banks), each thread adds CH entries of one row, the lanes of a row add up
-// by two or three exchanges and the waves' partials in order.  170
-// instructions a thread for 48 values; the transposed shuffles took 500.
-// Fixed order.  buf: the FFT buffer (its readers have passed a barrier).
+// Workgroup sums of the per-thread sums into red[kNSum]; buf: the FFT buffer
+// (its readers have passed a barrier).
 template <int NTHR, int CH>
 __device__ __forceinline__ void deriv_reduce(const double (&acc)[kNSum], double* buf, double* red, bool extra)
 {
-    static_assert(kNMain % CH == 0 && 64 % CH == 0, "whole chunks");
-    constexpr int NW = NTHR / 64, ROW = NTHR + 1;
-    __shared__ double part[kNSum][NW];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-#pragma unroll
-    for (int k0 = 0; k0 < kNMain; k0 += CH)
-    {
-        if (k0) __syncthreads();
-#pragma unroll
-        for (int v = 0; v < CH; v++) buf[v * ROW + t] = acc[k0 + v];
-        __syncthreads();
-        const int v = t % CH;
-        const double* row = buf + v * ROW + (t / CH) * CH;
-        double s = 0.0;
-#pragma unroll
-        for (int i = 0; i < CH; i++) s += row[i];
-#pragma unroll
-        for (int d = CH; d < 64; d *= 2) s += __shfl_xor(s, d, 64);
-        if (lane < CH) part[k0 + v][wave] = s;
-    }
-    if (extra)
-    {
-        const double s = wave_sum(acc[kNMain]);
-        if (lane == 0) part[kNMain][wave] = s;
-    }
-    __syncthreads();
-    if (t < kNSum)
-    {
-        double s = 0.0;
-        if (t < kNMain || extra)
-            for (int i = 0; i < NW; i++) s += part[t][i];
-        red[t] = s;
-    }
+    block_sum_rows<NTHR, CH, kNMain>(acc, buf, red);
+    const double s = extra ? block_sum<NTHR>(acc[kNMain]) : 0.0;
+    if (threadIdx.x == 0) red[kNMain] = s;
     __syncthreads();
 }
 

@@ -346,12 +346,9 @@ __device__ __forceinline__ void fd_tdi_xyz(double c1, double s1, double2 P, cons
     Z = ch(d[2].x - d[4].x, d[2].y - d[4].y, d[3].x, d[3].y);
 }
 
-template <int N>
-__device__ __forceinline__ void fd_tdi(const UcbConst& c, int m, int fmt, const double2* d, double2* out)
+__device__ __forceinline__ void fd_tdi_channels(double c1, double s1, double2 P, int fmt, const double2* d,
+                                                double2* out)
 {
-    double s1, c1;
-    fd_tdi_phase<N>(c, m, c1, s1);
-    const double2 P = fd_tdi_prefactor<N>(c, m, fmt, c1, s1);
     double2 X, Y, Z;
     fd_tdi_xyz(c1, s1, P, d, X, Y, Z);
     double2 A = make_double2((Z.x - X.x) * kSQRT1_2, (Z.y - X.y) * kSQRT1_2);
@@ -366,6 +363,14 @@ __device__ __forceinline__ void fd_tdi(const UcbConst& c, int m, int fmt, const 
     out[2] = Z;
     out[3] = A;
     out[4] = E;
+}
+
+template <int N>
+__device__ __forceinline__ void fd_tdi(const UcbConst& c, int m, int fmt, const double2* d, double2* out)
+{
+    double s1, c1;
+    fd_tdi_phase<N>(c, m, c1, s1);
+    fd_tdi_channels(c1, s1, fd_tdi_prefactor<N>(c, m, fmt, c1, s1), fmt, d, out);
 }
 
 }  // namespace glass

@@ -14,11 +14,16 @@
 // (psi, phase) pairs) go through the batched template pipeline (slow series
 // -> LDS FFTs -> TDI) one after another and stay in registers, one bin per
 // thread; then the projections N^i = (s|A^i) and the Gram M^ij = (A^i|A^j)
-// for X and for A+E are summed over the workgroup, and thread 0 inverts the
-// two 4x4 Grams, forms F = N^T M^-1 N / 2 and the maximum-likelihood
-// extrinsic parameters.  Cells are bucketed by their filter length
-// N = ucb_bandwidth(f0, fdot, cos theta, A = 1e-22) into one kernel per
-// power-of-two class, as the proposal evaluations are.
+// for X and for A+E are summed over the workgroup.  Cells are bucketed by
+// their filter length N = ucb_bandwidth(f0, fdot, cos theta, A = 1e-22) into
+// one kernel per power-of-two class, as the proposal evaluations are.
+//
+// Vector issue bounds it, and at the usual 64 bins a cell is one wave, so
+// what one lane does costs as much as what all do: the constants of a cell
+// before the filters, and after them the inverses of its two 4x4 Grams, F =
+// N^T M^-1 N / 2 and the maximum-likelihood extrinsic parameters, are kernels
+// of one thread per cell.  The filters share their sample (FilterSample).
+// 102,400 cells of 64 bins: 1.28 -> 0.53 ms.
 //
 // The 4x4 inverse is Gauss-Jordan elimination with partial pivoting in
 // place of LAPACKE dgetrf/dgetri (utils/src/glass_math.c:501-523); the two
@@ -54,7 +59,12 @@ struct FstatDev
     int fmt;
     const double* pos;
     const double2* tw;
-    double fp[4][4];  // per filter: ln A, cos iota, psi, phase
+    // per filter: the factors of the plus and cross tensors as ucb_setup
+    // forms them, the phase (0 for the first) with its cosine and sine
+    struct Filter
+    {
+        double DPr, DPi, DCr, DCi, phase, cph, sph;
+    } f[4];
 };
 
 struct Cells
@@ -63,7 +73,13 @@ struct Cells
     double* lx;          // [n] F-statistic of X
     double* lae;         // [n] F-statistic of A, E
     double* fpar;        // [n][4]: A, iota, psi, phase of the A,E fit
+    UcbConst* pc;        // [n] template constants of the first filter
+    double* sums;        // [n][kFsSum]
+    int* cls;            // [n] class (kFsClass: none)
 };
+
+// Sums of one cell: N of X and of A, E, then the upper triangles of M.
+constexpr int kFsSum = 28;
 
 // Gauss-Jordan inverse with partial pivoting of a 4x4 matrix (in place)
 __host__ __device__ inline void invert4(double m[4][4])
@@ -136,9 +152,9 @@ __device__ inline void fstat_params(const double M[4][4], const double* N, doubl
 // per block (an LDS histogram, then one global atomic per class per
 // block): the cells of a segment mostly share one filter length, and one
 // global atomic per cell on that class's counter serialises the launch.
-__global__ __launch_bounds__(256) void fstat_align_kernel(int n, const double* __restrict__ cell, FstatDev D,
-                                                          int* __restrict__ cls, int* __restrict__ list, int cap,
-                                                          int* __restrict__ err)
+__global__ __launch_bounds__(256) void fstat_align_kernel(int n, FstatDev D,
+                                                          Cells C, int* __restrict__ cls, int* __restrict__ list,
+                                                          int cap, int* __restrict__ err)
 {
     __shared__ int hist[kFsClass + 1], base[kFsClass + 1];
     if (threadIdx.x <= kFsClass) hist[threadIdx.x] = 0;
@@ -147,10 +163,15 @@ __global__ __launch_bounds__(256) void fstat_align_kernel(int n, const double* _
     int k = -1, slot = 0;
     if (e < n)
     {
-        const double f0 = cell[(size_t)e * 4], fdot = cell[(size_t)e * 4 + 1], theta = cell[(size_t)e * 4 + 2];
+        const double f0 = C.cell[(size_t)e * 4], fdot = C.cell[(size_t)e * 4 + 1];
+        const double theta = C.cell[(size_t)e * 4 + 2], phi = C.cell[(size_t)e * 4 + 3];
         const int N = ucb_bandwidth(D.L, D.fstar, f0, fdot, cos(theta), 1.e-22, D.T, D.NFFT);
         k = 31 - __clz(N) - 4;  // log2(N) - 4
         if (k < 0 || k >= kFsClass || (N & (N - 1))) k = kFsClass;
+        C.cls[e] = k;
+        // amplitude and polarisation come with each filter
+        const double p[8] = {f0 * D.T, cos(theta), phi, 0.0, 0.0, 0.0, D.f[0].phase, fdot * (D.T * D.T)};
+        ucb_setup(p, 8, D.T, D.t0, D.L, D.fstar, C.pc[e]);
         slot = atomicAdd(&hist[k], 1);
     }
     __syncthreads();
@@ -160,117 +181,270 @@ __global__ __launch_bounds__(256) void fstat_align_kernel(int n, const double* _
     if (k >= 0 && k < kFsClass) list[(size_t)k * cap + base[k] + slot] = e;
 }
 
-template <int N, int NTHR>
-__global__ __launch_bounds__(NTHR) void fstat_kernel(const int* __restrict__ list, const int* __restrict__ count,
-                                                     FstatDev D, Cells C)
+// One slow sample of all four filters.  They differ in the polarisation
+// tensor's factors and in the constant phase subtracted in arg2, whose rounding
+// (~1e-10 rad at 3 mHz and 2 yr, independent in each filter) the results keep:
+// with the quadrature filters as exact quarter turns of the others F moves by
+// up to 1e-9.  arg2 of filter k is that of the first less phase_k plus a
+// delta, so its factor exp(i arg2) is the first's turned by phase_k times 1 +
+// i delta (delta^2 < 1e-18).  What the filters share is formed once: ~350
+// instructions, and 90 for each filter instead of 400.
+struct FilterSample
 {
-    constexpr int PER = (N + NTHR - 1) / NTHR;  // bins per thread
-    __shared__ double2 lds[FdShape<N>::LDS];
-    if ((int)blockIdx.x >= *count) return;
-    const int e = list[blockIdx.x];
-    const double f0 = C.cell[(size_t)e * 4], fdot = C.cell[(size_t)e * 4 + 1];
-    const double theta = C.cell[(size_t)e * 4 + 2], phi = C.cell[(size_t)e * 4 + 3];
-    const long q = (long)(f0 * D.T);
-    double2 hx[PER][4], ha[PER][4], he[PER][4];
-    // the four filters' constants, one lane each (the same code on four lanes
-    // of the first wave: one setup's latency instead of four in turn)
-    __shared__ UcbConst sc4[4];
-    if (threadIdx.x < 4)
+    double2 B[3][2];      // spacecraft i, link h: amplitude exp(i arg2) S exp(-i arg1) (the first's arg2)
+    double dp[3], dc[3];  // arms 12, 13, 23
+    double delta[3][3];   // filter 1..3, spacecraft
+
+    __device__ __forceinline__ FilterSample(const UcbConst& c, const FstatDev& D, double t,
+                                            const double* __restrict__ pos)
     {
-        const int fi = threadIdx.x;
-        double p[8] = {f0 * D.T,    cos(theta),   phi,          D.fp[fi][0],
-                       D.fp[fi][1], D.fp[fi][2], D.fp[fi][3], fdot * (D.T * D.T)};
-        ucb_setup(p, 8, D.T, D.t0, D.L, D.fstar, sc4[fi]);
-    }
-    __syncthreads();
-    for (int fi = 0; fi < 4; fi++)
-    {
-        const UcbConst& k = sc4[fi];
-        if (fi) __syncthreads();  // the last filter's LDS reads
-        fd_link_bins<N, false>(
-            HeldConst{k}, lds, D.pos, kPosNF / N, D.tw, kTwN / N, [](int) {}, [&](int kk, int m, const double2* dl) {
-                double2 v[5];
-                fd_tdi<N>(k, m, D.fmt, dl, v);
-                hx[kk][fi] = v[0];
-                ha[kk][fi] = v[3];
-                he[kk][fi] = v[4];
-            });
-    }
-    // projections and Gram sums (get_N, get_M), the reference's term order
-    double nx[4] = {0, 0, 0, 0}, nae[4] = {0, 0, 0, 0}, mx[10], mae[10];
-    for (int i = 0; i < 10; i++) mx[i] = mae[i] = 0.0;
-    const long qo = q - D.qmin0;
-    {
+        const double x[3] = {pos[0], pos[1], pos[2]}, y[3] = {pos[3], pos[4], pos[5]}, z[3] = {pos[6], pos[7], pos[8]};
+        double a2[3], hf[3], ae[3];
+        double dft;
+        {
 #pragma clang fp contract(off)
+            dft = c.df * t;
+        }
 #pragma unroll
-        for (int kk = 0; kk < PER; kk++)
+        for (int i = 0; i < 3; i++)
         {
-            const int m = FdShape<N>::bin(kk);
-            const long kb = qo + m - N / 2;
-            if (m >= N || !(kb > 0 && kb < D.NFFT)) continue;
-            const double c = D.C00[kb];
-            const double2 dX = D.X[kb], dA = D.A[kb], dE = D.E[kb];
-            for (int i = 0; i < 4; i++)
+            double xi;
             {
-                nx[i] += (dX.x * hx[kk][i].x + dX.y * hx[kk][i].y) / c;
-                nae[i] += (dA.x * ha[kk][i].x + dA.y * ha[kk][i].y + dE.x * he[kk][i].x + dE.y * he[kk][i].y) / c;
-            }
-            int t = 0;
-            for (int i = 0; i < 4; i++)
-                for (int j = i; j < 4; j++, t++)
+                // as ucb_slow_sample_to forms it for each filter
+#pragma clang fp contract(off)
+                const double kdotx = div_by_recip(x[i] * c.k[0] + y[i] * c.k[1] + z[i] * c.k[2], kCLIGHT, kInvCLIGHT);
+                xi = t - kdotx;
+                const double w = c.pi2f0 * xi, chirp = c.pidfdt * xi * xi;
+                a2[i] = w - c.phi0 - dft;
+                a2[i] += chirp;
+#pragma unroll
+                for (int k = 1; k < 4; k++)
                 {
-                    mx[t] += 4.0 * (hx[kk][i].x * hx[kk][j].x + hx[kk][i].y * hx[kk][j].y) / c;
-                    mae[t] += 4.0 * (ha[kk][i].x * ha[kk][j].x + ha[kk][i].y * ha[kk][j].y) / c +
-                              4.0 * (he[kk][i].x * he[kk][j].x + he[kk][i].y * he[kk][j].y) / c;
+                    double a = w - D.f[k].phase - dft;
+                    a += chirp;
+                    delta[k - 1][i] = (a - a2[i]) + D.f[k].phase;
                 }
+            }
+            hf[i] = fma(c.dfh, xi, c.f0h);
+            ae[i] = fma(c.aevq, xi, 0.25);
+        }
+        double kr[3];
+#pragma unroll
+        for (int m = 0; m < 3; m++)
+        {
+            const int i0 = m < 2 ? 0 : 1, i1 = m == 0 ? 1 : 2;
+            const double r0 = x[i1] - x[i0], r1 = y[i1] - y[i0], r2 = z[i1] - z[i0];
+            const double ru = r0 * c.ua[0] + r1 * c.ua[1] + r2 * c.ua[2];
+            const double rv = r0 * c.va[0] + r1 * c.va[1];
+            kr[m] = r0 * c.ka[0] + r1 * c.ka[1] + r2 * c.ka[2];
+            dp[m] = rv * rv - ru * ru;
+            dc[m] = 2.0 * ru * rv;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        double sn[3], cs[3];
+        unsigned fl[3];
+        sincos_half<3>(a2, sn, cs, fl);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+        {
+            const double a = flip_sign(ae[i], fl[i]), wr = a * cs[i], wi = a * sn[i];
+            const double ka = i == 0 ? kr[0] : (i == 1 ? -kr[0] : -kr[1]);
+            const double kb = i == 0 ? kr[1] : (i == 1 ? kr[2] : -kr[2]);
+            const double arg[2] = {fma(hf[i], ka, hf[i]), fma(hf[i], kb, hf[i])};
+            double fr[2], fi[2];
+            sinc_phase<2>(arg, c.wide, fr, fi);
+#pragma unroll
+            for (int h = 0; h < 2; h++) B[i][h] = make_double2(wr * fr[h] - wi * fi[h], wr * fi[h] + wi * fr[h]);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    // the 28 workgroup sums in one pass (one barrier instead of 56)
-    constexpr int B = NTHR < 64 ? 64 : NTHR;
-    __shared__ double tot[28];
+
+    // out(l, value) of filter k's five series, as ucb_slow_sample_to
+    template <typename Out>
+    __device__ __forceinline__ void filter(const FstatDev::Filter& f, int k, Out&& out) const
     {
-        double v[28];
+        double2 T1[3];
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-        {
-            v[i] = nx[i];
-            v[4 + i] = nae[i];
-        }
+        for (int m = 0; m < 3; m++)
+            T1[m] = make_double2(dp[m] * f.DPr + dc[m] * f.DCr, dp[m] * f.DPi + dc[m] * f.DCi);
+        double2 d23;
 #pragma unroll
-        for (int i = 0; i < 10; i++)
+        for (int q = 0; q < 3; q++)
         {
-            v[8 + i] = mx[i];
-            v[18 + i] = mae[i];
+            const int i = q == 0 ? 1 : (q == 1 ? 0 : 2);
+            double2 r = make_double2(1.0, 0.0);
+            if (k > 0)
+            {
+                const double e = delta[k > 0 ? k - 1 : 0][i];
+                r = make_double2(fma(e, f.sph, f.cph), fma(e, f.cph, -f.sph));
+            }
+            double2 d[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+            {
+                const int m = i == 0 ? h : (i == 1 ? 2 * h : 1 + h);
+                const double2 b = k > 0 ? cmul(B[i][h], r) : B[i][h];
+                d[h] = cmul(T1[m], b);
+            }
+            if (i == 1) d23 = d[1];
+            out(i, make_double2(d[0].x - d23.x, d[0].y - d23.y));
+            if (i != 1) out(i == 0 ? 3 : 4, make_double2(d[1].x - d23.x, d[1].y - d23.y));
         }
-        block_sum_many<B, 28>(v, tot);
     }
-    if (threadIdx.x != 0) return;
+};
+
+// The constants of a cell's filter: the first's with its own amplitude and phase.
+struct FilterConst
+{
+    LoadedConst base;
+    const FstatDev& D;
+    int k;
+    __device__ __forceinline__ UcbConst operator()() const
+    {
+        UcbConst c = base();
+        const FstatDev::Filter& f = D.f[k];
+        c.DPr = f.DPr;
+        c.DPi = f.DPi;
+        c.DCr = f.DCr;
+        c.DCi = f.DCi;
+        c.phi0 = f.phase;
+        return c;
+    }
+};
+
+// Terms of one bin from the filters' X, A, E, with the weight 1/c.
+__device__ __forceinline__ void fstat_bin(const FstatDev& D, long kb, const double2 (&h)[4][3], double (&v)[kFsSum])
+{
+    const double w = 1.0 / D.C00[kb];
+    const double2 dX = D.X[kb], dA = D.A[kb], dE = D.E[kb];
+    auto re = [](double2 a, double2 b) { return a.x * b.x + a.y * b.y; };
+    int t = 8;
+#pragma unroll
     for (int i = 0; i < 4; i++)
     {
-        nx[i] = tot[i];
-        nae[i] = tot[4 + i];
-    }
-    for (int i = 0; i < 10; i++)
-    {
-        mx[i] = tot[8 + i];
-        mae[i] = tot[18 + i];
-    }
-    double MX[4][4], MA[4][4];
-    int t = 0;
-    for (int i = 0; i < 4; i++)
+        double2 u[3];
+#pragma unroll
+        for (int ch = 0; ch < 3; ch++) u[ch] = make_double2(w * h[i][ch].x, w * h[i][ch].y);
+        v[i] += re(dX, u[0]);
+        v[4 + i] += re(dA, u[1]) + re(dE, u[2]);
+#pragma unroll
         for (int j = i; j < 4; j++, t++)
         {
-            MX[i][j] = MX[j][i] = mx[t];
-            MA[i][j] = MA[j][i] = mae[t];
+            v[t] += 4.0 * re(u[0], h[j][0]);
+            v[10 + t] += 4.0 * (re(u[1], h[j][1]) + re(u[2], h[j][2]));
         }
+    }
+}
+
+// Three waves per SIMD up to 512 bins: the compiler's choice is a few vector
+// registers above the 168 that allows.
+template <int N>
+__global__ __launch_bounds__(fd_threads(N)) __attribute__((amdgpu_waves_per_eu(N <= 512 ? 3 : 1, 8))) void fstat_kernel(
+    const int* __restrict__ list, const int* __restrict__ count, FstatDev D, Cells C)
+{
+    using S = FdShape<N>;
+    constexpr int CH = 8, ROWS = CH * (S::NTHR + 1) / 2 + 1;
+    __shared__ double2 lds[S::LDS > ROWS ? S::LDS : ROWS];
+    if ((int)blockIdx.x >= *count) return;
+    const int e = list[blockIdx.x];
+    const LoadedConst k{C.pc + e};
+    const long qo = (long)(C.cell[(size_t)e * 4] * D.T) - D.qmin0 - N / 2;  // segment bin of template bin 0
+    double v[kFsSum];
+#pragma unroll
+    for (int i = 0; i < kFsSum; i++) v[i] = 0.0;
+    if constexpr (S::P == 1)
+    {
+        const int t = S::lane();
+        const bool on = t < N;
+        const int ts = wave_fft_slot(t), tb = wave_fft_slot((t + N / 2) & (N - 1));
+        const int n = on ? t : 0;
+        const FilterSample s(k(), D, ucb_sample_time(D.T, D.t0, n, N), D.pos + (size_t)n * (kPosNF / N) * 9);
+        double2 h[4][3], P;
+        double c1, s1;
+        {
+            const UcbConst& c = k();
+            fd_tdi_phase<N>(c, t, c1, s1);
+            P = fd_tdi_prefactor<N>(c, t, D.fmt, c1, s1);
+        }
+#pragma unroll
+        for (int f = 0; f < 4; f++)
+        {
+            if (f) __syncthreads();  // the last filter's LDS reads
+            if (on) s.filter(D.f[f], f, [&](int l, double2 x) { lds[l * S::PN + ts] = x; });
+            __syncthreads();
+            wave_fft<N, kNLink, S::NTHR, true>(lds, opaque(D.tw), kTwN / N);
+            double2 d[kNLink], o[5];
+#pragma unroll
+            for (int l = 0; l < kNLink; l++) d[l] = lds[l * S::PN + tb];
+            fd_tdi_channels(c1, s1, P, D.fmt, d, o);
+            h[f][0] = o[0];
+            h[f][1] = o[3];
+            h[f][2] = o[4];
+        }
+        const long kb = qo + t;
+        if (on && kb > 0 && kb < D.NFFT) fstat_bin(D, kb, h, v);
+    }
+    else
+    {
+        double2 h[S::Q][4][3];
+#pragma unroll
+        for (int f = 0; f < 4; f++)
+        {
+            if (f) __syncthreads();  // the last filter's LDS reads
+            fd_link_bins<N, false>(
+                FilterConst{k, D, f}, lds, D.pos, kPosNF / N, D.tw, kTwN / N, [](int) {},
+                [&](int s, int m, const double2* dl) {
+                    double2 o[5];
+                    fd_tdi<N>(k(), m, D.fmt, dl, o);
+                    h[s][f][0] = o[0];
+                    h[s][f][1] = o[3];
+                    h[s][f][2] = o[4];
+                });
+        }
+#pragma unroll
+        for (int s = 0; s < S::Q; s++)
+        {
+            const long kb = qo + S::bin(s);
+            if (kb > 0 && kb < D.NFFT) fstat_bin(D, kb, h[s], v);
+        }
+    }
+    __syncthreads();
+    block_sum_rows<S::NTHR, CH, kFsSum>(v, (double*)lds, C.sums + (size_t)e * kFsSum);
+}
+
+// F-statistics and extrinsic parameters of the cells, one thread each; cells
+// no class holds get NaN.
+__global__ __launch_bounds__(64) void fstat_fit_kernel(int n, Cells C)
+{
+    const int e = blockIdx.x * 64 + threadIdx.x;
+    if (e >= n) return;
+    if (C.cls[e] >= kFsClass)
+    {
+        C.lx[e] = C.lae[e] = NAN;
+        for (int k = 0; k < 4; k++) C.fpar[(size_t)e * 4 + k] = NAN;
+        return;
+    }
+    const double* v = C.sums + (size_t)e * kFsSum;
+    double nx[4], nae[4], MX[4][4], MA[4][4];
+#pragma unroll
     for (int i = 0; i < 4; i++)
     {
-        nx[i] *= 4.0;
-        nae[i] *= 4.0;
+        nx[i] = 4.0 * v[i];
+        nae[i] = 4.0 * v[4 + i];
     }
+    int t = 8;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = i; j < 4; j++, t++)
+        {
+            MX[i][j] = MX[j][i] = v[t];
+            MA[i][j] = MA[j][i] = v[10 + t];
+        }
     invert4(MX);
-    invert4(MA);
     C.lx[e] = fstat_value(MX, nx);
+    invert4(MA);
     C.lae[e] = fstat_value(MA, nae);
     fstat_params(MA, nae, C.fpar + (size_t)e * 4);
 }
@@ -289,7 +463,9 @@ struct glass_hip_fstat
     std::vector<void*> allocs;
     double* cells = nullptr;
     double *lx = nullptr, *lae = nullptr, *fpar = nullptr;
-    int *cls = nullptr, *list = nullptr;
+    int *cls = nullptr, *list = nullptr, *kcls = nullptr;
+    UcbConst* pc = nullptr;
+    double* sums = nullptr;
 };
 
 template <typename T>
@@ -349,10 +525,10 @@ extern "C" int glass_hip_fstat_create(glass_hip_fstat** out, const glass_hip_orb
     const double psi[4] = {0.0, M_PI_4, 0.0, M_PI_4}, ph[4] = {0.0, M_PI, 3.0 * M_PI_2, M_PI_2};
     for (int i = 0; i < 4; i++)
     {
-        D.fp[i][0] = log(2.0);
-        D.fp[i][1] = cos(M_PI_2);
-        D.fp[i][2] = psi[i];
-        D.fp[i][3] = ph[i];
+        const double p[8] = {1.0, 0.0, 0.0, log(2.0), cos(M_PI_2), psi[i], ph[i], 0.0};
+        UcbConst c;
+        ucb_setup(p, 8, T, t0, orbit->L, orbit->fstar, c);
+        D.f[i] = {c.DPr, c.DPi, c.DCr, c.DCi, ph[i], cos(ph[i]), sin(ph[i])};
     }
     F->cap = max_cells;
     const size_t nb = sizeof(double) * 2 * (size_t)NFFT;
@@ -362,7 +538,9 @@ extern "C" int glass_hip_fstat_create(glass_hip_fstat** out, const glass_hip_orb
         (rc = falloc(F, &dE, 2 * (size_t)NFFT)) || (rc = falloc(F, &dC, NFFT)) ||
         (rc = falloc(F, &F->cells, 4 * (size_t)max_cells)) || (rc = falloc(F, &F->lx, max_cells)) ||
         (rc = falloc(F, &F->lae, max_cells)) || (rc = falloc(F, &F->fpar, 4 * (size_t)max_cells)) ||
-        (rc = falloc(F, &F->cls, kFsClass + 1)) || (rc = falloc(F, &F->list, (size_t)kFsClass * max_cells)))
+        (rc = falloc(F, &F->cls, kFsClass + 1)) || (rc = falloc(F, &F->list, (size_t)kFsClass * max_cells)) ||
+        (rc = falloc(F, &F->kcls, max_cells)) || (rc = falloc(F, &F->pc, max_cells)) ||
+        (rc = falloc(F, &F->sums, (size_t)kFsSum * max_cells)))
     {
         glass_hip_fstat_destroy(F);
         return rc;
@@ -398,34 +576,25 @@ __global__ void fs_zero_kernel(int* p, int n)
     if (i < n) p[i] = 0;
 }
 
-__global__ void fs_nan_kernel(int n, double* lx, double* lae, double* fpar)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    lx[i] = lae[i] = NAN;
-    for (int k = 0; k < 4; k++) fpar[(size_t)i * 4 + k] = NAN;
-}
-
 static int fstat_launch(glass_hip_fstat* F, int n, const double* cells, double* lx, double* lae, double* fpar,
                         hipStream_t s)
 {
     fs_zero_kernel<<<1, 64, 0, s>>>(F->cls, kFsClass + 1);
-    fs_nan_kernel<<<(n + 255) / 256, 256, 0, s>>>(n, lx, lae, fpar);
-    fstat_align_kernel<<<(n + 255) / 256, 256, 0, s>>>(n, cells, F->D, F->cls, F->list, F->cap,
-                                                       F->cls + kFsClass);
+    const Cells C{cells, lx, lae, fpar, F->pc, F->sums, F->kcls};
+    fstat_align_kernel<<<(n + 255) / 256, 256, 0, s>>>(n, F->D, C, F->cls, F->list, F->cap, F->cls + kFsClass);
     // the class counts decide the grids: only non-empty classes launch, one
     // workgroup per cell (an empty class's full grid of immediately
     // exiting workgroups costs 80-160 us)
     int cnt[kFsClass + 1];
     GH_CHECK(hipMemcpyAsync(cnt, F->cls, sizeof(cnt), hipMemcpyDeviceToHost, s));
     GH_CHECK(hipStreamSynchronize(s));
-    Cells C{cells, lx, lae, fpar};
-#define FS_L(kk, NN)                                                                                            \
-    if (cnt[kk] > 0)                                                                                            \
-        fstat_kernel<NN, fd_threads(NN)><<<cnt[kk], fd_threads(NN), 0, s>>>(F->list + (size_t)kk * F->cap,     \
-                                                                            F->cls + kk, F->D, C);
+#define FS_L(kk, NN)                                                                                        \
+    if (cnt[kk] > 0)                                                                                        \
+        fstat_kernel<NN><<<cnt[kk], fd_threads(NN), 0, s>>>(F->list + (size_t)kk * F->cap, F->cls + kk,     \
+                                                            F->D, C);
     FS_L(0, 16) FS_L(1, 32) FS_L(2, 64) FS_L(3, 128) FS_L(4, 256) FS_L(5, 512) FS_L(6, 1024) FS_L(7, 2048)
 #undef FS_L
+    fstat_fit_kernel<<<(n + 63) / 64, 64, 0, s>>>(n, C);
     GH_CHECK(hipGetLastError());
     return GLASS_HIP_OK;
 }
