@@ -257,6 +257,103 @@ GH_HD inline void sincos_cr(double x, double* s, double* c)
     *c = v.c;
 }
 
+// sin(pi j / 128), j = 0..64, as double-double (values computed at 250-bit
+// precision for this library).
+constexpr dd_t kSinTab[65] = {
+    {0.0, 0.0}, {0.024541228522912288, -9.186849012577878e-20},
+    {0.049067674327418015, -6.79610372051828e-19}, {0.07356456359966743, -2.7784941506273593e-18},
+    {0.0980171403295606, -1.634582362244256e-18}, {0.1224106751992162, 2.8354501489965335e-18},
+    {0.14673047445536175, 3.726947147046568e-18}, {0.17096188876030122, 9.19199801817591e-18},
+    {0.19509032201612828, -7.991079068461731e-18}, {0.2191012401568698, -3.6513812299150776e-19},
+    {0.2429801799032639, -8.751431529719663e-18}, {0.26671275747489837, 2.0941222578826688e-17},
+    {0.2902846772544624, -1.892797870777425e-17}, {0.31368174039889146, 1.4560447299968912e-17},
+    {0.33688985339222005, -4.200094003347509e-19}, {0.35989503653498817, -1.7601687123839282e-17},
+    {0.3826834323650898, -1.0050772696461588e-17}, {0.40524131400498986, 9.911140194289988e-18},
+    {0.4275550934302821, 9.411189816295473e-18}, {0.4496113296546066, 4.883192423203524e-18},
+    {0.47139673682599764, 6.516678136069013e-18}, {0.49289819222978404, -1.0257831676562186e-18},
+    {0.5141027441932218, -4.5712707523615624e-17}, {0.5349976198870973, -5.3683132708358134e-17},
+    {0.5555702330196022, 4.709410940561677e-17}, {0.5758081914178453, -3.7909495458942734e-17},
+    {0.5956993044924334, -1.3438641936579467e-17}, {0.6152315905806268, 2.623141776726695e-17},
+    {0.6343932841636455, 1.0420901929280035e-17}, {0.6531728429537768, 8.569564206002624e-18},
+    {0.6715589548470184, -4.048903774929669e-17}, {0.6895405447370669, -1.588932329480679e-17},
+    {0.7071067811865476, -4.833646656726457e-17}, {0.7242470829514669, 2.9198471334403004e-17},
+    {0.7409511253549591, -1.4708616952297345e-17}, {0.7572088465064846, -1.9909098777335502e-17},
+    {0.773010453362737, -3.256590703364977e-17}, {0.7883464276266062, 3.439699315405971e-17},
+    {0.8032075314806449, -3.306060980481491e-17}, {0.8175848131515837, -1.4883149812426772e-17},
+    {0.8314696123025452, 1.4073856984728024e-18}, {0.8448535652497071, -4.363136029687964e-17},
+    {0.8577286100002721, -4.818344793633662e-17}, {0.8700869911087115, -4.188851086854997e-17},
+    {0.881921264348355, -1.9843248405890562e-17}, {0.8932243011955153, -4.116123915190891e-18},
+    {0.9039892931234433, -6.609754468748431e-18}, {0.9142097557035307, -3.631618252781442e-17},
+    {0.9238795325112867, 1.7645047084336677e-17}, {0.9329927988347388, 4.2041415555384355e-17},
+    {0.9415440651830208, -2.789637954769834e-17}, {0.9495281805930367, -7.55441519280433e-18},
+    {0.9569403357322088, 4.05538698618757e-17}, {0.9637760657954398, 2.646395056122003e-17},
+    {0.970031253194544, 1.8365300348428844e-17}, {0.9757021300385286, -2.5572556081259686e-17},
+    {0.9807852804032304, 1.8546939997825006e-17}, {0.9852776423889412, 2.3155637027900207e-17},
+    {0.989176509964781, -4.098730993704711e-17}, {0.99247953459871, 3.1093055095428906e-17},
+    {0.9951847266721969, -4.248691367830441e-17}, {0.9972904566786902, 9.164769537110173e-18},
+    {0.9987954562051724, -1.2291693337075465e-17}, {0.9996988186962042, -2.985148640379975e-17},
+    {1.0, 0.0},
+};
+
+// sin(pi i / 128) for i = 0..255, the table of sincos_tab.
+GH_HD inline dd_t sin_tab_entry(int i)
+{
+    const int q = i & 127;
+    const dd_t v = kSinTab[q <= 64 ? q : 128 - q];
+    return i & 128 ? dd_neg(v) : v;
+}
+
+// As sincos_cr (rounded to nearest but for ~1e-5 of arguments, |x| < 2^29,
+// else NaN) from a table of sin_tab_entry: x = k pi/128 + r reduced exactly,
+// |r| <= pi/256, and the sum formulas with the table's double-doubles.  Only
+// the leading terms sin r ~ r and cos r - 1 ~ -r^2/2 are carried in
+// double-double; what is left is below 4e-7, so that its rounding is below
+// 2^-74.  About 110 instructions, 371 for sincos_cr.
+GH_HD inline sc_t sincos_tab(double x, const dd_t* tab)
+{
+#pragma clang fp contract(off)
+    constexpr double kInvP = 40.74366543152521, P1 = 0.02454369260617026, P2 = 9.567553118338697e-19, P3 = -2.3396639138424529e-35;
+    constexpr double kRound = 6755399441055744.0;  // 1.5 2^52: the sum's low bits are the integer
+    const double ks = fma(x, kInvP, kRound), k = ks - kRound;
+    unsigned long long kb;
+    __builtin_memcpy(&kb, &ks, sizeof kb);
+    const int j = (int)(kb & 255);
+    const dd_t p1 = dd_prod(k, P1);
+    // x - p1.h is exact (Sterbenz)
+    dd_t r = dd_sum(x - p1.h, -p1.l);
+    {
+        const dd_t p2 = dd_prod(k, P2), t = dd_sum(r.h, -p2.h);
+        const double l = t.l + ((r.l - p2.l) - k * P3);
+        r.h = t.h + l;
+        r.l = l - (r.h - t.h);
+    }
+    const double p = r.h * r.h, e = fma(r.h, r.h, -p) + 2.0 * (r.h * r.l);  // r^2
+    // sin r - r.h and cos r - 1 + p/2
+    double q = fma(p, 1.0 / 362880.0, -1.0 / 5040.0);
+    q = fma(q, p, 1.0 / 120.0);
+    q = fma(q, p, -1.0 / 6.0);
+    const double sr = fma(r.h * p, q, fma(-0.5 * p, r.l, r.l));
+    q = fma(p, 1.0 / 40320.0, -1.0 / 720.0);
+    q = fma(q, p, 1.0 / 24.0);
+    const double cr = fma(p * p, q, -0.5 * e), ch = -0.5 * p;
+    const dd_t S = tab[j], C = tab[(j + 64) & 255];
+    sc_t o;
+    {
+        const dd_t t = dd_prod(C.h, r.h), u = dd_prod(S.h, ch), a = dd_sum(S.h, t.h), b = dd_sum(a.h, u.h);
+        double l = fma(C.h, sr, fma(C.l, r.h, fma(S.h, cr, fma(S.l, ch, S.l))));
+        l = (t.l + u.l) + l;
+        o.s = b.h + ((a.l + b.l) + l);
+    }
+    {
+        const dd_t t = dd_prod(-S.h, r.h), u = dd_prod(C.h, ch), a = dd_sum(C.h, t.h), b = dd_sum(a.h, u.h);
+        double l = fma(-S.h, sr, fma(-S.l, r.h, fma(C.h, cr, fma(C.l, ch, C.l))));
+        l = (t.l + u.l) + l;
+        o.c = b.h + ((a.l + b.l) + l);
+    }
+    if (!(fabs(x) < 536870912.0)) o.s = o.c = __builtin_nan("");
+    return o;
+}
+
 // atan(k/8), k = 0..8, and 2^(j/64), j = 0..63, as double-double (values
 // computed at 200-bit precision for this library).
 constexpr dd_t kAtanTab[9] = {

@@ -8,9 +8,7 @@
 //                     phase splines, phase at spacecraft 1, the 24 delayed
 //                     one-arm terms of X,Y,Z (LISA_spline_response), their
 //                     amplitude/phase (extract_amplitude_and_phase,
-//                     unwrap_phase) and the six TDI splines.  The serial
-//                     parts (tridiagonal sweeps, sign-flip scan, unwrap)
-//                     run one spline / channel per lane, side by side.
+//                     unwrap_phase) and the six TDI splines.
 //  K2 layer_kernel  : the heterodyned series at NT*(L+1) samples (LDS),
 //                     a packed real FFT (X+iY in one complex FFT, Z as
 //                     half-length), per layer the Meyer-windowed band and
@@ -38,7 +36,7 @@ namespace wdm {
 
 // ------------------------------------------------------------ TDI table --
 
-__constant__ TdiTerm c_tdi[8] = {
+constexpr TdiTerm kTdi[8] = {
     {0, 2, 1, +1, 0, 1, -1, 1, 2, 2.0, 2.0},
     {1, 2, 1, -1, 0, 2, +1, 1, 2, 1.0, 2.0},
     {2, 1, 2, +1, 1, 1, -1, 0, 1, 1.0, 2.0},
@@ -84,7 +82,7 @@ void spline_host(int N, const double* x, const double* y, double* c)
 
 // x-only terms of the recurrence: dx | l | mu | 1/l (N each; the
 // reciprocals correctly rounded, for spline_sweep's division)
-static void spline_prep_host(int N, const double* x, double* p)
+static void spline_prep_host(int N, const double* x, double* p, int* warm)
 {
 #pragma clang fp contract(off)
     double *dx = p, *l = p + N, *mu = p + 2 * N, *rl = p + 3 * N;
@@ -98,6 +96,20 @@ static void spline_prep_host(int N, const double* x, double* p)
         mu[i] = dx[i] / l[i];
     }
     for (int i = 0; i < N; i++) rl[i] = 1.0 / l[i];
+    // knots after which either recurrence holds less than 2^-80 of what it
+    // started from (42 on even knots)
+    *warm = 1;
+    for (int i = 1; i < N - 1; i++)
+    {
+        double f = 1.0, b = 1.0;
+        int n = 0;
+        for (int j = i; j < N - 1 && (f > 0x1p-80 || b > 0x1p-80); j++, n++)
+        {
+            f *= dx[j - 1] / l[j];
+            b *= mu[j];
+        }
+        if (n > *warm) *warm = n;
+    }
 }
 
 // ------------------------------------------------------ host: geometry --
@@ -164,6 +176,7 @@ struct Geo
     const double* prep_o;  // 4 x Norb  dx | l | mu | 1/l on the orbit knots
     const double* tssb;    // Norb response times t0 + i Tobs/(Norb-1)
     const double* prep_s;  // 4 x Norb  on the response times
+    int warm_o, warm_s;    // spline_prep_host's warm of both
     const double* resp;    // Norb x 24: x[3][3]/c, n[3][3], L[3] at tssb
     // per layer count L (slot L; a forced count Lf in slot kForcedSlot):
     const double* ds[kForcedSlot + 1];   // N_ds x 5: t, r0x, r0y, r0z, dx
@@ -230,10 +243,10 @@ static int geo_build(GeoHost& G, const glass_hip_wdm& w, int Norb, const double*
     g.ods = ot[1] - ot[0];
     std::vector<double> oc(9 * 4 * N), prep_o(4 * N), tssb(N), prep_s(4 * N), resp(24 * N, 0.0);
     for (int s = 0; s < 9; s++) spline_host(N, ot.data(), pos + s * N, oc.data() + 4 * s * N);
-    spline_prep_host(N, ot.data(), prep_o.data());
+    spline_prep_host(N, ot.data(), prep_o.data(), &g.warm_o);
     const double dts = Tobs / (double)(N - 1);
     for (int i = 0; i < N; i++) tssb[i] = t0 + i * dts;
-    spline_prep_host(N, tssb.data(), prep_s.data());
+    spline_prep_host(N, tssb.data(), prep_s.data(), &g.warm_s);
     if (tssb[0] < ot[0] || tssb[N - 1] > ot[N - 1])
     {
         set_error("wavelet waveform: response times [%g, %g] outside the orbit knots [%g, %g]",
@@ -352,16 +365,16 @@ __host__ __device__ inline size_t scratch_doubles(int N) { return 64 + 28 * (siz
 
 constexpr int kRespThreads = 256;
 
-// LDS of K1 in doubles: ssb 8N | M,Mf 6N | As 3N | flip,pjump 6N | phase_sc N.
-// The sweep scratch of the splines lives in regions dead by then: the two
-// barycentre sweeps use M,Mf (not yet written), the six TDI sweeps use ssb
-// (z) and As + flip (y2), dead after the signed amplitude/phase step.
-// Then the sign-flip scan's knot flags: per channel three bit masks (local
-// minimum, the d2 and d3 tests) of kMaxKnots bits.
+// LDS of K1 in doubles: sine table 512 | ssb 8N | M,Mf 6N | As 3N | z 3N |
+// phase_sc N.  The splines' right-hand sides and sweeps live in regions dead by
+// then: the two barycentre splines in M,Mf (not yet written), the six TDI
+// splines in ssb (right-hand sides, then y2) and As + z (the forward sweeps),
+// dead after the signed amplitude/phase step.  Then the sign-flip scan's knot
+// flags: per channel the d2 and d3 tests and the flips, kMaxKnots bits each.
 constexpr int kFlagWords = kMaxKnots / 64;
 __host__ __device__ inline size_t resp_lds_bytes(int N)
 {
-    return sizeof(double) * 24 * (size_t)N + sizeof(Hdr) + sizeof(unsigned long long) * 9 * kFlagWords;
+    return sizeof(double) * (512 + 21 * (size_t)N) + sizeof(unsigned long long) * 9 * kFlagWords;
 }
 
 // Per-template constants, one thread per template, into each template's
@@ -387,30 +400,51 @@ __device__ inline void spline_alpha(int N, const double* __restrict__ prep, cons
     z[i] = 3.0 * ((y[i + 1] - y[i]) / dx[i] - (y[i] - y[i - 1]) / dx[i - 1]);
 }
 
-// One lane's tridiagonal sweep of that spline, z holding the alpha_i of
-// spline_alpha: writes z and y2 (N each).  Only the recurrence itself is
-// serial; its division by l_i goes through the precomputed 1/l_i.
-__device__ inline void spline_sweep(int N, const double* __restrict__ prep, double* z, double* y2)
+// The tridiagonal sweeps of that spline over chunk c of kSweepChunks, one lane
+// each: alpha (spline_alpha) -> z, and after a barrier z -> y2.  Only the
+// recurrence itself is serial (its division by l_i goes through the precomputed
+// 1/l_i) and it forgets: each knot keeps 0.27 of the one before, so a chunk that
+// starts `warm` knots early from zero holds the value of the whole sweep (2^-80
+// of it is left out, 2^-27 of its last bit).  62 dependent steps for 202 knots
+// instead of 202.
+constexpr int kSweepChunks = 10;
+__device__ inline void sweep_range(int N, int c, int* lo, int* hi)
+{
+    const int len = (N - 2 + kSweepChunks - 1) / kSweepChunks;
+    *lo = 1 + c * len;
+    *hi = min(N - 1, *lo + len);
+}
+__device__ inline void spline_forward(int N, const double* __restrict__ prep, const double* alpha, double* z, int c,
+                                      int warm)
 {
 #pragma clang fp contract(off)
-    const double *dx = prep, *l = prep + N, *mu = prep + 2 * N, *rl = prep + 3 * N;
-    z[0] = 0.0;
+    const double *dx = prep, *l = prep + N, *rl = prep + 3 * N;
+    int lo, hi;
+    sweep_range(N, c, &lo, &hi);
+    if (c == 0) z[0] = 0.0;
     double zp = 0.0;
 #pragma unroll 4
-    for (int i = 1; i < N - 1; i++)
+    for (int i = max(1, lo - warm); i < hi; i++)
     {
-        const double alpha = z[i];
-        zp = div_by_recip(alpha - dx[i - 1] * zp, l[i], rl[i]);
-        z[i] = zp;
+        zp = div_by_recip(alpha[i] - dx[i - 1] * zp, l[i], rl[i]);
+        if (i >= lo) z[i] = zp;
     }
-    z[N - 1] = 0.0;
+}
+__device__ inline void spline_backward(int N, const double* __restrict__ prep, const double* z, double* y2, int c,
+                                       int warm)
+{
+#pragma clang fp contract(off)
+    const double* mu = prep + 2 * N;
+    int lo, hi;
+    sweep_range(N, c, &lo, &hi);
+    if (c == 0) lo = 0;
+    if (c == kSweepChunks - 1) y2[N - 1] = 0.0;
     double yn = 0.0;
-    y2[N - 1] = 0.0;
 #pragma unroll 4
-    for (int i = N - 2; i >= 0; i--)
+    for (int i = min(N - 2, hi - 1 + warm); i >= lo; i--)
     {
         yn = z[i] - mu[i] * yn;
-        y2[i] = yn;
+        if (i < hi) y2[i] = yn;
     }
 }
 
@@ -430,14 +464,16 @@ __device__ inline void spline_finish(int N, int i, const double* __restrict__ pr
     *y3o = (y2[i + 1] - y2[i]) / (3.0 * dx);
 }
 
-// a[i] of a 3-element register array for a runtime i in 0..2, by selects
-// (an indexed private array would live in scratch memory)
-__device__ inline double pick3(const double (&a)[3], int i) { return i == 0 ? a[0] : (i == 1 ? a[1] : a[2]); }
-
-// four waves per SIMD (128 VGPRs): four 256-thread workgroups per CU,
-// as many as the 24N-double LDS footprint allows
-__global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) resp_kernel(Geo g, int n, const double* __restrict__ params,
-                                                            double* __restrict__ scratch)
+// Vector issue bounds it (65% busy), most of it in the 24 delayed terms of
+// a knot.  Their sine and cosine come from a table in LDS (sincos_tab); the
+// vertices and arms are permuted for the channel as they are loaded, so the
+// eight terms are written out without selects; and what is serial along the
+// knots, which one wave worked while three waited, is cut into chunks (the
+// splines), bits (the flips) and a prefix sum (the unwrapping).  4096 templates
+// of 202 knots: 718 -> 362 us.  Four waves per SIMD (128 VGPRs): four 256-thread
+// workgroups per CU, as many as the LDS allows.
+__global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) resp_kernel(
+    Geo g, int n, double* __restrict__ scratch)
 {
 #pragma clang fp contract(off)
     const int e = blockIdx.x;
@@ -445,20 +481,22 @@ __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_
     extern __shared__ double lds[];
     const int N = g.Norb;
     const int tid = threadIdx.x;
-    double* ssb = lds;               // amp y0..y3 | phase y0..y3
+    dd_t* tab = (dd_t*)lds;          // sin_tab_entry
+    double* ssb = lds + 512;         // amp y0..y3 | phase y0..y3
     double* Mx = ssb + 8 * N;        // M X,Y,Z | Mf X,Y,Z
-    double* As = Mx + 6 * N;         // |M| X,Y,Z
-    double* fl = As + 3 * N;         // flip X,Y,Z | pjump X,Y,Z
-    double* phsc = fl + 6 * N;       // phase at spacecraft 1
-    Hdr* H = (Hdr*)(phsc + N);
-    unsigned long long* flg = (unsigned long long*)(H + 1);  // 9 x kFlagWords
+    double* As = Mx + 6 * N;         // |M| X,Y,Z, and 3N more
+    double* phsc = As + 6 * N;       // phase at spacecraft 1
+    unsigned long long* flg = (unsigned long long*)(phsc + N);  // 9 x kFlagWords
     double* scr = scratch + scratch_doubles(N) * (size_t)e;
-    (void)params;
 
-    // the header hdr_kernel wrote
-    for (int i = tid; i < (int)(sizeof(Hdr) / sizeof(double)); i += kRespThreads) ((double*)H)[i] = scr[i];
-    __syncthreads();
-    const Hdr h = *H;
+    // the header hdr_kernel wrote, by scalar loads
+    Hdr h;
+    {
+        auto hs = (const __attribute__((address_space(4))) double*)scr;
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(Hdr) / sizeof(double)); i++) ((double*)&h)[i] = hs[i];
+    }
+    for (int i = tid; i < 256; i += kRespThreads) tab[i] = sin_tab_entry(i);
     // barycentre amplitude and phase at the orbit knots
     for (int i = tid; i < N; i += kRespThreads)
     {
@@ -473,7 +511,13 @@ __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_
         spline_alpha(N, g.prep_o, ssb + 4 * N * sp, Mx + N * sp, i);
     }
     __syncthreads();
-    if (tid < 2) spline_sweep(N, g.prep_o, Mx + N * tid, ssb + 4 * N * tid + 2 * N);
+    {
+        const int sp = tid / kSweepChunks, c = tid % kSweepChunks;
+        double* z = Mx + (2 + sp) * N;
+        if (sp < 2) spline_forward(N, g.prep_o, Mx + N * sp, z, c, g.warm_o);
+        __syncthreads();
+        if (sp < 2) spline_backward(N, g.prep_o, z, ssb + 4 * N * sp + 2 * N, c, g.warm_o);
+    }
     __syncthreads();
     for (int i = tid; i < 2 * N; i += kRespThreads)
     {
@@ -483,6 +527,12 @@ __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_
     }
     __syncthreads();
     const double* cph = ssb + 4 * N;
+    const double rds = 1.0 / g.ods;
+    // even_index with the division by the knot spacing through its reciprocal
+    auto knot = [&](double x) {
+        const int j = (int)floor(div_by_recip(x - g.ot0, g.ods, rds));
+        return min(max(j, 0), N - 1);
+    };
     // export the barycentre phase spline for the layer kernel
     for (int i = tid; i < 4 * N; i += kRespThreads) scr[64 + i] = cph[i];
     // phase at spacecraft 1 (LISA_spacecraft_to_barycenter_time, flag -1)
@@ -492,66 +542,66 @@ __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_
         double kdotr = 0.0;
         for (int i = 0; i < 3; i++) kdotr += h.k[i] * r[i];
         const double tsc = g.tssb[m] - kdotr;
-        const int j = even_index(tsc, g.ot0, g.ods, N);
+        const int j = knot(tsc);
         phsc[m] = spline_at(cph, N, j, tsc - g.ot[j]);
     }
-    // the X, Y, Z responses: items (sample m, channel ch)
+    // the X, Y, Z responses: items (sample m, channel ch), vertex and arm i of
+    // the channel's permutation being (ch + i) mod 3
     for (int it = tid; it < 3 * N; it += kRespThreads)
     {
         const int m = it / 3, ch = it % 3;
         const double* r = g.resp + 24 * m;
-        const double* x = r;          // x[i][j] at 3i+j
-        const double* nn = r + 9;
-        const double* L = r + 18;
-        double kr[3], kn[3], App[3], Apm[3], Acp[3], Acm[3];
+        double kr[3], L[3], App[3], Apm[3], Acp[3], Acm[3];
+#pragma unroll
         for (int i = 0; i < 3; i++)
         {
+            const int v = ch + i < 3 ? ch + i : ch + i - 3;
+            const double *x = r + 3 * v, *nn = r + 9 + 3 * v;
+            L[i] = r[18 + v];
             kr[i] = 0.0;
-            for (int j = 0; j < 3; j++) kr[i] += h.k[j] * x[3 * i + j];
-        }
-        for (int i = 0; i < 3; i++)
-        {
-            kn[i] = 0.0;
-            for (int j = 0; j < 3; j++) kn[i] += h.k[j] * nn[3 * i + j];
-        }
-        for (int i = 0; i < 3; i++)
-        {
-            double dp = 0.0, dc = 0.0;
+            double kn = 0.0;
+#pragma unroll
             for (int j = 0; j < 3; j++)
+            {
+                kr[i] += h.k[j] * x[j];
+                kn += h.k[j] * nn[j];
+            }
+            double dp = 0.0, dc = 0.0;
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+#pragma unroll
                 for (int l = 0; l < 3; l++)
                 {
-                    dp += (nn[3 * i + j] * nn[3 * i + l]) * h.ep[3 * j + l];
-                    dc += (nn[3 * i + j] * nn[3 * i + l]) * h.ec[3 * j + l];
+                    dp += (nn[j] * nn[l]) * h.ep[3 * j + l];
+                    dc += (nn[j] * nn[l]) * h.ec[3 * j + l];
                 }
-            App[i] = dp / (1.0 + kn[i]);
-            Apm[i] = dp / (1.0 - kn[i]);
-            Acp[i] = dc / (1.0 + kn[i]);
-            Acm[i] = dc / (1.0 - kn[i]);
+            const double bp = 1.0 + kn, bm = 1.0 - kn, rp = 1.0 / bp, rm = 1.0 / bm;
+            App[i] = div_by_recip(dp, bp, rp);
+            Apm[i] = div_by_recip(dp, bm, rm);
+            Acp[i] = div_by_recip(dc, bp, rp);
+            Acm[i] = div_by_recip(dc, bm, rm);
         }
         const double t = g.tssb[m];
         double M = 0.0, Mf = 0.0;
-#pragma unroll 1
+#pragma unroll
         for (int q = 0; q < 8; q++)
         {
-            const TdiTerm T = c_tdi[q];
-            // vertex permutation of channel ch: vtx[i] = (ch + i) mod 3
-            const int vv = (ch + T.v) % 3, v1 = (ch + T.i1) % 3, v2 = (ch + T.i2) % 3;
-            const double te = t - pick3(kr, vv) - T.m1 * L[v1] - T.m2 * L[v2];
-            const int j = even_index(te, g.ot0, g.ods, N);
+            const TdiTerm T = kTdi[q];
+            const double te = t - kr[T.v] - T.m1 * L[T.i1] - T.m2 * L[T.i2];
+            const int j = knot(te);
             const double dx = te - g.ot[j];
             const double a = spline_at(ssb, N, j, dx);
             const double ph = spline_at(cph, N, j, dx);
             // correctly rounded: the channel sums cancel by (f/f*)^2, which
             // would magnify one-ulp differences of sin/cos
-            double sp, cp;
-            sincos_cr(ph, &sp, &cp);
+            const sc_t sc = sincos_tab(ph, tab);
+            const double sp = sc.s, cp = sc.c;
             const double hp = a * (h.Ap * h.c2p * cp + h.Ac * h.s2p * sp);
             const double hc = a * (h.Ac * h.c2p * sp - h.Ap * h.s2p * cp);
             const double hpf = a * (-h.Ap * h.c2p * sp + h.Ac * h.s2p * cp);
             const double hcf = a * (h.Ac * h.c2p * cp + h.Ap * h.s2p * sp);
-            const int j1 = (ch + T.j1) % 3, j2 = (ch + T.j2) % 3;
-            const double P1 = T.pm1 ? pick3(App, j1) : pick3(Apm, j1), Q1 = T.pm1 ? pick3(Acp, j1) : pick3(Acm, j1);
-            const double P2 = T.pm2 ? pick3(App, j2) : pick3(Apm, j2), Q2 = T.pm2 ? pick3(Acp, j2) : pick3(Acm, j2);
+            const double P1 = T.pm1 ? App[T.j1] : Apm[T.j1], Q1 = T.pm1 ? Acp[T.j1] : Acm[T.j1];
+            const double P2 = T.pm2 ? App[T.j2] : Apm[T.j2], Q2 = T.pm2 ? Acp[T.j2] : Acm[T.j2];
             double v;
             v = hp * P1 + hc * Q1;
             M = T.s1 > 0 ? M + v : M - v;
@@ -561,6 +611,7 @@ __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_
             Mf = T.s1 > 0 ? Mf + v : Mf - v;
             v = hpf * P2 + hcf * Q2;
             Mf = T.s2 > 0 ? Mf + v : Mf - v;
+            __builtin_amdgcn_sched_barrier(0);  // one term's temporaries at a time
         }
         Mx[ch * N + m] = M;
         Mx[(3 + ch) * N + m] = Mf;
@@ -568,128 +619,133 @@ __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_
     }
     __syncthreads();
     // sign flips of the amplitude (extract_amplitude_and_phase,
-    // utils/src/glass_math.c:1244-1296).  The tests at each knot (a local
-    // minimum of |M|, then |d2/d1| < 0.1 and |d3/d1| < 0.1) need no state:
-    // every wave evaluates 64 knots of a channel at once into ballot masks;
-    // one lane per channel then walks the knots in the reference's order
-    // (a d2 hit skips the next knot), holding the running flip and phase
-    // jump in registers.
+    // utils/src/glass_math.c:1244-1296): at a local minimum of |M| the tests
+    // |d2/d1| < 0.1 (the amplitude and its phase jump flip at the next knot,
+    // which is then skipped) and |d3/d1| < 0.1 (they flip at this one).  The
+    // tests need no state: every wave evaluates 64 knots of a channel into
+    // ballot masks.  One lane per channel walks the knots that pass one, in
+    // the reference's order, and leaves a mask of the flips.
+    const int NWd = (N + 63) / 64, lane = tid & 63;
+    for (int b = tid >> 6; b < 3 * NWd; b += kRespThreads / 64)
     {
-        const int NWd = (N + 63) / 64, lane = tid & 63;
-        for (int b = tid >> 6; b < 3 * NWd; b += kRespThreads / 64)
+        const int ch = b / NWd, w = b % NWd, i = w * 64 + lane;
+        bool t2 = false, t3 = false;
+        if (i >= 1 && i <= N - 2)
         {
-            const int ch = b / NWd, w = b % NWd, i = w * 64 + lane;
-            bool mn = false, t2 = false, t3 = false;
-            if (i >= 1 && i <= N - 2)
+            const double* A = As + ch * N;
+            if (A[i] < A[i - 1] && A[i] < A[i + 1])
             {
-                const double* A = As + ch * N;
-                mn = A[i] < A[i - 1] && A[i] < A[i + 1];
-                if (mn)
-                {
-                    const double d1 = A[i + 1] + A[i - 1] - 2.0 * A[i];
-                    const double d2 = -A[i + 1] + A[i - 1] - 2.0 * A[i];
-                    const double d3 = -A[i + 1] + A[i - 1] + 2.0 * A[i];
-                    t2 = fabs(d2 / d1) < 0.1;
-                    t3 = fabs(d3 / d1) < 0.1;
-                }
+                const double d1 = A[i + 1] + A[i - 1] - 2.0 * A[i];
+                const double d2 = -A[i + 1] + A[i - 1] - 2.0 * A[i];
+                const double d3 = -A[i + 1] + A[i - 1] + 2.0 * A[i];
+                t2 = fabs(d2 / d1) < 0.1;
+                t3 = fabs(d3 / d1) < 0.1;
             }
-            const unsigned long long m0 = __ballot(mn), m2 = __ballot(t2), m3 = __ballot(t3);
-            if (lane == 0)
-            {
-                flg[(ch * 3 + 0) * kFlagWords + w] = m0;
-                flg[(ch * 3 + 1) * kFlagWords + w] = m2;
-                flg[(ch * 3 + 2) * kFlagWords + w] = m3;
-            }
+        }
+        const unsigned long long m2 = __ballot(t2), m3 = __ballot(t3);
+        if (lane == 0)
+        {
+            flg[(ch * 3 + 0) * kFlagWords + w] = m2;
+            flg[(ch * 3 + 1) * kFlagWords + w] = m3;
+            flg[(ch * 3 + 2) * kFlagWords + w] = 0;
         }
     }
     __syncthreads();
     if (tid < 3)
     {
-        const unsigned long long* fm = flg + tid * 3 * kFlagWords;
-        double* flip = fl + tid * N;
-        double* pj = fl + (3 + tid) * N;
-        flip[0] = 1.0;
-        pj[0] = 0.0;
-        double pf = 1.0, pp = 0.0;  // flip[i-1], pj[i-1]
-        int wc = -1;
-        unsigned long long wm = 0, w2 = 0, w3 = 0;
+        const unsigned long long *f2 = flg + tid * 3 * kFlagWords, *f3 = f2 + kFlagWords;
+        unsigned long long* fl = flg + tid * 3 * kFlagWords + 2 * kFlagWords;
         int i = 1;
-        do
+        while (i < N - 1)
         {
-            double cf = pf, cp = pp;  // flip[i] = flip[i-1]
             const int w = i >> 6;
-            if (w != wc)
+            const unsigned long long m = (f2[w] | f3[w]) >> (i & 63);
+            if (!m)
             {
-                wc = w;
-                wm = fm[w];
-                w2 = fm[kFlagWords + w];
-                w3 = fm[2 * kFlagWords + w];
+                i = (w + 1) * 64;
+                continue;
             }
-            const unsigned long long bit = 1ull << (i & 63);
-            if (wm & bit)
-            {
-                const bool b2 = (w2 & bit) != 0, b3 = (w3 & bit) != 0;
-                if (b2)
-                {
-                    // flip[i+1] = -flip[i], pj[i+1] = pj[i] + pi; i++
-                    flip[i] = cf;
-                    pj[i] = cp;
-                    pf = cf;
-                    pp = cp;
-                    cf = -1.0 * cf;
-                    cp = cp + M_PI;
-                    i++;
-                }
-                if (b3)
-                {
-                    // flip[i] = -flip[i-1], pj[i] = pj[i-1] + pi
-                    cf = -1.0 * pf;
-                    cp = pp + M_PI;
-                }
-            }
-            flip[i] = cf;
-            pj[i] = cp;
-            pf = cf;
-            pp = cp;
-            i++;
-        } while (i < N - 1);
-        flip[N - 1] = flip[N - 2];
-        pj[N - 1] = pj[N - 2];
+            i += __ffsll(m) - 1;
+            const bool b2 = (f2[w] >> (i & 63)) & 1;  // else b3
+            const int at = b2 ? i + 1 : i;
+            if (at < N) fl[at >> 6] |= 1ull << (at & 63);
+            i = at + 1;
+        }
     }
     __syncthreads();
-    // signed amplitude and phase relative to the spacecraft-1 carrier
+    // signed amplitude and phase relative to the spacecraft-1 carrier; the
+    // last knot has the flips of the one before
     for (int it = tid; it < 3 * N; it += kRespThreads)
     {
-        const int ch = it / N, i = it % N;
+        const int ch = it / N, i = it % N, k = min(i, N - 2);
+        const unsigned long long* fl = flg + ch * 3 * kFlagWords + 2 * kFlagWords;
+        int flips = __popcll(fl[k >> 6] << (63 - (k & 63)));
+        for (int w = 0; w < k >> 6; w++) flips += __popcll(fl[w]);
+        double pj = 0.0;
+        for (int w = 0; w < flips; w++) pj += M_PI;
         const double M = Mx[ch * N + i], Mf = Mx[(3 + ch) * N + i];
         const double v = remainder(phsc[i], PI2);
-        Mx[ch * N + i] = fl[ch * N + i] * As[ch * N + i];
-        Mx[(3 + ch) * N + i] = -atan2_cr(Mf, M) + fl[(3 + ch) * N + i] - v;
+        Mx[ch * N + i] = flips & 1 ? -As[ch * N + i] : As[ch * N + i];
+        Mx[(3 + ch) * N + i] = -atan2_cr(Mf, M) + pj - v;
     }
     __syncthreads();
-    // unwrap_phase (utils/src/glass_math.c:1034-1052)
-    if (tid < 3)
+    // unwrap_phase (utils/src/glass_math.c:1034-1052), one wave per channel:
+    // the turns added at a knot are those of the one before and the difference
+    // of the two phases in turns, rounded, so they are a prefix sum.  Where a
+    // difference is within 1e-6 of half a turn (or is NaN) the rounding of the
+    // unwrapped phase decides, and one lane walks the knots.
+    if (tid < 192)
     {
         constexpr double kInvPI2 = 1.0 / PI2;  // correctly rounded (compile time)
-        double* ph = Mx + (3 + tid) * N;
-        double v = ph[0];
-#pragma unroll 4
-        for (int i = 0; i < N; i++)
+        double* ph = Mx + (3 + (tid >> 6)) * N;
+        bool near = false;
+        for (int i = 1 + lane; i < N; i += 64)
         {
-            double u = ph[i];
-            const double q = rint(div_by_recip(fabs(u - v), PI2, kInvPI2));
-            if (q > 0.0)
+            const double f = (ph[i - 1] - ph[i]) * kInvPI2;
+            near = near || !(fabs(f - rint(f)) < 0.499999);
+        }
+        if (__ballot(near) == 0)
+        {
+            double turns = 0.0, last = ph[0];
+            for (int i0 = 0; i0 < N; i0 += 64)
             {
-                if (v > u) u += q * PI2;
-                else u -= q * PI2;
+                const int i = i0 + lane;
+                const double p = ph[min(i, N - 1)];
+                double b = __shfl_up(p, 1, 64);
+                if (lane == 0) b = last;
+                double d = rint((b - p) * kInvPI2);
+#pragma unroll
+                for (int w = 1; w < 64; w <<= 1)
+                {
+                    const double o = __shfl_up(d, w, 64);
+                    if (lane >= w) d += o;
+                }
+                d += turns;
+                if (i < N) ph[i] = p + d * PI2;
+                turns = __shfl(d, 63, 64);
+                last = __shfl(p, 63, 64);
             }
-            v = u;
-            ph[i] = u;
+        }
+        else if (lane == 0)
+        {
+            double v = ph[0];
+#pragma unroll 4
+            for (int i = 0; i < N; i++)
+            {
+                double u = ph[i];
+                const double q = rint(div_by_recip(fabs(u - v), PI2, kInvPI2));
+                if (q > 0.0)
+                {
+                    if (v > u) u += q * PI2;
+                    else u -= q * PI2;
+                }
+                v = u;
+                ph[i] = u;
+            }
         }
     }
     __syncthreads();
     // six TDI splines on the response times: spline s = 2*ch + (0 amp, 1 phase)
-    double* y2s = As;  // 6N over As and the flip half of fl
     for (int it = tid; it < 6 * (N - 2); it += kRespThreads)
     {
         const int sp = it / (N - 2), i = 1 + it % (N - 2);
@@ -697,14 +753,19 @@ __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_
         spline_alpha(N, g.prep_s, Mx + (3 * ph + ch) * N, ssb + sp * N, i);
     }
     __syncthreads();
-    if (tid < 6) spline_sweep(N, g.prep_s, ssb + tid * N, y2s + tid * N);
+    {
+        const int sp = tid / kSweepChunks, c = tid % kSweepChunks;
+        if (sp < 6) spline_forward(N, g.prep_s, ssb + sp * N, As + sp * N, c, g.warm_s);
+        __syncthreads();
+        if (sp < 6) spline_backward(N, g.prep_s, As + sp * N, ssb + sp * N, c, g.warm_s);
+    }
     __syncthreads();
     for (int it = tid; it < 6 * N; it += kRespThreads)
     {
         const int s = it / N, i = it % N;
         const int ch = s >> 1, ph = s & 1;
         const double* y0 = Mx + (3 * ph + ch) * N;
-        const double* y2 = y2s + s * N;
+        const double* y2 = ssb + s * N;
         double y1, y3;
         spline_finish(N, i, g.prep_s, y0, y2, &y1, &y3);
         double* c = scr + 64 + 4 * N + 4 * (size_t)N * s;
@@ -1195,8 +1256,7 @@ static int launch_templates(const GeoHost& G, int n, const double* d_params, dou
     const Geo& g = G.g;
     if (n <= 0) return GLASS_HIP_OK;
     hipLaunchKernelGGL(hdr_kernel, dim3((n + 255) / 256), dim3(256), 0, s, g, n, d_params, d_scratch);
-    hipLaunchKernelGGL(resp_kernel, dim3(n), dim3(kRespThreads), resp_lds_bytes(g.Norb), s, g, n, d_params,
-                       d_scratch);
+    hipLaunchKernelGGL(resp_kernel, dim3(n), dim3(kRespThreads), resp_lds_bytes(g.Norb), s, g, n, d_scratch);
     GH_CHECK(hipGetLastError());
     if (g.NT >= 1024 || g.Lf > 0)
     {

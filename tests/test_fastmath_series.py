@@ -29,12 +29,18 @@ def fm(tmp_path_factory):
                    ' double a[1] = {x[i]}, r[1], m[1], s[1], c[1], d[1];'
                    ' glass::sinc_phase<1>(a, w, r, m); glass::sinc_values<true, 1>(a, w, s, c, d);'
                    ' double* q = o + 5 * i; q[0] = r[0]; q[1] = m[0]; q[2] = s[0]; q[3] = c[0]; q[4] = d[0]; } }\n')
+    with src.open("a") as f:
+        f.write('extern "C" void f_sctab(const double* x, double* s, double* c, int n) {'
+                ' glass::dd_t t[256]; for (int i = 0; i < 256; i++) t[i] = glass::sin_tab_entry(i);'
+                ' for (int i = 0; i < n; i++) { glass::sc_t v = glass::sincos_tab(x[i], t);'
+                ' s[i] = v.s; c[i] = v.c; } }\n')
     so = d / "fs.so"
     subprocess.run(["g++", "-O2", "-ffp-contract=off", "-std=c++17", "-shared", "-fPIC", "-I",
                     os.path.join(ROOT, "glass_amd", "csrc"), str(src), "-o", str(so)], check=True)
     L = ctypes.CDLL(str(so))
     dp = ctypes.POINTER(ctypes.c_double)
     L.f_sincos.argtypes = [dp, dp, dp, ctypes.c_int]
+    L.f_sctab.argtypes = [dp, dp, dp, ctypes.c_int]
     L.f_sinc.argtypes = [dp, ctypes.c_double, dp, ctypes.c_int]
     return L, dp
 
@@ -76,3 +82,25 @@ def test_transfer_function(fm, fmax):
     # s, c, d and fr to 3 units; fi = x s s carries 2 |sin x| times the error
     # of s and two roundings of at most 0.73
     assert np.all(worst <= np.array([3, 4.5, 3, 3, 3]) * EPS), worst / EPS
+
+
+@pytest.mark.parametrize("lo,hi", [(-0.05, 0.05), (-7.0, 7.0), (1e5, 2e6), (-5.3e8, 5.3e8)])
+def test_sincos_tab_correctly_rounded(fm, lo, hi):
+    """Errors below 2^-72 against half an ulp of a result that is mostly above
+    2^-6: fewer than one in 2^13 arguments may round the other way, and those
+    by one unit; 8000 arguments hold at most a handful."""
+    L, dp = fm
+    x = np.random.default_rng(17).uniform(lo, hi, 8000)
+    x[:4] = 0.0, np.pi / 2, np.pi / 128 * 1.5, -np.pi
+    s, c = np.empty_like(x), np.empty_like(x)
+    L.f_sctab(x.ctypes.data_as(dp), s.ctypes.data_as(dp), c.ctypes.data_as(dp), len(x))
+    off = 0
+    for f, got in ((mp.sin, s), (mp.cos, c)):
+        ref = np.array([float(f(mp.mpf(v))) for v in x])
+        bad = got != ref
+        off += int(bad.sum())
+        assert np.all(np.abs(got - ref) <= np.spacing(np.abs(ref)))
+    assert off <= 4, off
+    y = np.array([2.0 ** 29, np.inf, -np.inf, np.nan])
+    L.f_sctab(y.ctypes.data_as(dp), s.ctypes.data_as(dp), c.ctypes.data_as(dp), len(y))
+    assert np.isnan(s[:4]).all() and np.isnan(c[:4]).all()
