@@ -259,14 +259,14 @@ __device__ __forceinline__ void lds_fft(double2* buf, const double2* __restrict_
 __host__ __device__ constexpr int wave_fft_slot(int n) { return n + (n >> 3); }
 __host__ __device__ constexpr int wave_fft_stride(int N) { return N + N / 8; }
 
-template <int N, int NL, int R, int NTHR>
+template <int N, int NL, int R, int NTHR, int PAD>
 __device__ __forceinline__ void wave_fft_stage(double2* buf, int Ns, const double2* __restrict__ tw, int twstride,
                                                int unit, int lane)
 {
     constexpr int SPW = 512 / N;      // series in a unit
     constexpr int NB = N / R;         // butterflies in a series
     constexpr int PER = 8 / R;        // butterflies a lane
-    constexpr int PN = wave_fft_stride(N);
+    constexpr int PN = wave_fft_stride(N) + PAD;
     double2 v[PER][R];
     double2 w[PER][R - 1];
     if (Ns > 1)
@@ -315,12 +315,14 @@ __device__ __forceinline__ void wave_fft_stage(double2* buf, int Ns, const doubl
     wave_lds_sync();
 }
 
-// All units of NL series.  The caller has synchronised the input; ends with
-// a workgroup barrier.  TIGHT: a stage's twiddles are loaded in that stage
-// and not before (28 registers instead of up to 56), for callers that hold
-// other series meanwhile.
-template <int N, int NL, int NTHR, bool TIGHT = false>
-__device__ __forceinline__ void wave_fft(double2* buf, const double2* __restrict__ tw, int twstride)
+// All units of NL series, the first on wave `first`.  The caller has
+// synchronised the input, and does so again before other waves' results are
+// read.  TIGHT: a stage's twiddles are loaded in that stage and not before (28
+// registers instead of up to 56), for callers that hold other series meanwhile.
+// PAD: slots between two series besides (1 where lanes side by side read the
+// same point of different series).
+template <int N, int NL, int NTHR, bool TIGHT = false, int PAD = 0>
+__device__ __forceinline__ void wave_fft_units(double2* buf, const double2* __restrict__ tw, int twstride, int first)
 {
     static_assert(N >= 16 && N <= 512 && (N & (N - 1)) == 0 && NTHR % 64 == 0, "powers of two, 16 to 512 points");
     constexpr int SPW = 512 / N, UNITS = (NL + SPW - 1) / SPW, NW = NTHR / 64;
@@ -333,22 +335,29 @@ __device__ __forceinline__ void wave_fft(double2* buf, const double2* __restrict
     if constexpr (TIGHT) asm volatile("" : "+v"(lane));
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 #pragma unroll 1
-    for (int u = wave; u < UNITS; u += NW)
+    for (int u = wave < first ? wave - first + NW : wave - first; u < UNITS; u += NW)
     {
         int Ns = 1;
 #pragma unroll
         for (int s = 0; s < N8; s++)
         {
-            wave_fft_stage<N, NL, 8, NTHR>(buf, Ns, TIGHT ? opaque(tw) : tw, twstride, u, lane);
+            wave_fft_stage<N, NL, 8, NTHR, PAD>(buf, Ns, TIGHT ? opaque(tw) : tw, twstride, u, lane);
             Ns *= 8;
         }
 #pragma unroll
         for (int s = 0; s < N4; s++)
         {
-            wave_fft_stage<N, NL, 4, NTHR>(buf, Ns, TIGHT ? opaque(tw) : tw, twstride, u, lane);
+            wave_fft_stage<N, NL, 4, NTHR, PAD>(buf, Ns, TIGHT ? opaque(tw) : tw, twstride, u, lane);
             Ns *= 4;
         }
     }
+}
+
+// ... from the first wave on, with a workgroup barrier at the end.
+template <int N, int NL, int NTHR, bool TIGHT = false>
+__device__ __forceinline__ void wave_fft(double2* buf, const double2* __restrict__ tw, int twstride)
+{
+    wave_fft_units<N, NL, NTHR, TIGHT>(buf, tw, twstride, 0);
     __syncthreads();
 }
 

@@ -464,6 +464,16 @@ __device__ inline void spline_finish(int N, int i, const double* __restrict__ pr
     *y3o = (y2[i + 1] - y2[i]) / (3.0 * dx);
 }
 
+// A template's header by scalar loads.
+__device__ __forceinline__ Hdr load_hdr(const double* scr)
+{
+    Hdr h;
+    auto hs = (const __attribute__((address_space(4))) double*)scr;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(Hdr) / sizeof(double)); i++) ((double*)&h)[i] = hs[i];
+    return h;
+}
+
 // Vector issue bounds it (65% busy), most of it in the 24 delayed terms of
 // a knot.  Their sine and cosine come from a table in LDS (sincos_tab); the
 // vertices and arms are permuted for the channel as they are loaded, so the
@@ -490,12 +500,7 @@ __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_
     double* scr = scratch + scratch_doubles(N) * (size_t)e;
 
     // the header hdr_kernel wrote, by scalar loads
-    Hdr h;
-    {
-        auto hs = (const __attribute__((address_space(4))) double*)scr;
-#pragma unroll
-        for (int i = 0; i < (int)(sizeof(Hdr) / sizeof(double)); i++) ((double*)&h)[i] = hs[i];
-    }
+    const Hdr h = load_hdr(scr);
     for (int i = tid; i < 256; i += kRespThreads) tab[i] = sin_tab_entry(i);
     // barycentre amplitude and phase at the orbit knots
     for (int i = tid; i < N; i += kRespThreads)
@@ -778,11 +783,6 @@ __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_
 
 // ---------------------------------------------------------- K2: layers --
 
-// 512 threads: the kernel's 74 KB of LDS (NT 512) admits two workgroups
-// per CU, so 512-thread workgroups give four waves per SIMD where 256-thread
-// ones gave two (111 VGPRs allow four)
-constexpr int kLayerThreads = 512;
-
 struct LayerArgs
 {
     const double* data;   // 3 planes of npix (NULL: no inner products)
@@ -853,160 +853,282 @@ __device__ inline int block_exclusive_scan(int v, int* ws)
     return ws[w] + x - v;
 }
 
-template <int NT, int L>
-__device__ void layer_body(const Geo& g, const Hdr& h, int e, const LayerArgs& a, double2* U, double2* V,
-                           double2* B, int* cnt, const double* __restrict__ scr)
+// Doubles of a template's splines (phase at the barycentre, six TDI splines)
+// staged in LDS for its samples, where they fit: a sample gathers 29 of them,
+// from L2 a vector-memory instruction each.
+__host__ __device__ constexpr int spline_doubles(int N) { return 28 * N; }
+constexpr int kStagedKnots = 320;  // 72 KB
+
+// Sample i of the heterodyned X, Y, Z series (ds, dsi: tables of its layer
+// count).
+__device__ __forceinline__ void series_sample(const Geo& g, const Hdr& h, const double* __restrict__ ds,
+                                              const int* __restrict__ dsi, int i, const double* cph,
+                                              const double* ctdi, double rds, double (&x)[3])
 {
-    constexpr int NDS = NT * (L + 1);
-    constexpr int M = NDS / 2;
-    const int tid = threadIdx.x;
-    const int N = g.Norb;
-    const double* cph = scr + 64;
-    const double* ctdi = scr + 64 + 4 * N;
-    const double* ds = g.ds[L];
-    const int* dsi = g.dsi[L];
-    {
 #pragma clang fp contract(off)
-        const double w0 = PI2 * h.fhet;
-        for (int i = tid; i < NDS; i += kLayerThreads)
-        {
-            const double* e5 = ds + 5 * (size_t)i;
-            const double t = e5[0];
-            double kdotr = 0.0;
-            for (int d = 0; d < 3; d++) kdotr += h.k[d] * e5[1 + d];
-            const double tsc = t - kdotr;
-            const int j = even_index(tsc, g.ot0, g.ods, N);
-            const double phase_ds = spline_at(cph, N, j, tsc - g.ot[j]);
-            const double phase_het = w0 * t;
-            const int si = dsi[i];
-            const double sdx = e5[4];
-            double x[3];
-            for (int ch = 0; ch < 3; ch++)
-            {
-                const double* ca = ctdi + 4 * (size_t)N * (2 * ch);
-                const double* cp = ctdi + 4 * (size_t)N * (2 * ch + 1);
-                const double Amp = spline_at(ca, N, si, sdx);
-                double Phase = spline_at(cp, N, si, sdx);
-                Phase += phase_ds;
-                Phase -= phase_het;
-                double s, c;
-                sincos_red(Phase, &s, &c);
-                x[ch] = Amp * c;
-            }
-            U[i] = make_double2(x[0], x[1]);
-            if (i & 1) V[i >> 1].y = x[2];
-            else V[i >> 1].x = x[2];
-        }
+    const int N = g.Norb;
+    const double* e5 = ds + 5 * (size_t)i;
+    const double t = e5[0];
+    double kdotr = 0.0;
+#pragma unroll
+    for (int d = 0; d < 3; d++) kdotr += h.k[d] * e5[1 + d];
+    const double tsc = t - kdotr;
+    // even_index with the division by the knot spacing through its reciprocal
+    int j = (int)floor(div_by_recip(tsc - g.ot0, g.ods, rds));
+    j = min(max(j, 0), N - 1);
+    const double phase_ds = spline_at(cph, N, j, tsc - g.ot[j]);
+    const double phase_het = PI2 * h.fhet * t;
+    const int si = dsi[i];
+    const double sdx = e5[4];
+#pragma unroll
+    for (int ch = 0; ch < 3; ch++)
+    {
+        const double Amp = spline_at(ctdi + 4 * N * (2 * ch), N, si, sdx);
+        double Phase = spline_at(ctdi + 4 * N * (2 * ch + 1), N, si, sdx);
+        Phase += phase_ds;
+        Phase -= phase_het;
+        double s, c;
+        sincos_red(Phase, &s, &c);
+        x[ch] = Amp * c;
     }
+}
+
+// The first decimation of thread t's samples n = t + NT p, p < P, of the packed
+// series: u (X + i Y, P NT points) into P series of NT points, U[P k + r] =
+// FFT(ur)[k], and z (Z, two samples a point: lanes 2n and 2n + 1 hold one) into P
+// of NT/2.  pu(r, v): point t of series r; pv(r, v): point t/2, called by one of
+// the two lanes.  tw: P NT-th roots, tws apart.
+template <int NT, int P, typename PU, typename PV>
+__device__ __forceinline__ void series_dif(double2 (&u)[P], const double (&z)[P], int t,
+                                           const double2* __restrict__ tw, int tws, PU&& pu, PV&& pv)
+{
+    double2 y[P], v[P];
+    radix_butterfly<P>(u, y);
+    pu(0, y[0]);
+#pragma unroll
+    for (int r = 1; r < P; r++) pu(r, cmul(y[r], tw[r * t * tws]));
+    const bool odd = t & 1;
+#pragma unroll
+    for (int p = 0; p < P; p++)
+    {
+        const double o = __shfl_xor(z[p], 1, 64);
+        v[p] = odd ? make_double2(o, z[p]) : make_double2(z[p], o);
+    }
+    radix_butterfly<P>(v, y);
+#pragma unroll
+    for (int r = 0; r < P; r++)
+        if (odd == ((r & 1) != 0)) pv(r, r == 0 ? y[0] : cmul(y[r], tw[r * (t >> 1) * 2 * tws]));
+}
+
+// The windowed and conjugated X, Y, Z spectra of bin k (0 < k < NDS/2) from U
+// and V.  w: exp(-2 pi i k / NDS).  The inverse transforms are forward ones of
+// the conjugates.
+__device__ __forceinline__ void band_bin(double2 ua, double2 ub, double2 va, double2 vb, double2 w, double wt,
+                                         double2 (&o)[3])
+{
+    // X = (U[k] + conj U[NDS-k]) / 2 ; Y = (U[k] - conj U[NDS-k]) / (2i)
+    wt *= 0.5;
+    o[0] = make_double2(wt * (ua.x + ub.x), -wt * (ua.y - ub.y));
+    o[1] = make_double2(wt * (ua.y + ub.y), wt * (ua.x - ub.x));
+    const double2 E = make_double2(va.x + vb.x, va.y - vb.y), O = make_double2(va.y + vb.y, -(va.x - vb.x));
+    o[2] = make_double2(wt * (E.x + (w.x * O.x - w.y * O.y)), -wt * (E.y + (w.x * O.y + w.y * O.x)));
+}
+
+// Pixel value at time n of layer m from the inverse transform r (conjugated).
+__device__ __forceinline__ double pixel_value(double2 r, int NT, int NF, int m, int n, double norm)
+{
+    const double re = r.x / NT, im = -r.y / NT;  // a power of two
+    if (m == 0 || m == NF) return (n % 2 == 0) ? re * M_SQRT2 * norm : 0.0;
+    const int sgn = (m % 2 == 0) ? 1 : -1;
+    return ((n + m) % 2 == 0) ? re * norm : sgn * im * norm;
+}
+
+// The pixel list of template e (ucb/src/glass_ucb_waveform.c:1189-1212):
+// candidates in (time i, layer j) order, kept when kmin <= k < kmax; returns
+// their count, which it stores.  cnt: NTHR/64 + 1 ints of LDS.
+template <int NT, int L, int NTHR>
+__device__ __forceinline__ int pixel_list(const Geo& g, const Hdr& h, int e, const LayerArgs& a, int* cnt)
+{
+    constexpr int NC = NT * L;
+    int* lst = a.list + (size_t)e * a.vcap;
+    const int tid = threadIdx.x, k0 = h.jmin * NT;
+    if (k0 >= g.kmin && k0 + NC <= g.kmax)
+    {
+        // all of them, but for a band at the grid's edge
+        for (int c = tid; c < NC; c += NTHR) lst[c] = c / L + (h.jmin + c % L) * NT - g.kmin;
+        if (tid == 0) a.nwave[e] = NC;
+        return NC;
+    }
+    constexpr int PER = (NC + NTHR - 1) / NTHR;
+    const int c0 = tid * PER;
+    int mine = 0;
+    for (int c = c0; c < c0 + PER && c < NC; c++)
+    {
+        const int k = c / L + (h.jmin + c % L) * NT;
+        mine += (k >= g.kmin && k < g.kmax);
+    }
+    int pos = block_exclusive_scan<NTHR>(mine, cnt);
+    if (tid == 0) a.nwave[e] = cnt[NTHR / 64];
+    for (int c = c0; c < c0 + PER && c < NC; c++)
+    {
+        const int k = c / L + (h.jmin + c % L) * NT;
+        if (k >= g.kmin && k < g.kmax) lst[pos++] = k - g.kmin;
+    }
+    __threadfence_block();
     __syncthreads();
-    // forward FFTs: U (NDS) and V (NDS/2)
+    return cnt[NTHR / 64];
+}
+
+// wavelet_nwip terms of pixel k (index into the data planes): snr^2 = sum h^T
+// C h; the logL change of adding the template to a zero model with the
+// reference's edge rule (gaussian_log_likelhood_wavelet,
+// utils/src/glass_model.c:805-855).
+__device__ __forceinline__ void pixel_terms(const Geo& g, const LayerArgs& a, int k, const double (&hv)[3],
+                                            double& hh, double& dl)
+{
+    double C[3][3];
+    C[0][0] = a.invC[k];
+    C[1][1] = a.invC[(size_t)a.npix + k];
+    C[2][2] = a.invC[2 * (size_t)a.npix + k];
+    C[0][1] = C[1][0] = a.invC[3 * (size_t)a.npix + k];
+    C[0][2] = C[2][0] = a.invC[4 * (size_t)a.npix + k];
+    C[1][2] = C[2][1] = a.invC[5 * (size_t)a.npix + k];
+    const double d[3] = {a.data[k], a.data[(size_t)a.npix + k], a.data[2 * (size_t)a.npix + k]};
+    double th = 0.0, tdh = 0.0, tdd = 0.0;
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+        {
+            th += hv[p] * hv[q] * C[p][q];
+            tdh += d[p] * hv[q] * C[p][q];
+            tdd += d[p] * d[q] * C[p][q];
+        }
+    hh += th;
+    const int i = (k + g.kmin) % g.NT;
+    if (k >= 0 && k < a.npix) dl += (i < g.imin || i > g.imax) ? 0.5 * tdd : tdh - 0.5 * th;
+}
+
+// One template per workgroup of NT threads (NT 256, 512).  Barriers and latency
+// bound it, not work: with transforms spread over the workgroup (152 barriers a
+// template) the vector units were 28% busy.  So each thread holds its L + 1
+// samples of the series through a first decimation, each wave transforms whole
+// series of NT points by itself, and the pixels go from the inverse transforms
+// to the inner products in registers; six barriers are left.  LDS: up to eight
+// series; three layers' nine bands go in two turns.  4096 templates of 512
+// time pixels: 457 -> 297 us.
+template <int NT, int L>
+__device__ __forceinline__ void layer_body(const Geo& g, const Hdr& h, int e, const LayerArgs& a, double2* lds,
+                                           int* cnt, const double* __restrict__ scr)
+{
+    constexpr int P = L + 1, NDS = NT * P, NTHR = NT;
+    constexpr int PU = wave_fft_stride(NT) + 1, PV = wave_fft_stride(NT / 2) + 1;
+    constexpr int UU = (P * NT + 511) / 512;  // waves the X, Y series take
+    const int t = threadIdx.x, N = g.Norb;
     const bool three = (NDS % 3) == 0;
     const double2* twU = three ? g.tw3 : g.tw;
     const int tsU = (three ? kTw3N : kTwN) / NDS;
-    lds_fft<NDS, 1, kLayerThreads>(U, twU, tsU);
-    lds_fft<M, 1, kLayerThreads>(V, twU, tsU * 2);
-    // pixel list (ucb/src/glass_ucb_waveform.c:1189-1212): candidates in
-    // (time i, layer j) order, kept when kmin <= k < kmax
-    int* lst = a.list + (size_t)e * a.vcap;
+    const int Nw = pixel_list<NT, L, NTHR>(g, h, e, a, cnt);
+    double2 *U = lds, *V = lds + P * PU;
     {
-        constexpr int NC = NT * L;
-        constexpr int PER = (NC + kLayerThreads - 1) / kLayerThreads;
-        const int c0 = tid * PER;
-        int mine = 0;
-        for (int c = c0; c < c0 + PER && c < NC; c++)
+        const double* cs = scr + 64;
+        const double rds = 1.0 / g.ods;
+        double2 u[P];
+        double z[P];
+        if (N <= kStagedKnots)
         {
-            const int k = c / L + (h.jmin + c % L) * NT;
-            mine += (k >= g.kmin && k < g.kmax);
+            double* c = (double*)lds;
+            for (int i = t; i < spline_doubles(N); i += NTHR) c[i] = cs[i];
+            __syncthreads();
+#pragma unroll
+            for (int p = 0; p < P; p++)
+            {
+                double x[3];
+                series_sample(g, h, g.ds[L], g.dsi[L], t + NT * p, c, c + 4 * N, rds, x);
+                u[p] = make_double2(x[0], x[1]);
+                z[p] = x[2];
+            }
+            __syncthreads();
         }
-        int pos = block_exclusive_scan<kLayerThreads>(mine, cnt);
-        if (tid == 0) a.nwave[e] = cnt[kLayerThreads / 64];
-        for (int c = c0; c < c0 + PER && c < NC; c++)
-        {
-            const int k = c / L + (h.jmin + c % L) * NT;
-            if (k >= g.kmin && k < g.kmax) lst[pos++] = k - g.kmin;
-        }
+        else
+#pragma unroll
+            for (int p = 0; p < P; p++)
+            {
+                double x[3];
+                series_sample(g, h, g.ds[L], g.dsi[L], t + NT * p, cs, cs + 4 * N, rds, x);
+                u[p] = make_double2(x[0], x[1]);
+                z[p] = x[2];
+            }
+        series_dif<NT, P>(
+            u, z, t, twU, tsU, [&](int r, double2 v) { U[r * PU + wave_fft_slot(t)] = v; },
+            [&](int r, double2 v) { V[r * PV + wave_fft_slot(t >> 1)] = v; });
     }
     __syncthreads();
-    const int Nw = cnt[kLayerThreads / 64];
+    wave_fft_units<NT, P, NTHR, true, 1>(U, g.tw, kTwN / NT, 0);
+    wave_fft_units<NT / 2, P, NTHR, true, 1>(V, g.tw, kTwN / (NT / 2), UU);
+    __syncthreads();
+    // the bands of the L layers: bin k = P j + r of U is point j of series r
+    double2 b[L][3];
     const double* win = g.win[L];
+#pragma unroll
+    for (int off = 0; off < L; off++)
+    {
+        const int j = t - NT / 2, k = (off + 1) * NT / 2 + j, m = h.jmin + off;
+        b[off][0] = b[off][1] = b[off][2] = make_double2(0.0, 0.0);
+        if (t > 0)
+        {
+            double wt = win[j < 0 ? -j : j];
+            if (j == 0 && (m == 0 || m == g.NF)) wt /= 2.0;
+            auto at = [&](const double2* s, int stride, int q) { return s[(q % P) * stride + wave_fft_slot(q / P)]; };
+            band_bin(at(U, PU, k), at(U, PU, NDS - k), at(V, PV, k), at(V, PV, NDS / 2 - k), twU[k * tsU], wt, b[off]);
+        }
+    }
+    // the inverse transforms, CB channels at a time; thread t takes the pixels
+    // c = t + NTHR i, time c / L of layer c % L
+    constexpr int CB = 3 * L <= 8 ? 3 : 2;
+    double hv[L][3];
     const double norm = sqrt((double)g.NF) / (L + 1.0);
     double* vals = a.values + (size_t)e * 3 * a.vcap;
-    for (int ch = 0; ch < 3; ch++)
+#pragma unroll
+    for (int c0 = 0; c0 < 3; c0 += CB)
     {
-        // windowed bands of the L layers, conjugated so the forward FFT
-        // gives the conjugate of the inverse transform
-        for (int it = tid; it < L * NT; it += kLayerThreads)
-        {
-            const int off = it / NT, jj = it % NT;
-            const int j = jj - NT / 2;
-            const int m = h.jmin + off;
-            const int center = (off + 1) * NT / 2;
-            const int idx = center + j;
-            double2 v = make_double2(0.0, 0.0);
-            if (jj > 0 && idx >= 0 && idx <= NDS / 2)
-            {
-                double wt = win[j < 0 ? -j : j];
-                if (j == 0 && (m == 0 || m == g.NF)) wt /= 2.0;
-                const double2 S = spectrum<NDS>(ch, idx, U, V, twU, tsU);
-                v = make_double2(wt * S.x, -(wt * S.y));
-            }
-            B[off * NT + jj] = v;
-        }
+        constexpr int kCh = CB;
+        const int nch = c0 + kCh <= 3 ? kCh : 3 - c0;
+        __syncthreads();  // the readers of what is in LDS
+#pragma unroll
+        for (int ch = 0; ch < 3; ch++)
+            if (ch >= c0 && ch < c0 + nch)
+#pragma unroll
+                for (int off = 0; off < L; off++) lds[((ch - c0) * L + off) * PU + wave_fft_slot(t)] = b[off][ch];
         __syncthreads();
-        lds_fft<NT, L, kLayerThreads>(B, g.tw, kTwN / NT);
-        for (int it = tid; it < L * NT; it += kLayerThreads)
-        {
-            const int n = it / L, off = it % L;
-            const int m = h.jmin + off;
-            const double2 r = B[off * NT + n];
-            const double re = r.x / NT, im = -r.y / NT;
-            double val;
-            if (m == 0 || m == g.NF) val = (n % 2 == 0) ? re * M_SQRT2 * norm : 0.0;
-            else
-            {
-                const int sgn = (m % 2 == 0) ? 1 : -1;
-                val = ((n + m) % 2 == 0) ? re * norm : sgn * im * norm;
-            }
-            const int pos = n * L + off;
-            if (pos < Nw) vals[ch * a.vcap + pos] = val;
-        }
+        wave_fft_units<NT, kCh * L, NTHR, true, 1>(lds, g.tw, kTwN / NT, 0);
         __syncthreads();
+#pragma unroll
+        for (int i = 0; i < L; i++)
+        {
+            const int c = t + NTHR * i, n = c / L, off = c % L;
+#pragma unroll
+            for (int ch = 0; ch < 3; ch++)
+                if (ch >= c0 && ch < c0 + nch)
+                {
+                    const double2 r = lds[((ch - c0) * L + off) * PU + wave_fft_slot(n)];
+                    hv[i][ch] = pixel_value(r, NT, g.NF, h.jmin + off, n, norm);
+                    if (c < Nw) vals[ch * a.vcap + c] = hv[i][ch];
+                }
+        }
     }
     if (!a.data) return;
-    __threadfence_block();
-    __syncthreads();
-    // wavelet_nwip terms over the pixel list: snr^2 = sum h^T C h; the
-    // logL change of adding the template to a zero model with the
-    // reference's edge rule (gaussian_log_likelhood_wavelet,
-    // utils/src/glass_model.c:805-855)
+    const int* lst = a.list + (size_t)e * a.vcap;
     double hh = 0.0, dl = 0.0;
-    for (int t = tid; t < Nw; t += kLayerThreads)
+#pragma unroll
+    for (int i = 0; i < L; i++)
     {
-        const int k = lst[t];
-        const double hv[3] = {vals[t], vals[a.vcap + t], vals[2 * a.vcap + t]};
-        double C[3][3];
-        C[0][0] = a.invC[k];
-        C[1][1] = a.invC[(size_t)a.npix + k];
-        C[2][2] = a.invC[2 * (size_t)a.npix + k];
-        C[0][1] = C[1][0] = a.invC[3 * (size_t)a.npix + k];
-        C[0][2] = C[2][0] = a.invC[4 * (size_t)a.npix + k];
-        C[1][2] = C[2][1] = a.invC[5 * (size_t)a.npix + k];
-        const double d[3] = {a.data[k], a.data[(size_t)a.npix + k], a.data[2 * (size_t)a.npix + k]};
-        double th = 0.0, tdh = 0.0, tdd = 0.0;
-        for (int p = 0; p < 3; p++)
-            for (int q = 0; q < 3; q++)
-            {
-                th += hv[p] * hv[q] * C[p][q];
-                tdh += d[p] * hv[q] * C[p][q];
-                tdd += d[p] * d[q] * C[p][q];
-            }
-        hh += th;
-        const int i = (k + g.kmin) % g.NT;
-        if (k >= 0 && k < a.npix) dl += (i < g.imin || i > g.imax) ? 0.5 * tdd : tdh - 0.5 * th;
+        const int c = t + NTHR * i;
+        if (c < Nw) pixel_terms(g, a, Nw == NT * L ? c / L + (h.jmin + c % L) * NT - g.kmin : lst[c], hv[i], hh, dl);
     }
-    hh = block_sum<kLayerThreads>(hh);
-    dl = block_sum<kLayerThreads>(dl);
-    if (tid == 0)
+    hh = block_sum<NTHR>(hh);
+    dl = block_sum<NTHR>(dl);
+    if (t == 0)
     {
         a.snr[e] = sqrt(hh);
         a.dlogL[e] = dl;
@@ -1014,31 +1136,27 @@ __device__ void layer_body(const Geo& g, const Hdr& h, int e, const LayerArgs& a
 }
 
 template <int NT>
-__global__ void __launch_bounds__(kLayerThreads) layer_kernel(Geo g, int n, LayerArgs a,
-                                                              const double* __restrict__ scratch)
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 8))) layer_kernel(
+    Geo g, int n, LayerArgs a, const double* __restrict__ scratch)
 {
     const int e = blockIdx.x;
     if (e >= n) return;
     extern __shared__ double2 lds2[];
+    __shared__ int cnt[NT / 64 + 1];
     const double* scr = scratch + scratch_doubles(g.Norb) * (size_t)e;
-    __shared__ Hdr H;
-    if (threadIdx.x == 0) H = *(const Hdr*)scr;
-    __syncthreads();
-    const Hdr h = H;
-    // LDS: U (4 NT) | V (2 NT) | B (3 NT); list counts in static LDS
-    __shared__ int cnt[kLayerThreads + 1];
-    double2* U = lds2;
-    double2* V = U + 4 * NT;
-    double2* B = V + 2 * NT;
-    if (h.L == 1) layer_body<NT, 1>(g, h, e, a, U, V, B, cnt, scr);
-    else if (h.L == 2) layer_body<NT, 2>(g, h, e, a, U, V, B, cnt, scr);
-    else layer_body<NT, 3>(g, h, e, a, U, V, B, cnt, scr);
+    const Hdr h = load_hdr(scr);
+    if (h.L == 1) layer_body<NT, 1>(g, h, e, a, lds2, cnt, scr);
+    else if (h.L == 2) layer_body<NT, 2>(g, h, e, a, lds2, cnt, scr);
+    else layer_body<NT, 3>(g, h, e, a, lds2, cnt, scr);
 }
 
+// eight series, or the staged splines of N knots
 template <int NT>
-constexpr size_t layer_lds_bytes()
+static size_t layer_lds_bytes(int N)
 {
-    return sizeof(double2) * 9 * NT;
+    const size_t series = sizeof(double2) * 8 * (wave_fft_stride(NT) + 1);
+    const size_t staged = N <= kStagedKnots ? sizeof(double) * spline_doubles(N) : 0;
+    return series > staged ? series : staged;
 }
 
 // ---------------------------------------------- K2 for NT of 1024..4096 --
@@ -1284,11 +1402,9 @@ static int launch_templates(const GeoHost& G, int n, const double* d_params, dou
                                d_scratch);
     }
     else if (g.NT == 512)
-        hipLaunchKernelGGL(layer_kernel<512>, dim3(n), dim3(kLayerThreads), layer_lds_bytes<512>(), s, g, n, a,
-                           d_scratch);
+        hipLaunchKernelGGL(layer_kernel<512>, dim3(n), dim3(512), layer_lds_bytes<512>(g.Norb), s, g, n, a, d_scratch);
     else
-        hipLaunchKernelGGL(layer_kernel<256>, dim3(n), dim3(kLayerThreads), layer_lds_bytes<256>(), s, g, n, a,
-                           d_scratch);
+        hipLaunchKernelGGL(layer_kernel<256>, dim3(n), dim3(256), layer_lds_bytes<256>(g.Norb), s, g, n, a, d_scratch);
     GH_CHECK(hipGetLastError());
     return GLASS_HIP_OK;
 }
@@ -1314,7 +1430,9 @@ static int set_lds_limits()
         if (hipFuncSetAttribute((const void*)resp_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)resp_lds_bytes(kMaxKnots)) != hipSuccess ||
             hipFuncSetAttribute((const void*)layer_kernel<512>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)layer_lds_bytes<512>()) != hipSuccess ||
+                                (int)layer_lds_bytes<512>(kStagedKnots)) != hipSuccess ||
+            hipFuncSetAttribute((const void*)layer_kernel<256>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)layer_lds_bytes<256>(kStagedKnots)) != hipSuccess ||
             hipFuncSetAttribute((const void*)layer_kernel_big<4096>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)(sizeof(double2) * 4096)) != hipSuccess)
         {
