@@ -1161,23 +1161,267 @@ static size_t layer_lds_bytes(int N)
 
 // ---------------------------------------------- K2 for NT of 1024..4096 --
 //
-// The heterodyned series of NT (L+1) <= 16384 samples and its spectrum do
-// not fit one workgroup's LDS: they live in a global scratch slice per
-// workgroup (U = X + iY and V = Z packed as before, each with a partner
-// buffer) and are transformed by ping-pong Stockham stages through L2, with
-// the same butterflies, twiddle values and stage order as the LDS path.
-// The windowed band of each layer (NT points, 64 KB at NT = 4096) is
-// inverse-transformed in LDS, one layer at a time.  Workgroups stride over
-// the templates.
+// The heterodyned series of NT (L+1) <= 16384 samples and its spectrum do not
+// fit one workgroup's LDS: they live in a global slice per template (U = X + i
+// Y, then V = Z packed as above), the L + 1 series of NT and NT/2 points that a
+// first decimation in registers leaves.  Four kernels, each with a template's
+// work on several workgroups: the samples and their decimation; one workgroup a
+// series, cut once more to 512 points a wave; one a channel for the bands and
+// their inverse transforms; the pixel list and inner products.  (One workgroup
+// for all of a template, with ping-pong stages of the whole series through L2
+// and a fifth of the CUs holding a second one, left the vector units 10% busy.)
+// 300 templates of 4096 time pixels: 651 -> 273 us.
+
+constexpr int kSeriesThreads = 512;
+constexpr int kSumThreads = 1024;
+
+// double2 per scratch slice: U (NDS) and V (NDS / 2), NDS = NT (L + 1) at
+// three layers; with a forced count each with its partner (below)
+__host__ __device__ inline size_t big_layer_slice(int NT, int Lf = 0)
+{
+    return Lf > 0 ? 3 * (size_t)NT * (size_t)(Lf + 1) : 6 * (size_t)NT;
+}
+
+// f(integral constant L) of a template's layer count
+template <typename F>
+__device__ __forceinline__ void with_layers(int L, F&& f)
+{
+    if (L == 1) f(std::integral_constant<int, 1>());
+    else if (L == 2) f(std::integral_constant<int, 2>());
+    else f(std::integral_constant<int, 3>());
+}
+
+template <int NT>
+__global__ void __launch_bounds__(kSeriesThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) series_kernel_big(
+    Geo g, int e0, LayerArgs a, const double* __restrict__ scratch)
+{
+    extern __shared__ double ldss[];  // the splines, where staged
+    const int N = g.Norb, t = blockIdx.x * kSeriesThreads + threadIdx.x;
+    const double* scr = scratch + scratch_doubles(N) * (size_t)(e0 + blockIdx.y);
+    const Hdr h = load_hdr(scr);
+    double2* S = a.big + a.bigslice * (size_t)blockIdx.y;
+    const double* cs = scr + 64;
+    const bool staged = N <= kStagedKnots;
+    if (staged)
+    {
+        for (int i = threadIdx.x; i < spline_doubles(N); i += kSeriesThreads) ldss[i] = cs[i];
+        __syncthreads();
+    }
+    with_layers(h.L, [&](auto l) {
+        constexpr int L = decltype(l)::value, P = L + 1, NDS = NT * P;
+        const double rds = 1.0 / g.ods;
+        double2 u[P];
+        double z[P];
+        if (staged)
+#pragma unroll
+            for (int p = 0; p < P; p++)
+            {
+                double x[3];
+                series_sample(g, h, g.ds[L], g.dsi[L], t + NT * p, ldss, ldss + 4 * N, rds, x);
+                u[p] = make_double2(x[0], x[1]);
+                z[p] = x[2];
+            }
+        else
+#pragma unroll
+            for (int p = 0; p < P; p++)
+            {
+                double x[3];
+                series_sample(g, h, g.ds[L], g.dsi[L], t + NT * p, cs, cs + 4 * N, rds, x);
+                u[p] = make_double2(x[0], x[1]);
+                z[p] = x[2];
+            }
+        const bool three = P == 3;
+        series_dif<NT, P>(
+            u, z, t, three ? g.tw3 : g.tw16, (three ? kTw3N : kTw16N) / NDS,
+            [&](int r, double2 v) { S[r * NT + t] = v; },
+            [&](int r, double2 v) { S[NDS + r * (NT / 2) + (t >> 1)] = v; });
+    });
+}
+
+// A forward transform of M = 512 P points whose points t + 512 p thread t of
+// 512 brings in x: P series of 512 in lds, one a wave; get(i) is point t + 512 i
+// of the result, after the call (no barrier after the reads).
+template <int M>
+struct SplitFft
+{
+    static constexpr int P = M / 512, PN = wave_fft_stride(512) + 1;
+    static constexpr size_t kBytes = sizeof(double2) * P * PN;
+    double2* lds;
+    __device__ __forceinline__ SplitFft(double2 (&x)[P], double2* buf, const double2* __restrict__ tw, int t) : lds(buf)
+    {
+        double2* o = lds + wave_fft_slot(t);
+        if constexpr (P == 1)
+            o[0] = x[0];
+        else
+        {
+            double2 y[P];
+            radix_butterfly<P>(x, y);
+            o[0] = y[0];
+#pragma unroll
+            for (int r = 1; r < P; r++) o[r * PN] = cmul(y[r], tw[r * t * (kTwN / M)]);
+        }
+        __syncthreads();
+        wave_fft_units<512, P, 512, true, 1>(lds, tw, kTwN / 512, 0);
+        __syncthreads();
+    }
+    __device__ __forceinline__ double2 get(int b) const { return lds[(b % P) * PN + wave_fft_slot(b / P)]; }
+};
+
+template <int M>
+__device__ __forceinline__ void fft_in_place(double2* S, double2* lds, const double2* __restrict__ tw)
+{
+    const int t = threadIdx.x;
+    double2 x[M / 512];
+#pragma unroll
+    for (int p = 0; p < M / 512; p++) x[p] = S[t + 512 * p];
+    const SplitFft<M> f(x, lds, tw, t);
+#pragma unroll
+    for (int p = 0; p < M / 512; p++) S[t + 512 * p] = f.get(t + 512 * p);
+}
+
+// blockIdx.x 0..3: series of U, 4..7: of V
+template <int NT>
+__global__ void __launch_bounds__(512) fft_kernel_big(Geo g, int e0, LayerArgs a, const double* __restrict__ scratch)
+{
+    extern __shared__ double2 ldsb[];
+    const int P = load_hdr(scratch + scratch_doubles(g.Norb) * (size_t)(e0 + blockIdx.y)).L + 1, r = blockIdx.x & 3;
+    if (r >= P) return;
+    double2* S = a.big + a.bigslice * (size_t)blockIdx.y;
+    if (blockIdx.x < 4)
+        fft_in_place<NT>(S + r * NT, ldsb, g.tw);
+    else
+        fft_in_place<NT / 2>(S + P * NT + r * (NT / 2), ldsb, g.tw);
+}
+
+// Pixels of a template's list: its candidates inside the grid.
+__device__ __forceinline__ int pixel_count(const Geo& g, const Hdr& h, int L)
+{
+    int n = 0;
+    for (int off = 0; off < L; off++)
+    {
+        const int k0 = (h.jmin + off) * g.NT;
+        n += max(0, min(g.kmax, k0 + g.NT) - max(g.kmin, k0));
+    }
+    return n;
+}
+
+// blockIdx.x: channel
+template <int NT>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 8))) band_kernel_big(
+    Geo g, int e0, LayerArgs a, const double* __restrict__ scratch)
+{
+    extern __shared__ double2 ldsb[];
+    const int e = e0 + blockIdx.y, ch = blockIdx.x, t = threadIdx.x;
+    const Hdr h = load_hdr(scratch + scratch_doubles(g.Norb) * (size_t)e);
+    const double2* S = a.big + a.bigslice * (size_t)blockIdx.y;
+    with_layers(h.L, [&](auto l) {
+        constexpr int L = decltype(l)::value, P = L + 1, NDS = NT * P, Q = NT / 512;
+        const double2 *U = S, *V = S + NDS;
+        const bool three = P == 3;
+        const double2* twU = three ? g.tw3 : g.tw16;
+        const int tsU = (three ? kTw3N : kTw16N) / NDS;
+        const double* win = g.win[L];
+        const double norm = sqrt((double)g.NF) / (L + 1.0);
+        const int Nw = pixel_count(g, h, L);
+        double val[L][Q];
+#pragma unroll
+        for (int off = 0; off < L; off++)
+        {
+            const int m = h.jmin + off;
+            double2 x[Q];
+#pragma unroll
+            for (int p = 0; p < Q; p++)
+            {
+                const int jj = t + 512 * p, j = jj - NT / 2, k = off * (NT / 2) + jj;
+                x[p] = make_double2(0.0, 0.0);
+                if (jj > 0)
+                {
+                    double wt = win[j < 0 ? -j : j];
+                    if (j == 0 && (m == 0 || m == g.NF)) wt /= 2.0;
+                    auto at = [&](const double2* s, int len, int q) { return s[(q % P) * len + q / P]; };
+                    const double2 none = make_double2(0.0, 0.0);
+                    double2 o[3];
+                    if (ch < 2)
+                    {
+                        band_bin(at(U, NT, k), at(U, NT, NDS - k), none, none, none, wt, o);
+                        x[p] = ch == 0 ? o[0] : o[1];
+                    }
+                    else
+                    {
+                        band_bin(none, none, at(V, NT / 2, k), at(V, NT / 2, NDS / 2 - k), twU[k * tsU], wt, o);
+                        x[p] = o[2];
+                    }
+                }
+            }
+            if (off) __syncthreads();  // the last layer's reads
+            const SplitFft<NT> f(x, ldsb, g.tw, t);
+#pragma unroll
+            for (int p = 0; p < Q; p++)
+                val[off][p] = pixel_value(f.get(t + 512 * p), NT, g.NF, m, t + 512 * p, norm);
+        }
+        double* vals = a.values + (size_t)(3 * (size_t)e + ch) * a.vcap;
+#pragma unroll
+        for (int p = 0; p < Q; p++)
+#pragma unroll
+            for (int off = 0; off < L; off++)
+            {
+                const int pos = (t + 512 * p) * L + off;
+                if (pos < Nw) vals[pos] = val[off][p];
+            }
+    });
+}
+
+template <int NT>
+__global__ void __launch_bounds__(kSumThreads) sum_kernel_big(Geo g, int e0, LayerArgs a,
+                                                              const double* __restrict__ scratch)
+{
+    __shared__ int cnt[kSumThreads / 64 + 1];
+    const int e = e0 + blockIdx.x, t = threadIdx.x;
+    const Hdr h = load_hdr(scratch + scratch_doubles(g.Norb) * (size_t)e);
+    with_layers(h.L, [&](auto l) {
+        constexpr int L = decltype(l)::value;
+        const int Nw = pixel_list<NT, L, kSumThreads>(g, h, e, a, cnt);
+        if (!a.data) return;
+        const int* lst = a.list + (size_t)e * a.vcap;
+        const double* vals = a.values + (size_t)e * 3 * a.vcap;
+        double hh = 0.0, dl = 0.0;
+        for (int c = t; c < Nw; c += kSumThreads)
+        {
+            const double hv[3] = {vals[c], vals[a.vcap + c], vals[2 * a.vcap + c]};
+            pixel_terms(g, a, Nw == NT * L ? c / L + (h.jmin + c % L) * NT - g.kmin : lst[c], hv, hh, dl);
+        }
+        hh = block_sum<kSumThreads>(hh);
+        dl = block_sum<kSumThreads>(dl);
+        if (t == 0)
+        {
+            a.snr[e] = sqrt(hh);
+            a.dlogL[e] = dl;
+        }
+    });
+}
+
+template <int NT>
+static void launch_big(const Geo& g, int n, const LayerArgs& a, const double* d_scratch, hipStream_t s)
+{
+    const size_t staged = g.Norb <= kStagedKnots ? sizeof(double) * spline_doubles(g.Norb) : 0;
+    for (int e0 = 0; e0 < n; e0 += a.nbig)
+    {
+        const int m = std::min(a.nbig, n - e0);
+        series_kernel_big<NT><<<dim3(NT / kSeriesThreads, m), kSeriesThreads, staged, s>>>(g, e0, a, d_scratch);
+        fft_kernel_big<NT><<<dim3(8, m), 512, SplitFft<NT>::kBytes, s>>>(g, e0, a, d_scratch);
+        band_kernel_big<NT><<<dim3(3, m), 512, SplitFft<NT>::kBytes, s>>>(g, e0, a, d_scratch);
+        sum_kernel_big<NT><<<m, kSumThreads, 0, s>>>(g, e0, a, d_scratch);
+    }
+}
+
+// ------------------------------------------- K2 for forced layer counts --
+//
+// Series of up to 32768 samples: U and V with a partner buffer each in a
+// global slice per workgroup, transformed by ping-pong Stockham stages through
+// L2; each layer's band is inverse-transformed in LDS, one layer at a time.
+// Workgroups stride over the templates.
 
 constexpr int kBigLayerThreads = 512;
-
-// double2 per scratch slice: U and partner (NDS each) and V and partner
-// (NDS / 2 each), NDS = NT (L + 1) at the largest L (3, or a forced count)
-__host__ __device__ inline size_t big_layer_slice(int NT, int Lmax = kMaxLayers)
-{
-    return 3 * (size_t)NT * (size_t)((Lmax > kMaxLayers ? Lmax : kMaxLayers) + 1);
-}
 
 template <int NT, int L>
 __device__ void layer_body_big(const Geo& g, const Hdr& h, int e, const LayerArgs& a, double2* G0, double2* B,
@@ -1186,7 +1430,7 @@ __device__ void layer_body_big(const Geo& g, const Hdr& h, int e, const LayerArg
     constexpr int NDS = NT * (L + 1);
     constexpr int M = NDS / 2;
     constexpr int NTHR = kBigLayerThreads;
-    constexpr int SLOT = L > kMaxLayers ? kForcedSlot : L;
+    constexpr int SLOT = kForcedSlot;
     const int tid = threadIdx.x;
     const int N = g.Norb;
     const double* cph = scr + 64;
@@ -1232,9 +1476,8 @@ __device__ void layer_body_big(const Geo& g, const Hdr& h, int e, const LayerArg
     }
     __threadfence_block();
     __syncthreads();
-    const bool three = (NDS % 3) == 0;
-    const double2* twU = three ? g.tw3 : (NDS > kTw16N ? g.tw32 : g.tw16);
-    const int tsU = (three ? kTw3N : (NDS > kTw16N ? kTw32N : kTw16N)) / NDS;
+    const double2* twU = NDS > kTw16N ? g.tw32 : g.tw16;
+    const int tsU = (NDS > kTw16N ? kTw32N : kTw16N) / NDS;
     const double2* U = pingpong_fft<NDS, NTHR>(Ua, Ub, twU, tsU);
     const double2* V = pingpong_fft<M, NTHR>(Va, Vb, twU, tsU * 2);
     int* lst = a.list + (size_t)e * a.vcap;
@@ -1352,17 +1595,11 @@ __global__ void __launch_bounds__(kBigLayerThreads) layer_kernel_big(Geo g, int 
         if (threadIdx.x == 0) H = *(const Hdr*)scr;
         __syncthreads();
         const Hdr h = H;
-        if (h.L == 1) layer_body_big<NT, 1>(g, h, e, a, G0, ldsb, cnt, scr);
-        else if (h.L == 2) layer_body_big<NT, 2>(g, h, e, a, G0, ldsb, cnt, scr);
-        else if (h.L == 3) layer_body_big<NT, 3>(g, h, e, a, G0, ldsb, cnt, scr);
-        else if constexpr (NT <= 512)
-        {
-            // forced layer counts (forced_layers_ok)
-            if (h.L == 7) layer_body_big<NT, 7>(g, h, e, a, G0, ldsb, cnt, scr);
-            else if (h.L == 15) layer_body_big<NT, 15>(g, h, e, a, G0, ldsb, cnt, scr);
-            else if (h.L == 31) layer_body_big<NT, 31>(g, h, e, a, G0, ldsb, cnt, scr);
-            else if (h.L == 63) layer_body_big<NT, 63>(g, h, e, a, G0, ldsb, cnt, scr);
-        }
+        // the counts of forced_layers_ok
+        if (h.L == 7) layer_body_big<NT, 7>(g, h, e, a, G0, ldsb, cnt, scr);
+        else if (h.L == 15) layer_body_big<NT, 15>(g, h, e, a, G0, ldsb, cnt, scr);
+        else if (h.L == 31) layer_body_big<NT, 31>(g, h, e, a, G0, ldsb, cnt, scr);
+        else if (h.L == 63) layer_body_big<NT, 63>(g, h, e, a, G0, ldsb, cnt, scr);
     }
 }
 
@@ -1383,23 +1620,21 @@ static int launch_templates(const GeoHost& G, int n, const double* d_params, dou
             set_error("wavelet templates: NT = %d (forced layers %d) needs the long-series scratch", g.NT, g.Lf);
             return GLASS_HIP_EINVAL;
         }
-        const int grid = n < a.nbig ? n : a.nbig;
-        const size_t lds = sizeof(double2) * (size_t)g.NT;
-        if (g.NT == 256)
-            hipLaunchKernelGGL(layer_kernel_big<256>, dim3(grid), dim3(kBigLayerThreads), lds, s, g, n, a,
-                               d_scratch);
-        else if (g.NT == 512)
-            hipLaunchKernelGGL(layer_kernel_big<512>, dim3(grid), dim3(kBigLayerThreads), lds, s, g, n, a,
-                               d_scratch);
+        if (g.Lf > 0)
+        {
+            const int grid = n < a.nbig ? n : a.nbig;
+            const size_t lds = sizeof(double2) * (size_t)g.NT;
+            if (g.NT == 256)
+                layer_kernel_big<256><<<grid, kBigLayerThreads, lds, s>>>(g, n, a, d_scratch);
+            else
+                layer_kernel_big<512><<<grid, kBigLayerThreads, lds, s>>>(g, n, a, d_scratch);
+        }
         else if (g.NT == 1024)
-            hipLaunchKernelGGL(layer_kernel_big<1024>, dim3(grid), dim3(kBigLayerThreads), lds, s, g, n, a,
-                               d_scratch);
+            launch_big<1024>(g, n, a, d_scratch, s);
         else if (g.NT == 2048)
-            hipLaunchKernelGGL(layer_kernel_big<2048>, dim3(grid), dim3(kBigLayerThreads), lds, s, g, n, a,
-                               d_scratch);
+            launch_big<2048>(g, n, a, d_scratch, s);
         else
-            hipLaunchKernelGGL(layer_kernel_big<4096>, dim3(grid), dim3(kBigLayerThreads), lds, s, g, n, a,
-                               d_scratch);
+            launch_big<4096>(g, n, a, d_scratch, s);
     }
     else if (g.NT == 512)
         hipLaunchKernelGGL(layer_kernel<512>, dim3(n), dim3(512), layer_lds_bytes<512>(g.Norb), s, g, n, a, d_scratch);
@@ -1427,14 +1662,17 @@ static int set_lds_limits()
     static std::once_flag once;
     static int rc = GLASS_HIP_OK;
     std::call_once(once, [] {
-        if (hipFuncSetAttribute((const void*)resp_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)resp_lds_bytes(kMaxKnots)) != hipSuccess ||
-            hipFuncSetAttribute((const void*)layer_kernel<512>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)layer_lds_bytes<512>(kStagedKnots)) != hipSuccess ||
-            hipFuncSetAttribute((const void*)layer_kernel<256>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)layer_lds_bytes<256>(kStagedKnots)) != hipSuccess ||
-            hipFuncSetAttribute((const void*)layer_kernel_big<4096>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(sizeof(double2) * 4096)) != hipSuccess)
+        auto allow_lds = [](auto* f, size_t bytes) {
+            return hipFuncSetAttribute((const void*)f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) ==
+                   hipSuccess;
+        };
+        const size_t staged = sizeof(double) * spline_doubles(kStagedKnots);
+        if (!allow_lds(resp_kernel, resp_lds_bytes(kMaxKnots)) ||
+            !allow_lds(layer_kernel<512>, layer_lds_bytes<512>(kStagedKnots)) ||
+            !allow_lds(layer_kernel<256>, layer_lds_bytes<256>(kStagedKnots)) ||
+            !allow_lds(series_kernel_big<1024>, staged) || !allow_lds(series_kernel_big<2048>, staged) ||
+            !allow_lds(series_kernel_big<4096>, staged) || !allow_lds(fft_kernel_big<4096>, SplitFft<4096>::kBytes) ||
+            !allow_lds(band_kernel_big<4096>, SplitFft<4096>::kBytes))
         {
             set_error("hipFuncSetAttribute (dynamic LDS) failed");
             rc = GLASS_HIP_ERUNTIME;
@@ -1864,8 +2102,7 @@ static int wdm_batch_create(glass_hip_wdm_batch** plan, const glass_hip_wdm* w, 
     }
     if (NT >= 1024 || layers > 0)
     {
-        // the layer kernel strides over the templates with two workgroups
-        // per CU, each with its own long-series slice
+        // long-series slices of as many templates as are in flight at a time
         int ncu = 0;
         GH_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, P->device));
         P->nbig = std::min(max_templates, 2 * std::max(ncu, 1));
