@@ -406,19 +406,33 @@ __device__ inline void spline_alpha(int N, const double* __restrict__ prep, cons
 // 1/l_i) and it forgets: each knot keeps 0.27 of the one before, so a chunk that
 // starts `warm` knots early from zero holds the value of the whole sweep (2^-80
 // of it is left out, 2^-27 of its last bit).  62 dependent steps for 202 knots
-// instead of 202.
+// instead of 202.  The x-only terms come from LDS: a step that waits for L2 takes
+// 380 cycles, five times its arithmetic.
 constexpr int kSweepChunks = 10;
+struct SweepTerms
+{
+    double *dx, *l, *mu, *rl;
+    // from prep (spline_prep_host), by the whole workgroup
+    __device__ __forceinline__ void fill(int N, const double* __restrict__ prep) const
+    {
+        for (int i = threadIdx.x; i < N; i += kRespThreads)
+        {
+            dx[i] = prep[i];
+            l[i] = prep[N + i];
+            mu[i] = prep[2 * N + i];
+            rl[i] = prep[3 * N + i];
+        }
+    }
+};
 __device__ inline void sweep_range(int N, int c, int* lo, int* hi)
 {
     const int len = (N - 2 + kSweepChunks - 1) / kSweepChunks;
     *lo = 1 + c * len;
     *hi = min(N - 1, *lo + len);
 }
-__device__ inline void spline_forward(int N, const double* __restrict__ prep, const double* alpha, double* z, int c,
-                                      int warm)
+__device__ inline void spline_forward(int N, const SweepTerms& s, const double* alpha, double* z, int c, int warm)
 {
 #pragma clang fp contract(off)
-    const double *dx = prep, *l = prep + N, *rl = prep + 3 * N;
     int lo, hi;
     sweep_range(N, c, &lo, &hi);
     if (c == 0) z[0] = 0.0;
@@ -426,15 +440,13 @@ __device__ inline void spline_forward(int N, const double* __restrict__ prep, co
 #pragma unroll 4
     for (int i = max(1, lo - warm); i < hi; i++)
     {
-        zp = div_by_recip(alpha[i] - dx[i - 1] * zp, l[i], rl[i]);
+        zp = div_by_recip(alpha[i] - s.dx[i - 1] * zp, s.l[i], s.rl[i]);
         if (i >= lo) z[i] = zp;
     }
 }
-__device__ inline void spline_backward(int N, const double* __restrict__ prep, const double* z, double* y2, int c,
-                                       int warm)
+__device__ inline void spline_backward(int N, const SweepTerms& s, const double* z, double* y2, int c, int warm)
 {
 #pragma clang fp contract(off)
-    const double* mu = prep + 2 * N;
     int lo, hi;
     sweep_range(N, c, &lo, &hi);
     if (c == 0) lo = 0;
@@ -443,7 +455,7 @@ __device__ inline void spline_backward(int N, const double* __restrict__ prep, c
 #pragma unroll 4
     for (int i = min(N - 2, hi - 1 + warm); i >= lo; i--)
     {
-        yn = z[i] - mu[i] * yn;
+        yn = z[i] - s.mu[i] * yn;
         if (i < hi) y2[i] = yn;
     }
 }
@@ -480,7 +492,7 @@ __device__ __forceinline__ Hdr load_hdr(const double* scr)
 // eight terms are written out without selects; and what is serial along the
 // knots, which one wave worked while three waited, is cut into chunks (the
 // splines), bits (the flips) and a prefix sum (the unwrapping).  4096 templates
-// of 202 knots: 718 -> 362 us.  Four waves per SIMD (128 VGPRs): four 256-thread
+// of 202 knots: 718 -> 338 us.  Four waves per SIMD (128 VGPRs): four 256-thread
 // workgroups per CU, as many as the LDS allows.
 __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) resp_kernel(
     Geo g, int n, double* __restrict__ scratch)
@@ -515,13 +527,15 @@ __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_
         const int sp = it / (N - 2), i = 1 + it % (N - 2);
         spline_alpha(N, g.prep_o, ssb + 4 * N * sp, Mx + N * sp, i);
     }
+    const SweepTerms to{As, As + N, As + 2 * N, As + 3 * N};  // not yet written
+    to.fill(N, g.prep_o);
     __syncthreads();
     {
         const int sp = tid / kSweepChunks, c = tid % kSweepChunks;
         double* z = Mx + (2 + sp) * N;
-        if (sp < 2) spline_forward(N, g.prep_o, Mx + N * sp, z, c, g.warm_o);
+        if (sp < 2) spline_forward(N, to, Mx + N * sp, z, c, g.warm_o);
         __syncthreads();
-        if (sp < 2) spline_backward(N, g.prep_o, z, ssb + 4 * N * sp + 2 * N, c, g.warm_o);
+        if (sp < 2) spline_backward(N, to, z, ssb + 4 * N * sp + 2 * N, c, g.warm_o);
     }
     __syncthreads();
     for (int i = tid; i < 2 * N; i += kRespThreads)
@@ -757,12 +771,15 @@ __global__ void __launch_bounds__(kRespThreads) __attribute__((amdgpu_waves_per_
         const int ch = sp >> 1, ph = sp & 1;
         spline_alpha(N, g.prep_s, Mx + (3 * ph + ch) * N, ssb + sp * N, i);
     }
+    static_assert(kMaxKnots <= 512, "mu in the sine table's place");
+    const SweepTerms ts{ssb + 6 * N, ssb + 7 * N, lds, phsc};  // what they held is dead
+    ts.fill(N, g.prep_s);
     __syncthreads();
     {
         const int sp = tid / kSweepChunks, c = tid % kSweepChunks;
-        if (sp < 6) spline_forward(N, g.prep_s, ssb + sp * N, As + sp * N, c, g.warm_s);
+        if (sp < 6) spline_forward(N, ts, ssb + sp * N, As + sp * N, c, g.warm_s);
         __syncthreads();
-        if (sp < 6) spline_backward(N, g.prep_s, As + sp * N, ssb + sp * N, c, g.warm_s);
+        if (sp < 6) spline_backward(N, ts, As + sp * N, ssb + sp * N, c, g.warm_s);
     }
     __syncthreads();
     for (int it = tid; it < 6 * N; it += kRespThreads)
@@ -983,17 +1000,28 @@ __device__ __forceinline__ int pixel_list(const Geo& g, const Hdr& h, int e, con
 // C h; the logL change of adding the template to a zero model with the
 // reference's edge rule (gaussian_log_likelhood_wavelet,
 // utils/src/glass_model.c:805-855).
-__device__ __forceinline__ void pixel_terms(const Geo& g, const LayerArgs& a, int k, const double (&hv)[3],
-                                            double& hh, double& dl)
+struct PixelData
 {
+    double w[6], d[3];  // invC and data planes
+    __device__ __forceinline__ void load(const LayerArgs& a, int k)
+    {
+#pragma unroll
+        for (int p = 0; p < 6; p++) w[p] = a.invC[p * (size_t)a.npix + k];
+#pragma unroll
+        for (int p = 0; p < 3; p++) d[p] = a.data[p * (size_t)a.npix + k];
+    }
+};
+__device__ __forceinline__ void pixel_terms(const Geo& g, const LayerArgs& a, int k, const PixelData& x,
+                                            const double (&hv)[3], double& hh, double& dl)
+{
+    const double* d = x.d;
     double C[3][3];
-    C[0][0] = a.invC[k];
-    C[1][1] = a.invC[(size_t)a.npix + k];
-    C[2][2] = a.invC[2 * (size_t)a.npix + k];
-    C[0][1] = C[1][0] = a.invC[3 * (size_t)a.npix + k];
-    C[0][2] = C[2][0] = a.invC[4 * (size_t)a.npix + k];
-    C[1][2] = C[2][1] = a.invC[5 * (size_t)a.npix + k];
-    const double d[3] = {a.data[k], a.data[(size_t)a.npix + k], a.data[2 * (size_t)a.npix + k]};
+    C[0][0] = x.w[0];
+    C[1][1] = x.w[1];
+    C[2][2] = x.w[2];
+    C[0][1] = C[1][0] = x.w[3];
+    C[0][2] = C[2][0] = x.w[4];
+    C[1][2] = C[2][1] = x.w[5];
     double th = 0.0, tdh = 0.0, tdd = 0.0;
 #pragma unroll
     for (int p = 0; p < 3; p++)
@@ -1038,6 +1066,7 @@ __device__ __forceinline__ void layer_body(const Geo& g, const Hdr& h, int e, co
         if (N <= kStagedKnots)
         {
             double* c = (double*)lds;
+#pragma unroll 8
             for (int i = t; i < spline_doubles(N); i += NTHR) c[i] = cs[i];
             __syncthreads();
 #pragma unroll
@@ -1087,6 +1116,14 @@ __device__ __forceinline__ void layer_body(const Geo& g, const Hdr& h, int e, co
     // c = t + NTHR i, time c / L of layer c % L
     constexpr int CB = 3 * L <= 8 ? 3 : 2;
     double hv[L][3];
+    // the pixels' data, loaded during the inverse transforms (all registers are
+    // taken where there are three layers)
+    constexpr bool EARLY = L <= 2;
+    PixelData x[L];
+    auto pixel = [&](int i) {
+        const int c = t + NTHR * i;
+        return Nw == NT * L ? c / L + (h.jmin + c % L) * NT - g.kmin : a.list[(size_t)e * a.vcap + c];
+    };
     const double norm = sqrt((double)g.NF) / (L + 1.0);
     double* vals = a.values + (size_t)e * 3 * a.vcap;
 #pragma unroll
@@ -1100,6 +1137,10 @@ __device__ __forceinline__ void layer_body(const Geo& g, const Hdr& h, int e, co
             if (ch >= c0 && ch < c0 + nch)
 #pragma unroll
                 for (int off = 0; off < L; off++) lds[((ch - c0) * L + off) * PU + wave_fft_slot(t)] = b[off][ch];
+        if (EARLY && a.data)
+#pragma unroll
+            for (int i = 0; i < L; i++)
+                if (t + NTHR * i < Nw) x[i].load(a, pixel(i));
         __syncthreads();
         wave_fft_units<NT, kCh * L, NTHR, true, 1>(lds, g.tw, kTwN / NT, 0);
         __syncthreads();
@@ -1118,13 +1159,14 @@ __device__ __forceinline__ void layer_body(const Geo& g, const Hdr& h, int e, co
         }
     }
     if (!a.data) return;
-    const int* lst = a.list + (size_t)e * a.vcap;
     double hh = 0.0, dl = 0.0;
 #pragma unroll
     for (int i = 0; i < L; i++)
     {
-        const int c = t + NTHR * i;
-        if (c < Nw) pixel_terms(g, a, Nw == NT * L ? c / L + (h.jmin + c % L) * NT - g.kmin : lst[c], hv[i], hh, dl);
+        if (t + NTHR * i >= Nw) continue;
+        const int k = pixel(i);
+        if (!EARLY) x[i].load(a, k);
+        pixel_terms(g, a, k, x[i], hv[i], hh, dl);
     }
     hh = block_sum<NTHR>(hh);
     dl = block_sum<NTHR>(dl);
@@ -1170,7 +1212,7 @@ static size_t layer_lds_bytes(int N)
 // their inverse transforms; the pixel list and inner products.  (One workgroup
 // for all of a template, with ping-pong stages of the whole series through L2
 // and a fifth of the CUs holding a second one, left the vector units 10% busy.)
-// 300 templates of 4096 time pixels: 651 -> 273 us.
+// 300 templates of 4096 time pixels: 651 -> 271 us.
 
 constexpr int kSeriesThreads = 512;
 constexpr int kSumThreads = 1024;
@@ -1204,6 +1246,7 @@ __global__ void __launch_bounds__(kSeriesThreads) __attribute__((amdgpu_waves_pe
     const bool staged = N <= kStagedKnots;
     if (staged)
     {
+#pragma unroll 8
         for (int i = threadIdx.x; i < spline_doubles(N); i += kSeriesThreads) ldss[i] = cs[i];
         __syncthreads();
     }
@@ -1388,7 +1431,10 @@ __global__ void __launch_bounds__(kSumThreads) sum_kernel_big(Geo g, int e0, Lay
         for (int c = t; c < Nw; c += kSumThreads)
         {
             const double hv[3] = {vals[c], vals[a.vcap + c], vals[2 * a.vcap + c]};
-            pixel_terms(g, a, Nw == NT * L ? c / L + (h.jmin + c % L) * NT - g.kmin : lst[c], hv, hh, dl);
+            const int k = Nw == NT * L ? c / L + (h.jmin + c % L) * NT - g.kmin : lst[c];
+            PixelData x;
+            x.load(a, k);
+            pixel_terms(g, a, k, x, hv, hh, dl);
         }
         hh = block_sum<kSumThreads>(hh);
         dl = block_sum<kSumThreads>(dl);
