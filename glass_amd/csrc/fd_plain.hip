@@ -186,23 +186,21 @@ static int ucb_waveform_dropin(const glass_hip_orbit* ao, const glass_hip_numeri
     int rc;
     if ((rc = ctx_get(&cx))) return rc;
     const size_t outb = sizeof(double2) * 5 * (size_t)BW;
-    if ((rc = cx->dbuf.ensure(outb + 128))) return rc;
+    // parameters and template in the pinned buffer itself: two copies around a
+    // kernel of 10 us took longer than it
     if ((rc = cx->hbuf.ensure(outb + 128))) return rc;
-    double* hp = (double*)cx->hbuf.p;
-    double* dp = (double*)((char*)cx->dbuf.p + outb);
-    memcpy(hp + 10 * BW, params, sizeof(double) * NParams);
-    GH_CHECK(hipMemcpyAsync(dp, hp + 10 * BW, sizeof(double) * NParams, hipMemcpyHostToDevice, cx->stream));
+    double *hp = (double*)cx->hbuf.p, *dp = hp + 10 * BW;
+    double2* out = (double2*)hp;
+    memcpy(dp, params, sizeof(double) * NParams);
     if (ao)
-        rc = fd_waveform_launch(1, dp, NParams, T, t0, *ao, BW, fmt, (double2*)cx->dbuf.p, cx->stream);
+        rc = fd_waveform_launch(1, dp, NParams, T, t0, *ao, BW, fmt, out, cx->stream);
     else
     {
         const double* pos = nullptr;
         if (!(rc = numeric_positions(*no, T, t0, BW, &pos)))
-            rc = fd_waveform_launch_pos(1, dp, NParams, T, t0, no->L, no->fstar, pos, BW, fmt, (double2*)cx->dbuf.p,
-                                        cx->stream);
+            rc = fd_waveform_launch_pos(1, dp, NParams, T, t0, no->L, no->fstar, pos, BW, fmt, out, cx->stream);
     }
     if (rc) return rc;
-    GH_CHECK(hipMemcpyAsync(hp, cx->dbuf.p, outb, hipMemcpyDeviceToHost, cx->stream));
     GH_CHECK(hipStreamSynchronize(cx->stream));
     double* outs[5] = {X, Y, Z, A, E};
     for (int ch = 0; ch < (all ? 5 : 1); ch++) memcpy(outs[ch], hp + (size_t)ch * 2 * BW, sizeof(double) * 2 * BW);

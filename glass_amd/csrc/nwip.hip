@@ -5,7 +5,13 @@
 //
 // Streaming, HBM-bound kernels: each block reduces a contiguous range of
 // bins with coalesced loads, writes one partial; a single-block pass sums
-// the partials in block order (deterministic).
+// the partials in block order (deterministic).  One block alone writes the
+// result.
+//
+// A call of a few hundred bins is bound by its launches and copies, not by its
+// bytes: results go to the pinned staging buffer, and inputs of up to
+// kInPlaceBytes are read from there (a waveform and a likelihood of 128 and 256
+// bins 79 -> 67 us with both).
 #include <cmath>
 #include <cstring>
 
@@ -30,7 +36,7 @@ struct NwipTerms
     int nterm;
 };
 
-__global__ __launch_bounds__(kRedThr) void nwip_kernel(NwipTerms T, int N, int chunk, double* part)
+__global__ __launch_bounds__(kRedThr) void nwip_kernel(NwipTerms T, int N, int chunk, double scale, double* part)
 {
     const int b0 = blockIdx.x * chunk, b1 = min(N, b0 + chunk);
     double acc = 0.0;
@@ -45,7 +51,7 @@ __global__ __launch_bounds__(kRedThr) void nwip_kernel(NwipTerms T, int N, int c
         acc += T.coef[t] * s;
     }
     acc = block_sum<kRedThr>(acc);
-    if (threadIdx.x == 0) part[blockIdx.x] = acc;
+    if (threadIdx.x == 0) part[blockIdx.x] = scale * acc;
 }
 
 __global__ __launch_bounds__(kRedThr) void sum_partials(const double* part, int n, double scale, double* out)
@@ -62,7 +68,7 @@ __global__ __launch_bounds__(kRedThr) void sum_partials(const double* part, int 
 __global__ __launch_bounds__(kRedThr) void logl3_kernel(const double2* __restrict__ dX, const double2* __restrict__ dY,
                                                         const double2* __restrict__ dZ, const double2* __restrict__ mX,
                                                         const double2* __restrict__ mY, const double2* __restrict__ mZ,
-                                                        const double* __restrict__ invC, int N, int chunk, double* part)
+                                                        const double* __restrict__ invC, int N, int chunk, double scale, double* part)
 {
     const int b0 = blockIdx.x * chunk, b1 = min(N, b0 + chunk);
     double acc = 0.0;
@@ -82,12 +88,12 @@ __global__ __launch_bounds__(kRedThr) void logl3_kernel(const double2* __restric
         acc += diag + 2.0 * off;
     }
     acc = block_sum<kRedThr>(acc);
-    if (threadIdx.x == 0) part[blockIdx.x] = acc;
+    if (threadIdx.x == 0) part[blockIdx.x] = scale * acc;
 }
 
 __global__ __launch_bounds__(kRedThr) void wnwip_kernel(const double* __restrict__ a, const double* __restrict__ b,
                                                         const double* __restrict__ w, const int* __restrict__ list,
-                                                        int N, int chunk, double* part)
+                                                        int N, int chunk, double scale, double* part)
 {
     const int b0 = blockIdx.x * chunk, b1 = min(N, b0 + chunk);
     double acc = 0.0;
@@ -97,7 +103,7 @@ __global__ __launch_bounds__(kRedThr) void wnwip_kernel(const double* __restrict
         acc += a[k] * b[k] * w[k];
     }
     acc = block_sum<kRedThr>(acc);
-    if (threadIdx.x == 0) part[blockIdx.x] = acc;
+    if (threadIdx.x == 0) part[blockIdx.x] = scale * acc;
 }
 
 // Per-bin analytic 3x3 inverse with Cholesky-like pivots and signed
@@ -138,48 +144,77 @@ static int grid_for(int N, int* chunk)
     return nb;
 }
 
+// Where the blocks of a reduction put their sums, and times what: the result
+// itself for a single block, else the partials that finish() adds up.
+struct Reduction
+{
+    int nb, chunk;
+    double scale, *out, *part, block_scale;
+    int init(ThreadCtx* cx, int N, double s, double* d_out)
+    {
+        if (int rc = cx->dpart.ensure(sizeof(double) * kMaxPart)) return rc;
+        nb = grid_for(N, &chunk);
+        scale = s;
+        out = d_out;
+        part = nb == 1 ? out : (double*)cx->dpart.p;
+        block_scale = nb == 1 ? scale : 1.0;
+        return GLASS_HIP_OK;
+    }
+    int finish(ThreadCtx* cx) const
+    {
+        if (nb > 1) sum_partials<<<1, kRedThr, 0, cx->stream>>>(part, nb, scale, out);
+        GH_CHECK(hipGetLastError());
+        return GLASS_HIP_OK;
+    }
+};
+
 // Device-pointer reductions (stream-ordered); result to *d_out.
 int nwip_terms_dev(const NwipTerms& T, int N, double scale, double* d_out, ThreadCtx* cx)
 {
-    int rc, chunk;
-    if ((rc = cx->dpart.ensure(sizeof(double) * kMaxPart))) return rc;
-    int nb = grid_for(N, &chunk);
-    nwip_kernel<<<nb, kRedThr, 0, cx->stream>>>(T, N, chunk, (double*)cx->dpart.p);
-    sum_partials<<<1, kRedThr, 0, cx->stream>>>((double*)cx->dpart.p, nb, scale, d_out);
-    GH_CHECK(hipGetLastError());
-    return GLASS_HIP_OK;
+    Reduction r;
+    if (int rc = r.init(cx, N, scale, d_out)) return rc;
+    nwip_kernel<<<r.nb, kRedThr, 0, cx->stream>>>(T, N, r.chunk, r.block_scale, r.part);
+    return r.finish(cx);
 }
 
-// Stage host arrays into the thread's device buffer; returns device ptrs.
-static int stage(ThreadCtx* cx, int n, const void* const* src, const size_t* bytes, void** dst, double** d_res)
+// Stages host arrays; returns the pointers for kernels, to the thread's device
+// buffer or, for a few, to the pinned buffer itself, and the result's place in
+// the pinned buffer.  The likelihood, which reads each bin once, gains at every
+// size measured (256 bins, 42 KB, 43 -> 35 us; 2048 bins, 336 KB, 54 -> 46; 8192
+// bins, 1.3 MB, 90 -> 80); snr reads its planes two or three times (256 bins, 24
+// KB, 35 -> 28 us, but 1024 bins, 96 KB, 44 -> 52).
+constexpr size_t kInPlaceBytes = 256 * 1024, kInPlaceReread = 32 * 1024;
+static int stage(ThreadCtx* cx, int n, const void* const* src, const size_t* bytes, void** dst, double** d_res,
+                 size_t limit = kInPlaceBytes)
 {
     size_t tot = 256;
     for (int i = 0; i < n; i++) tot += (bytes[i] + 255) & ~(size_t)255;
+    const bool in_place = tot <= limit;
     int rc;
-    if ((rc = cx->dbuf.ensure(tot))) return rc;
+    if (!in_place && (rc = cx->dbuf.ensure(tot))) return rc;
     if ((rc = cx->hbuf.ensure(tot))) return rc;
+    char* base = (char*)(in_place ? cx->hbuf.p : cx->dbuf.p);
     size_t off = 0;
     for (int i = 0; i < n; i++)
     {
         memcpy((char*)cx->hbuf.p + off, src[i], bytes[i]);
-        dst[i] = (char*)cx->dbuf.p + off;
+        dst[i] = base + off;
         off += (bytes[i] + 255) & ~(size_t)255;
     }
-    GH_CHECK(hipMemcpyAsync(cx->dbuf.p, cx->hbuf.p, off, hipMemcpyHostToDevice, cx->stream));
-    *d_res = (double*)((char*)cx->dbuf.p + off);
+    if (!in_place) GH_CHECK(hipMemcpyAsync(cx->dbuf.p, cx->hbuf.p, off, hipMemcpyHostToDevice, cx->stream));
+    *d_res = (double*)((char*)cx->hbuf.p + off);
     return GLASS_HIP_OK;
 }
 
-static double fetch_result(ThreadCtx* cx, double* d_res)
+// The result that the stream's kernels leave at res in the pinned buffer.
+static double fetch_result(ThreadCtx* cx, const double* res)
 {
-    double* h = (double*)((char*)cx->hbuf.p);
-    if (hipMemcpyAsync(h, d_res, sizeof(double), hipMemcpyDeviceToHost, cx->stream) != hipSuccess ||
-        hipStreamSynchronize(cx->stream) != hipSuccess)
+    if (hipStreamSynchronize(cx->stream) != hipSuccess)
     {
-        set_error("result copy failed");
+        set_error("reduction failed");
         return NAN;
     }
-    return h[0];
+    return *res;
 }
 
 }  // namespace glass
@@ -231,7 +266,7 @@ extern "C" double glass_hip_snr(const double* X, const double* Y, const double* 
     for (int i = 3; i < 9; i++) by[i] = sizeof(double) * N;
     void* d[9];
     double* dres;
-    if (stage(cx, 9, src, by, d, &dres)) return NAN;
+    if (stage(cx, 9, src, by, d, &dres, kInPlaceReread)) return NAN;
     NwipTerms T{};
     T.nterm = 6;
     const int ia[6] = {0, 1, 2, 0, 0, 1}, ib[6] = {0, 1, 2, 1, 2, 2};
@@ -268,17 +303,11 @@ extern "C" double glass_hip_wavelet_nwip(const double* a, const double* b, const
     void* d[4];
     double* dres;
     if (stage(cx, 4, src, by, d, &dres)) return NAN;
-    int rc, chunk;
-    if ((rc = cx->dpart.ensure(sizeof(double) * kMaxPart))) return NAN;
-    int nb = grid_for(N, &chunk);
-    wnwip_kernel<<<nb, kRedThr, 0, cx->stream>>>((const double*)d[0], (const double*)d[1], (const double*)d[2],
-                                                  (const int*)d[3], N, chunk, (double*)cx->dpart.p);
-    sum_partials<<<1, kRedThr, 0, cx->stream>>>((double*)cx->dpart.p, nb, 1.0, dres);
-    if (hipGetLastError() != hipSuccess)
-    {
-        set_error("wavelet_nwip launch failed");
-        return NAN;
-    }
+    Reduction r;
+    if (r.init(cx, N, 1.0, dres)) return NAN;
+    wnwip_kernel<<<r.nb, kRedThr, 0, cx->stream>>>((const double*)d[0], (const double*)d[1], (const double*)d[2],
+                                                   (const int*)d[3], N, r.chunk, r.block_scale, r.part);
+    if (r.finish(cx)) return NAN;
     return fetch_result(cx, dres);
 }
 
@@ -307,19 +336,13 @@ extern "C" double glass_hip_gaussian_log_likelihood(const double* dX, const doub
         size_t by[7] = {cb, cb, cb, cb, cb, cb, 9 * pb};
         void* d[7];
         if (stage(cx, 7, src, by, d, &dres)) return NAN;
-        int chunk;
-        if (cx->dpart.ensure(sizeof(double) * kMaxPart)) return NAN;
-        int nb = grid_for(NFFT, &chunk);
-        logl3_kernel<<<nb, kRedThr, 0, cx->stream>>>((const double2*)d[0], (const double2*)d[1], (const double2*)d[2],
-                                                      (const double2*)d[3], (const double2*)d[4], (const double2*)d[5],
-                                                      (const double*)d[6], NFFT, chunk, (double*)cx->dpart.p);
         // chi2 = 2 * sum; logL = -chi2/2
-        sum_partials<<<1, kRedThr, 0, cx->stream>>>((double*)cx->dpart.p, nb, -1.0, dres);
-        if (hipGetLastError() != hipSuccess)
-        {
-            set_error("logL launch failed");
-            return NAN;
-        }
+        Reduction r;
+        if (r.init(cx, NFFT, -1.0, dres)) return NAN;
+        logl3_kernel<<<r.nb, kRedThr, 0, cx->stream>>>((const double2*)d[0], (const double2*)d[1], (const double2*)d[2],
+                                                       (const double2*)d[3], (const double2*)d[4], (const double2*)d[5],
+                                                       (const double*)d[6], NFFT, r.chunk, r.block_scale, r.part);
+        if (r.finish(cx)) return NAN;
         return fetch_result(cx, dres);
     }
     // 1 channel (X) or 2 channels (A,E): diagonal terms only (glass_model.c:749-756)
@@ -337,7 +360,7 @@ extern "C" double glass_hip_gaussian_log_likelihood(const double* dX, const doub
     const void* src[6] = {dd[0], mm[0], invC, dd[nc - 1], mm[nc - 1], invC + 4 * (size_t)NFFT};
     size_t by[6] = {cb, cb, pb, cb, cb, pb};
     void* d[6];
-    if (stage(cx, 6, src, by, d, &dres)) return NAN;
+    if (stage(cx, 6, src, by, d, &dres, kInPlaceReread)) return NAN;
     // residual in place on the device copies of the data arrays
     // r = d - m via a 2-term expansion: (d-m).(d-m) = d.d - 2 d.m + m.m
     // would lose precision; use a dedicated pass instead.
@@ -391,7 +414,7 @@ namespace glass {
 // per pixel XX + 2 XY as snr_wavelet / gaussian_log_likelhood_wavelet
 // group it (utils/src/glass_math.c:428-438, utils/src/glass_model.c:839-853)
 __global__ __launch_bounds__(kRedThr) void wquad_kernel(const double* __restrict__ r, const double* __restrict__ C,
-                                                        int n, int chunk, double* part)
+                                                        int n, int chunk, double scale, double* part)
 {
     const int b0 = blockIdx.x * chunk, b1 = min(n, b0 + chunk);
     double acc = 0.0;
@@ -403,7 +426,7 @@ __global__ __launch_bounds__(kRedThr) void wquad_kernel(const double* __restrict
         acc += xx + 2.0 * xy;
     }
     acc = block_sum<kRedThr>(acc);
-    if (threadIdx.x == 0) part[blockIdx.x] = acc;
+    if (threadIdx.x == 0) part[blockIdx.x] = scale * acc;
 }
 
 // Stages n pixels of 9 planes (r: 3, C: 6) already laid out in the pinned
@@ -416,18 +439,12 @@ static double wquad_staged(ThreadCtx* cx, int n)
         set_error("wavelet staging copy failed");
         return NAN;
     }
-    int chunk;
-    if (cx->dpart.ensure(sizeof(double) * kMaxPart)) return NAN;
-    const int nb = grid_for(n, &chunk);
     const double* d = (const double*)cx->dbuf.p;
-    double* dres = (double*)((char*)cx->dbuf.p + ((planes + 255) & ~(size_t)255));
-    wquad_kernel<<<nb, kRedThr, 0, cx->stream>>>(d, d + 3 * (size_t)n, n, chunk, (double*)cx->dpart.p);
-    sum_partials<<<1, kRedThr, 0, cx->stream>>>((double*)cx->dpart.p, nb, 1.0, dres);
-    if (hipGetLastError() != hipSuccess)
-    {
-        set_error("wavelet reduction launch failed");
-        return NAN;
-    }
+    double* dres = (double*)cx->hbuf.p;  // the staged planes are on the device by then
+    Reduction r;
+    if (r.init(cx, n, 1.0, dres)) return NAN;
+    wquad_kernel<<<r.nb, kRedThr, 0, cx->stream>>>(d, d + 3 * (size_t)n, n, r.chunk, r.block_scale, r.part);
+    if (r.finish(cx)) return NAN;
     return fetch_result(cx, dres);
 }
 
