@@ -1,6 +1,6 @@
 // fd_plain.hip -- the per-call drop-in for ucb_waveform
 // (ucb/src/glass_ucb_waveform.c:738-1001): one workgroup builds one template
-// (slow series -> 6 LDS FFTs -> TDI) and writes X,Y,Z,A,E.
+// (slow series -> 5 LDS FFTs -> TDI) and writes X,Y,Z,A,E.
 #include <cmath>
 #include <cstring>
 #include <map>
