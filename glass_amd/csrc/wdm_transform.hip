@@ -269,10 +269,12 @@ __global__ void __launch_bounds__(NTH) layer_fwd_kernel(const double2* __restric
 }
 
 // Layers of up to 512 time pixels: a wave takes 512 / NT of them from the
-// spectrum to the pixels by itself, eight points a lane, with no barriers.
-// 4097 layers of 512: 22 us, as with a workgroup a layer; what is left is the
-// spectrum bins (two loads and a sine and cosine each).
-constexpr int kLayerWaves = 4;
+// spectrum to the pixels by itself, eight points a lane, with no barriers.  One
+// wave a workgroup, for 17 on a CU by their LDS (four to a workgroup make 16, and
+// the 4097 waves of 4096 layers of 512 then take a second turn: 21.8 us against
+// 19.8; a workgroup of 128 threads a layer took 21.8).  Forming the spectrum's bins
+// once, in a row pass that pairs rows k and M1 - k, moves 4 us from here to there.
+constexpr int kLayerWaves = 1;
 template <int NT, bool FROM_Z>
 __global__ void __launch_bounds__(64 * kLayerWaves) layer_wave_kernel(const double2* __restrict__ src,
                                                                       double* __restrict__ wdm, int NF,
