@@ -464,6 +464,7 @@ struct glass_hip_fstat
     double* cells = nullptr;
     double *lx = nullptr, *lae = nullptr, *fpar = nullptr;
     int *cls = nullptr, *list = nullptr, *kcls = nullptr;
+    char* work = nullptr;  // per cell constants, sums and class (Cells), one allocation
     UcbConst* pc = nullptr;
     double* sums = nullptr;
 };
@@ -539,12 +540,14 @@ extern "C" int glass_hip_fstat_create(glass_hip_fstat** out, const glass_hip_orb
         (rc = falloc(F, &F->cells, 4 * (size_t)max_cells)) || (rc = falloc(F, &F->lx, max_cells)) ||
         (rc = falloc(F, &F->lae, max_cells)) || (rc = falloc(F, &F->fpar, 4 * (size_t)max_cells)) ||
         (rc = falloc(F, &F->cls, kFsClass + 1)) || (rc = falloc(F, &F->list, (size_t)kFsClass * max_cells)) ||
-        (rc = falloc(F, &F->kcls, max_cells)) || (rc = falloc(F, &F->pc, max_cells)) ||
-        (rc = falloc(F, &F->sums, (size_t)kFsSum * max_cells)))
+        (rc = falloc(F, &F->work, (sizeof(UcbConst) + sizeof(double) * kFsSum + sizeof(int)) * (size_t)max_cells)))
     {
         glass_hip_fstat_destroy(F);
         return rc;
     }
+    F->pc = (UcbConst*)F->work;
+    F->sums = (double*)(F->pc + max_cells);
+    F->kcls = (int*)(F->sums + (size_t)kFsSum * max_cells);
     const double* pos = nullptr;
     const double2* tw = nullptr;
     if ((rc = positions(*orbit, T, t0, kPosNF, &pos)) || (rc = twiddles(&tw)))
