@@ -142,7 +142,7 @@ __global__ __launch_bounds__(fd_threads(N)) void adjoint_kernel(DerivArgs A)
         // bin m = P t + r is FFT index P k + r: per residue r the NT-point
         // transform over k, then sample n = t + NT p sums the residues with
         // w_N^{r t} w_P^{r p}
-        const int k = wave_fft_slot((t + NT / 2) & (NT - 1)), ts = wave_fft_slot(t);
+        const int k = S::place(t + NT / 2), ts = S::place(t);
         const bool on = NT >= 64 || t < NT;
 #pragma unroll
         for (int r = 0; r < P; r++)

@@ -56,6 +56,10 @@ struct FdShape
     static __device__ __forceinline__ int group() { return G == 1 ? 0 : threadIdx.x >> 9; }
     static __device__ __forceinline__ int residue(int s) { return G == 1 ? s : group() * (Q / 2) + s / 2 + Q * (s % 2); }
     static __device__ __forceinline__ int bin(int s) { return P * lane() + residue(s); }
+    // LDS place of thread t's point of a series.  A series of 16 or 32 points
+    // has fewer than its workgroup's 64 threads: the others get a place of it
+    // too, so that a read without a test stays within the series.
+    __host__ __device__ static constexpr int place(int t) { return wave_fft_slot(t & (NT - 1)); }
     // where the series of pass s waits
     static constexpr int slot(int s) { return G == 1 ? s : s / 2 + (Q / 2) * (s % 2); }
 };
