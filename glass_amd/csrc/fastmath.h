@@ -651,8 +651,9 @@ GH_HD inline void sinc_phase(const double (&x)[M], bool wide, double (&fr)[M], d
 }
 
 // Whether the transfer-function arguments of a template may leave |x| <=
-// 1.75, from its largest |f|/f*: they reach (1 + k.r/L)/2 times it, up to
-// 1.25 with the arm half as long again as L.
-GH_HD inline bool sinc_wide(double fmax) { return !(1.25 * fmax <= 1.75); }
+// 1.75, from its largest |f| and the factor (1 + k.r/L)/(2 f*) that the
+// orbit's arms reach.  With |f|/f* instead of |f| the factor is 1.25 for an arm
+// half as long again as L.
+GH_HD inline bool sinc_wide(double fmax, double reach = 1.25) { return !(reach * fmax <= 1.75); }
 
 }  // namespace glass

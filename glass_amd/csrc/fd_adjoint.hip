@@ -71,7 +71,7 @@ __global__ __launch_bounds__(fd_threads(N)) void adjoint_kernel(DerivArgs A)
     // the template constants and their derivatives on lanes of two waves,
     // so the two serial setups overlap (one wave at 32/64 bins: in turn)
     __shared__ UcbConst sc;
-    if (t == 0) ucb_setup(p, 8, A.T, A.t0, A.L, A.fstar, sc);
+    if (t == 0) ucb_setup(p, 8, A.T, A.t0, A.L, A.fstar, A.reach, sc);
     if (GRAD && t == (NTHR >= 128 ? 64 : 0)) ucb_diff_setup(p, A.T, sdd);
     __syncthreads();
     UcbConst c = sc;  // into scalar registers for the passes
@@ -288,6 +288,7 @@ extern "C" int glass_hip_fd_source_grad(const glass_hip_orbit* orbit, const char
     A.t0 = t0;
     A.L = orbit->L;
     A.fstar = orbit->fstar;
+    A.reach = analytic_reach(orbit->L, orbit->fstar, orbit->R, T, t0);
     A.pos = pos;
     A.tw = tw;
     A.fmt = fmt;

@@ -90,6 +90,7 @@ struct BatchDev
     struct EvalRec* rec;      // per-item places, written by align_kernel
     // constants
     double T, t0, L, fstar;
+    OrbitReach reach;
     const double* pos;      // positions table, kPosN samples
     const double* pos_soa;  // structure-of-arrays position blocks per series length
     const double2* tw;
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(kAlignOne) void align_kernel(int n, Items it, Batch
         bw_out[e] = BW;
         imin_out[e] = qmin - B.g_qmin[g];
         // the template constants and places of the class kernels, once per item
-        ucb_setup(p, 8, B.T, B.t0, B.L, B.fstar, B.pc[e]);
+        ucb_setup(p, 8, B.T, B.t0, B.L, B.fstar, B.reach, B.pc[e]);
         const int s = item_src(it, e), so = c * B.maxsrc + s;
         EvalRec r;
         r.tmpl = src_tmpl(B, c, s);
@@ -1193,6 +1194,7 @@ extern "C" int glass_hip_fd_batch_create_ex(glass_hip_fd_batch** plan, const gla
     B.t0 = t0;
     B.L = orbit->L;
     B.fstar = orbit->fstar;
+    B.reach = analytic_reach(orbit->L, orbit->fstar, orbit->R, T, t0);
     B.pos = pos;
     B.pos_soa = pos_soa;
     B.tw = tw;
@@ -1707,6 +1709,7 @@ extern "C" int glass_hip_fd_batch_derivs(glass_hip_fd_batch* P, int n, const int
     A.t0 = B.t0;
     A.L = B.L;
     A.fstar = B.fstar;
+    A.reach = B.reach;
     A.pos = B.pos;
     A.tw = B.tw;
     A.fmt = B.fmt;

@@ -4,6 +4,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "ucb_common.h"
+
 namespace glass {
 
 struct DerivArgs
@@ -42,6 +44,7 @@ struct DerivArgs
     double* outL;
     double* grad;
     double* fisher;
+    OrbitReach reach;
 };
 
 // deriv_kernel<N> over grid workgroups (N a power of two, 32..1024).

@@ -300,7 +300,7 @@ __device__ __forceinline__ void deriv_write(const UcbConst& c, const UcbDiff& dd
 template <int NTHR>
 __device__ __forceinline__ void deriv_setup(const double* p, const DerivArgs& A, UcbConst& sc, UcbDiff& sdd)
 {
-    if (threadIdx.x == 0) ucb_setup(p, 8, A.T, A.t0, A.L, A.fstar, sc);
+    if (threadIdx.x == 0) ucb_setup(p, 8, A.T, A.t0, A.L, A.fstar, A.reach, sc);
     if (threadIdx.x == (NTHR >= 128 ? 64 : 0)) ucb_diff_setup(p, A.T, sdd);
     __syncthreads();
 }
@@ -478,6 +478,7 @@ extern "C" int glass_hip_fd_source_derivs(const glass_hip_orbit* orbit, const ch
     A.t0 = t0;
     A.L = orbit->L;
     A.fstar = orbit->fstar;
+    A.reach = analytic_reach(orbit->L, orbit->fstar, orbit->R, T, t0);
     A.pos = pos;
     A.tw = tw;
     A.fmt = fmt;

@@ -17,12 +17,12 @@ namespace glass {
 template <int N, int NTHR>
 __global__ __launch_bounds__(NTHR) void fd_waveform_kernel(const double* __restrict__ params, int np,
                                                            double T, double t0, double L, double fstar,
-                                                           const double* __restrict__ pos, int posstride,
+                                                           OrbitReach reach, const double* __restrict__ pos, int posstride,
                                                            const double2* __restrict__ tw, int twstride,
                                                            int fmt, double2* __restrict__ out)
 {
     __shared__ double2 lds[FdShape<N>::LDS];
-    const UcbConst& c = ucb_setup_shared(params + (size_t)blockIdx.x * np, np, T, t0, L, fstar);
+    const UcbConst& c = ucb_setup_shared(params + (size_t)blockIdx.x * np, np, T, t0, L, fstar, reach);
     double2* o = out + (size_t)blockIdx.x * 5 * N;
     fd_link_bins<N, false>(
         HeldConst{c}, lds, pos, posstride, tw, twstride, [](int) {}, [&](int, int m, const double2* d) {
@@ -35,18 +35,19 @@ __global__ __launch_bounds__(NTHR) void fd_waveform_kernel(const double* __restr
 
 template <int N>
 static void launch_fd(int ntmpl, const double* params, int np, double T, double t0, double L,
-                      double fstar, const double* pos, int posstride, const double2* tw, int fmt,
+                      double fstar, OrbitReach reach, const double* pos, int posstride, const double2* tw, int fmt,
                       double2* out, hipStream_t s)
 {
     constexpr int NTHR = fd_threads(N);
-    fd_waveform_kernel<N, NTHR><<<ntmpl, NTHR, 0, s>>>(params, np, T, t0, L, fstar, pos, posstride, tw,
+    fd_waveform_kernel<N, NTHR><<<ntmpl, NTHR, 0, s>>>(params, np, T, t0, L, fstar, reach, pos, posstride, tw,
                                                         kTwN / N, fmt, out);
 }
 
 // The template kernel over ntmpl templates with the positions table pos
 // (9 doubles per slow sample, BW samples).
 static int fd_waveform_launch_pos(int ntmpl, const double* d_params, int np, double T, double t0, double L,
-                                  double fstar, const double* pos, int BW, int fmt, double2* d_out, hipStream_t s)
+                                  double fstar, OrbitReach reach, const double* pos, int BW, int fmt, double2* d_out,
+                                  hipStream_t s)
 {
     const double2* tw = nullptr;
     int rc;
@@ -54,7 +55,7 @@ static int fd_waveform_launch_pos(int ntmpl, const double* d_params, int np, dou
     switch (BW)
     {
 #define GH_CASE(n) \
-    case n: launch_fd<n>(ntmpl, d_params, np, T, t0, L, fstar, pos, 1, tw, fmt, d_out, s); break;
+    case n: launch_fd<n>(ntmpl, d_params, np, T, t0, L, fstar, reach, pos, 1, tw, fmt, d_out, s); break;
         GH_CASE(16) GH_CASE(32) GH_CASE(64) GH_CASE(128) GH_CASE(256) GH_CASE(512) GH_CASE(1024) GH_CASE(2048) GH_CASE(4096)
 #undef GH_CASE
         default: set_error("BW=%d unsupported (power of two 16..4096)", BW); return GLASS_HIP_EINVAL;
@@ -68,7 +69,8 @@ int fd_waveform_launch(int ntmpl, const double* d_params, int np, double T, doub
 {
     const double* pos = nullptr;
     if (int rc = positions(o, T, t0, BW, &pos)) return rc;
-    return fd_waveform_launch_pos(ntmpl, d_params, np, T, t0, o.L, o.fstar, pos, BW, fmt, d_out, s);
+    return fd_waveform_launch_pos(ntmpl, d_params, np, T, t0, o.L, o.fstar, analytic_reach(o.L, o.fstar, o.R, T, t0),
+                                  pos, BW, fmt, d_out, s);
 }
 
 namespace wdm {
@@ -81,10 +83,15 @@ void spline_host(int N, const double* x, const double* y, double* c);  // wdm_uc
 // spline_interpolation's binary search and cubic (:180-208), on the host in
 // the reference's operation order; the table is cached on the device per
 // (device, orbit data, T, t0, npos).
-static int numeric_positions(const glass_hip_numeric_orbit& o, double T, double t0, int npos, const double** out)
+static int numeric_positions(const glass_hip_numeric_orbit& o, double T, double t0, int npos, const double** out,
+                             OrbitReach* reach)
 {
+    struct Table
+    {
+        double *pos, arm, far;  // longest arm and largest distance in it
+    };
     static std::mutex mu;
-    static std::map<std::vector<double>, double*> cache;
+    static std::map<std::vector<double>, Table> cache;
     const int N = o.Norb;
     int dev = 0;
     GH_CHECK(hipGetDevice(&dev));
@@ -101,7 +108,8 @@ static int numeric_positions(const glass_hip_numeric_orbit& o, double T, double 
     auto it = cache.find(key);
     if (it != cache.end())
     {
-        *out = it->second;
+        *out = it->second.pos;
+        *reach = orbit_reach(o.L, o.fstar, T, t0, it->second.arm, it->second.far);
         return GLASS_HIP_OK;
     }
     for (int n = 1; n < N; n++)
@@ -134,11 +142,13 @@ static int numeric_positions(const glass_hip_numeric_orbit& o, double T, double 
             for (int d = 0; d < 3; d++)
                 h[9 * (size_t)n + 3 * d + sc] = wdm::spline_at(coef.data() + 4 * (size_t)N * (3 * sc + d), N, k, dx);
     }
-    double* dptr = nullptr;
-    GH_CHECK(hipMalloc(&dptr, sizeof(double) * h.size()));
-    GH_CHECK(hipMemcpy(dptr, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
-    cache[key] = dptr;
-    *out = dptr;
+    Table tab{nullptr, 0.0, 0.0};
+    positions_extent(h.data(), npos, &tab.arm, &tab.far);
+    GH_CHECK(hipMalloc(&tab.pos, sizeof(double) * h.size()));
+    GH_CHECK(hipMemcpy(tab.pos, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
+    cache[key] = tab;
+    *out = tab.pos;
+    *reach = orbit_reach(o.L, o.fstar, T, t0, tab.arm, tab.far);
     return GLASS_HIP_OK;
 }
 
@@ -197,8 +207,9 @@ static int ucb_waveform_dropin(const glass_hip_orbit* ao, const glass_hip_numeri
     else
     {
         const double* pos = nullptr;
-        if (!(rc = numeric_positions(*no, T, t0, BW, &pos)))
-            rc = fd_waveform_launch_pos(1, dp, NParams, T, t0, no->L, no->fstar, pos, BW, fmt, out, cx->stream);
+        OrbitReach reach;
+        if (!(rc = numeric_positions(*no, T, t0, BW, &pos, &reach)))
+            rc = fd_waveform_launch_pos(1, dp, NParams, T, t0, no->L, no->fstar, reach, pos, BW, fmt, out, cx->stream);
     }
     if (rc) return rc;
     GH_CHECK(hipStreamSynchronize(cx->stream));

@@ -131,11 +131,11 @@ struct LoadedConst
 // LDS; every thread reads them from there.  Synchronises the workgroup on
 // entry (readers of the previous template are done) and on exit.
 __device__ inline const UcbConst& ucb_setup_shared(const double* p, int np, double T, double t0, double L,
-                                                   double fstar)
+                                                   double fstar, OrbitReach reach)
 {
     __shared__ UcbConst sc;
     __syncthreads();
-    if (threadIdx.x == 0) ucb_setup(p, np, T, t0, L, fstar, sc);
+    if (threadIdx.x == 0) ucb_setup(p, np, T, t0, L, fstar, reach, sc);
     __syncthreads();
     return sc;
 }

@@ -56,6 +56,7 @@ struct FstatDev
     const double* C00;
     int NFFT, qmin0;
     double T, t0, L, fstar;
+    OrbitReach reach;
     int fmt;
     const double* pos;
     const double2* tw;
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(256) void fstat_align_kernel(int n, FstatDev D,
         C.cls[e] = k;
         // amplitude and polarisation come with each filter
         const double p[8] = {f0 * D.T, cos(theta), phi, 0.0, 0.0, 0.0, D.f[0].phase, fdot * (D.T * D.T)};
-        ucb_setup(p, 8, D.T, D.t0, D.L, D.fstar, C.pc[e]);
+        ucb_setup(p, 8, D.T, D.t0, D.L, D.fstar, D.reach, C.pc[e]);
         slot = atomicAdd(&hist[k], 1);
     }
     __syncthreads();
@@ -519,6 +520,7 @@ extern "C" int glass_hip_fstat_create(glass_hip_fstat** out, const glass_hip_orb
     D.t0 = t0;
     D.L = orbit->L;
     D.fstar = orbit->fstar;
+    D.reach = analytic_reach(orbit->L, orbit->fstar, orbit->R, T, t0);
     D.fmt = fmt;
     // the four filters of get_filters: amplitude 2, iota = pi/2 and
     // (psi, phase) = (0, 0), (pi/4, pi), (0, 3 pi/2), (pi/4, pi/2), mapped
@@ -528,7 +530,7 @@ extern "C" int glass_hip_fstat_create(glass_hip_fstat** out, const glass_hip_orb
     {
         const double p[8] = {1.0, 0.0, 0.0, log(2.0), cos(M_PI_2), psi[i], ph[i], 0.0};
         UcbConst c;
-        ucb_setup(p, 8, T, t0, orbit->L, orbit->fstar, c);
+        ucb_setup(p, 8, T, t0, orbit->L, orbit->fstar, D.reach, c);
         D.f[i] = {c.DPr, c.DPi, c.DCr, c.DCi, ph[i], cos(ph[i]), sin(ph[i])};
     }
     F->cap = max_cells;

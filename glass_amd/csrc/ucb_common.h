@@ -29,6 +29,50 @@ constexpr double kLARM = 2.5e9;
 constexpr double kSQRT1_2 = 0.70710678118654752440;
 constexpr double kINVSQ6 = 0.408248290463863;  // glass_lisa.c:436
 
+// What the spacecraft positions that a template reads reach.  L and f* come
+// from the caller, independent of the positions, so the bounds of the
+// transfer functions' arguments are taken from the positions themselves.
+struct OrbitReach
+{
+    double arg;   // largest argument over |f|: (1 + longest arm / L) / (2 f*), at least 1.25 / f*
+    double time;  // largest |time| at which a frequency is taken: |t0| + T and the light travel time
+                  // of the farthest spacecraft, at least 1000 s
+};
+
+// From the longest arm and the largest distance from the barycentre (metres);
+// a NaN stays one, and sinc_wide then takes the general path.
+inline OrbitReach orbit_reach(double L, double fstar, double T, double t0, double arm, double far)
+{
+    const double a = 0.5 * (1.0 + arm / fabs(L)), t = far * kInvCLIGHT;
+    return {(a <= 1.25 ? 1.25 : a) / fabs(fstar), fabs(t0) + T + (t <= 1000.0 ? 1000.0 : t)};
+}
+
+// The analytic orbit: spacecraft 2 |R| from a centre at 1 AU, arms of 2
+// sqrt(3) |R| (constant in its first order in the eccentricity).
+inline OrbitReach analytic_reach(double L, double fstar, double R, double T, double t0)
+{
+    return orbit_reach(L, fstar, T, t0, 1.001 * 2.0 * kSQ3 * fabs(R), kAU + 2.002 * fabs(R));
+}
+
+// Longest arm and largest distance in a table of n records x1 x2 x3 y1 y2 y3 z1
+// z2 z3 (NaN if one is).
+inline void positions_extent(const double* pos, int n, double* arm, double* far)
+{
+    double a = 0.0, r = 0.0;
+    for (const double* p = pos; p < pos + 9 * (size_t)n; p += 9)
+        for (int i = 0; i < 3; i++)
+        {
+            const int j = (i + 1) % 3;
+            const double dx = p[i] - p[j], dy = p[3 + i] - p[3 + j], dz = p[6 + i] - p[6 + j];
+            const double d = sqrt(dx * dx + dy * dy + dz * dz);
+            const double s = sqrt(p[i] * p[i] + p[3 + i] * p[3 + i] + p[6 + i] * p[6 + i]);
+            if (d > a || d != d) a = d;
+            if (s > r || s != s) r = s;
+        }
+    *arm = a;
+    *far = r;
+}
+
 // Per-template constants (glass_ucb_waveform.c:804-837).
 struct UcbConst
 {
@@ -56,7 +100,7 @@ struct UcbConst
 
 // glass_ucb_waveform.c:804-837 + LISA_polarization_tensor (glass_lisa.c:1566-1596)
 __host__ __device__ inline void ucb_setup(const double* p, int np, double T, double t0,
-                                          double L, double fstar, UcbConst& c)
+                                          double L, double fstar, OrbitReach reach, UcbConst& c)
 {
     // k feeds the phase through k.x: no contraction anywhere in the setup
 #pragma clang fp contract(off)
@@ -99,9 +143,7 @@ __host__ __device__ inline void ucb_setup(const double* p, int np, double T, dou
     c.ua[0] = u0 * c.invL;  c.ua[1] = u1 * c.invL;  c.ua[2] = u2 * c.invL;
     c.va[0] = v0 * c.invL;  c.va[1] = v1 * c.invL;
     for (int i = 0; i < 3; i++) c.ka[i] = c.k[i] * c.invL;
-    // times reach t0 + T and a light travel time of 1 AU beyond
-    const double tm = fabs(t0) + T + 1000.0;
-    c.wide = sinc_wide((fabs(c.f0) + (fabs(c.dfdt) + fabs(c.halfd2) * tm) * tm) * c.invfstar);
+    c.wide = sinc_wide(fabs(c.f0) + (fabs(c.dfdt) + fabs(c.halfd2) * reach.time) * reach.time, reach.arg);
     c.f0h = 0.5 * c.f0 * c.invfstar;
     c.dfh = 0.5 * c.dfdt * c.invfstar;
     c.d2h = 0.5 * c.halfd2 * c.invfstar;
