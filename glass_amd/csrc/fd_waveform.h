@@ -15,9 +15,11 @@
 // registers.  Each pass hands one bin per thread to the caller (m = P t + r),
 // so one bin's five values are live at a time.  NT = 512 is the length that
 // one wave transforms in three radix-8 passes (wave_fft).  At 2048 bins two
-// groups of threads share the P samples (FdShape).
+// groups of threads share the P samples (FdShape); at 4096 the template is cut
+// by its samples instead of its bins (fd_bins_by_sample).
 #pragma once
 #include "fft_lds.h"
+#include "runtime.h"
 #include "ucb_common.h"
 
 namespace glass {
@@ -50,12 +52,19 @@ struct FdShape
     static constexpr int NTHR = fd_threads(N, G);
     static constexpr int PN = wave_fft_stride(NT);
     static constexpr int LDS = G * kNLink * PN;       // double2 elements
+    // the template is cut by its samples
+    static constexpr bool BYSAMPLE = G == 2 && Q >= 4;
     // the thread's place in its group, and its bin in pass s: P t + the
-    // residue, of which the group g of two takes j = g Q/2 .. and j + Q
+    // residue, of which the group g of two takes j = g Q/2 .. and j + Q; cut
+    // by samples, t + NT (j + P/2) modulo N
     static __device__ __forceinline__ int lane() { return G == 1 ? threadIdx.x : threadIdx.x & 511; }
     static __device__ __forceinline__ int group() { return G == 1 ? 0 : threadIdx.x >> 9; }
-    static __device__ __forceinline__ int residue(int s) { return G == 1 ? s : group() * (Q / 2) + s / 2 + Q * (s % 2); }
-    static __device__ __forceinline__ int bin(int s) { return P * lane() + residue(s); }
+    __host__ __device__ static constexpr int residue(int g, int s) { return G == 1 ? s : g * (Q / 2) + s / 2 + Q * (s % 2); }
+    __host__ __device__ static constexpr int bin(int t, int g, int s)
+    {
+        return BYSAMPLE ? t + NT * ((residue(g, s) + P / 2) & (P - 1)) : P * t + residue(g, s);
+    }
+    static __device__ __forceinline__ int bin(int s) { return bin(lane(), group(), s); }
     // LDS place of thread t's point of a series.  A series of 16 or 32 points
     // has fewer than its workgroup's 64 threads: the others get a place of it
     // too, so that a read without a test stays within the series.
@@ -166,8 +175,9 @@ __device__ __forceinline__ void fd_dif(double2 (&x)[fd_series(N)][L], const doub
 // x_{g + 2q}, q < Q.  Each thread transforms its own (A_j from the even samples,
 // B_j from the odd, j < Q), hands half of the results to its partner through
 // LDS and combines the other half: X_j = A_j + w_P^j B_j, X_{j+Q} = A_j - w_P^j B_j,
-// left in the slots of FdShape.  lds: the groups' series rows.
-template <int N>
+// left in the slots of FdShape.  lds: the groups' series rows.  TURN: and times
+// w_N^{j t}, the points of the series to transform.
+template <int N, bool TURN = true>
 __device__ __forceinline__ void fd_dif2(double2 (&x)[fd_series(N) / 2][kNLink], double2* lds,
                                         const double2* __restrict__ tw, int tws)
 {
@@ -198,31 +208,86 @@ __device__ __forceinline__ void fd_dif2(double2 (&x)[fd_series(N) / 2][kNLink], 
         __syncthreads();
         const int j = g * H + i;
         const double2 wp = tw[j * S::NT * tws];  // w_P^j
-        const double2 w1 = tw[(j * t) * tws], w2 = tw[((j + Q) * t) * tws];
+        double2 w1, w2;
+        if constexpr (TURN) w1 = tw[(j * t) * tws], w2 = tw[((j + Q) * t) * tws];
 #pragma unroll
         for (int l = 0; l < kNLink; l++)
         {
             const double2 o = other[l * S::PN + t], h = pick(g, x[H + i][l], x[i][l]);
             const double2 a = pick(g, o, h), b = cmul(pick(g, h, o), wp);
-            x[i][l] = cmul(make_double2(a.x + b.x, a.y + b.y), w1);
-            x[H + i][l] = cmul(make_double2(a.x - b.x, a.y - b.y), w2);
+            x[i][l] = make_double2(a.x + b.x, a.y + b.y);
+            x[H + i][l] = make_double2(a.x - b.x, a.y - b.y);
+            if constexpr (TURN) x[i][l] = cmul(x[i][l], w1), x[H + i][l] = cmul(x[H + i][l], w2);
         }
     }
     __syncthreads();
 }
 
-// f(s, m, d) for every output bin m = FdShape::bin(s) of this thread: d[l] =
-// series l at bin m, FFT_l[(m + N/2) mod N] (glass_ucb_waveform.c:940-962);
-// the reference's 1/(2N) is part of fd_tdi's prefactor.  SOA: pos is the
-// N-sample structure-of-arrays block (9 rows of N samples); else the record
-// table read with stride posstride.  tws = entries of tw per N-th root.
-// pre(m) is called before the transform of bin m's pass, so that global
-// loads the caller issues there are in flight during it.  No barrier after
-// the last LDS reads: the caller passes one of its own before anything
-// writes lds again.
-template <int N, bool SOA, int GROUPS = fd_groups(N), typename K, typename Pre, typename F>
-__device__ __forceinline__ void fd_link_bins(const K& kget, double2* lds, const double* __restrict__ pos,
-                                             int posstride, const double2* __restrict__ tw, int tws, Pre&& pre, F&& f)
+// fd_link_bins (below) cut by the samples: series p is the samples n = P j + p,
+// whose transform Y_p enters bin j + NT r (FFT index) as w_N^{p j} w_P^{p r}
+// Y_p[j].  Each pass evaluates, transforms and turns one series a group, and the
+// groups' P sums come last (fd_dif2's exchange), so a thread's bins are 512
+// apart and the lanes of a wave read and write consecutive bins.  Cut by bins, a
+// thread's bins are P apart: each pass reads every line of the window, the stored
+// template and the weights for 16 of its 128 bytes, eight times 0.8 MB an item,
+// past the L2.  4080 evaluations of 4096 bins 2.67 -> 1.42 ms (1.65 with radix-4
+// transforms and bins 512 apart), 20,000 9.6 -> 5.9 ms; 300 in one launch 302 ->
+// 164 us.
+template <int N, bool SOA, typename K, typename Pre, typename F>
+__device__ __forceinline__ void fd_bins_by_sample(const K& kget, double2* lds, const double* __restrict__ pos,
+                                                  int posstride, const double2* __restrict__ tw, int tws, Pre&& pre,
+                                                  F&& f)
+{
+    using S = FdShape<N>;
+    constexpr int P = S::P, Q = S::Q, NT = S::NT, PN = S::PN;
+    constexpr int KS = SOA ? N : 1;
+    static_assert(S::BYSAMPLE && pos_soa_place(N, P * 5 + 3) == 3 * NT + 5, "positions in the samples' order");
+    const int t = S::lane();
+    // this thread's place of a series: it alone writes and, transformed, reads it
+    double2* own = lds + S::group() * kNLink * PN + S::place(t);
+    double2 x[Q][kNLink];
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+        for (int l = 0; l < kNLink; l++) x[q][l] = make_double2(0.0, 0.0);
+#pragma unroll 1
+    for (int q = 0; q < Q; q++)
+    {
+        const int p = S::group() + S::G * q, n = P * t + p;
+        const UcbConst& c = kget();
+        ucb_slow_sample_to<KS>(c, ucb_sample_time(c.T, c.t0, n, N),
+                               SOA ? pos + pos_soa_place(N, n) : pos + (size_t)n * posstride * 9,
+                               [&](int l, double2 v) { own[l * PN] = v; });
+        __syncthreads();
+        wave_fft<NT, S::G * kNLink, S::NTHR, true>(lds, opaque(tw), P * tws);
+        const double2 w = tw[(p * t) * tws];
+#pragma unroll
+        for (int l = 0; l < kNLink; l++)
+        {
+#pragma unroll
+            for (int i = 0; i + 1 < Q; i++) x[i][l] = x[i + 1][l];
+            x[Q - 1][l] = cmul(own[l * PN], w);
+        }
+    }
+    __syncthreads();
+    fd_dif2<N, false>(x, lds, tw, tws);
+#pragma unroll
+    for (int s = 0; s < Q; s++)
+    {
+        int u = t;  // fresh indices per bin
+        asm volatile("" : "+v"(u));
+        const int m = S::bin(u, S::group(), s);
+        pre(m);
+        f(s, m, x[S::slot(s)]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// ... and cut by the bins.
+template <int N, bool SOA, int GROUPS, typename K, typename Pre, typename F>
+__device__ __forceinline__ void fd_bins_by_bin(const K& kget, double2* lds, const double* __restrict__ pos,
+                                               int posstride, const double2* __restrict__ tw, int tws, Pre&& pre,
+                                               F&& f)
 {
     using S = FdShape<N, GROUPS>;
     constexpr int P = S::P, Q = S::Q, NT = S::NT, PN = S::PN;
@@ -272,7 +337,7 @@ __device__ __forceinline__ void fd_link_bins(const K& kget, double2* lds, const 
         if constexpr (P > 1) asm volatile("" : "+v"(u));
         // bin m = P t + r is FFT index (m + N/2) mod N = P k + r
         const int k = wave_fft_slot((u + NT / 2) & (NT - 1));
-        const int m = P * u + S::residue(s);
+        const int m = S::bin(u, S::group(), s);
         if (on) pre(m);
         wave_fft<NT, S::G * kNLink, S::NTHR, (P > 1)>(lds, opaque(tw), P * tws);
         double2 d[kNLink];
@@ -289,6 +354,26 @@ __device__ __forceinline__ void fd_link_bins(const K& kget, double2* lds, const 
         if (on) f(s, m, d);
         if (s + 1 < Q) __syncthreads();
     }
+}
+
+// f(s, m, d) for every output bin m = FdShape::bin(s) of this thread: d[l] =
+// series l at bin m, FFT_l[(m + N/2) mod N] (glass_ucb_waveform.c:940-962);
+// the reference's 1/(2N) is part of fd_tdi's prefactor.  SOA: pos is the
+// N-sample structure-of-arrays block (9 rows of N samples, pos_soa_place); else
+// the record table read with stride posstride.  tws = entries of tw per N-th root.
+// pre(m) is called before the transform of bin m's pass, so that global
+// loads the caller issues there are in flight during it.  No barrier after
+// the last LDS reads: the caller passes one of its own before anything
+// writes lds again.
+template <int N, bool SOA, int GROUPS = fd_groups(N), typename K, typename Pre, typename F>
+__device__ __forceinline__ void fd_link_bins(const K& kget, double2* lds, const double* __restrict__ pos,
+                                             int posstride, const double2* __restrict__ tw, int tws, Pre&& pre, F&& f)
+{
+    using S = FdShape<N, GROUPS>;
+    if constexpr (S::BYSAMPLE)
+        fd_bins_by_sample<N, SOA>(kget, lds, pos, posstride, tw, tws, pre, f);
+    else
+        fd_bins_by_bin<N, SOA, GROUPS>(kget, lds, pos, posstride, tw, tws, pre, f);
 }
 
 // exp(-i x) of x = f/f* at template bin m (f = (q + m - N/2)/T,

@@ -78,9 +78,12 @@ int positions(const glass_hip_orbit& o, double T, double t0, int npos, const dou
 // Spacecraft positions per series length N = kPosSoaMin..kPosSoaMax (powers
 // of two) in structure-of-arrays form: the block of N is 9 rows of N
 // samples (x1,x2,x3,y1,...,z3 at t0 + T n / N) at pos_soa_offset(N), so the
-// threads of a wave read consecutive samples of one coordinate.
+// threads of a wave read consecutive samples of one coordinate.  Sample n is at
+// pos_soa_place(N, n) of its rows: the 4096-bin kernels' lanes take every
+// eighth sample.
 constexpr int kPosSoaMin = 32, kPosSoaMax = 4096;
 __host__ __device__ constexpr int pos_soa_offset(int N) { return 9 * (N - kPosSoaMin); }
+__host__ __device__ constexpr int pos_soa_place(int N, int n) { return N < 4096 ? n : (n & 7) * (N / 8) + (n >> 3); }
 int positions_soa(const glass_hip_orbit& o, double T, double t0, const double** out);
 
 // Host restatement of analytic_orbits (utils/src/glass_lisa.c:77-124), used

@@ -209,7 +209,7 @@ int positions_soa(const glass_hip_orbit& o, double T, double t0, const double** 
     {
         double* blk = h.data() + pos_soa_offset(N);
         for (int n = 0; n < N; n++)
-            for (int k = 0; k < 9; k++) blk[(size_t)k * N + n] = fine[(size_t)n * (kPosSoaMax / N) * 9 + k];
+            for (int k = 0; k < 9; k++) blk[(size_t)k * N + pos_soa_place(N, n)] = fine[(size_t)n * (kPosSoaMax / N) * 9 + k];
     }
     double* d = nullptr;
     GH_CHECK(hipMalloc(&d, sizeof(double) * h.size()));

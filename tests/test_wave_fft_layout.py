@@ -33,6 +33,12 @@ template <int N> void shape()
     using S = FdShape<N>;
     printf("[%d, %d, %d, %d, %d, %d, [", N, S::NT, S::NTHR, S::PN, S::LDS, S::G);
     for (int t = 0; t < 2 * S::NTHR; t++) printf("%s%d", t ? "," : "", S::place(t));
+    printf("], [");
+    for (int s = 0; s < S::Q; s++)
+        for (int t = 0; t < S::G * (N < 512 ? N : 512); t++)
+            printf("%s%d", s || t ? "," : "", S::bin(t % 512, t / 512, s));
+    printf("], [");
+    for (int n = 0; n < N; n++) printf("%s%d", n ? "," : "", pos_soa_place(N, n));
     printf("]]");
 }
 int main()
@@ -73,7 +79,21 @@ def test_places_of_a_template(lay):
     test of its index: the adjoint's threads past a series of 32 points did
     read past the buffer."""
     assert [s[0] for s in lay["shapes"]] == [16 << k for k in range(9)]
-    for N, NT, NTHR, PN, LDS, G, place in lay["shapes"]:
+    for N, NT, NTHR, PN, LDS, G, place, _, _ in lay["shapes"]:
         assert max(place) < PN and LDS == 5 * G * PN, N
         per = [p for t, p in enumerate(place) if t < NT]
         assert len(set(per)) == NT and place[:NT] == lay["slot"][:NT], N
+
+
+def test_bins_of_a_template(lay):
+    """Each bin has one thread and pass, each sample one place in the positions'
+    rows.  At 4096 bins a wave's lanes take consecutive bins: eight apart, each
+    of eight passes read every line of the window (2.67 against 1.42 ms)."""
+    for N, NT, NTHR, PN, LDS, G, _, bins, pos in lay["shapes"]:
+        assert sorted(bins) == list(range(N)) and sorted(pos) == list(range(N)), N
+        if N == 4096:
+            b = np.array(bins).reshape(-1, 64)
+            assert np.all(np.diff(b, axis=1) == 1)
+            # thread t of a group takes sample 8 t + p in pass p
+            p = np.array(pos).reshape(512, 8)
+            assert np.all(np.diff(p, axis=0) == 1)
