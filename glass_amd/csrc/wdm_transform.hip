@@ -253,7 +253,7 @@ __device__ __forceinline__ void store_pixel(double* __restrict__ wdm, int NF, in
     }
 }
 
-// One layer m of wavelet_transform_freq a workgroup (NT of 1024 and more).
+// One layer m of wavelet_transform_freq a workgroup (layers_by_wave says when not).
 template <int NT, bool FROM_Z, int NTH = fft_threads(NT, 1)>
 __global__ void __launch_bounds__(NTH) layer_fwd_kernel(const double2* __restrict__ src, double* __restrict__ wdm,
                                                         int NF, const double* __restrict__ win, TwSel t)
@@ -268,12 +268,13 @@ __global__ void __launch_bounds__(NTH) layer_fwd_kernel(const double2* __restric
     for (int n = threadIdx.x; n < NT; n += NTH) store_pixel<NT>(wdm, NF, m, n, buf[n]);
 }
 
-// Layers of up to 512 time pixels: a wave takes 512 / NT of them from the
-// spectrum to the pixels by itself, eight points a lane, with no barriers.  One
-// wave a workgroup, for 17 on a CU by their LDS (four to a workgroup make 16, and
-// the 4097 waves of 4096 layers of 512 then take a second turn: 21.8 us against
-// 19.8; a workgroup of 128 threads a layer took 21.8).  Forming the spectrum's bins
-// once, in a row pass that pairs rows k and M1 - k, moves 4 us from here to there.
+// Layers of up to 512 time pixels, many of them: a wave takes 512 / NT of them
+// from the spectrum to the pixels by itself, eight points a lane, with no
+// barriers.  One wave a workgroup, for 17 on a CU by their LDS (four to a
+// workgroup make 16, and the 4097 waves of 4096 layers of 512 then take a second
+// turn: 21.8 us against 19.8; a workgroup of 128 threads a layer took 21.8).
+// Forming the spectrum's bins once, in a row pass that pairs rows k and M1 - k,
+// moves 4 us from here to there.
 constexpr int kLayerWaves = 1;
 template <int NT, bool FROM_Z>
 __global__ void __launch_bounds__(64 * kLayerWaves) layer_wave_kernel(const double2* __restrict__ src,
@@ -309,6 +310,18 @@ __global__ void __launch_bounds__(64 * kLayerWaves) layer_wave_kernel(const doub
         const int q = lane + 64 * p, m = m0 + q / NT;
         if (m <= NF) store_pixel<NT>(wdm, NF, m, q % NT, own[(q / NT) * PN + wave_fft_slot(q % NT)]);
     }
+}
+
+// Where waves take layers by themselves: a lane's eight points cost latency, so
+// the layers of few samples are spread over more threads (a workgroup a layer).
+// Whole transforms, a workgroup a layer / waves, us: of 2^14 samples 12.4-13.8 /
+// 13.7-15.6, of 2^17 12.4-15.4 / 15.4-16.7, of 2^19 26.8, 23.6, 22.2, 21.7, 22.6 /
+// 22.9, 22.9, 22.6, 22.9, 23.2 for 32 to 512 time pixels, of 2^20 38.7, 35.3,
+// 33.6, 34.6 / 33.3, 33.6, 33.7, 33.9 for 64 to 512, of 2^21 44.2, 41.2, 43.2 / 40.3,
+// 41.0, 41.9 for 128 to 512.
+constexpr bool layers_by_wave(int NF, int NT)
+{
+    return NT <= 512 && (long long)NF * NT >= (NT <= 64 ? 1 << 19 : 1 << 20);
 }
 
 // wavelet_transform_inverse_freq, first half: per layer the prefactors and
@@ -484,12 +497,19 @@ static int layers_fwd(const Plan& p, const double2* src, bool fromZ, const doubl
     const double2 *tw, *tw3;
     int rc;
     if ((rc = twiddles(&tw)) || (rc = twiddles3(&tw3))) return rc;
-    switch (p.NT)
-    {
-        GH_LAYER_WAVE(32) GH_LAYER_WAVE(64) GH_LAYER_WAVE(128) GH_LAYER_WAVE(256) GH_LAYER_WAVE(512)
-        GH_LAYER(1024) GH_LAYER(2048) GH_LAYER(4096)
-        default: return set_error("WDM transform: NT %d", p.NT), GLASS_HIP_EINVAL;
-    }
+    if (layers_by_wave(p.NF, p.NT))
+        switch (p.NT)
+        {
+            GH_LAYER_WAVE(32) GH_LAYER_WAVE(64) GH_LAYER_WAVE(128) GH_LAYER_WAVE(256) GH_LAYER_WAVE(512)
+            default: return set_error("WDM transform: NT %d", p.NT), GLASS_HIP_EINVAL;
+        }
+    else
+        switch (p.NT)
+        {
+            GH_LAYER(32) GH_LAYER(64) GH_LAYER(128) GH_LAYER(256) GH_LAYER(512) GH_LAYER(1024) GH_LAYER(2048)
+            GH_LAYER(4096)
+            default: return set_error("WDM transform: NT %d", p.NT), GLASS_HIP_EINVAL;
+        }
     GH_CHECK(hipGetLastError());
     return GLASS_HIP_OK;
 }

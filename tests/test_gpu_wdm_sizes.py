@@ -1,7 +1,8 @@
 """WDM transforms at the sizes that choose their kernels: columns and rows of 512
 to 4096 points (cut to series that a wave transforms), layers of 32 to 512 time
-pixels (several to a wave) and above.  Normwise 1e-12 against the oracle; the
-largest by the round trip."""
+pixels on both sides of the line above which waves take them (2^19 samples for
+up to 64 time pixels, 2^20 for more), and above.  Normwise 1e-12 against the
+oracle; the largest against the layers of its own spectrum."""
 import numpy as np
 import pytest
 
@@ -35,3 +36,10 @@ def test_largest_against_the_spectrum(gl, orc):
     b = W.wavelet_transform_freq(gw, np.fft.rfft(x).view(np.float64))
     scale = float(np.dot(a.ravel(), b.ravel()) / np.dot(b.ravel(), b.ravel()))
     assert normwise(a, b * scale) < 1e-12
+
+
+# the last below the line, 3 2^17 or 3 2^18 samples, and the first above it
+@pytest.mark.parametrize("NF,NT", [(12288, 32), (16384, 32), (6144, 64), (6144, 128), (8192, 128), (3072, 256),
+                                   (1536, 512), (2048, 512)])
+def test_layers_on_both_sides_of_the_line(orc, gl, NF, NT):
+    test_forward_sizes(orc, gl, NF, NT)
