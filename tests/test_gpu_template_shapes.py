@@ -47,16 +47,20 @@ def test_nine_parameters(gl, orc, fddot):
         assert normwise(h9, h8) > 1e-6
 
 
+@pytest.mark.parametrize("narrow", [False, True])
 @pytest.mark.parametrize("mode", [0, 1])
 @pytest.mark.parametrize("BW", [32, 64, 128, 256, 512, 1024])
-def test_adjoint_and_forward_mode(gl, BW, mode):
+def test_adjoint_and_forward_mode(gl, BW, mode, narrow):
     import torch
     from glass_amd.derivs import source_derivs, source_grad
-    T, n, W = synth.T_2YR, 5, BW + BW // 2 + 1
+    # narrow: a window of fewer bins than the template, which mode 1's weights
+    # by template bin leave too
+    T, n, W = synth.T_2YR, 5, BW // 2 + 3 if narrow else BW + BW // 2 + 1
     rng = np.random.default_rng(BW)
     P = np.stack([params(100 + i, f, T) for i, f in enumerate((2e-3, 9e-3, 21e-3, 45e-3, 80e-3))])
     # the last template leaves the window at both of its ends in turn
-    imin = torch.tensor([W // 4, 3, 0, -BW // 4, W - BW // 2], dtype=torch.int32, device="cuda")
+    imin = [-BW // 4, 2 - BW // 2, 0, 1, -3] if narrow else [W // 4, 3, 0, -BW // 4, W - BW // 2]
+    imin = torch.tensor(imin, dtype=torch.int32, device="cuda")
     A = rng.standard_normal((n, W, 3, 3))
     C = np.einsum("nwij,nwkj->nwik", A, A) + 3 * np.eye(3)
     ic = np.linalg.inv(C)
@@ -71,10 +75,10 @@ def test_adjoint_and_forward_mode(gl, BW, mode):
     L0, none = source_grad(o, T, p, BW, imin, invC, R, mode=mode, want_grad=False)
     assert none is None and torch.equal(F, F.transpose(1, 2))
     scale = g.abs().amax(1, keepdim=True)
-    if mode == 0:
-        # one likelihood, three kernels: sums in other orders of ~BW terms
-        assert torch.allclose(La, L, rtol=1e-11, atol=0) and torch.allclose(L0, L, rtol=1e-11, atol=0)
-        assert float(((ga - g).abs() / scale).max()) <= 1e-10
+    # one likelihood, three kernels, the same bins and weights in both modes:
+    # sums in other orders of ~BW terms
+    assert torch.allclose(La, L, rtol=1e-11, atol=0) and torch.allclose(L0, L, rtol=1e-11, atol=0)
+    assert float(((ga - g).abs() / scale).max()) <= 1e-10
     # central differences of L, step h: truncation h^2, rounding 1e-10/h
     for k, h in ((3, 1e-4), (5, 1e-4), (6, 1e-4), (0, 3e-5), (2, 1e-5)):
         up, dn = p.clone(), p.clone()
