@@ -37,13 +37,13 @@ def load(path):
 
 def tune(plan, n, cache=None, reps=3, fmt="sangria", retune=False):
     """Tiles for plan over its first n proposals: from the cache when the
-    key is there (applied with set_tiles), else measured (and stored).
+    key is there (applied as tuned tiles), else measured (and stored).
     Returns (tiles, ms per class or None when cached, from_cache)."""
     key = cache_key(plan, n, fmt)
     db = load(cache)
     if not retune and key in db:
         tiles = [tuple(t) for t in db[key]["tiles"]]
-        plan.set_tiles(tiles)
+        plan.set_tiles(tiles, tuned=True)
         return tiles, None, True
     tiles, ms = plan.autotune(n, reps=reps)
     if cache:

@@ -30,6 +30,8 @@ _EXTRA += [
     ("glass_hip_fd_batch_tile_candidates", [_i, _tp, _i, _ip], _i),
     ("glass_hip_fd_batch_get_tiles", [_vp, _tp], _i),
     ("glass_hip_fd_batch_set_tiles", [_vp, _tp], _i),
+    ("glass_hip_fd_batch_set_tuned_tiles", [_vp, _tp], _i),
+    ("glass_hip_fd_batch_one_launch", [_vp, _i], _i),
     ("glass_hip_fd_batch_autotune", [_vp, _i, _vp, _vp, _vp, _i, _tp, _dp, _vp], _i),
     ("glass_hip_fd_batch_derivs", [_vp, _i, _vp, _vp, _vp, _vp, _vp, _vp], _i),
     ("glass_hip_fd_batch_create_ex", [ctypes.POINTER(_vp), _vp, ctypes.c_char_p, _d, _d, _i, _ip, _ip, _dp, _dp,
@@ -213,9 +215,16 @@ class FdBatch:
         check(_L().glass_hip_fd_batch_get_tiles(self.h, t), "fd_batch_get_tiles")
         return [(x.nthr, x.gmul, x.waves) for x in t]
 
-    def set_tiles(self, tiles):
+    def set_tiles(self, tiles, tuned=False):
+        """tuned: tiles of an earlier autotune, for the class kernels of many
+        proposals; up to 1024 keep their one launch."""
         t = (Tile * NCLASS)(*[Tile(int(a), int(b), int(c)) for a, b, c in tiles])
-        check(_L().glass_hip_fd_batch_set_tiles(self.h, t), "fd_batch_set_tiles")
+        fn = _L().glass_hip_fd_batch_set_tuned_tiles if tuned else _L().glass_hip_fd_batch_set_tiles
+        check(fn(self.h, t), "fd_batch_set_tiles")
+
+    def one_launch(self, n):
+        """Whether n proposals are evaluated in one launch for all classes."""
+        return bool(_L().glass_hip_fd_batch_one_launch(self.h, int(n)))
 
     def autotune(self, n, reps=3):
         """Times every compiled tile of each BW class over the first n

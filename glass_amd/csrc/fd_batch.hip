@@ -713,6 +713,7 @@ struct glass_hip_fd_batch
     int ncu = 0;
     int tgrid[kNClass] = {0};
     glass_hip_tile tile[kNClass] = {};  // launch shape of each class's eval kernel
+    bool own_tiles = false;             // the caller chose them (not the default, nor an autotuner's)
     // graph cache
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -818,12 +819,13 @@ static bool tile_retired(int k, int nthr, int waves)
 // workgroup per slot, of 327,680: 74 of 32 bins 0.013 / 0.081 ms, 20,188 of
 // 64 bins 0.050 / 0.111, 23,671 of 2048 bins 2.85 / 3.13, 379 of 4096 bins
 // 0.24 / 0.46; but 130,042 of 512 bins 2.59 / 2.35.
+constexpr int kStrideGmul = 4;  // their grid multiplier for gmul 0
 constexpr bool eval_strides(int k) { return k < 2 || k > 5; }
 
 static int tile_grid(const glass_hip_fd_batch* P, int k, glass_hip_tile t, int n)
 {
     if (t.gmul <= 0 && !eval_strides(k)) return n;
-    const long long g = (long long)(t.gmul > 0 ? t.gmul : 4) * P->ncu * resident_per_cu(32 << k, t.nthr, t.waves);
+    const long long g = (long long)(t.gmul > 0 ? t.gmul : kStrideGmul) * P->ncu * resident_per_cu(32 << k, t.nthr, t.waves);
     return (int)(g < n ? g : n);
 }
 
@@ -868,16 +870,12 @@ static void launch_align(glass_hip_fd_batch* P, int n, const Items& it, double* 
 // eight launches of the classes, eager and replayed as a graph: 12 in 20, 37 /
 // 89, 81 us; 252 in 43, 47 / 94, 83; 1020 in 97, 104 / 139, 123; but 2040 in
 // 214, 222 / 206, 189, where the waves that end leave the CUs half empty.  The
-// class kernels run for a caller's own tiles and in the profiling mode, which
-// times them.
+// class kernels run for a caller's own tiles, and evaluate in the profiling mode,
+// which times them; tiles that an autotuner chose are for the class kernels of
+// more items and leave the line where it is.
 constexpr int kFewItems = 1024;
-static bool few_items(const glass_hip_fd_batch* P, int n)
-{
-    if (n > kFewItems || P->prof) return false;
-    for (int k = 0; k < kNClass; k++)
-        if (!default_tile(k, P->tile[k])) return false;
-    return true;
-}
+static bool few_items(const glass_hip_fd_batch* P, int n) { return n <= kFewItems && !P->own_tiles; }
+static bool few_evals(const glass_hip_fd_batch* P, int n) { return few_items(P, n) && !P->prof; }
 
 // alignment + per-class launches for items; mode 0: eval, 1: templates
 static int launch_items(glass_hip_fd_batch* P, int n, const Items& it, int mode, double* logl_out, double* snr_out,
@@ -890,7 +888,7 @@ static int launch_items(glass_hip_fd_batch* P, int n, const Items& it, int mode,
         return GLASS_HIP_EINVAL;
     }
     launch_align(P, n, it, mode == 0 ? logl_out : nullptr, mode == 0 ? snr_out : nullptr, s);
-    if (mode == 0 && few_items(P, n))
+    if (mode == 0 && few_evals(P, n))
     {
         EvalArgs A = eval_args(P, 32, it, logl_out, snr_out);
         A.pos = P->B.pos_soa;
@@ -1578,7 +1576,7 @@ extern "C" int glass_hip_fd_batch_get_tiles(glass_hip_fd_batch* P, glass_hip_til
     return GLASS_HIP_OK;
 }
 
-extern "C" int glass_hip_fd_batch_set_tiles(glass_hip_fd_batch* P, const glass_hip_tile* tiles)
+static int set_tiles(glass_hip_fd_batch* P, const glass_hip_tile* tiles, bool tuned)
 {
     if (!P || !tiles)
     {
@@ -1586,6 +1584,7 @@ extern "C" int glass_hip_fd_batch_set_tiles(glass_hip_fd_batch* P, const glass_h
         return GLASS_HIP_EINVAL;
     }
     glass_hip_tile use[kNClass];
+    bool own = false;
     for (int k = 0; k < kNClass; k++)
     {
         use[k] = tiles[k];
@@ -1600,8 +1599,28 @@ extern "C" int glass_hip_fd_batch_set_tiles(glass_hip_fd_batch* P, const glass_h
     }
     GH_CHECK(hipSetDevice(P->device));
     if (int rc = drop_graph(P)) return rc;
-    for (int k = 0; k < kNClass; k++) P->tile[k] = use[k];
+    for (int k = 0; k < kNClass; k++)
+    {
+        P->tile[k] = use[k];
+        own = own || !default_tile(k, use[k]);
+    }
+    P->own_tiles = own && !tuned;
     return GLASS_HIP_OK;
+}
+
+extern "C" int glass_hip_fd_batch_set_tiles(glass_hip_fd_batch* P, const glass_hip_tile* tiles)
+{
+    return set_tiles(P, tiles, false);
+}
+
+extern "C" int glass_hip_fd_batch_set_tuned_tiles(glass_hip_fd_batch* P, const glass_hip_tile* tiles)
+{
+    return set_tiles(P, tiles, true);
+}
+
+extern "C" int glass_hip_fd_batch_one_launch(const glass_hip_fd_batch* P, int n)
+{
+    return P && n > 0 && few_evals(P, n);
 }
 
 extern "C" int glass_hip_fd_batch_autotune(glass_hip_fd_batch* P, int nprop, const int* d_chain, const int* d_src,
@@ -1628,6 +1647,7 @@ extern "C" int glass_hip_fd_batch_autotune(glass_hip_fd_batch* P, int nprop, con
         return GLASS_HIP_EINVAL;
     }
     if (int rc = drop_graph(P)) return rc;
+    P->own_tiles = false;
     hipEvent_t e0, e1;
     GH_CHECK(hipEventCreate(&e0));
     GH_CHECK(hipEventCreate(&e1));
@@ -1645,6 +1665,8 @@ extern "C" int glass_hip_fd_batch_autotune(glass_hip_fd_batch* P, int nprop, con
             bms = 1e300;
             for (int c = 0; c < nc && c < 64 && !rc; c++)
             {
+                // the same launch as gmul 0
+                if (eval_strides(k) && cand[c].gmul == kStrideGmul) continue;
                 // one untimed launch, then reps timed ones; results go to
                 // the plan's own logL/snr buffers
                 if ((rc = launch_eval(P, k, cand[c], nprop, list, cntp, it, P->p_logl, P->p_snr, s))) break;

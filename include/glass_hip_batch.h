@@ -157,8 +157,17 @@ int glass_hip_fd_batch_tile_candidates(int k, glass_hip_tile *out, int max, int 
 int glass_hip_fd_batch_get_tiles(glass_hip_fd_batch *plan, glass_hip_tile *tiles);
 
 /* Sets all eight tiles (each a compiled candidate of its class, e.g. from
- * an earlier autotune); drops the captured graph. */
+ * an earlier autotune); drops the captured graph.  With tiles other than
+ * the defaults every evaluation and accept runs its class kernels. */
 int glass_hip_fd_batch_set_tiles(glass_hip_fd_batch *plan, const glass_hip_tile *tiles);
+
+/* The same for tiles that an earlier autotune chose: they are for the class
+ * kernels of many proposals, and up to 1024 keep their one launch. */
+int glass_hip_fd_batch_set_tuned_tiles(glass_hip_fd_batch *plan, const glass_hip_tile *tiles);
+
+/* 1 if the plan evaluates nprop proposals in one launch for all classes (up
+ * to 1024, unless the caller set tiles of its own or profiles), else 0. */
+int glass_hip_fd_batch_one_launch(const glass_hip_fd_batch *plan, int nprop);
 
 /* Autotuner: buckets the nprop proposals (device arrays, as for an eval)
  * into BW classes, times every compiled tile of each non-empty class over

@@ -75,3 +75,46 @@ def test_line_between_them(gl, orc, concurrent):
         for i in range(2):
             assert _rel(a[i], b[i][:1020]) < 1e-12 and bool((a[i] == c[i]).all())
     plan.close()
+
+
+def test_tuned_tiles_leave_a_few_proposals_in_one_launch(gl, orc, tmp_path):
+    """An autotuner's tiles are for the class kernels of many proposals; with a
+    caller's own every evaluation and accept runs those."""
+    from glass_amd import autotune
+    from glass_amd.batch import NCLASS, tile_candidates
+    cfg = make_cfg(orc, seed=31, ngroup=5, ntemp=2, nprop=103, windows=(512, 1024, 2048), f_lo=0.5e-3, f_hi=9e-3)
+    plan = new_plan(gl, cfg, 1030)
+    plan.set_proposals(cfg["p_chain"], cfg["p_src"], cfg["p_params"])
+    assert plan.one_launch(1) and plan.one_launch(1024) and not plan.one_launch(1025)
+    ref = [x.clone() for x in plan.eval(500)]
+    other = [tile_candidates(k)[1] for k in range(NCLASS)]
+    assert other != plan.tiles()
+    plan.set_tiles(other)
+    assert not plan.one_launch(1) and plan.tiles() == other
+    plan.set_tiles(other, tuned=True)
+    assert plan.one_launch(1024) and plan.tiles() == other
+    for got in (plan.eval(500), plan.eval(500, graph=True)):
+        assert all(bool((a == b).all()) for a, b in zip(got, ref))
+    cache = str(tmp_path / "tiles.json")
+    for _ in range(2):  # measured, then from the cache
+        plan.set_tiles(other)
+        tiles, _, cached = autotune.tune(plan, 1030, cache=cache, reps=1)
+        assert plan.tiles() == tiles and plan.one_launch(1024) and not plan.one_launch(1025)
+    assert cached
+    plan.profile(True)
+    assert not plan.one_launch(1)
+    plan.profile(False)
+    plan.close()
+
+
+@pytest.mark.parametrize("k", [0, 1, 6, 7])
+def test_autotuner_times_a_launch_once(gl, orc, k):
+    """Where the default grid strides, gmul 0 and 4 are the same launch: the
+    tuner keeps gmul 0 for it."""
+    cfg = make_cfg(orc, seed=37, ngroup=6, ntemp=2, nprop=4, windows=(64, 4096, 6000), f_lo=0.5e-3, f_hi=20e-3)
+    plan = new_plan(gl, cfg, len(cfg["p_chain"]))
+    plan.set_proposals(cfg["p_chain"], cfg["p_src"], cfg["p_params"])
+    for _ in range(4):
+        tiles, _ = plan.autotune(len(cfg["p_chain"]), reps=1)
+        assert tiles[k][1] != 4
+    plan.close()
