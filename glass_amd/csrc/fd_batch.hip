@@ -396,9 +396,8 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(MINW, 8)))
 // first: (class k, template bins N, workgroup threads, waves per SIMD).
 #ifndef GH_EVAL_TILES
 #define GH_EVAL_TILES(X)                                                                                      \
-    X(0, 32, 64, 1) X(1, 64, 64, 1) X(1, 64, 64, 6) X(2, 128, 128, 1) X(2, 128, 128, 6) X(3, 256, 256, 1)    \
-    X(3, 256, 256, 6) X(3, 256, 256, 8) X(4, 512, 512, 6) X(4, 512, 512, 1) X(4, 512, 512, 8)                \
-    X(5, 1024, 512, 4) X(5, 1024, 512, 5) X(6, 2048, 1024, 1) X(7, 4096, 1024, 1)
+    X(0, 32, 64, 1) X(1, 64, 64, 1) X(1, 64, 64, 6) X(2, 128, 128, 1) X(3, 256, 256, 1) X(4, 512, 512, 6)    \
+    X(4, 512, 512, 1) X(5, 1024, 512, 4) X(5, 1024, 512, 5) X(6, 2048, 1024, 1) X(7, 4096, 1024, 1)
 #endif
 
 // Template of each listed item into its source's slot.  LOOP: the grid
@@ -800,12 +799,14 @@ static bool tile_compiled(int k, int nthr, int waves)
 }
 
 // Shapes of class k that earlier builds compiled (other thread counts of the
-// same kernels): a caller's saved choice of one runs as the default shape
-// with its grid multiplier.
+// same kernels, and waves that the compiler did not grant or that the default
+// has: 128 bins with 6, 256 with 6 and 8, 512 with 8): a caller's saved choice of
+// one runs as the default shape with its grid multiplier.
 static bool tile_retired(int k, int nthr, int waves)
 {
-    static constexpr int shape[][3] = {{2, 64, 1},  {3, 128, 1},  {3, 128, 4}, {3, 256, 5}, {4, 256, 1},
-                                       {5, 512, 1}, {5, 1024, 1}, {5, 256, 1}, {6, 512, 1}, {7, 512, 1}};
+    static constexpr int shape[][3] = {{2, 64, 1},  {2, 128, 6},  {3, 128, 1}, {3, 128, 4}, {3, 256, 5},
+                                       {3, 256, 6}, {3, 256, 8},  {4, 256, 1}, {4, 512, 8}, {5, 512, 1},
+                                       {5, 1024, 1}, {5, 256, 1}, {6, 512, 1}, {7, 512, 1}};
     for (const auto& x : shape)
         if (x[0] == k && x[1] == nthr && x[2] == waves) return true;
     return false;
@@ -814,11 +815,15 @@ static bool tile_retired(int k, int nthr, int waves)
 // Classes whose default grid strides.  The grid cannot know how many of the n
 // proposals are in a class; a slot that is not costs the launch of an empty
 // workgroup, 0.2 ns of 64 threads and 0.7 ns of 1024 (0.07 and 0.22 ms of
-// 327,680), while striding costs the 128- to 1024-bin kernels 6 to 10% an
-// item (the loop holds 30 more vector registers).  Striding against one
-// workgroup per slot, of 327,680: 74 of 32 bins 0.013 / 0.081 ms, 20,188 of
-// 64 bins 0.050 / 0.111, 23,671 of 2048 bins 2.85 / 3.13, 379 of 4096 bins
-// 0.24 / 0.46; but 130,042 of 512 bins 2.59 / 2.35.
+// 327,680), while the striding loop holds more vector registers.  A workgroup a
+// slot against striding, of 327,680 mixed proposals: 74 of 32 bins 0.080 / 0.012
+// ms, 20,188 of 64 bins 0.108 / 0.049, 23,671 of 2048 bins 3.1 / 2.8, 379 of 4096
+// bins 0.46 / 0.17; and where all proposals are of one length: 20,000 of 64 bins 96
+// / 99 us, of 2048 2.51 / 2.53 ms, of 4096 5.65 / 5.72.  In between one workgroup a
+// slot: of 60,000 of one length 128 bins 266 / 303 us, 256 bins 0.51 / 0.62 ms, 512
+// bins 1.04 / 1.19, 1024 bins 2.36 / 2.96; of the mixed proposals 37,679 of 128 bins
+// 0.19 / 0.17, 74,247 of 256 bins 0.59 / 0.66, 130,042 of 512 bins 2.33 / 2.53,
+// 41,400 of 1024 bins 1.80 / 1.75.
 constexpr int kStrideGmul = 4;  // their grid multiplier for gmul 0
 constexpr bool eval_strides(int k) { return k < 2 || k > 5; }
 

@@ -98,6 +98,11 @@ def test_retired_tiles_run_as_the_default(gl, orc):
     base = plan.tiles()
     l0, s0 = (x.clone() for x in plan.eval(E))
     old = list(base)
+    for k, nthr, waves in ((2, 128, 6), (3, 256, 6), (3, 256, 8), (4, 512, 8)):  # copies of the default
+        old[k] = (nthr, 1, waves)
+        plan.set_tiles(old)
+        assert plan.tiles()[k] == (base[k][0], 1, base[k][2])
+    old = list(base)
     old[3], old[4], old[5], old[6] = (128, 2, 4), (256, 0, 1), (1024, 1, 1), (512, 4, 1)
     plan.set_tiles(old)
     now = plan.tiles()
