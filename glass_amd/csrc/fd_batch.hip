@@ -870,14 +870,17 @@ static void launch_align(glass_hip_fd_batch* P, int n, const Items& it, double* 
                                                                        P->cls_list, P->cls_cap, logl_out, snr_out);
 }
 
-// Items that one launch of all classes takes: four per CU.  Evaluating
-// proposals of 2- and 4-year windows (512 to 4096 bins) in one launch against
-// eight launches of the classes, eager and replayed as a graph: 12 in 20, 37 /
-// 89, 81 us; 252 in 43, 47 / 94, 83; 1020 in 97, 104 / 139, 123; but 2040 in
-// 214, 222 / 206, 189, where the waves that end leave the CUs half empty.  The
-// class kernels run for a caller's own tiles, and evaluate in the profiling mode,
-// which times them; tiles that an autotuner chose are for the class kernels of
-// more items and leave the line where it is.
+// Items that one launch of all classes takes: four per CU.  Evaluating in one
+// launch against eight launches of the classes, eager and replayed as a graph, us:
+// 2-year windows of 512 to 4096 bins, 12 proposals 21, 38 / 105, 91; 252 in 40, 44 /
+// 114, 100; 1020 in 71, 78 / 119, 127; 2040 in 117, 124 / 145, 127; 1-year windows of
+// 96 to 256 bins, 12 in 21, 33 / 72, 62; 1020 in 26, 34 / 78, 67; 2040 in 35, 42 / 77,
+// 66.  Templates of 2048 and 4096 bins alone take the same time either way from
+// about 1000 on (0.19 and 0.36 us each), where the launches no longer count and the
+// class kernels need fewer registers: the line is there.  The class kernels run for
+// a caller's own tiles, and evaluate in the profiling mode, which times them; tiles
+// that an autotuner chose are for the class kernels of more items and leave the line
+// where it is.
 constexpr int kFewItems = 1024;
 static bool few_items(const glass_hip_fd_batch* P, int n) { return n <= kFewItems && !P->own_tiles; }
 static bool few_evals(const glass_hip_fd_batch* P, int n) { return few_items(P, n) && !P->prof; }

@@ -26,13 +26,13 @@ constexpr int kMaxPart = 1024;
 
 // Generic weighted sum of products: term t of bin n is
 // a_t[n] . b_t[n] * w_t[n] * coef_t  with complex a,b (Re a conj b).
-// Used for fourier_nwip (1 term) and snr (6 terms).
+// Used for fourier_nwip (1 term) and the likelihood of 1 or 2 channels.
 struct NwipTerms
 {
-    const double2* a[6];
-    const double2* b[6];
-    const double* w[6];
-    double coef[6];
+    const double2* a[2];
+    const double2* b[2];
+    const double* w[2];
+    double coef[2];
     int nterm;
 };
 
@@ -60,6 +60,32 @@ __global__ __launch_bounds__(kRedThr) void sum_partials(const double* part, int 
     for (int i = threadIdx.x; i < n; i += kRedThr) s += part[i];
     s = block_sum<kRedThr>(s);
     if (threadIdx.x == 0) out[0] = scale * s;
+}
+
+// sum_n XX w0 + YY w1 + ZZ w2 + 2 (XY w3 + XZ w4 + YZ w5), every plane read once:
+// the planes may lie in pinned host memory, where the six terms one after the
+// other, each waiting for its own reads, made snr of 64 bins slower than copying
+// them first.
+struct SnrPlanes
+{
+    const double2* h[3];
+    const double* w[6];
+};
+__global__ __launch_bounds__(kRedThr) void snr3_kernel(SnrPlanes P, int N, int chunk, double scale, double* part)
+{
+    const int b0 = blockIdx.x * chunk, b1 = min(N, b0 + chunk);
+    double acc = 0.0;
+    for (int n = b0 + threadIdx.x; n < b1; n += kRedThr)
+    {
+        const double2 x = P.h[0][n], y = P.h[1][n], z = P.h[2][n];
+        const double diag = (x.x * x.x + x.y * x.y) * P.w[0][n] + (y.x * y.x + y.y * y.y) * P.w[1][n] +
+                            (z.x * z.x + z.y * z.y) * P.w[2][n];
+        const double off = (x.x * y.x + x.y * y.y) * P.w[3][n] + (x.x * z.x + x.y * z.y) * P.w[4][n] +
+                           (y.x * z.x + y.y * z.y) * P.w[5][n];
+        acc += diag + 2.0 * off;
+    }
+    acc = block_sum<kRedThr>(acc);
+    if (threadIdx.x == 0) part[blockIdx.x] = scale * acc;
 }
 
 // chi^2 of the 3-channel residual r = d - m over NFFT bins:
@@ -181,8 +207,9 @@ int nwip_terms_dev(const NwipTerms& T, int N, double scale, double* d_out, Threa
 // buffer or, for a few, to the pinned buffer itself, and the result's place in
 // the pinned buffer.  The likelihood, which reads each bin once, gains at every
 // size measured (256 bins, 42 KB, 43 -> 35 us; 2048 bins, 336 KB, 54 -> 46; 8192
-// bins, 1.3 MB, 90 -> 80); snr reads its planes two or three times (256 bins, 24
-// KB, 35 -> 28 us, but 1024 bins, 96 KB, 44 -> 52).
+// bins, 1.3 MB, 90 -> 80), and snr (64 bins, 6 KB, 22 -> 21;
+// 1024 bins, 96 KB, 31 -> 26); the likelihood of one or two channels reads its
+// planes twice (two channels of 1024 bins 46 -> 48).
 constexpr size_t kInPlaceBytes = 256 * 1024, kInPlaceReread = 32 * 1024;
 static int stage(ThreadCtx* cx, int n, const void* const* src, const size_t* bytes, void** dst, double** d_res,
                  size_t limit = kInPlaceBytes)
@@ -266,18 +293,14 @@ extern "C" double glass_hip_snr(const double* X, const double* Y, const double* 
     for (int i = 3; i < 9; i++) by[i] = sizeof(double) * N;
     void* d[9];
     double* dres;
-    if (stage(cx, 9, src, by, d, &dres, kInPlaceReread)) return NAN;
-    NwipTerms T{};
-    T.nterm = 6;
-    const int ia[6] = {0, 1, 2, 0, 0, 1}, ib[6] = {0, 1, 2, 1, 2, 2};
-    for (int t = 0; t < 6; t++)
-    {
-        T.a[t] = (const double2*)d[ia[t]];
-        T.b[t] = (const double2*)d[ib[t]];
-        T.w[t] = (const double*)d[3 + t];
-        T.coef[t] = t < 3 ? 1.0 : 2.0;
-    }
-    if (nwip_terms_dev(T, N, 2.0, dres, cx)) return NAN;
+    if (stage(cx, 9, src, by, d, &dres)) return NAN;
+    SnrPlanes P;
+    for (int i = 0; i < 3; i++) P.h[i] = (const double2*)d[i];
+    for (int i = 0; i < 6; i++) P.w[i] = (const double*)d[3 + i];
+    Reduction r;
+    if (r.init(cx, N, 2.0, dres)) return NAN;
+    snr3_kernel<<<r.nb, kRedThr, 0, cx->stream>>>(P, N, r.chunk, r.block_scale, r.part);
+    if (r.finish(cx)) return NAN;
     return sqrt(fetch_result(cx, dres));
 }
 
