@@ -205,12 +205,17 @@ int nwip_terms_dev(const NwipTerms& T, int N, double scale, double* d_out, Threa
 
 // Stages host arrays; returns the pointers for kernels, to the thread's device
 // buffer or, for a few, to the pinned buffer itself, and the result's place in
-// the pinned buffer.  The likelihood, which reads each bin once, gains at every
-// size measured (256 bins, 42 KB, 43 -> 35 us; 2048 bins, 336 KB, 54 -> 46; 8192
-// bins, 1.3 MB, 90 -> 80), and snr (64 bins, 6 KB, 22 -> 21;
-// 1024 bins, 96 KB, 31 -> 26); the likelihood of one or two channels reads its
-// planes twice (two channels of 1024 bins 46 -> 48).
-constexpr size_t kInPlaceBytes = 256 * 1024, kInPlaceReread = 32 * 1024;
+// the pinned buffer.  Kernels that read each plane once gain at every size
+// measured, us after the copy / in place: the likelihood of 256 bins (42 KB) 39 /
+// 34, of 2048 (336 KB) 52 / 46, of 32,768 (5.4 MB) 233 / 215; snr of 64 bins 22 / 21,
+// of 1024 (96 KB) 31 / 26, of 32,768 (3.1 MB) 129 / 128; fourier_nwip of 64 bins 21 /
+// 19, of 4096 (160 KB) 33 / 27, of 32,768 (1.3 MB) 72 / 68; wavelet_nwip, which
+// gathers by its list, of 1024 of 1024 pixels 30 / 29, of 512 of 512 23 / 24, of 2048 of
+// 32,768 59 / 48; the likelihood of one channel of 64 bins 35 / 34, of 1024 43 / 40,
+// of 32,768 (1.3 MB) 123 / 111.  That of two channels, which subtracts in place and
+// reads again one channel after the other, gains less and then loses: 256 bins (25
+// KB) 42 / 39, 1024 (96 KB) 46 / 48, 16,384 88 / 97.
+constexpr size_t kInPlaceBytes = 6 * 1024 * 1024, kInPlaceReread = 32 * 1024;
 static int stage(ThreadCtx* cx, int n, const void* const* src, const size_t* bytes, void** dst, double** d_res,
                  size_t limit = kInPlaceBytes)
 {
@@ -383,7 +388,7 @@ extern "C" double glass_hip_gaussian_log_likelihood(const double* dX, const doub
     const void* src[6] = {dd[0], mm[0], invC, dd[nc - 1], mm[nc - 1], invC + 4 * (size_t)NFFT};
     size_t by[6] = {cb, cb, pb, cb, cb, pb};
     void* d[6];
-    if (stage(cx, 6, src, by, d, &dres, kInPlaceReread)) return NAN;
+    if (stage(cx, 6, src, by, d, &dres, nc == 1 ? kInPlaceBytes : kInPlaceReread)) return NAN;
     // residual in place on the device copies of the data arrays
     // r = d - m via a 2-term expansion: (d-m).(d-m) = d.d - 2 d.m + m.m
     // would lose precision; use a dedicated pass instead.
