@@ -596,6 +596,7 @@ __global__ __launch_bounds__(256) void accept_add_old_kernel(int nacc, Items it,
     const int a = blockIdx.x;
     if (a >= nacc || (it.dn && a >= *it.dn)) return;
     const int c = item_chain(it, a), s = item_src(it, a), so = c * B.maxsrc + s;
+    if (s < 0) return;  // left out, as accept_few_kernel and the template kernels do
     const int g = B.c_group[c], W = B.g_W[g], cap = B.g_cap[g];
     accept_add_old(B.resid + (size_t)B.c_roff[c] * 3, W, src_tmpl(B, c, s), cap, B.s_imin[so], B.s_bw[so]);
 }
@@ -608,6 +609,7 @@ __global__ __launch_bounds__(256) void accept_sub_new_kernel(int nacc, Items it,
     const int a = blockIdx.x;
     if (a >= nacc || (it.dn && a >= *it.dn)) return;
     const int c = item_chain(it, a), s = item_src(it, a);
+    if (s < 0) return;
     const int g = B.c_group[c], W = B.g_W[g], cap = B.g_cap[g];
     const int in = imin_new[a], bn = bw_new[a];
     double2* R = B.resid + (size_t)B.c_roff[c] * 3;

@@ -118,3 +118,32 @@ def test_autotuner_times_a_launch_once(gl, orc, k):
         tiles, _ = plan.autotune(len(cfg["p_chain"]), reps=1)
         assert tiles[k][1] != 4
     plan.close()
+
+
+def test_accepting_a_left_out_item_changes_nothing(gl, orc):
+    """An accepted item without a source (negative index) is left out: in one
+    launch, and in the launches per length of more than 1024."""
+    cfg = make_cfg(orc, seed=41, ngroup=103, ntemp=10, nprop=1, windows=(64, 100, 256), f_lo=0.5e-3, f_hi=2e-3)
+    n = len(cfg["p_chain"])
+    assert n == 1030 and len(set(cfg["p_chain"])) == n
+    src = cfg["p_src"].copy()
+    src[[0, 511, 1029]] = -1
+    out = []
+    for parts in ([n], [515, n - 515]):
+        plan = new_plan(gl, cfg, n)
+        plan.set_proposals(cfg["p_chain"], src, cfg["p_params"])
+        before = plan.state()
+        plan.eval(n)
+        a = 0
+        for m in parts:
+            plan.accept(np.arange(a, a + m))
+            a += m
+        after = plan.state()
+        same = np.all(before[1] == after[1], axis=(1, 2)) & (before[0] == after[0])
+        assert sorted(np.flatnonzero(same)) == sorted(cfg["p_chain"][[0, 511, 1029]])
+        plan.refresh()
+        fresh = plan.state()
+        assert np.max(np.abs(fresh[0] / after[0] - 1)) < 1e-9
+        out.append(after)
+        plan.close()
+    assert np.max(np.abs(out[0][0] / out[1][0] - 1)) < 1e-12 and np.array_equal(out[0][1], out[1][1])
