@@ -181,6 +181,12 @@ static int ucb_waveform_dropin(const glass_hip_orbit* ao, const glass_hip_numeri
         set_error("ucb_waveform: bad arguments");
         return GLASS_HIP_EINVAL;
     }
+    // before the staging buffer, which BW sizes
+    if (BW < 16 || BW > 4096 || (BW & (BW - 1)))
+    {
+        set_error("BW=%d unsupported (power of two 16..4096)", BW);
+        return GLASS_HIP_EINVAL;
+    }
     if (no && (no->Norb < 4 || !no->t || !no->x || !no->y || !no->z || !(no->L > 0) || !(no->fstar > 0)))
     {
         set_error("ucb_waveform_numeric: bad orbit (Norb %d, L %g, fstar %g)", no->Norb, no->L, no->fstar);

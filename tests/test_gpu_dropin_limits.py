@@ -53,3 +53,16 @@ def test_wavelet_nwip(gl, nmax, n):
     lst = rng.permutation(nmax)[:n].astype(np.int32)
     ref = np.sum((np.asarray(a, np.longdouble) ** 2 * w)[lst])
     assert abs(gl.wavelet_nwip(a, a, w, lst) - ref) <= TOL * ref
+
+
+@pytest.mark.parametrize("BW", [-4096, -1, 0, 8, 24, 8192])
+def test_waveform_of_an_unsupported_length_is_refused(gl, BW):
+    """... before anything is written to the staging buffer that BW sizes."""
+    import ctypes
+    o = gl.analytic_orbit()
+    p = np.full(8, 0.3)
+    out = np.full((5, 16), 7.0)
+    dp = ctypes.POINTER(ctypes.c_double)
+    rows = [r.ctypes.data_as(dp) for r in out]
+    rc = gl.lib().glass_hip_ucb_waveform(ctypes.byref(o), b"sangria", 3e7, 0.0, p.ctypes.data_as(dp), 8, *rows, BW, 3)
+    assert rc != 0 and f"BW={BW} unsupported" in gl.last_error() and np.all(out == 7.0)
