@@ -97,3 +97,95 @@ def test_bins_of_a_template(lay):
             # thread t of a group takes sample 8 t + p in pass p
             p = np.array(pos).reshape(512, 8)
             assert np.all(np.diff(p, axis=0) == 1)
+
+
+def schedule(N):
+    """Radices of wave_fft_units: eights, then one or two fours."""
+    log2 = N.bit_length() - 1
+    n4 = {0: 0, 2: 1, 1: 2}[log2 % 3]
+    return [8] * ((log2 - 2 * n4) // 3) + [4] * n4
+
+
+def stage(N, NL, R, Ns, unit, slot, PN):
+    """Every butterfly of a unit: (lane, reads, writes) as places of the buffer,
+    its first place and the offsets from it as the kernel forms them."""
+    SPW, NB, PER = 512 // N, N // R, 8 // R
+    out = []
+    for lane in range(64):
+        for p in range(PER):
+            b = lane + 64 * p
+            l, j = unit * SPW + b // NB, b % NB
+            if NL % SPW and l >= NL:
+                continue
+            base = (j // Ns) * Ns * R + j % Ns
+            rd = [l * PN + slot[j] + slot[m * NB] for m in range(R)]
+            wr = [l * PN + slot[base] + slot[m * Ns] for m in range(R)]
+            assert rd == [l * PN + slot[j + m * NB] for m in range(R)]
+            assert wr == [l * PN + slot[base + m * Ns] for m in range(R)]
+            out.append((lane, j, rd, wr))
+    return out
+
+
+# (series, waves, padding, first wave) in use: the five or fifteen series of the
+# templates and their derivatives, two groups' ten, the wavelet kernels' padded
+# ones (whose half-length series start at another wave), the split transforms'
+# eight and a layer pass' one wave
+CASES = [(5, 1, 0, 0), (5, 4, 0, 0), (5, 8, 0, 0), (10, 16, 0, 0), (15, 8, 0, 0), (15, 1, 0, 0), (1, 1, 0, 0), (8, 8, 1, 0),
+         (2, 8, 1, 2), (3, 8, 1, 3), (4, 8, 1, 4), (3, 4, 1, 2), (6, 8, 1, 0), (9, 8, 1, 0), (16, 1, 0, 0)]
+
+
+@pytest.mark.parametrize("N", [16, 32, 64, 128, 256, 512])
+@pytest.mark.parametrize("NL,waves,pad,first", CASES)
+def test_stages_stay_within_a_wave(lay, N, NL, waves, pad, first):
+    slot, PN = lay["slot"], lay["stride"][str(N)] + pad
+    SPW = 512 // N
+    units = (NL + SPW - 1) // SPW
+    # u = wave - first (mod waves), striding by the waves
+    owner = {}
+    for w in range(waves):
+        for u in range(w - first if w >= first else w - first + waves, units, waves):
+            assert u not in owner
+            owner[u] = w
+    assert sorted(owner) == list(range(units))
+    every = sorted(l * PN + slot[n] for l in range(NL) for n in range(N))
+    assert len(set(every)) == NL * N and every[-1] < NL * PN
+    Ns = 1
+    for R in schedule(N):
+        reads, writes, of = [], [], {}
+        for u in range(units):
+            for lane, j, rd, wr in stage(N, NL, R, Ns, u, slot, PN):
+                reads += rd
+                writes += wr
+                for e in rd + wr:
+                    assert of.setdefault(e, owner[u]) == owner[u]
+        assert sorted(reads) == every and sorted(writes) == every
+        Ns *= R
+    assert Ns == N
+
+
+@pytest.mark.parametrize("N", [16, 32, 64, 128, 256, 512])
+def test_stages_give_the_transform(lay, N):
+    slot, PN, NL = lay["slot"], lay["stride"][str(N)], 512 // N + 1
+    rng = np.random.default_rng(N)
+    x = rng.standard_normal((NL, N)) + 1j * rng.standard_normal((NL, N))
+    buf = np.full(NL * PN, np.nan + 0j)
+    for l in range(NL):
+        buf[[l * PN + s for s in slot[:N]]] = x[l]
+    Ns = 1
+    for R in schedule(N):
+        for u in range((NL * N + 511) // 512):
+            done = []
+            for lane, j, rd, wr in stage(N, NL, R, Ns, u, slot, PN):
+                tw = np.exp(-2j * np.pi * (j % Ns) * np.arange(R) / (R * Ns))
+                done.append((wr, np.fft.fft(buf[rd] * tw)))
+            for wr, y in done:
+                buf[wr] = y
+        Ns *= R
+    got = np.array([[buf[l * PN + slot[k]] for k in range(N)] for l in range(NL)])
+    assert np.max(np.abs(got - np.fft.fft(x, axis=1))) < 1e-12 * np.sqrt(N)
+
+
+def test_checker_sees_offsets_that_do_not_add_up(lay):
+    slot = [n + n // 6 for n in range(512)]
+    with pytest.raises(AssertionError):
+        stage(64, 8, 8, 8, 0, slot, 80)
