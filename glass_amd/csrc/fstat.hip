@@ -82,6 +82,13 @@ struct Cells
 // Sums of one cell: N of X and of A, E, then the upper triangles of M.
 constexpr int kFsSum = 28;
 
+// Cells that a new plan has work buffers for (constants, sums, class and lists, 692
+// bytes a cell).  A call with more grows them; where there is no memory for that it
+// evaluates the cells in turns (408,800 cells 2.02 ms at once, 2.12 in four turns).
+// With buffers for its whole capacity a plan of 2^20 cells, the Python default,
+// held 0.8 GB and took 12 ms to create and close; now 0.2 GB and 1 to 3 ms.
+constexpr int kFsTurn = 131072;
+
 // Gauss-Jordan inverse with partial pivoting of a 4x4 matrix (in place)
 __host__ __device__ inline void invert4(double m[4][4])
 {
@@ -460,12 +467,14 @@ struct glass_hip_fstat
 {
     int device = 0;
     FstatDev D{};
-    int cap = 0;
+    int cap = 0, turn = 0;  // cells a call, and at a time
     std::vector<void*> allocs;
     double* cells = nullptr;
     double *lx = nullptr, *lae = nullptr, *fpar = nullptr;
     int *cls = nullptr, *list = nullptr, *kcls = nullptr;
-    char* work = nullptr;  // per cell constants, sums and class (Cells), one allocation
+    // per cell constants, sums and class (Cells) and the class lists of turn
+    // cells, one allocation
+    char* work = nullptr;
     UcbConst* pc = nullptr;
     double* sums = nullptr;
 };
@@ -484,12 +493,34 @@ static int falloc(glass_hip_fstat* F, T** p, size_t n)
     return GLASS_HIP_OK;
 }
 
+// Work buffers for n cells in place of the ones the plan has (which stay if there
+// is no memory for them; hipFree waits for the kernels that use them).
+static bool work_buffers(glass_hip_fstat* F, int n)
+{
+    const size_t c = n;
+    char* w = nullptr;
+    if (hipMalloc(&w, c * (sizeof(UcbConst) + sizeof(double) * kFsSum + sizeof(int) * (1 + kFsClass))) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (F->work) (void)hipFree(F->work);
+    F->work = w;
+    F->turn = n;
+    F->pc = (UcbConst*)w;
+    F->sums = (double*)(F->pc + c);
+    F->kcls = (int*)(F->sums + kFsSum * c);
+    F->list = F->kcls + c;
+    return true;
+}
+
 extern "C" int glass_hip_fstat_destroy(glass_hip_fstat* F)
 {
     if (!F) return GLASS_HIP_OK;
     (void)hipSetDevice(F->device);
     (void)hipDeviceSynchronize();
     for (void* p : F->allocs) (void)hipFree(p);
+    if (F->work) (void)hipFree(F->work);
     delete F;
     return GLASS_HIP_OK;
 }
@@ -541,15 +572,17 @@ extern "C" int glass_hip_fstat_create(glass_hip_fstat** out, const glass_hip_orb
         (rc = falloc(F, &dE, 2 * (size_t)NFFT)) || (rc = falloc(F, &dC, NFFT)) ||
         (rc = falloc(F, &F->cells, 4 * (size_t)max_cells)) || (rc = falloc(F, &F->lx, max_cells)) ||
         (rc = falloc(F, &F->lae, max_cells)) || (rc = falloc(F, &F->fpar, 4 * (size_t)max_cells)) ||
-        (rc = falloc(F, &F->cls, kFsClass + 1)) || (rc = falloc(F, &F->list, (size_t)kFsClass * max_cells)) ||
-        (rc = falloc(F, &F->work, (sizeof(UcbConst) + sizeof(double) * kFsSum + sizeof(int)) * (size_t)max_cells)))
+        (rc = falloc(F, &F->cls, kFsClass + 1)))
     {
         glass_hip_fstat_destroy(F);
         return rc;
     }
-    F->pc = (UcbConst*)F->work;
-    F->sums = (double*)(F->pc + max_cells);
-    F->kcls = (int*)(F->sums + (size_t)kFsSum * max_cells);
+    if (!work_buffers(F, max_cells < kFsTurn ? max_cells : kFsTurn))
+    {
+        set_error("fstat: no memory for the work buffers of %d cells", max_cells < kFsTurn ? max_cells : kFsTurn);
+        glass_hip_fstat_destroy(F);
+        return GLASS_HIP_ERUNTIME;
+    }
     const double* pos = nullptr;
     const double2* tw = nullptr;
     if ((rc = positions(*orbit, T, t0, kPosNF, &pos)) || (rc = twiddles(&tw)))
@@ -581,12 +614,13 @@ __global__ void fs_zero_kernel(int* p, int n)
     if (i < n) p[i] = 0;
 }
 
-static int fstat_launch(glass_hip_fstat* F, int n, const double* cells, double* lx, double* lae, double* fpar,
-                        hipStream_t s)
+// n <= F->turn cells; first: the count of cells without a class starts at zero.
+static int fstat_turn(glass_hip_fstat* F, int n, const double* cells, double* lx, double* lae, double* fpar, bool first,
+                      hipStream_t s)
 {
-    fs_zero_kernel<<<1, 64, 0, s>>>(F->cls, kFsClass + 1);
+    fs_zero_kernel<<<1, 64, 0, s>>>(F->cls, first ? kFsClass + 1 : kFsClass);
     const Cells C{cells, lx, lae, fpar, F->pc, F->sums, F->kcls};
-    fstat_align_kernel<<<(n + 255) / 256, 256, 0, s>>>(n, F->D, C, F->cls, F->list, F->cap, F->cls + kFsClass);
+    fstat_align_kernel<<<(n + 255) / 256, 256, 0, s>>>(n, F->D, C, F->cls, F->list, F->turn, F->cls + kFsClass);
     // the class counts decide the grids: only non-empty classes launch, one
     // workgroup per cell (an empty class's full grid of immediately
     // exiting workgroups costs 80-160 us)
@@ -595,12 +629,23 @@ static int fstat_launch(glass_hip_fstat* F, int n, const double* cells, double* 
     GH_CHECK(hipStreamSynchronize(s));
 #define FS_L(kk, NN)                                                                                        \
     if (cnt[kk] > 0)                                                                                        \
-        fstat_kernel<NN><<<cnt[kk], fd_threads(NN), 0, s>>>(F->list + (size_t)kk * F->cap, F->cls + kk,     \
+        fstat_kernel<NN><<<cnt[kk], fd_threads(NN), 0, s>>>(F->list + (size_t)kk * F->turn, F->cls + kk,    \
                                                             F->D, C);
     FS_L(0, 16) FS_L(1, 32) FS_L(2, 64) FS_L(3, 128) FS_L(4, 256) FS_L(5, 512) FS_L(6, 1024) FS_L(7, 2048)
 #undef FS_L
     fstat_fit_kernel<<<(n + 63) / 64, 64, 0, s>>>(n, C);
     GH_CHECK(hipGetLastError());
+    return GLASS_HIP_OK;
+}
+
+static int fstat_launch(glass_hip_fstat* F, int n, const double* cells, double* lx, double* lae, double* fpar,
+                        hipStream_t s)
+{
+    if (n > F->turn) work_buffers(F, n);
+    for (int o = 0; o < n; o += F->turn)
+        if (int rc = fstat_turn(F, n - o < F->turn ? n - o : F->turn, cells + 4 * (size_t)o, lx + o, lae + o,
+                                fpar + 4 * (size_t)o, o == 0, s))
+            return rc;
     return GLASS_HIP_OK;
 }
 

@@ -68,3 +68,31 @@ def test_mixed_lengths_and_none(gl, orc):
             rx, ra, rp, _ = fd.logl(*cells[c])
             assert abs(lx[c] - rx) < 1e-10 * abs(rx) and abs(la[c] - ra) < 1e-10 * abs(ra)
     F.close()
+
+
+def test_more_cells_than_a_new_plan_has_buffers_for(gl, orc):
+    """A new plan has work buffers for 131,072 cells: more give what their parts
+    give, bit for bit, before and after the buffers have grown."""
+    import torch
+    from glass_amd.fstat import Fstat
+    T, NFFT, n, turn = YEAR, 3000, 131072 * 2 + 77, 131072
+    rng = np.random.default_rng(9)
+    f = 3e-3
+    qmin0 = int(f * T) - NFFT // 2
+    C00 = np.full(NFFT, 1e-40)
+    X, A, E = (1e-20 * (rng.standard_normal(NFFT) + 1j * rng.standard_normal(NFFT)) for _ in range(3))
+    cells = np.stack([f + rng.uniform(-0.2, 0.2, n) * NFFT / T, np.zeros(n), np.arccos(rng.uniform(-1, 1, n)),
+                      rng.uniform(0, 2 * np.pi, n)], axis=1)
+    F = Fstat(gl.analytic_orbit(), "sangria", T, 0.0, qmin0, X, A, E, C00, max_cells=n)
+    c = torch.tensor(cells, device="cuda")
+    before = F.eval(c[:turn])
+    whole = F.eval(c)
+    assert all(torch.equal(w[:turn], p) for w, p in zip(whole, before))
+    for a, b in ((0, 1000), (turn - 500, turn + 500), (turn, 2 * turn), (2 * turn - 3, n)):
+        part = F.eval(c[a:b])
+        assert all(torch.equal(w[a:b], p) for w, p in zip(whole, part))
+    fd = orc.FstatData(T, qmin0, X, A, E, C00, orbit=orc.analytic_orbit())
+    for e in (0, turn - 1, turn, n - 1):
+        rx, ra, *_ = fd.logl(*cells[e])
+        assert abs(float(whole[0][e]) / rx - 1) < 1e-10 and abs(float(whole[1][e]) / ra - 1) < 1e-10
+    F.close()
