@@ -36,7 +36,7 @@ FP64_PEAK_TFLOPS = 78.6
 # HBM bytes per launch of the batched per-class kernels, measured with rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE on this workload and scaled by the same counters on a 256 MiB device copy (fetch x2.00,
 # write x1.00): profiles/eval_kernel_batched_fd_sweep.md.  Keyed by template bins N.
-MEASURED_TRAFFIC = {512: 2.3867e9, 1024: 1.8406e9, 2048: 2.1160e9, 256: 8.4900e8, 4096: 8.4510e8,
+MEASURED_TRAFFIC = {512: 2.3867e9, 1024: 1.8406e9, 2048: 2.1160e9, 256: 8.4900e8, 4096: 3.6360e8,
                     128: 2.4090e8, 64: 8.0450e7, 32: 1.7480e6}
 
 # HBM bytes per launch of logl_chunk_kernel on the inner-product leg (rocprofv3 --pmc FETCH_SIZE and

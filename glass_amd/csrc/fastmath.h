@@ -11,11 +11,19 @@
 //    outside it the result is NaN, so a misuse poisons the likelihood
 //    instead of passing silently.  No platform libm call is inlined, which
 //    keeps the register footprint of the callers small.
+//  * sincos_half: sin and cos up to a common sign (reduction mod pi, minimax
+//    polynomials), the slow series' phase factors; sinc_values, sinc_phase:
+//    the transfer functions sin(x)/x, cos x and their derivative, x less a
+//    multiple of pi where a template's frequency needs it (sinc_wide).
+//  * sincos_cr, atan2_cr, exp_cr: correctly rounded, for the wavelet response;
+//    sincos_tab: the same sine and cosine from a table.
 //  * sinc_ratio(x) = sin(x)/x by its Taylor series in x^2 through x^24
-//    (|x| <= 1.75, truncation < 1e-19); larger |x| use sincos_red.
+//    (|x| <= 1.75, truncation < 1e-19), larger |x| by sincos_red: one argument
+//    of any size by another series, which the tests hold beside glibc.
 //
-// Accuracy is checked against glibc on the CPU (tests/test_fastmath.py):
-// a few ulp, far inside the 1e-12 waveform budget.
+// Accuracy is checked on the CPU against glibc (tests/test_fastmath.py) and 150-bit
+// values (tests/test_fastmath_series.py): a few ulp, far inside the 1e-12 waveform
+// budget.
 #pragma once
 #include <math.h>
 

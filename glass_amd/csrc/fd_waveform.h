@@ -30,7 +30,7 @@ constexpr int kNLink = 5;  // series of a template
 // eight series of one group would take 233 VGPRs and more (one workgroup of
 // eight waves per CU, the vector units 34% busy); each group holds half.
 // 23,671 fused evaluations of 2048 bins 2.93 -> 2.81 ms, 379 of 4096 bins 0.39
-// -> 0.24 ms.
+// -> 0.24 ms (0.17 cut by samples).
 constexpr int fd_groups(int N) { return N >= 2048 ? 2 : 1; }
 
 // Series of a template of N bins (P).

@@ -12,8 +12,9 @@
 // contiguous loads), a twiddle, row FFTs of length M2 over TR adjacent rows
 // with the output written in natural order (TR*16-byte contiguous stores).
 // The layer kernel then forms the needed bins of the real spectrum from Z[k]
-// and Z[M-k] on the fly.  All FFTs run in LDS (fft_lds.h); one workgroup
-// per layer writes its NT pixels contiguously.
+// and Z[M-k] on the fly.  All FFTs run in LDS (fft_lds.h); a workgroup, or where
+// there are many short layers a wave (layers_by_wave), writes a layer's NT pixels
+// contiguously.
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -270,9 +271,11 @@ __global__ void __launch_bounds__(NTH) layer_fwd_kernel(const double2* __restric
 
 // Layers of up to 512 time pixels, many of them: a wave takes 512 / NT of them
 // from the spectrum to the pixels by itself, eight points a lane, with no
-// barriers.  One wave a workgroup, for 17 on a CU by their LDS (four to a
-// workgroup make 16, and the 4097 waves of 4096 layers of 512 then take a second
-// turn: 21.8 us against 19.8; a workgroup of 128 threads a layer took 21.8).
+// barriers.  One wave a workgroup, for 17 on a CU by their LDS, where four to a
+// workgroup make 16: two and four were as fast within 1% at 2^19 to 2^23 samples of
+// 32 to 512 time pixels, but for 4096 layers of 512 (4097 waves, a second turn for
+// the last: 43.2 and 43.4 us the transform, 41.8 with one) and 12,288 of 128 (40.8,
+// 40.1, 39.9).  A workgroup of 128 threads a layer took 2 us more there.
 // Forming the spectrum's bins once, in a row pass that pairs rows k and M1 - k,
 // moves 4 us from here to there.
 constexpr int kLayerWaves = 1;

@@ -3,17 +3,23 @@
 // wavelet_nwip-based inner products, snr_wavelet and the wavelet
 // likelihood, as drop-ins and as a batched device API.
 //
-// Layout of the computation (one template per workgroup, two kernels):
-//  K1 resp_kernel   : on the Norb orbit knots -- barycentre amplitude and
-//                     phase splines, phase at spacecraft 1, the 24 delayed
-//                     one-arm terms of X,Y,Z (LISA_spline_response), their
-//                     amplitude/phase (extract_amplitude_and_phase,
-//                     unwrap_phase) and the six TDI splines.
-//  K2 layer_kernel  : the heterodyned series at NT*(L+1) samples (LDS),
-//                     a packed real FFT (X+iY in one complex FFT, Z as
-//                     half-length), per layer the Meyer-windowed band and
-//                     an inverse FFT of NT, the pixel list, then the fused
-//                     inner products against data and invC.
+// Layout of the computation:
+//  hdr_kernel       : one thread per template, its header (layers, heterodyne).
+//  K1 resp_kernel   : one workgroup per template, on the Norb orbit knots --
+//                     barycentre amplitude and phase splines, phase at
+//                     spacecraft 1, the 24 delayed one-arm terms of X,Y,Z
+//                     (LISA_spline_response), their amplitude/phase
+//                     (extract_amplitude_and_phase, unwrap_phase) and the six
+//                     TDI splines.
+//  K2               : the heterodyned series at NT*(L+1) samples, a packed
+//                     real FFT (X+iY in one complex FFT, Z as half-length),
+//                     per layer the Meyer-windowed band and an inverse FFT of
+//                     NT, the pixel list, then the inner products against data
+//                     and invC.  NT of 256 and 512: layer_kernel, one workgroup
+//                     per template, from LDS.  NT of 1024 to 4096: series_,
+//                     fft_, band_ and sum_kernel_big, several workgroups per
+//                     template, through a global slice.  Forced layer counts:
+//                     layer_kernel_big, ping-pong transforms through L2.
 // Everything that depends only on the orbit and the time grids (knots,
 // spline x-terms, spacecraft geometry at the knots, spacecraft 1 at the
 // downsampled times, interval indices) is tabulated once on the host with
