@@ -493,8 +493,8 @@ static int falloc(glass_hip_fstat* F, T** p, size_t n)
     return GLASS_HIP_OK;
 }
 
-// Work buffers for n cells in place of the ones the plan has (which stay if there
-// is no memory for them; hipFree waits for the kernels that use them).
+// Work buffers for n cells in place of the ones the plan has, which stay if there
+// is no memory for them.
 static bool work_buffers(glass_hip_fstat* F, int n)
 {
     const size_t c = n;
@@ -504,7 +504,11 @@ static bool work_buffers(glass_hip_fstat* F, int n)
         (void)hipGetLastError();
         return false;
     }
-    if (F->work) (void)hipFree(F->work);
+    if (F->work)
+    {
+        (void)hipDeviceSynchronize();  // an earlier call's kernels use them
+        (void)hipFree(F->work);
+    }
     F->work = w;
     F->turn = n;
     F->pc = (UcbConst*)w;
